@@ -538,6 +538,61 @@ int tk_expert_tail_embed(const void* x, int ldx, const void* norm_w, const void*
                          int K, const void* emb_w, const void* emb_b, int emb_n, int emb_act, void* emb_out, int emb_ld,
                          int emb_dtype, void* stream);
 
+/* ---- persistent denoising loop ------------------------------------------------------------- */
+/* The whole flow-matching loop of the SmolVLA-shaped expert (hidden 720, 15 query / 5 K/V heads of 64, feed-forward
+ * 2048, 32 action columns) in one launch whose blocks stay resident: per Euler step the folded suffix embedding, every
+ * expert layer (self-attention over [prefix; action tokens], cross-attention over the prefix's projected K/V), the
+ * final norm, the action projection and x += dt * v (tybok/policies/smolvla/models/flow_matching.py:316-350,406-644,
+ * vlm_with_expert.py:166-408).  Same operands as the launches it replaces (tk_bf16w_linear, tk_expert_attn,
+ * tk_expert_cross_attn_fused, tk_fp8w_norm_gated_ffn, tk_expert_tail); 1 / rms of a norm multiplies the products'
+ * fp32 accumulators instead of the bf16 operands. */
+#define TK_SV_MAX_LAYERS 20
+typedef struct tk_sv_weights {
+  const void* wqkv; /* tk_pack_bf16_weight(rope_half = 32): q | k | v rows (1600), cross layers: q rows only (960) */
+  const void* wo;   /* tk_pack_bf16_weight of [720, 960] */
+  const void* wgu;  /* tk_pack_fp8_gate_up of [2048, 720] x 2 */
+  const void* wd;   /* tk_pack_fp8_weight of [720, 2048] */
+  const float *sg, *su, *sd;
+  const void *norm_in, *norm_post; /* bf16 [720] */
+  int cross;
+} tk_sv_weights;
+/* Bytes of one layer's weights in the launch's own order, and the once-per-model transform of layer `layer` into
+ * `blob` (layers * tk_sv_denoise_layer_bytes() bytes, 16-byte aligned). */
+size_t tk_sv_denoise_layer_bytes(void);
+int tk_sv_denoise_pack(const tk_sv_weights* w, int layer, void* blob, size_t blob_bytes, void* stream);
+/* One layer's cached prefix: keys bf16 [P, 5, 64] (element strides k_sl, k_sh) and values transposed bf16
+ * [5, 64, >= P rounded up to 32] (vt_sh, vt_sd), strides multiples of 8; cross layers: the hi planes, and the lo planes
+ * of the same strides. */
+typedef struct tk_sv_cache {
+  const void *k, *k_lo, *vt, *vt_lo;
+  int k_sl, k_sh, vt_sh, vt_sd;
+} tk_sv_cache;
+typedef struct tk_sv_denoise_args {
+  int layers, steps; /* layers <= TK_SV_MAX_LAYERS */
+  int M, P;          /* action tokens (<= 64), prefix tokens; ceil(P / 32) + ceil(M / 32) <= 16 */
+  unsigned cross_mask; /* bit l: layer l is a cross layer; layer 0 must not be one */
+  float dt, eps;
+  const float* x0; /* fp32 [M, 32]: the noise */
+  float* out;      /* fp32 [M, 32]: x after the last step */
+  const void* pad; /* uint8 [P] (1 = valid) or NULL */
+  const int *pos, *pos0;            /* int32 [M]: rotary positions of the self and of the cross layers (clamped) */
+  const float *rope_cos, *rope_sin; /* fp32 [positions, 32] */
+  int positions;
+  const float *emb_w, *emb_b;   /* folded first linear of the suffix embedding: fp32 [720, 32], [steps, 720]; SiLU follows */
+  const float *time_w, *time_b; /* its second linear: fp32 [720, 720], [720] */
+  const float *act_w, *act_b;   /* action projection: fp32 [32, 720], [32] or NULL */
+  const void* blob;             /* tk_sv_denoise_pack of every layer, then the closing norm's weight, fp32 [720] */
+  void* xchg;                   /* tk_sv_denoise_xchg_bytes(layers) bytes, 16-byte aligned; one launch at a time */
+  size_t xchg_bytes;
+  tk_sv_cache cache[TK_SV_MAX_LAYERS];
+} tk_sv_denoise_args;
+size_t tk_sv_denoise_xchg_bytes(int layers);
+/* `args` is a host structure, read before the call returns.  The launch needs one free compute unit per block (256
+ * blocks: TK_EINVAL on a smaller device) and waits between its blocks, each wait bounded by tk_set_handoff_spin(): if
+ * other work keeps blocks from running that long, the launch ends with NaNs in `out` and the caller falls back to the
+ * separate launches. */
+int tk_sv_denoise(const tk_sv_denoise_args* args, void* stream);
+
 /* ---- diagnostics: helpers of the tests and the benchmark; no policy path calls them -------------- */
 /* out_f32[256] = value of every e4m3fn code as decoded by the device's conversion instruction
  * (the weight path of the GEMM); used to assert the OCP (not FNUZ) flavour on the box. */

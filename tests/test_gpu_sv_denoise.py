@@ -1,0 +1,101 @@
+"""The SmolVLA flow-matching loop as one persistent launch against the launches per layer it replaces, at the edges of
+its row groups and key tiles; what a launch that cannot get its waits answered leaves behind; its argument checks."""
+
+import os
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, os.path.join(HERE, "golden"))
+
+import cases  # noqa: E402
+
+import tybok_amd.ops as tk  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def model():
+    from tybok_amd.policies.smolvla.model import SmolVLAModel
+
+    cfg, sd, _ = cases.smolvla_build(cases.SMOLVLA_CASES["small"])
+    m = SmolVLAModel(cfg, sd, "cuda", fused_expert=True, fp8_expert_mlp=True, fp8_llm_mlp=True, fused_prefill=True)
+    assert m.denoise_plan is not None and m.persistent_loop
+    return m
+
+
+def _case(model, m, p):
+    g = torch.Generator().manual_seed(1000 * m + p)
+    kv = [torch.randn(model.num_layers, 1, p, 5, 64, generator=g).to(torch.bfloat16).cuda() for _ in range(2)]
+    pad = torch.rand(1, p, generator=g).cuda() > 0.2
+    pad[0, 0] = True
+    pos = tuple((int(pad.sum()) * k + torch.arange(m)).to(torch.int32).cuda() for k in (1, 0))
+    return torch.randn(m, 32, generator=g).cuda(), model.attention_caches(*kv, None), pad, pos
+
+
+def _run(model, x, caches, pad, pos):
+    return model.denoise_plan.run(x, model.num_steps, -1.0 / model.num_steps, model.suffix_b_all, caches, pad[0], *pos)
+
+
+# rows: one row group, a full one, one more row, three and a bit, all four; keys: a single one, tile edges, the most tiles
+@pytest.mark.parametrize("m,p", [(1, 1), (16, 32), (17, 33), (50, 241), (33, 255), (50, 448), (64, 448)])
+@torch.inference_mode()
+def test_one_launch_matches_the_launches_per_layer(model, m, p):
+    x, caches, pad, pos = _case(model, m, p)
+    want = x[None]
+    for step in range(model.num_steps):
+        want = model.fused_euler_step(pad, caches, want, step, pos, -1.0 / model.num_steps)
+    got = _run(model, x, caches, pad, pos)
+    assert torch.isfinite(got).all()
+    rel = float((got - want[0]).norm() / (want[0] - x).norm())
+    print(f"M={m} P={p}: relative difference of the flow {rel:.3g}")
+    assert rel < 2e-2  # bf16 rounding: the launches per layer and the plain torch path differ by 5e-3 - 1.2e-2 here
+    assert torch.equal(got, _run(model, x, caches, pad, pos))  # both exchange sets start clean again
+
+
+@torch.inference_mode()
+def test_a_run_whose_waits_give_up_ends_with_nans_and_leaves_nothing_behind(model):
+    # forced from the host: with a bound of zero polls no wave waits; every block still runs to its end
+    case = _case(model, 50, 65)
+    want = _run(model, *case)
+    prev = tk.set_handoff_spin(0)
+    try:
+        lost = _run(model, *case)
+        torch.cuda.synchronize()
+    finally:
+        tk.set_handoff_spin(prev)
+    assert torch.isnan(lost).any()
+    assert torch.equal(_run(model, *case), want)
+
+
+def test_engine_repeats_a_starved_request_layer_by_layer(tmp_path, monkeypatch):
+    from tybok_amd.policies.synthetic import write_smolvla_checkpoint
+    from tybok_amd.registry import create_engine
+
+    flags = dict(tl_fused_expert=True, tl_fp8_expert_mlp=True, tl_fp8_llm_mlp=True, tl_llm_fused_attn=True)
+    ckpt = write_smolvla_checkpoint(str(tmp_path), cameras=1, seed=5, num_vlm_layers=2, vision_layers=1, num_steps=2)
+    engine = create_engine(ckpt, device="cuda", graph=False, warmup=False, **flags)
+    frame, noise = engine._profile_frame(), torch.zeros(1, 50, 6)
+    engine.model.persistent_loop = False
+    want = engine.predict_action_chunk(frame, noise=noise)
+    engine.model.persistent_loop = True
+    monkeypatch.setattr(engine.model.denoise_plan, "run", lambda x0, *a: torch.full_like(x0, float("nan")))
+    assert np.array_equal(engine.predict_action_chunk(frame, noise=noise), want)
+    assert engine.model.persistent_loop is False
+    # a request that is itself NaN says nothing about the launch
+    engine.model.persistent_loop = True
+    assert np.isnan(engine.predict_action_chunk(frame, noise=noise * float("nan"))).any()
+    assert engine.model.persistent_loop is True
+
+
+def test_bad_arguments_are_refused(model):
+    x, caches, pad, pos = _case(model, 50, 65)
+    with pytest.raises(ValueError):
+        _run(model, torch.zeros(65, 32, device="cuda"), caches, pad, pos)
+    with pytest.raises(ValueError):
+        _run(model, x, caches, pad, (pos[0].long(), pos[1]))
+    assert not tk.SvDenoisePlan.covers(50, 449) and tk.SvDenoisePlan.covers(64, 448)

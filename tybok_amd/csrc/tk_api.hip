@@ -1460,6 +1460,77 @@ int tk_add_layer_norm_f16(const void* x, int ldx, const void* r, int ldr, void* 
   return layer_norm_impl("add_layer_norm_f16", x, ldx, TK_F32, r, ldr, xsum, ldxs, w, b, TK_F32, eps, y, ldy, M, K, stream, 1);
 }
 
+size_t tk_sv_denoise_xchg_bytes(int layers) {
+  return layers < 1 || layers > kSvMaxLayers ? 0 : tk_sv_denoise_exchange_bytes(layers);
+}
+size_t tk_sv_denoise_layer_bytes(void) { return tk_sv_denoise_blob_bytes(); }
+
+int tk_sv_denoise_pack(const tk_sv_weights* w, int layer, void* blob, size_t blob_bytes, void* stream) {
+  if (!w || layer < 0 || layer >= kSvMaxLayers) return fail(TK_EINVAL, "sv_pack: layer=%d (0..%d)", layer, kSvMaxLayers - 1);
+  if (!w->wqkv || !w->wo || !w->wgu || !w->wd || !w->sg || !w->su || !w->sd || !w->norm_in || !w->norm_post) return fail(TK_EINVAL, "sv_pack: null pointer");
+  if (!aligned16(w->wqkv) || !aligned16(w->wo) || !aligned16(w->wgu) || !aligned16(w->wd)) return fail(TK_EINVAL, "sv_pack: packed weights must be 16-byte aligned");
+  const size_t lb = tk_sv_denoise_blob_bytes();
+  if (!blob || !aligned16(blob) || blob_bytes < (size_t)(layer + 1) * lb)
+    return fail(TK_EWORKSPACE, "sv_pack: blob of %zu bytes, %zu needed", blob_bytes, (size_t)(layer + 1) * lb);
+  SvPackArgs a = {(const uint8_t*)w->wqkv, (const uint8_t*)w->wo, (const uint8_t*)w->wgu, (const uint8_t*)w->wd, w->sg, w->su, w->sd,
+                  (const unsigned short*)w->norm_in, (const unsigned short*)w->norm_post, w->cross != 0, (uint8_t*)blob + (size_t)layer * lb};
+  if (tk_launch_sv_pack(a, (hipStream_t)stream)) return fail(TK_ELAUNCH, "sv_pack: launch failed");
+  return TK_OK;
+}
+
+int tk_sv_denoise(const tk_sv_denoise_args* h, void* stream) {
+  static_assert(kSvMaxLayers == TK_SV_MAX_LAYERS, "the public and the internal layer limits agree");
+  if (!h) return fail(TK_EINVAL, "sv_denoise: null argument");
+  if (h->layers < 1 || h->layers > kSvMaxLayers || h->steps < 1) return fail(TK_EINVAL, "sv_denoise: layers=%d (1..%d), steps=%d", h->layers, kSvMaxLayers, h->steps);
+  if (h->M < 1 || h->M > 64 || h->P < 1) return fail(TK_EINVAL, "sv_denoise: M=%d (1..64), P=%d", h->M, h->P);
+  if ((h->P + 31) / 32 + (h->M + 31) / 32 > tk_sv_denoise_max_key_tiles())
+    return fail(TK_EINVAL, "sv_denoise: P=%d, M=%d: more than %d key tiles", h->P, h->M, tk_sv_denoise_max_key_tiles());
+  if (h->cross_mask & 1u) return fail(TK_EINVAL, "sv_denoise: layer 0 must be a self layer");
+  if (!h->x0 || !h->out || !h->pos || !h->pos0 || !h->rope_cos || !h->rope_sin || h->positions < 1 || !h->emb_w || !h->emb_b || !h->time_w || !h->time_b || !h->act_w || !h->blob)
+    return fail(TK_EINVAL, "sv_denoise: null pointer");
+  if (!aligned16(h->time_w) || !aligned16(h->act_w) || !aligned16(h->blob) || !aligned8(h->time_b) || !aligned8(h->rope_cos) || !aligned8(h->rope_sin))
+    return fail(TK_EINVAL, "sv_denoise: time_w, act_w, blob must be 16-byte, time_b and the rotary tables 8-byte aligned");
+  if (!h->xchg || !aligned16(h->xchg) || h->xchg_bytes < tk_sv_denoise_exchange_bytes(h->layers))
+    return fail(TK_EWORKSPACE, "sv_denoise: exchange buffer of %zu bytes, %zu needed", h->xchg_bytes, tk_sv_denoise_exchange_bytes(h->layers));
+  if (device_cus() < 256) return fail(TK_EINVAL, "sv_denoise: %d compute units, 256 needed", device_cus());
+  SvDenoiseArgs a = {};
+  for (int l = 0; l < h->layers; ++l) {
+    const tk_sv_cache& s = h->cache[l];
+    const bool cross = (h->cross_mask >> l) & 1u;
+    if (!s.k || !s.vt || (cross && (!s.k_lo || !s.vt_lo))) return fail(TK_EINVAL, "sv_denoise: layer %d: null prefix cache", l);
+    if (!aligned16(s.k) || !aligned16(s.vt) || (cross && (!aligned16(s.k_lo) || !aligned16(s.vt_lo)))) return fail(TK_EINVAL, "sv_denoise: layer %d: misaligned prefix cache", l);
+    if (s.k_sl % 8 || s.k_sh % 8 || s.vt_sh % 8 || s.vt_sd % 8 || s.k_sl < 0 || s.k_sh < 0 || s.vt_sd < (h->P + 31) / 32 * 32 || s.vt_sh < 0)
+      return fail(TK_EINVAL, "sv_denoise: layer %d: bad key / value strides %d %d %d %d", l, s.k_sl, s.k_sh, s.vt_sh, s.vt_sd);
+    a.cache[l] = SvCache{(const unsigned short*)s.k, (const unsigned short*)s.k_lo, (const unsigned short*)s.vt, (const unsigned short*)s.vt_lo, s.k_sl, s.k_sh, s.vt_sh, s.vt_sd};
+  }
+  a.layers = h->layers;
+  a.steps = h->steps;
+  a.M = h->M;
+  a.P = h->P;
+  a.cross_mask = h->cross_mask;
+  a.dt = h->dt;
+  a.eps = h->eps;
+  a.x0 = h->x0;
+  a.out = h->out;
+  a.pad = (const uint8_t*)h->pad;
+  a.pos = h->pos;
+  a.pos0 = h->pos0;
+  a.rope_cos = h->rope_cos;
+  a.rope_sin = h->rope_sin;
+  a.positions = h->positions;
+  a.emb_w = h->emb_w;
+  a.emb_b = h->emb_b;
+  a.time_w = h->time_w;
+  a.time_b = h->time_b;
+  a.act_w = h->act_w;
+  a.act_b = h->act_b;
+  a.blob = (const uint8_t*)h->blob;
+  a.xchg = h->xchg;
+  a.spin = g_handoff_spin.load(std::memory_order_relaxed);
+  if (tk_launch_sv_denoise(a, (hipStream_t)stream)) return fail(TK_ELAUNCH, "sv_denoise: launch failed");
+  return TK_OK;
+}
+
 int tk_debug_stream_read(const void* src, size_t bytes, int blocks, void* sink, void* stream) {
   if (!src || !aligned16(src) || blocks <= 0 || blocks > 65536) return fail(TK_EINVAL, "stream_read: null or unaligned source, or blocks=%d out of range", blocks);
   if (bytes == 0 || bytes % ((size_t)blocks * 4096)) return fail(TK_EINVAL, "stream_read: bytes=%zu must be a positive multiple of blocks * 4096", bytes);

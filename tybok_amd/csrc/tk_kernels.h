@@ -324,3 +324,46 @@ int tk_launch_attn_px(AttnArgs a, int D, hipStream_t st);
 int tk_attn_px_max_tiles();
 int tk_launch_attn_cross_px(AttnArgs a, hipStream_t st);
 int tk_launch_kv_prepare(KvPrepArgs p, hipStream_t st);
+
+// ---- persistent denoising loop (denoise_smolvla.hip) ----
+constexpr int kSvMaxLayers = 20;
+struct SvPackArgs {
+  const uint8_t* wqkv;  // packed bf16: q | k | v (self) or q (cross), rotary pair order
+  const uint8_t* wo;    // packed bf16
+  const uint8_t* wgu;   // packed fp8, gate / up tiles interleaved
+  const uint8_t* wd;    // packed fp8
+  const float *sg, *su, *sd;
+  const unsigned short *norm_in, *norm_post;
+  int cross;
+  uint8_t* blob;  // this layer's part
+};
+struct SvCache {
+  // prefix K [P, G, D] (element strides k_sl, k_sh) and V^T [G, D, P rounded up to 32] (strides vt_sh, vt_sd); cross
+  // layers: hi planes, and the lo planes of the same layout
+  const unsigned short *k, *k_lo, *vt, *vt_lo;
+  int k_sl, k_sh, vt_sh, vt_sd;
+};
+struct SvDenoiseArgs {
+  int layers, steps, M, P;
+  unsigned cross_mask;  // bit l: layer l is a cross layer
+  float dt, eps;
+  const float* x0;  // fp32 [M, 32]
+  float* out;       // fp32 [M, 32]
+  const uint8_t* pad;  // [P] 0 / 1 or nullptr
+  const int *pos, *pos0;  // int32 [M]: rotary positions of the self and of the cross layers
+  const float *rope_cos, *rope_sin;  // fp32 [positions, 32]
+  int positions;
+  const float *emb_w, *emb_b;    // folded suffix embedding: fp32 [720, 32], [steps, 720]
+  const float *time_w, *time_b;  // fp32 [720, 720], [720]
+  const float *act_w, *act_b;    // fp32 [32, 720], [32] or nullptr
+  const uint8_t* blob;  // layers * tk_sv_denoise_blob_bytes(), then the closing norm's weight in fp32
+  void* xchg;           // tk_sv_denoise_exchange_bytes(layers)
+  int spin;             // polls of a waiting wave before it gives up
+  SvCache cache[kSvMaxLayers];
+};
+size_t tk_sv_denoise_exchange_bytes(int layers);
+size_t tk_sv_denoise_blob_bytes();
+int tk_sv_denoise_max_key_tiles();
+int tk_launch_sv_pack(const SvPackArgs& a, hipStream_t st);
+int tk_launch_sv_denoise(const SvDenoiseArgs& a, hipStream_t st);
+int tk_launch_fill_ones(void* p, size_t bytes, hipStream_t st);

@@ -148,10 +148,43 @@ SIGNATURES: dict[str, tuple] = {
          c_int, c_void_p, c_int, c_int, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
          c_int, c_int, c_int, c_void_p, c_size_t, c_void_p],
     ),  # fmt: skip
+    "tk_sv_denoise_xchg_bytes": (c_size_t, [c_int]),
+    "tk_sv_denoise_layer_bytes": (c_size_t, []),
+    "tk_sv_denoise_pack": (c_int, [c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
+    "tk_sv_denoise": (c_int, [c_void_p, c_void_p]),
     "tk_debug_decode_fp8": (c_int, [c_void_p, c_void_p]),
     "tk_debug_stream_read": (c_int, [c_void_p, c_size_t, c_int, c_void_p, c_void_p]),
     "tk_debug_fp8w_gemm_cut": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }
+
+SV_MAX_LAYERS = 20
+
+
+class SvWeights(ctypes.Structure):
+    """``tk_sv_weights``"""
+
+    _fields_ = [*((n, c_void_p) for n in ("wqkv", "wo", "wgu", "wd", "sg", "su", "sd", "norm_in", "norm_post")), ("cross", c_int)]
+
+
+class SvCache(ctypes.Structure):
+    """``tk_sv_cache``"""
+
+    _fields_ = [*((n, c_void_p) for n in ("k", "k_lo", "vt", "vt_lo")), *((n, c_int) for n in ("k_sl", "k_sh", "vt_sh", "vt_sd"))]
+
+
+class SvDenoiseArgs(ctypes.Structure):
+    """``tk_sv_denoise_args``"""
+
+    _fields_ = [
+        *((n, c_int) for n in ("layers", "steps", "M", "P")),
+        ("cross_mask", ctypes.c_uint),
+        *((n, c_float) for n in ("dt", "eps")),
+        *((n, c_void_p) for n in ("x0", "out", "pad", "pos", "pos0", "rope_cos", "rope_sin")),
+        ("positions", c_int),
+        *((n, c_void_p) for n in ("emb_w", "emb_b", "time_w", "time_b", "act_w", "act_b", "blob", "xchg")),
+        ("xchg_bytes", c_size_t),
+        ("cache", SvCache * SV_MAX_LAYERS),
+    ]
 
 
 def library_path() -> str:

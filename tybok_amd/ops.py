@@ -7,11 +7,13 @@ capture's private pool).
 
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
 
 from . import native
+from .graph import launch_turn
 
 ACT = {"silu": 0, "gelu_tanh": 1}
 MASK_NONE, MASK_BIDIR, MASK_CAUSAL = 0, 1, 2
@@ -322,8 +324,6 @@ def w8a8_gated_ffn(
 def w8a8_ffn_intermediates(ws: Workspace, m: int, k: int, i: int) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
     """Views of what the last :func:`w8a8_gated_ffn` of this shape left in ``ws``: the bf16 intermediate ``[m, i]``,
     its e4m3fn codes ``[m, i]`` and their fp32 row scales ``[m]``."""
-    import ctypes
-
     offs = [ctypes.c_size_t() for _ in range(3)]
     native.check(native.lib().tk_w8a8_ffn_layout(m, k, i, *(ctypes.addressof(o) for o in offs)), "tk_w8a8_ffn_layout")
     h_off, h8_off, sh_off = (int(o.value) for o in offs)
@@ -642,8 +642,6 @@ def project_prefix_kv_layers(ks, vs, wks, wvs, d: int) -> list[PrefixKV]:
     """:func:`project_prefix_kv` for several layers (at most 16) in one launch: lists of per-layer ``k, v [P, KV]`` views
     (one shape and row stride) and ``wk, wv [N, KV]`` fp32 weights -> one :class:`PrefixKV` per layer (views of stacked
     planes).  Same bits as one call per layer."""
-    import ctypes
-
     lib = native.lib()
     bf = torch.bfloat16
     n_layers = len(ks)
@@ -954,6 +952,98 @@ def expert_tail(
     )  # fmt: skip
     native.check(rc, "tk_expert_tail")
     return v, x_new
+
+
+def _launch_alone(launch, device) -> None:
+    """Launch a grid whose blocks wait for each other (a recorded one takes its turn when it is replayed)."""
+    if torch.cuda.is_current_stream_capturing():
+        launch()
+    else:
+        with launch_turn(device):
+            launch()
+
+
+class SvDenoisePlan:
+    """The SmolVLA-shaped expert's weights laid out for :meth:`run`, the flow-matching loop as one persistent launch
+    (``tk_sv_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).
+
+    ``layers``: one dict per expert layer -- ``wqkv``, ``wo`` (:class:`PackedBf16Weight`), ``wgu``
+    (:class:`PackedGateUp`), ``wd`` (:class:`PackedWeight`), ``norm_in``, ``norm_post`` (bf16 ``[720]``), ``cross``."""
+
+    HIDDEN, HEADS, KV_HEADS, HEAD_DIM, FFN, ACTION = 720, 15, 5, 64, 2048, 32
+    MAX_TOKENS, MAX_TILES = 64, 16
+
+    def __init__(self, layers, *, time_w, time_b, act_w, act_b, norm_out, emb_w, rope: RopeTables, eps: float, device):
+        e, f = self.HIDDEN, self.FFN
+        nq, nkv = self.HEADS * self.HEAD_DIM, self.KV_HEADS * self.HEAD_DIM
+        if not 1 <= len(layers) <= native.SV_MAX_LAYERS or layers[0]["cross"]:
+            raise ValueError(f"1..{native.SV_MAX_LAYERS} layers, the first one a self layer")
+        for d in layers:
+            n = nq if d["cross"] else nq + 2 * nkv
+            shapes = ((d["wqkv"], n, e), (d["wo"], e, nq), (d["wd"], e, f))
+            if any((w.n, w.k) != (n_, k_) for w, n_, k_ in shapes) or (d["wgu"].i, d["wgu"].k) != (f, e) or d["wqkv"].rope_half != 32 or d["wo"].rope_half:
+                raise ValueError("expert layer of another shape")
+            if any(d[k].dtype != torch.bfloat16 or d[k].numel() != e or not d[k].is_contiguous() for k in ("norm_in", "norm_post")):
+                raise ValueError("norm weights must be contiguous bf16 [720]")
+        fp32 = ((time_w, (e, e)), (time_b, (e,)), (act_w, (self.ACTION, e)), (emb_w, (e, self.ACTION)))
+        if any(t.dtype != torch.float32 or tuple(t.shape) != shape or not t.is_contiguous() for t, shape in fp32) or norm_out.dtype != torch.bfloat16:
+            raise ValueError("time / action / embedding weights must be contiguous fp32 of the expert's shapes")
+        self._keep = (time_w, time_b, act_w, act_b, emb_w, rope)
+        lib = native.lib()
+        nbytes, lbytes = int(lib.tk_sv_denoise_xchg_bytes(len(layers))), int(lib.tk_sv_denoise_layer_bytes())
+        self._xchg = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        # the layers' weights in the launch's own order, the closing norm's behind them
+        self._blob = torch.empty(len(layers) * lbytes + 4 * e, dtype=torch.uint8, device=device)
+        self._blob[len(layers) * lbytes :] = norm_out.float().view(torch.uint8)
+        a = self._args = native.SvDenoiseArgs()
+        a.layers, a.eps = len(layers), float(eps)
+        a.rope_cos, a.rope_sin, a.positions = rope.cos.data_ptr(), rope.sin.data_ptr(), rope.positions
+        a.emb_w, a.time_w, a.time_b = emb_w.data_ptr(), time_w.data_ptr(), time_b.data_ptr()
+        a.act_w, a.act_b = act_w.data_ptr(), _ptr(act_b)
+        a.blob, a.xchg, a.xchg_bytes = self._blob.data_ptr(), self._xchg.data_ptr(), nbytes
+        a.cross_mask = sum(1 << i for i, d in enumerate(layers) if d["cross"])
+        for i, d in enumerate(layers):
+            w = native.SvWeights(
+                *(d[k].data.data_ptr() for k in ("wqkv", "wo", "wgu", "wd")), d["wgu"].scale_gate.data_ptr(), d["wgu"].scale_up.data_ptr(),
+                d["wd"].scale.data_ptr(), d["norm_in"].data_ptr(), d["norm_post"].data_ptr(), int(d["cross"]),
+            )  # fmt: skip
+            native.check(lib.tk_sv_denoise_pack(ctypes.addressof(w), i, self._blob.data_ptr(), self._blob.numel(), _stream()), "tk_sv_denoise_pack")
+
+    @classmethod
+    def covers(cls, tokens: int, prefix: int) -> bool:
+        """Whether a run of that many action tokens over that long a prefix is one launch."""
+        return 1 <= tokens <= cls.MAX_TOKENS and prefix >= 1 and (prefix + 31) // 32 + (tokens + 31) // 32 <= cls.MAX_TILES
+
+    def run(self, x0: torch.Tensor, steps: int, dt: float, emb_b: torch.Tensor, caches, pad: torch.Tensor, pos: torch.Tensor, pos0: torch.Tensor) -> torch.Tensor:
+        """``x0 [M, 32]`` fp32 after ``steps`` Euler steps of size ``dt``; ``emb_b`` fp32 ``[steps, 720]``, ``caches`` a
+        :class:`PrefixKV` per layer (cross layers with lo planes), ``pad`` bool ``[P]``, ``pos`` / ``pos0`` int32 ``[M]``."""
+        a = self._args
+        m, p = x0.shape[0], caches[0].length
+        if x0.dtype != torch.float32 or x0.shape[1] != self.ACTION or not x0.is_contiguous() or not self.covers(m, p) or len(caches) != a.layers:
+            raise ValueError("x0 must be contiguous fp32 [M <= 64, 32], one prefix cache per layer")
+        if emb_b.dtype != torch.float32 or emb_b.shape[0] < steps or emb_b.shape[1] != self.HIDDEN or not emb_b.is_contiguous():
+            raise ValueError("emb_b must be contiguous fp32 [steps, 720]")
+        if pad.dtype not in (torch.bool, torch.uint8) or pad.numel() != p or not pad.is_contiguous():
+            raise ValueError("pad must be a contiguous bool / uint8 [P]")
+        for t in (pos, pos0):
+            if t.dtype != torch.int32 or t.numel() != m or not t.is_contiguous():
+                raise ValueError("positions must be contiguous int32 [M]")
+        g, d = self.KV_HEADS, self.HEAD_DIM
+        for i, (cache, c) in enumerate(zip(caches, a.cache)):
+            k, vt = cache.k, cache.vt
+            if k.shape != (p, g, d) or k.stride(2) != 1 or k.dtype != torch.bfloat16 or vt.shape[:2] != (g, d) or vt.stride(2) != 1 or vt.shape[2] < _pad32(p):
+                raise ValueError("prefix caches must be bf16 [P, 5, 64] keys and [5, 64, >= P rounded up to 32] values")
+            if (a.cross_mask >> i) & 1:
+                if cache.k_lo is None or cache.k_lo.stride() != k.stride() or cache.vt_lo.stride() != vt.stride():
+                    raise ValueError("cross layers need lo planes of the hi planes' layout")
+                c.k_lo, c.vt_lo = cache.k_lo.data_ptr(), cache.vt_lo.data_ptr()
+            c.k, c.vt = k.data_ptr(), vt.data_ptr()
+            c.k_sl, c.k_sh, c.vt_sh, c.vt_sd = k.stride(0), k.stride(1), vt.stride(0), vt.stride(1)
+        out = torch.empty_like(x0)
+        a.steps, a.M, a.P, a.dt = int(steps), m, p, float(dt)
+        a.x0, a.out, a.pad, a.pos, a.pos0, a.emb_b = x0.data_ptr(), out.data_ptr(), pad.data_ptr(), pos.data_ptr(), pos0.data_ptr(), emb_b.data_ptr()
+        _launch_alone(lambda: native.check(native.lib().tk_sv_denoise(ctypes.addressof(a), _stream()), "tk_sv_denoise"), x0.device)
+        return out
 
 
 def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:

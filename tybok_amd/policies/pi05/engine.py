@@ -238,8 +238,7 @@ class PI05Engine(ChunkRuntime, PolicyEngine):
     def predict_action_chunk(self, frame: dict[str, Any], noise: torch.Tensor | None = None, *, return_normalized: bool = False, **rtc: Any) -> Any:
         if any(v is not None for v in rtc.values()):
             raise NotImplementedError("Real-Time Chunking guidance arguments are not supported by this backend")
-        actions = self._robot_actions(frame, noise)
-        chunk = self._to_robot_units(actions)
+        actions, chunk = self._robot_actions(frame, noise)
         return (chunk, actions.cpu().numpy()[0]) if return_normalized else chunk
 
     @torch.inference_mode()

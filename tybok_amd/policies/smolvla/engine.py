@@ -180,7 +180,7 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
 
     @torch.inference_mode()
     def predict_action_chunk(self, frame: dict[str, Any], noise: torch.Tensor | None = None) -> np.ndarray:
-        return self._to_robot_units(self._robot_actions(frame, noise))
+        return self._robot_actions(frame, noise)[1]
 
     @torch.inference_mode()
     def select_action(self, frame: dict[str, Any], noise: torch.Tensor | None = None) -> np.ndarray:

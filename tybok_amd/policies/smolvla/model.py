@@ -181,6 +181,10 @@ class SmolVLAModel:
         self.rope_cos = torch.cos(radians).to(self.device)
         self.rope_tables = tk.RopeTables(self.rope_cos, self.rope_sin) if self.fused_expert or self.fused_prefill else None
         self.set_num_steps(cfg.num_steps)
+        # the whole Euler loop as one persistent launch (None: the launches per layer); a request that finds it starved of
+        # compute units by other work is repeated with it off
+        self.denoise_plan = self._denoise_plan()
+        self.persistent_loop = self.denoise_plan is not None
         v = cfg.vlm_config.vision_config
         side = v.image_size // v.patch_size
         self.vis_pos = torch.arange(side * side, device=self.device)
@@ -210,6 +214,27 @@ class SmolVLAModel:
         self._img_scale_value = float(torch.tensor(t.hidden_size**0.5, dtype=BF16))  # the same bf16-rounded factor, on the host
         self.patch_w = self.p[VIS + "embeddings.patch_embedding.weight"].reshape(v.hidden_size, -1)
 
+    def _denoise_plan(self):
+        """The expert's weights for the flow-matching loop as one persistent launch, or None where the expert has
+        another shape than the one that launch is built for (or is not on the fused fp8 tiers)."""
+        pl, p = tk.SvDenoisePlan, self.p
+        dims = (self.cfg.expert_hidden_size, self.heads, self.kv_heads, self.head_dim, self.cfg.expert_intermediate_size, self.cfg.max_action_dim)
+        if not (self.fused_expert and all(m.fp8 and m.act == "silu" for m in self.exp_mlp)) or self.cfg.is_cross_layer(0):
+            return None
+        if dims != (pl.HIDDEN, pl.HEADS, pl.KV_HEADS, pl.HEAD_DIM, pl.FFN, pl.ACTION) or not 1 <= self.num_layers <= 20:
+            return None
+        if torch.cuda.get_device_properties(self.device).multi_processor_count < 256:
+            return None
+        layers = []
+        for i in range(self.num_layers):
+            lp, mlp = f"{EXP}layers.{i}.", self.exp_mlp[i]
+            layers.append(dict(wqkv=self.exp_qkv[i], wo=self.exp_o[i], wgu=mlp.wgu, wd=mlp.wd, norm_in=self.p[lp + "input_layernorm.weight"],
+                               norm_post=self.p[lp + "post_attention_layernorm.weight"], cross=self.cfg.is_cross_layer(i)))  # fmt: skip
+        return pl(
+            layers, time_w=p["action_time_mlp_out.weight"], time_b=p["action_time_mlp_out.bias"], act_w=p["action_out_proj.weight"],
+            act_b=p["action_out_proj.bias"], norm_out=p[EXP + "norm.weight"], emb_w=self.suffix_w, rope=self.rope_tables, eps=self.eps, device=self.device,
+        )  # fmt: skip
+
     def set_num_steps(self, n: int) -> None:
         self.num_steps = int(n)
         dt = -1.0 / self.num_steps
@@ -233,6 +258,7 @@ class SmolVLAModel:
             w_a, w_t = w_mlp[:, :e], w_mlp[:, e:]
             self.suffix_w = (w_a @ w_in).float().contiguous()
             self.suffix_b = [(w_a @ b_in + w_t @ te[0].to(torch.float64) + b_mlp).float().contiguous() for te in self.time_embs]
+            self.suffix_b_all = torch.stack(self.suffix_b).contiguous()  # [steps (Heun: 2 steps), hidden]
 
     def _pack_attention_weights(self, stack: str, q_only) -> tuple[list, list]:
         """bf16 attention weights of a decoder stack in tile order: q|k|v concatenated (or q alone
@@ -734,7 +760,14 @@ class SmolVLAModel:
         return x_t
 
     def sample_actions_core(self, embs, pads, att, noise, trace: dict | None = None) -> torch.Tensor:
-        if self.overlap and getattr(self.cfg, "sampler", "euler") == "euler" and trace is None and embs.shape[0] == 1 and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous():
+        euler = getattr(self.cfg, "sampler", "euler") == "euler"
+        # the loop as one launch: also where step 0 was asked to overlap the prefill (all ten steps of it take less time
+        # than nine of the other path's)
+        one_launch = (
+            euler and self.persistent_loop and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous()
+            and tk.SvDenoisePlan.covers(noise.shape[1], embs.shape[1])
+        )  # fmt: skip
+        if self.overlap and euler and not one_launch and trace is None and embs.shape[0] == 1 and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous():
             return self._sample_actions_overlapped(embs, pads, att, noise)
         vt = suf_pos = None
         fused = self.fused_expert and noise.shape[0] == 1
@@ -756,8 +789,8 @@ class SmolVLAModel:
                 positions = tuple(t[0].clamp(0, _ROPE_POSITIONS - 1).to(torch.int32) for t in positions)
         caches = self.attention_caches(keys, values, ekv, vt) if self.fused_expert and noise.shape[0] == 1 else None
         fused_loop = caches is not None and x_t.dtype == torch.float32 and x_t.is_contiguous()
-        if getattr(self.cfg, "sampler", "euler") == "heun":
-            # predictor at t, corrector at t + dt, then x <- x + (dt / 2) (v0 + v1)
+        if not euler:
+            # Heun: predictor at t, corrector at t + dt, then x <- x + (dt / 2) (v0 + v1)
             # (tybok/policies/smolvla/models/flow_matching.py:596-625)
             for step in range(self.num_steps):
                 if fused_loop:
@@ -768,6 +801,8 @@ class SmolVLAModel:
                     v1 = self.denoise_step(pads, keys, values, ekv, x_t + dt * v0, self.time_embs[2 * step + 1], positions, caches)
                 x_t = x_t + (dt * 0.5) * (v0 + v1)
             return x_t
+        if fused_loop and one_launch:
+            return self.denoise_plan.run(x_t[0], self.num_steps, dt, self.suffix_b_all, caches, pads[0], *positions)[None]
         h = None
         carry = fused_loop and self._fused_embed_ok(x_t)
         for step in range(self.num_steps):
