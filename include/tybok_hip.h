@@ -593,6 +593,44 @@ size_t tk_sv_denoise_xchg_bytes(int layers);
  * separate launches. */
 int tk_sv_denoise(const tk_sv_denoise_args* args, void* stream);
 
+/* The same for the pi0.5 expert (hidden 1024, 8 query heads of 256 over one K/V head, feed-forward 4096, AdaRMS norms
+ * with gated residuals, 32 action columns; tybok/policies/pi05/models/flow_matching.py:505-556).  The caller lays out:
+ *  - blob, per layer tk_pi_denoise_layer_bytes() bytes.  A piece of 1 KiB holds 16 output columns x 32 inputs, 16 bytes
+ *    per lane l = 16 g + r: inputs 8 g .. of column r.  q|k|v bf16 [share 80][tile 2][k tile 32]: shares 0..63 head s / 8,
+ *    columns 16 (s % 8) .. of both rotary halves, 64..71 the same of k, 72..79 32 columns of v; o bf16 [tile 64][k tile
+ *    64]; gate / up [pair 256][k tile 32], a lane's 8 gate codes then its 8 up codes; down [tile 64][k tile pair 64], a
+ *    lane's 8 codes of both; fp32 row scales of gate, up and down;
+ *  - mods, fp32 per (step, layer) tk_pi_denoise_mod_floats(): input norm scale, its gate, second norm's scale, its gate
+ *    (1024 each); the shift vectors through the weights they meet: q|k|v (in share order), gate, up (row scales
+ *    included).  Entry `layers` of a step: final norm's scale; first 32 q|k|v values: final shift . act_w^T + bias. */
+#define TK_PI_MAX_LAYERS 24
+typedef struct tk_pi_cache {
+  const void *k, *vt; /* bf16 [P, 256] of row stride k_sl, bf16 [256, >= P rounded up to 32] of row stride vt_sd; multiples of 8 */
+  int k_sl, vt_sd;
+} tk_pi_cache;
+typedef struct tk_pi_denoise_args {
+  int layers, steps; /* 2 <= layers <= TK_PI_MAX_LAYERS */
+  int M, P;          /* action tokens (<= 64), prefix tokens; ceil(P / 32) + ceil(M / 32) <= 40 */
+  float dt, eps;
+  const float* x0;
+  float* out;
+  const void* pad; /* uint8 [P] (1 = valid) or NULL */
+  const int* pos;  /* int32 [M] (clamped) */
+  const float *rope_cos, *rope_sin; /* fp32 [positions, 128]; bf16 arithmetic */
+  int positions;
+  const float *emb_w, *emb_b; /* fp32 [1024, 32], [1024] */
+  const float* act_w;         /* fp32 [32, 1024] */
+  const float* mods;
+  const void* blob;
+  void* xchg; /* tk_pi_denoise_xchg_bytes() bytes, 16-byte aligned; one launch at a time */
+  size_t xchg_bytes;
+  tk_pi_cache cache[TK_PI_MAX_LAYERS];
+} tk_pi_denoise_args;
+size_t tk_pi_denoise_xchg_bytes(void);
+size_t tk_pi_denoise_layer_bytes(void);
+size_t tk_pi_denoise_mod_floats(void);
+int tk_pi_denoise(const tk_pi_denoise_args* args, void* stream);
+
 /* ---- diagnostics: helpers of the tests and the benchmark; no policy path calls them -------------- */
 /* out_f32[256] = value of every e4m3fn code as decoded by the device's conversion instruction
  * (the weight path of the GEMM); used to assert the OCP (not FNUZ) flavour on the box. */

@@ -1,0 +1,86 @@
+"""The pi0.5 flow-matching loop as one persistent launch against the launches per layer it replaces, at the edges of its
+row groups, key tiles and key splits; what a launch that cannot get its waits answered leaves behind; argument checks."""
+
+import os
+import sys
+
+import pytest
+import torch
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+sys.path.insert(0, os.path.join(HERE, "golden"))
+
+import cases  # noqa: E402
+
+import tybok_amd.ops as tk  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def model():
+    from tybok_amd.policies.pi05.model import PI05Model
+
+    cfg, sd, _ = cases.pi05_build(cases.PI05_CASES["small"])
+    m = PI05Model(cfg, sd, "cuda", fused_expert=True, fp8_expert_mlp=True, fp8_llm_mlp=True, fused_prefill=True)
+    assert m.denoise_plan is not None and m.persistent_loop
+    return m
+
+
+def _case(model, m, p):
+    g = torch.Generator().manual_seed(1000 * m + p)
+    depth = model.ed["depth"]
+    kv = [tuple(torch.randn(1, 1, p, 256, generator=g).to(torch.bfloat16).cuda() for _ in range(2)) for _ in range(depth)]
+    pad = torch.rand(1, p, generator=g).cuda() > 0.2
+    pos = (int(pad.sum()) + torch.arange(m)).to(torch.int32).cuda()
+    return torch.randn(m, 32, generator=g).cuda(), model.attention_caches(kv), pad, pos
+
+
+def _run(model, x, caches, pad, pos):
+    return model.denoise_plan.run(x, -1.0 / model.num_steps, caches, pad[0], pos)
+
+
+# rows: one row group, a full one, one more row, two and a bit, all four; keys: a single one and fewer tiles than splits
+# (empty splits), tile edges, the most tiles
+@pytest.mark.parametrize("m,p", [(1, 1), (16, 32), (17, 33), (50, 275), (50, 712), (33, 223), (50, 968), (64, 1216)])
+@torch.inference_mode()
+def test_one_launch_matches_the_launches_per_layer(model, m, p):
+    x, caches, pad, pos = _case(model, m, p)
+    model.vt_suf = torch.zeros(1, 256, (m + 31) // 32 * 32, dtype=torch.bfloat16, device="cuda")
+    want = x
+    for step in range(model.num_steps):
+        hidden = model.lin("action_in_proj", want).to(torch.bfloat16)
+        hidden = model._denoise_layers_fused(pad, caches, hidden, pos, step)
+        _, want = tk.expert_tail(
+            hidden, model.p["action_out_proj.weight"], model.p["action_out_proj.bias"], ada=model.final_split[step], eps=1e-6, x_t=want, dt=-1.0 / model.num_steps
+        )
+    got = _run(model, x, caches, pad, pos)
+    assert torch.isfinite(got).all()
+    rel = float((got - want).norm() / (want - x).norm())
+    print(f"M={m} P={p}: relative difference of the flow {rel:.3g}")
+    assert rel < 2e-2  # bf16 rounding: residual rows, logits and rotary products round to bf16 there, fp32 here (3.1e-3 - 3.5e-3)
+    assert torch.equal(got, _run(model, x, caches, pad, pos))  # the exchange buffers start clean again
+
+
+@torch.inference_mode()
+def test_a_run_whose_waits_give_up_ends_with_nans_and_leaves_nothing_behind(model):
+    # forced from the host: with a bound of zero polls no wave waits; every block still runs to its end
+    case = _case(model, 50, 65)
+    want = _run(model, *case)
+    prev = tk.set_handoff_spin(0)
+    try:
+        lost = _run(model, *case)
+        torch.cuda.synchronize()
+    finally:
+        tk.set_handoff_spin(prev)
+    assert torch.isnan(lost).any()
+    assert torch.equal(_run(model, *case), want)
+
+
+def test_bad_arguments_are_refused(model):
+    x, caches, pad, pos = _case(model, 50, 65)
+    with pytest.raises(ValueError):
+        _run(model, torch.zeros(65, 32, device="cuda"), caches, pad, pos)
+    with pytest.raises(ValueError):
+        _run(model, x, caches, pad, pos.long())
+    assert not tk.PiDenoisePlan.covers(50, 1217) and tk.PiDenoisePlan.covers(64, 1216)

@@ -1531,6 +1531,56 @@ int tk_sv_denoise(const tk_sv_denoise_args* h, void* stream) {
   return TK_OK;
 }
 
+size_t tk_pi_denoise_xchg_bytes(void) { return tk_pi_denoise_exchange_bytes(); }
+size_t tk_pi_denoise_layer_bytes(void) { return tk_pi_denoise_blob_bytes(); }
+size_t tk_pi_denoise_mod_floats(void) { return tk_pi_denoise_mod_bytes() / 4; }
+
+int tk_pi_denoise(const tk_pi_denoise_args* h, void* stream) {
+  static_assert(kPiMaxLayers == TK_PI_MAX_LAYERS, "the public and the internal layer limits agree");
+  if (!h) return fail(TK_EINVAL, "pi_denoise: null argument");
+  if (h->layers < 2 || h->layers > kPiMaxLayers || h->steps < 1 || h->steps > 1000)
+    return fail(TK_EINVAL, "pi_denoise: layers=%d (2..%d), steps=%d (1..1000)", h->layers, kPiMaxLayers, h->steps);
+  if (h->M < 1 || h->M > 64 || h->P < 1 || (h->P + 31) / 32 + (h->M + 31) / 32 > tk_pi_denoise_max_key_tiles())
+    return fail(TK_EINVAL, "pi_denoise: M=%d (1..64), P=%d: at most %d key tiles", h->M, h->P, tk_pi_denoise_max_key_tiles());
+  if (!h->x0 || !h->out || !h->pos || !h->rope_cos || !h->rope_sin || h->positions < 1 || !h->emb_w || !h->emb_b || !h->act_w || !h->mods || !h->blob)
+    return fail(TK_EINVAL, "pi_denoise: null pointer");
+  if (!aligned16(h->act_w) || !aligned16(h->blob) || !aligned16(h->mods) || !aligned8(h->emb_b) || !aligned8(h->rope_cos) || !aligned8(h->rope_sin))
+    return fail(TK_EINVAL, "pi_denoise: act_w, mods, blob must be 16-byte, emb_b and the rotary tables 8-byte aligned");
+  if (!h->xchg || !aligned16(h->xchg) || h->xchg_bytes < tk_pi_denoise_exchange_bytes())
+    return fail(TK_EWORKSPACE, "pi_denoise: exchange buffer of %zu bytes, %zu needed", h->xchg_bytes, tk_pi_denoise_exchange_bytes());
+  if (device_cus() < 256) return fail(TK_EINVAL, "pi_denoise: %d compute units, 256 needed", device_cus());
+  PiDenoiseArgs a = {};
+  for (int l = 0; l < h->layers; ++l) {
+    const tk_pi_cache& s = h->cache[l];
+    if (!s.k || !s.vt || !aligned16(s.k) || !aligned16(s.vt)) return fail(TK_EINVAL, "pi_denoise: layer %d: null or misaligned prefix cache", l);
+    if (s.k_sl % 8 || s.vt_sd % 8 || s.k_sl < 256 || s.k_sl > (1 << 16) || s.vt_sd < (h->P + 31) / 32 * 32 || s.vt_sd > (1 << 16))
+      return fail(TK_EINVAL, "pi_denoise: layer %d: bad key / value strides %d %d", l, s.k_sl, s.vt_sd);
+    a.cache[l] = PiCache{(const unsigned short*)s.k, (const unsigned short*)s.vt, s.k_sl, s.vt_sd};
+  }
+  a.layers = h->layers;
+  a.steps = h->steps;
+  a.M = h->M;
+  a.P = h->P;
+  a.dt = h->dt;
+  a.eps = h->eps;
+  a.x0 = h->x0;
+  a.out = h->out;
+  a.pad = (const uint8_t*)h->pad;
+  a.pos = h->pos;
+  a.rope_cos = h->rope_cos;
+  a.rope_sin = h->rope_sin;
+  a.positions = h->positions;
+  a.emb_w = h->emb_w;
+  a.emb_b = h->emb_b;
+  a.act_w = h->act_w;
+  a.mods = h->mods;
+  a.blob = (const uint8_t*)h->blob;
+  a.xchg = h->xchg;
+  a.spin = g_handoff_spin.load(std::memory_order_relaxed);
+  if (tk_launch_pi_denoise(a, (hipStream_t)stream)) return fail(TK_ELAUNCH, "pi_denoise: launch failed");
+  return TK_OK;
+}
+
 int tk_debug_stream_read(const void* src, size_t bytes, int blocks, void* sink, void* stream) {
   if (!src || !aligned16(src) || blocks <= 0 || blocks > 65536) return fail(TK_EINVAL, "stream_read: null or unaligned source, or blocks=%d out of range", blocks);
   if (bytes == 0 || bytes % ((size_t)blocks * 4096)) return fail(TK_EINVAL, "stream_read: bytes=%zu must be a positive multiple of blocks * 4096", bytes);

@@ -367,3 +367,32 @@ int tk_sv_denoise_max_key_tiles();
 int tk_launch_sv_pack(const SvPackArgs& a, hipStream_t st);
 int tk_launch_sv_denoise(const SvDenoiseArgs& a, hipStream_t st);
 int tk_launch_fill_ones(void* p, size_t bytes, hipStream_t st);
+
+// ---- persistent denoising loop of pi0.5 (denoise_pi05.hip) ----
+constexpr int kPiMaxLayers = 24;
+struct PiCache {
+  const unsigned short *k, *vt;  // prefix K [P, 256] (row stride k_sl) and V^T [256, P rounded up to 32] (row stride vt_sd)
+  int k_sl, vt_sd;
+};
+struct PiDenoiseArgs {
+  int layers, steps, M, P;
+  float dt, eps;
+  const float* x0;  // fp32 [M, 32]
+  float* out;       // fp32 [M, 32]
+  const uint8_t* pad;  // [P] 0 / 1 or nullptr
+  const int* pos;      // int32 [M]
+  const float *rope_cos, *rope_sin;  // fp32 [positions, 128] holding bf16 values
+  int positions;
+  const float *emb_w, *emb_b;  // action embedding: fp32 [1024, 32], [1024]
+  const float* act_w;          // action projection: fp32 [32, 1024]
+  const float* mods;           // [steps][layers + 1] of tk_pi_denoise_mod_bytes()
+  const uint8_t* blob;         // [layers] of tk_pi_denoise_blob_bytes()
+  void* xchg;                  // tk_pi_denoise_exchange_bytes()
+  int spin;                    // polls of a waiting wave before it gives up
+  PiCache cache[kPiMaxLayers];
+};
+size_t tk_pi_denoise_exchange_bytes();
+size_t tk_pi_denoise_blob_bytes();
+size_t tk_pi_denoise_mod_bytes();
+int tk_pi_denoise_max_key_tiles();
+int tk_launch_pi_denoise(const PiDenoiseArgs& a, hipStream_t st);

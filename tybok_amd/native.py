@@ -152,6 +152,10 @@ SIGNATURES: dict[str, tuple] = {
     "tk_sv_denoise_layer_bytes": (c_size_t, []),
     "tk_sv_denoise_pack": (c_int, [c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
     "tk_sv_denoise": (c_int, [c_void_p, c_void_p]),
+    "tk_pi_denoise_xchg_bytes": (c_size_t, []),
+    "tk_pi_denoise_layer_bytes": (c_size_t, []),
+    "tk_pi_denoise_mod_floats": (c_size_t, []),
+    "tk_pi_denoise": (c_int, [c_void_p, c_void_p]),
     "tk_debug_decode_fp8": (c_int, [c_void_p, c_void_p]),
     "tk_debug_stream_read": (c_int, [c_void_p, c_size_t, c_int, c_void_p, c_void_p]),
     "tk_debug_fp8w_gemm_cut": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
@@ -184,6 +188,29 @@ class SvDenoiseArgs(ctypes.Structure):
         *((n, c_void_p) for n in ("emb_w", "emb_b", "time_w", "time_b", "act_w", "act_b", "blob", "xchg")),
         ("xchg_bytes", c_size_t),
         ("cache", SvCache * SV_MAX_LAYERS),
+    ]
+
+
+PI_MAX_LAYERS = 24
+
+
+class PiCache(ctypes.Structure):
+    """``tk_pi_cache``"""
+
+    _fields_ = [*((n, c_void_p) for n in ("k", "vt")), *((n, c_int) for n in ("k_sl", "vt_sd"))]
+
+
+class PiDenoiseArgs(ctypes.Structure):
+    """``tk_pi_denoise_args``"""
+
+    _fields_ = [
+        *((n, c_int) for n in ("layers", "steps", "M", "P")),
+        *((n, c_float) for n in ("dt", "eps")),
+        *((n, c_void_p) for n in ("x0", "out", "pad", "pos", "rope_cos", "rope_sin")),
+        ("positions", c_int),
+        *((n, c_void_p) for n in ("emb_w", "emb_b", "act_w", "mods", "blob", "xchg")),
+        ("xchg_bytes", c_size_t),
+        ("cache", PiCache * PI_MAX_LAYERS),
     ]
 
 

@@ -1046,6 +1046,114 @@ class SvDenoisePlan:
         return out
 
 
+def _operand_tiles(w: torch.Tensor) -> torch.Tensor:
+    """``[N, K]`` -> ``[N / 16, K / 32, 4, 16, 8]``: per 16 rows x 32 columns the 8 columns ``8 g ..`` of row ``r``, the
+    order in which the persistent launches read a matrix operand."""
+    n, k = w.shape
+    return w.view(n // 16, 16, k // 32, 4, 8).permute(0, 2, 3, 1, 4)
+
+
+def _unpack_fp8_tiles(data: torch.Tensor, n: int, k: int) -> torch.Tensor:
+    """The ``[n, k]`` e4m3fn bytes of a packed matrix (``n``, ``k`` multiples of 32)."""
+    return data.view(-1)[: n * k].view(n // 32, k // 32, 2, 32, 16).permute(0, 3, 1, 2, 4).reshape(n, k)
+
+
+class PiDenoisePlan:
+    """The pi0.5 expert's weights laid out for :meth:`run`, the flow-matching loop as one persistent launch
+    (``tk_pi_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).
+
+    ``layers``: one dict per expert layer -- ``q``, ``k``, ``v``, ``o`` (bf16 matrices), ``wgu`` (:class:`PackedGateUp`),
+    ``wd`` (:class:`PackedWeight`)."""
+
+    HIDDEN, HEADS, KV_HEADS, HEAD_DIM, FFN, ACTION = 1024, 8, 1, 256, 4096, 32
+    MAX_TOKENS, MAX_TILES = 64, 40
+
+    def __init__(self, layers, *, act_w, act_b, emb_w, emb_b, rope: RopeTables, eps: float, device):
+        e, f, d, nq = self.HIDDEN, self.FFN, self.HEAD_DIM, self.HEADS * self.HEAD_DIM
+        if not 2 <= len(layers) <= native.PI_MAX_LAYERS:
+            raise ValueError(f"2..{native.PI_MAX_LAYERS} layers")
+        for w in layers:
+            bf16 = ((w["q"], (nq, e)), (w["k"], (d, e)), (w["v"], (d, e)), (w["o"], (e, nq)))
+            if any(t.dtype != torch.bfloat16 or tuple(t.shape) != s for t, s in bf16) or (w["wgu"].i, w["wgu"].k, w["wd"].n, w["wd"].k) != (f, e, e, f):
+                raise ValueError("expert layer of another shape")
+        fp32 = ((act_w, (self.ACTION, e)), (act_b, (self.ACTION,)), (emb_w, (e, self.ACTION)), (emb_b, (e,)))
+        if any(t.dtype != torch.float32 or tuple(t.shape) != s or not t.is_contiguous() for t, s in fp32):
+            raise ValueError("action projections must be contiguous fp32 of the expert's shapes")
+        lib = native.lib()
+        nbytes, lbytes = int(lib.tk_pi_denoise_xchg_bytes()), int(lib.tk_pi_denoise_layer_bytes())
+        self._keep = (act_w, act_b, emb_w, emb_b, rope)
+        self._xchg = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        self._blob = torch.empty(len(layers), lbytes, dtype=torch.uint8, device=device)
+        self._mod_floats, self._mods, self._steps = int(lib.tk_pi_denoise_mod_floats()), None, 0
+        # q|k|v rows in the order of the launch's shares: a rotary pair of 16-row tiles per share of q and k
+        pair = torch.arange(d, device=device).view(2, d // 32, 16).transpose(0, 1).reshape(-1)
+        self._rows = torch.cat([h * d + pair for h in range(self.HEADS + 1)] + [torch.arange(nq + d, nq + 2 * d, device=device)])
+        for w, out in zip(layers, self._blob):
+            gate, up = _unpack_fp8_tiles(w["wgu"].data, 2 * f, e).view(f // 32, 2, 32, e).unbind(1)
+            gu = torch.stack([_operand_tiles(t.reshape(f, e)) for t in (gate, up)], dim=-2)
+            down = _operand_tiles(_unpack_fp8_tiles(w["wd"].data, e, f)).reshape(e // 16, f // 64, 2, 4, 16, 8).permute(0, 1, 3, 4, 2, 5)
+            qkv = torch.cat([w["q"], w["k"], w["v"]])[self._rows]
+            parts = [_operand_tiles(qkv), _operand_tiles(w["o"]), gu, down, w["wgu"].scale_gate, w["wgu"].scale_up, w["wd"].scale]
+            torch.cat([t.contiguous().view(torch.uint8).view(-1) for t in parts], out=out)
+        a = self._args = native.PiDenoiseArgs()
+        a.layers, a.eps = len(layers), float(eps)
+        a.rope_cos, a.rope_sin, a.positions = rope.cos.data_ptr(), rope.sin.data_ptr(), rope.positions
+        a.emb_w, a.emb_b, a.act_w = emb_w.data_ptr(), emb_b.data_ptr(), act_w.data_ptr()
+        a.blob, a.xchg, a.xchg_bytes = self._blob.data_ptr(), self._xchg.data_ptr(), nbytes
+
+    def set_modulations(self, mods, final) -> None:
+        """Per step ``mods[step][layer] = ((scale, shift, gate) of the input norm, the same of the second norm)`` and
+        ``final[step] = (scale, shift)``, as the launches per layer take them (once per number of steps).  The shifts go
+        through the weights here: ``W . shift`` is a constant of the step.  In double precision, layer by layer."""
+        e, f, d, nq, steps, depth = self.HIDDEN, self.FFN, self.HEAD_DIM, self.HEADS * self.HEAD_DIM, len(mods), self._args.layers
+        act_w, act_b = self._keep[:2]
+        out = torch.zeros(steps, depth + 1, self._mod_floats, dtype=torch.float32, device=self._blob.device)
+        col = lambda i, norm, part: torch.stack([mods[s][i][norm][part].float() for s in range(steps)])  # noqa: E731
+        n_qkv, n_gu = 2 * (nq + 2 * d) * e, 2 * f * e
+        for i in range(depth):
+            blob = self._blob[i]
+            w = blob[:n_qkv].view(torch.bfloat16).view(-1, e // 32, 4, 16, 8).permute(0, 3, 1, 2, 4).reshape(-1, e)
+            lo = n_qkv + 2 * e * nq
+            gu = blob[lo : lo + n_gu].view(torch.float8_e4m3fn).float().view(f // 16, e // 32, 4, 16, 2, 8).permute(4, 0, 3, 1, 2, 5).reshape(2 * f, e)
+            sc = blob[lo + n_gu + e * f :].view(torch.float32)[: 2 * f]
+            parts = [col(i, 0, 0), col(i, 0, 2), col(i, 1, 0), col(i, 1, 2), (col(i, 0, 1).double() @ w.double().t()).float(),
+                     ((col(i, 1, 1).double() @ gu.double().t()) * sc.double()).float()]  # fmt: skip
+            out[:, i] = torch.cat(parts, dim=1)
+        out[:, depth, :e] = torch.stack([s for s, _ in final])
+        shift = torch.stack([s for _, s in final]).double()
+        out[:, depth, 4 * e : 4 * e + self.ACTION] = (shift @ act_w.double().t() + act_b.double()).float()
+        self._mods, self._steps = out, steps
+
+    @classmethod
+    def covers(cls, tokens: int, prefix: int) -> bool:
+        """Whether a run of that many action tokens over that long a prefix is one launch."""
+        return 1 <= tokens <= cls.MAX_TOKENS and prefix >= 1 and (prefix + 31) // 32 + (tokens + 31) // 32 <= cls.MAX_TILES
+
+    def run(self, x0: torch.Tensor, dt: float, caches, pad: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
+        """``x0 [M, 32]`` fp32 after the modulations' number of Euler steps of size ``dt``; ``caches`` a :class:`PrefixKV`
+        per layer, ``pad`` bool ``[P]``, ``pos`` int32 ``[M]``."""
+        a = self._args
+        m, p, d = x0.shape[0], caches[0].length, self.HEAD_DIM
+        if self._mods is None:
+            raise RuntimeError("set_modulations() first")
+        if x0.dtype != torch.float32 or x0.shape[1] != self.ACTION or not x0.is_contiguous() or not self.covers(m, p) or len(caches) != a.layers:
+            raise ValueError("x0 must be contiguous fp32 [M <= 64, 32], one prefix cache per layer")
+        if pad.dtype not in (torch.bool, torch.uint8) or pad.numel() != p or not pad.is_contiguous():
+            raise ValueError("pad must be a contiguous bool / uint8 [P]")
+        if pos.dtype != torch.int32 or pos.numel() != m or not pos.is_contiguous():
+            raise ValueError("positions must be contiguous int32 [M]")
+        for cache, c in zip(caches, a.cache):
+            k, vt = cache.k, cache.vt
+            if k.shape != (p, 1, d) or k.stride(2) != 1 or k.dtype != torch.bfloat16 or vt.shape[:2] != (1, d) or vt.stride(2) != 1 or vt.shape[2] < _pad32(p):
+                raise ValueError("prefix caches must be bf16 [P, 1, 256] keys and [1, 256, >= P rounded up to 32] values")
+            c.k, c.vt, c.k_sl, c.vt_sd = k.data_ptr(), vt.data_ptr(), k.stride(0), vt.stride(1)
+        out = torch.empty_like(x0)
+        a.steps, a.M, a.P, a.dt = self._steps, m, p, float(dt)
+        a.x0, a.out, a.pad, a.pos, a.mods = x0.data_ptr(), out.data_ptr(), pad.data_ptr(), pos.data_ptr(), self._mods.data_ptr()
+        _launch_alone(lambda: native.check(native.lib().tk_pi_denoise(ctypes.addressof(a), _stream()), "tk_pi_denoise"), x0.device)
+        return out
+
+
 def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float, out_dtype: torch.dtype = torch.bfloat16) -> torch.Tensor:
     """``bf16(LayerNorm(x) * w + b)`` over the last dim of ``x [..., K]`` (fp32 with fp32 parameters, or
     bf16 with bf16 parameters; contiguous rows), statistics in fp32.  One launch, bf16 result -- or, for fp32 rows

@@ -187,7 +187,30 @@ class PI05Model:
             # the MLP-only tiers: fc1 / fc2 on the many-row kernel in their 16-bit type (bf16 or fp16)
             if all(w.shape[1] % 16 == 0 and w.shape[0] % 8 == 0 for w, _ in self.vis_lowp.values()):
                 self.vis_dense = {n: (tk.pack_bf16_weight(w), b.contiguous()) for n, (w, b) in self.vis_lowp.items()}
+        # the whole Euler loop as one persistent launch (None: the launches per layer); a request that finds it starved of
+        # compute units by other work is repeated with it off
+        self.denoise_plan = self._denoise_plan()
+        self.persistent_loop = self.denoise_plan is not None
         self.set_num_steps(cfg.num_steps)
+
+    def _denoise_plan(self):
+        """The expert's weights for the flow-matching loop as one persistent launch, or None where the expert has
+        another shape than the one that launch is built for (or is not on the fused fp8 tiers)."""
+        pl, p, ed = tk.PiDenoisePlan, self.p, self.ed
+        if not (self.fused_expert and all(m.fp8 and m.act == "gelu_tanh" for m in self.exp_mlp)):
+            return None
+        dims = (ed["width"], ed["num_heads"], ed["num_kv_heads"], self.head_dim, self.exp_mlp[0].wgu.i, p["action_out_proj.weight"].shape[0])
+        if dims != (pl.HIDDEN, pl.HEADS, pl.KV_HEADS, pl.HEAD_DIM, pl.FFN, pl.ACTION) or not 2 <= ed["depth"] <= 24:
+            return None
+        ends = [p[f"action_{n}_proj.{t}"] for n in ("out", "in") for t in ("weight", "bias")]
+        if any(t.dtype != torch.float32 for t in ends) or torch.cuda.get_device_properties(self.device).multi_processor_count < 256:
+            return None
+        layers = []
+        for i in range(ed["depth"]):
+            lp = f"{EXP}layers.{i}.self_attn."
+            layers.append(dict({n: p[f"{lp}{n}_proj.weight"].to(BF16) for n in "qkvo"}, wgu=self.exp_mlp[i].wgu, wd=self.exp_mlp[i].wd))
+        act_w, act_b, emb_w, emb_b = (t.contiguous() for t in ends)
+        return pl(layers, act_w=act_w, act_b=act_b, emb_w=emb_w, emb_b=emb_b, rope=self.rope_tables_hip, eps=EPS, device=self.device)
 
     def lin(self, name: str, x: torch.Tensor) -> torch.Tensor:
         return F.linear(x, self.p[name + ".weight"], self.p.get(name + ".bias"))
@@ -224,6 +247,8 @@ class PI05Model:
                 self.final_mods.append(final)
                 self.mods_split.append(mods_split)
                 self.final_split.append(final_split)
+            if self.denoise_plan is not None:
+                self.denoise_plan.set_modulations(self.mods_split, self.final_split)
 
     def velocity_at(self, prefix_pad, kv, x_t, t: float) -> torch.Tensor:
         """One velocity evaluation at an arbitrary flow time (the per-step tables hold only the Euler
@@ -632,6 +657,8 @@ class PI05Model:
                 self.vt_suf = torch.zeros(kv[0][0].shape[1], self.head_dim, (s + 31) // 32 * 32, dtype=BF16, device=self.device)
             # clamp(sum(pad) + arange(s)): from the prefill's bookkeeping launch, or a launch of its own
             pos32 = suf_pos if suf_pos is not None else tk.prefix_meta(pads[0].contiguous(), None, _ROPE_POSITIONS, s, want_mask=False)[2]
+            if self.persistent_loop and tk.PiDenoisePlan.covers(s, pads.shape[1]):
+                return self.denoise_plan.run(x_t[0], dt, caches, pads[0], pos32)[None]
             # (`action_in_proj` stays the library's fp32 product + cast, two launches a step: carried in the tail launch
             # of the step before -- tk_expert_tail_embed -- it sums its 32 terms in another order, and that re-draw of
             # a few bf16 roundings moved one frame's maximum error from under to over the cap held for this path)
