@@ -16,15 +16,16 @@
 //           P4  h = silu(g) * u of norm(hidden) . Wgu^T           64 blocks, two gate / up pairs of 16 columns each
 //           P5  hidden += h . Wd^T                                45 blocks
 //
-// Rows: 16 per block (four row groups, each on two XCDs: the exchange of a group is 0.3 us cheaper there than across
-// all eight), so a block's share of a phase's input is 23 - 64 KiB.  Inside a block the 16 waves split K; the partial
+// Rows: 16 per block (four row groups), so a block's share of a phase's input is 23 - 64 KiB.  The four blocks of one
+// column share are on one XCD, whose L2 then fetches their weights once: the loop 2.74 -> 2.55 ms against a row group on
+// two XCDs of its own, although a hand-off inside two XCDs is 0.3 us shorter.  Inside a block the 16 waves split K; the partial
 // tiles meet in LDS once per phase.  With four waves on every SIMD an instruction costs 16 cycles of the phase, so what
 // 64 blocks would repeat is done once by the producer: hidden rows are exchanged as bf16(x * w) with the NEXT norm's
 // weight, beside the row's partial sums of squares; 1 / rms is a factor of the whole row and multiplies the accumulator.
 // The residual stream never leaves its owner's registers and stays fp32 there.
 //
-// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.8 ms, against 4.7 ms of the launches per layer.
-// A self layer takes 17 us, a cross layer 18 us: of its five hand-offs 1.3 - 2 us each, the attention 2.5 us, the other
+// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.55 ms, against 4.7 ms of the launches per layer.
+// A layer takes 16 us: of its five hand-offs 1.3 - 2 us each, the attention 2.5 us, the other
 // phases 0.8 - 1.2 us each from their input's arrival; the cross layer's attention blocks load 216 KiB (query weights,
 // K and V hi + lo planes) at the 60 B/ns a compute unit gets, 3.5 us.
 #include <math.h>
@@ -86,8 +87,8 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   cx.r = cx.lane & 15;
   cx.spin = a.spin;
   cx.dead = 0;
-  // blocks land round-robin on the XCDs: a row group on two of them
-  int rt = (blockIdx.x & 7) >> 1, c = ((blockIdx.x >> 3) << 1) | (blockIdx.x & 1);
+  // blocks land round-robin on the XCDs: the row groups' blocks of one column share are on one
+  int rt = blockIdx.x >> 6, c = blockIdx.x & 63;
   if (rt * 16 >= a.M) return;
   const int set_b = HEAD_B + a.layers * LAYER_B;
   cx.rs = make_rsrc(a.xchg, PW_B + 2u * (unsigned)set_b);
@@ -108,6 +109,9 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   // for data that the blocks `from` .. (and the extra ones) produce in phase `id`
   enum { PH_E0, PH_E1, PH_E2, PH_P1, PH_P2, PH_P3, PH_P4, PH_P5 };
   auto id_of = [&](int step, int l, int ph) { return (step * (a.layers + 1) + l + 1) * 8 + ph; };  // E phases: l = -1
+  // (everything asked for has arrived by then: told so, the compiler does not wait for the progress store's acknowledgement
+  // where it next uses a loaded register)
+  auto arrived = [&]() { __builtin_amdgcn_s_waitcnt(0x0f70); };  // vmcnt(0)
   auto announce = [&](int id) {
     if (tid == 0) st_x(cx.rs, (unsigned)id, 0, OFF_PW + rt * kProgressBytes + c * 128);
   };
@@ -415,6 +419,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
     gate(kHid, in_id);
     i32x4 st;
     wait_tiles<2, KE>(x, cx, in_base + rt * X_B, wave, 16, [&] { ask_stats(st, in_base); });
+    arrived();
     announce(id);
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -547,6 +552,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       i32x4 v[3];
       gate(kHid, id_of(step, -1, PH_E1));
       wait_tiles<3, NE>(v, cx, cur + OFF_HE + rt * HE_B, wave, 16, [] {});
+      arrived();
       announce(id_of(step, -1, PH_E2));
       f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -666,6 +672,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         i32x4 v[2];
         gate(kAtt, id_of(step, l, PH_P2));
         wait_tiles<2, KO>(v, cx, base + OFF_ATT + rt * ATT_B, wave, 16, [] {});
+        arrived();
         announce(id_of(step, l, PH_P3));
         const f32x4 acc = mfma(wB[1], v[1], mfma(wB[0], v[0], f32x4{0.f, 0.f, 0.f, 0.f}));
         *(f32x4*)(part() + wave * 1024 + lane * 16) = acc;
@@ -697,6 +704,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
             wu[i] = fp8x8_to_bf16x8(wC[i][2], wC[i][3]);
           }
         });
+        arrived();
         announce(id_of(step, l, PH_P4));
         f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
@@ -737,6 +745,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
 #pragma unroll
           for (int i = 0; i < 4; ++i) wd[i] = fp8x8_to_bf16x8(wD[i >> 1][2 * (i & 1)], wD[i >> 1][2 * (i & 1) + 1]);
         });
+        arrived();
         announce(id_of(step, l, PH_P5));
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
