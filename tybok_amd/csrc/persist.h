@@ -9,7 +9,8 @@
 // 1.9 us with acknowledged stores + flags, and 3 us or more between the first wait of one dependent launch and that
 // of the next.  Buffers come in two sets, used by alternate denoising steps; a block rewrites its words of the idle
 // set with ones one step after they were read (every path from "written" to "rewritten" runs through data that all
-// readers produced after their reads), so a word is always clean before it is used again.
+// readers produced after their reads), so a word is always clean before it is used again.  (The pi0.5 loop keeps a ring
+// of four layers instead: a layer's words are rewritten at the end of the next one and used again two layers later.)
 //
 // GATE.  Loads that come back empty cost the compute unit's memory pipe as much as real ones (its sixteen waves asking
 // for a phase's whole input keep it busy for 0.4 - 1 us), so nobody asks before there is something to expect: every block
