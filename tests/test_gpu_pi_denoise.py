@@ -84,3 +84,17 @@ def test_bad_arguments_are_refused(model):
     with pytest.raises(ValueError):
         _run(model, x, caches, pad, pos.long())
     assert not tk.PiDenoisePlan.covers(50, 1217) and tk.PiDenoisePlan.covers(64, 1216)
+
+
+@torch.inference_mode()
+def test_more_steps_than_one_launch_takes_run_layer_by_layer(model):
+    cfg, _, inp = cases.pi05_build(cases.PI05_CASES["small"])
+    steps = model.num_steps
+    model.set_num_steps(1001)
+    try:
+        args = ([t.cuda() for t in inp["images"]], [t.cuda() for t in inp["img_masks"]], inp["lang_tokens"].cuda(), inp["lang_masks"].cuda(), inp["noise"].cuda())
+        assert torch.isfinite(model.sample_actions(*args)).all()
+    finally:
+        model.set_num_steps(steps)
+    assert not tk.PiDenoisePlan.covers(50, 275, 1001) and tk.PiDenoisePlan.covers(50, 275, 1000)
+    assert not tk.SvDenoisePlan.covers(50, 241, 1001) and tk.SvDenoisePlan.covers(50, 241, 1000)

@@ -963,6 +963,9 @@ def _launch_alone(launch, device) -> None:
             launch()
 
 
+DENOISE_MAX_STEPS = 1000  # Euler steps of one denoising launch
+
+
 class SvDenoisePlan:
     """The SmolVLA-shaped expert's weights laid out for :meth:`run`, the flow-matching loop as one persistent launch
     (``tk_sv_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).
@@ -1010,9 +1013,10 @@ class SvDenoisePlan:
             native.check(lib.tk_sv_denoise_pack(ctypes.addressof(w), i, self._blob.data_ptr(), self._blob.numel(), _stream()), "tk_sv_denoise_pack")
 
     @classmethod
-    def covers(cls, tokens: int, prefix: int) -> bool:
-        """Whether a run of that many action tokens over that long a prefix is one launch."""
-        return 1 <= tokens <= cls.MAX_TOKENS and prefix >= 1 and (prefix + 31) // 32 + (tokens + 31) // 32 <= cls.MAX_TILES
+    def covers(cls, tokens: int, prefix: int, steps: int = 1) -> bool:
+        """Whether ``steps`` steps of that many action tokens over that long a prefix are one launch."""
+        tiles = (prefix + 31) // 32 + (tokens + 31) // 32
+        return 1 <= tokens <= cls.MAX_TOKENS and prefix >= 1 and tiles <= cls.MAX_TILES and 1 <= steps <= DENOISE_MAX_STEPS
 
     def run(self, x0: torch.Tensor, steps: int, dt: float, emb_b: torch.Tensor, caches, pad: torch.Tensor, pos: torch.Tensor, pos0: torch.Tensor) -> torch.Tensor:
         """``x0 [M, 32]`` fp32 after ``steps`` Euler steps of size ``dt``; ``emb_b`` fp32 ``[steps, 720]``, ``caches`` a
@@ -1125,9 +1129,10 @@ class PiDenoisePlan:
         self._mods, self._steps = out, steps
 
     @classmethod
-    def covers(cls, tokens: int, prefix: int) -> bool:
-        """Whether a run of that many action tokens over that long a prefix is one launch."""
-        return 1 <= tokens <= cls.MAX_TOKENS and prefix >= 1 and (prefix + 31) // 32 + (tokens + 31) // 32 <= cls.MAX_TILES
+    def covers(cls, tokens: int, prefix: int, steps: int = 1) -> bool:
+        """Whether ``steps`` steps of that many action tokens over that long a prefix are one launch."""
+        tiles = (prefix + 31) // 32 + (tokens + 31) // 32
+        return 1 <= tokens <= cls.MAX_TOKENS and prefix >= 1 and tiles <= cls.MAX_TILES and 1 <= steps <= DENOISE_MAX_STEPS
 
     def run(self, x0: torch.Tensor, dt: float, caches, pad: torch.Tensor, pos: torch.Tensor) -> torch.Tensor:
         """``x0 [M, 32]`` fp32 after the modulations' number of Euler steps of size ``dt``; ``caches`` a :class:`PrefixKV`

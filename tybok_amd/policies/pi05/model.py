@@ -247,7 +247,7 @@ class PI05Model:
                 self.final_mods.append(final)
                 self.mods_split.append(mods_split)
                 self.final_split.append(final_split)
-            if self.denoise_plan is not None:
+            if self.denoise_plan is not None and self.num_steps <= tk.DENOISE_MAX_STEPS:  # (more: the launches per layer)
                 self.denoise_plan.set_modulations(self.mods_split, self.final_split)
 
     def velocity_at(self, prefix_pad, kv, x_t, t: float) -> torch.Tensor:
@@ -657,7 +657,7 @@ class PI05Model:
                 self.vt_suf = torch.zeros(kv[0][0].shape[1], self.head_dim, (s + 31) // 32 * 32, dtype=BF16, device=self.device)
             # clamp(sum(pad) + arange(s)): from the prefill's bookkeeping launch, or a launch of its own
             pos32 = suf_pos if suf_pos is not None else tk.prefix_meta(pads[0].contiguous(), None, _ROPE_POSITIONS, s, want_mask=False)[2]
-            if self.persistent_loop and tk.PiDenoisePlan.covers(s, pads.shape[1]):
+            if self.persistent_loop and tk.PiDenoisePlan.covers(s, pads.shape[1], self.num_steps):
                 return self.denoise_plan.run(x_t[0], dt, caches, pads[0], pos32)[None]
             # (`action_in_proj` stays the library's fp32 product + cast, two launches a step: carried in the tail launch
             # of the step before -- tk_expert_tail_embed -- it sums its 32 terms in another order, and that re-draw of

@@ -765,7 +765,7 @@ class SmolVLAModel:
         # than nine of the other path's)
         one_launch = (
             euler and self.persistent_loop and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous()
-            and tk.SvDenoisePlan.covers(noise.shape[1], embs.shape[1])
+            and tk.SvDenoisePlan.covers(noise.shape[1], embs.shape[1], self.num_steps)
         )  # fmt: skip
         if self.overlap and euler and not one_launch and trace is None and embs.shape[0] == 1 and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous():
             return self._sample_actions_overlapped(embs, pads, att, noise)
