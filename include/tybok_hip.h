@@ -547,6 +547,7 @@ int tk_expert_tail_embed(const void* x, int ldx, const void* norm_w, const void*
  * tk_expert_cross_attn_fused, tk_fp8w_norm_gated_ffn, tk_expert_tail); 1 / rms of a norm multiplies the products'
  * fp32 accumulators instead of the bf16 operands. */
 #define TK_SV_MAX_LAYERS 20
+#define TK_DENOISE_MAX_STEPS 1000
 typedef struct tk_sv_weights {
   const void* wqkv; /* tk_pack_bf16_weight(rope_half = 32): q | k | v rows (1600), cross layers: q rows only (960) */
   const void* wo;   /* tk_pack_bf16_weight of [720, 960] */
@@ -561,14 +562,16 @@ typedef struct tk_sv_weights {
 size_t tk_sv_denoise_layer_bytes(void);
 int tk_sv_denoise_pack(const tk_sv_weights* w, int layer, void* blob, size_t blob_bytes, void* stream);
 /* One layer's cached prefix: keys bf16 [P, 5, 64] (element strides k_sl, k_sh) and values transposed bf16
- * [5, 64, >= P rounded up to 32] (vt_sh, vt_sd), strides multiples of 8; cross layers: the hi planes, and the lo planes
- * of the same strides. */
+ * [5, 64, >= P rounded up to 32] (vt_sh, vt_sd), strides multiples of 8, k_sl and vt_sd at most TK_SV_MAX_ROW_STRIDE,
+ * k_sh and vt_sh at most TK_SV_MAX_HEAD_STRIDE; cross layers: the hi planes, and the lo planes of the same strides. */
+#define TK_SV_MAX_ROW_STRIDE (1 << 16)
+#define TK_SV_MAX_HEAD_STRIDE (1 << 20)
 typedef struct tk_sv_cache {
   const void *k, *k_lo, *vt, *vt_lo;
   int k_sl, k_sh, vt_sh, vt_sd;
 } tk_sv_cache;
 typedef struct tk_sv_denoise_args {
-  int layers, steps; /* layers <= TK_SV_MAX_LAYERS */
+  int layers, steps; /* layers <= TK_SV_MAX_LAYERS, steps <= TK_DENOISE_MAX_STEPS */
   int M, P;          /* action tokens (<= 64), prefix tokens; ceil(P / 32) + ceil(M / 32) <= 16 */
   unsigned cross_mask; /* bit l: layer l is a cross layer; layer 0 must not be one */
   float dt, eps;
@@ -609,7 +612,7 @@ typedef struct tk_pi_cache {
   int k_sl, vt_sd;
 } tk_pi_cache;
 typedef struct tk_pi_denoise_args {
-  int layers, steps; /* 2 <= layers <= TK_PI_MAX_LAYERS */
+  int layers, steps; /* 2 <= layers <= TK_PI_MAX_LAYERS, steps <= TK_DENOISE_MAX_STEPS */
   int M, P;          /* action tokens (<= 64), prefix tokens; ceil(P / 32) + ceil(M / 32) <= 40 */
   float dt, eps;
   const float* x0;

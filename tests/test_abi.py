@@ -215,6 +215,50 @@ def test_arguments_are_checked_on_the_host(name, args, code, fragment):
     assert fragment in message, message
 
 
+def _loop_args(kind, cache=None, **kw):
+    """Arguments both denoising loops accept (stand-in pointers), with ``kw`` and the first layer's ``cache`` changed."""
+    from tybok_amd import native
+
+    a = native.SvDenoiseArgs() if kind == "sv" else native.PiDenoiseArgs()
+    a.layers, a.steps, a.M, a.P, a.positions, a.xchg_bytes = 2, 10, 50, 241, 300, 1 << 40
+    for name, ctype in a._fields_:
+        if ctype is ctypes.c_void_p:
+            setattr(a, name, P)
+    for c in a.cache[:2]:
+        c.k, c.vt = P, P
+        c.k_sl, c.vt_sd = (320, 256)
+        if kind == "sv":
+            c.k_sh, c.vt_sh = 64, 64 * 256
+    for name, value in kw.items():
+        setattr(a, name, value)
+    for name, value in (cache or {}).items():
+        setattr(a.cache[0], name, value)
+    return a
+
+
+@pytest.mark.parametrize("kind,change,fragment", [
+    ("sv", dict(steps=1001), "steps=1001"),
+    ("sv", dict(cache=dict(k_sl=1 << 22)), "strides"),  # 240 rows of it: 2 GB, a byte offset beyond 32 bits
+    ("sv", dict(cache=dict(vt_sd=1 << 25)), "strides"),
+    ("sv", dict(cache=dict(k_sh=1 << 28)), "strides"),
+    ("sv", dict(cache=dict(vt_sh=1 << 28)), "strides"),
+    ("pi", dict(steps=1001), "steps=1001"),
+    ("pi", dict(cache=dict(k_sl=1 << 22)), "strides"),
+    ("pi", dict(cache=dict(vt_sd=1 << 25)), "strides"),
+])  # fmt: skip
+def test_a_loops_sizes_are_bounded_on_the_host(kind, change, fragment):
+    # strides and steps whose byte offsets and progress words would leave 32 bits never reach the kernel
+    from tybok_amd import native
+
+    if not os.path.exists(native.library_path()):
+        pytest.skip("libtybok_hip.so not built")
+    lib = native.lib()
+    args = _loop_args(kind, **change)
+    rc = getattr(lib, f"tk_{kind}_denoise")(ctypes.addressof(args), None)
+    message = lib.tk_last_error().decode()
+    assert rc == -1 and fragment in message, (rc, message)
+
+
 @pytest.mark.parametrize("compiler,flags", [("gcc", ["-std=c99", "-x", "c"]), ("g++", ["-std=c++17", "-x", "c++"])])
 def test_header_is_plain_c_and_cxx(tmp_path, compiler, flags):
     # the boundary is a C ABI: the header must be usable from C (cgo, ctypes generators, C hosts) and from C++

@@ -1481,7 +1481,8 @@ int tk_sv_denoise_pack(const tk_sv_weights* w, int layer, void* blob, size_t blo
 int tk_sv_denoise(const tk_sv_denoise_args* h, void* stream) {
   static_assert(kSvMaxLayers == TK_SV_MAX_LAYERS, "the public and the internal layer limits agree");
   if (!h) return fail(TK_EINVAL, "sv_denoise: null argument");
-  if (h->layers < 1 || h->layers > kSvMaxLayers || h->steps < 1) return fail(TK_EINVAL, "sv_denoise: layers=%d (1..%d), steps=%d", h->layers, kSvMaxLayers, h->steps);
+  if (h->layers < 1 || h->layers > kSvMaxLayers || h->steps < 1 || h->steps > TK_DENOISE_MAX_STEPS)
+    return fail(TK_EINVAL, "sv_denoise: layers=%d (1..%d), steps=%d (1..%d)", h->layers, kSvMaxLayers, h->steps, TK_DENOISE_MAX_STEPS);
   if (h->M < 1 || h->M > 64 || h->P < 1) return fail(TK_EINVAL, "sv_denoise: M=%d (1..64), P=%d", h->M, h->P);
   if ((h->P + 31) / 32 + (h->M + 31) / 32 > tk_sv_denoise_max_key_tiles())
     return fail(TK_EINVAL, "sv_denoise: P=%d, M=%d: more than %d key tiles", h->P, h->M, tk_sv_denoise_max_key_tiles());
@@ -1499,7 +1500,9 @@ int tk_sv_denoise(const tk_sv_denoise_args* h, void* stream) {
     const bool cross = (h->cross_mask >> l) & 1u;
     if (!s.k || !s.vt || (cross && (!s.k_lo || !s.vt_lo))) return fail(TK_EINVAL, "sv_denoise: layer %d: null prefix cache", l);
     if (!aligned16(s.k) || !aligned16(s.vt) || (cross && (!aligned16(s.k_lo) || !aligned16(s.vt_lo)))) return fail(TK_EINVAL, "sv_denoise: layer %d: misaligned prefix cache", l);
-    if (s.k_sl % 8 || s.k_sh % 8 || s.vt_sh % 8 || s.vt_sd % 8 || s.k_sl < 0 || s.k_sh < 0 || s.vt_sd < (h->P + 31) / 32 * 32 || s.vt_sh < 0)
+    // upper bounds: the kernel forms byte offsets in 32 bits (at most 511 rows, 4 heads further: 75 MB)
+    if (s.k_sl % 8 || s.k_sh % 8 || s.vt_sh % 8 || s.vt_sd % 8 || s.k_sl < 0 || s.k_sh < 0 || s.vt_sd < (h->P + 31) / 32 * 32 || s.vt_sh < 0 ||
+        s.k_sl > TK_SV_MAX_ROW_STRIDE || s.vt_sd > TK_SV_MAX_ROW_STRIDE || s.k_sh > TK_SV_MAX_HEAD_STRIDE || s.vt_sh > TK_SV_MAX_HEAD_STRIDE)
       return fail(TK_EINVAL, "sv_denoise: layer %d: bad key / value strides %d %d %d %d", l, s.k_sl, s.k_sh, s.vt_sh, s.vt_sd);
     a.cache[l] = SvCache{(const unsigned short*)s.k, (const unsigned short*)s.k_lo, (const unsigned short*)s.vt, (const unsigned short*)s.vt_lo, s.k_sl, s.k_sh, s.vt_sh, s.vt_sd};
   }
@@ -1538,8 +1541,8 @@ size_t tk_pi_denoise_mod_floats(void) { return tk_pi_denoise_mod_bytes() / 4; }
 int tk_pi_denoise(const tk_pi_denoise_args* h, void* stream) {
   static_assert(kPiMaxLayers == TK_PI_MAX_LAYERS, "the public and the internal layer limits agree");
   if (!h) return fail(TK_EINVAL, "pi_denoise: null argument");
-  if (h->layers < 2 || h->layers > kPiMaxLayers || h->steps < 1 || h->steps > 1000)
-    return fail(TK_EINVAL, "pi_denoise: layers=%d (2..%d), steps=%d (1..1000)", h->layers, kPiMaxLayers, h->steps);
+  if (h->layers < 2 || h->layers > kPiMaxLayers || h->steps < 1 || h->steps > TK_DENOISE_MAX_STEPS)
+    return fail(TK_EINVAL, "pi_denoise: layers=%d (2..%d), steps=%d (1..%d)", h->layers, kPiMaxLayers, h->steps, TK_DENOISE_MAX_STEPS);
   if (h->M < 1 || h->M > 64 || h->P < 1 || (h->P + 31) / 32 + (h->M + 31) / 32 > tk_pi_denoise_max_key_tiles())
     return fail(TK_EINVAL, "pi_denoise: M=%d (1..64), P=%d: at most %d key tiles", h->M, h->P, tk_pi_denoise_max_key_tiles());
   if (!h->x0 || !h->out || !h->pos || !h->rope_cos || !h->rope_sin || h->positions < 1 || !h->emb_w || !h->emb_b || !h->act_w || !h->mods || !h->blob)
