@@ -157,7 +157,8 @@ int tk_fp8w_norm_gated_ffn(const void* x, int ldx, const void* norm_w, float nor
  * launch boundary it replaces (measured: 10.9 against 8.6 us per FFN), so the single-launch form is OFF unless
  * asked for.  The three calls below have no counterpart in the reference:
  *   tk_set_ffn_fusion(on): 1 runs the action chunk's FFN as one launch; returns the previous setting (default 0).
- *   tk_set_handoff_spin(polls): how often a waiting block polls before it gives up (default 200000, about 0.1 s);
+ *   tk_set_handoff_spin(polls): how often a waiting block polls before it gives up (default 200000, about 0.1 s; the
+ *     denoising launches carry a bound of their own);
  *     returns the previous value.  A block that gives up sets the workspace's sticky error word (int32 at byte
  *     offset tk_workspace_handoff_error_offset()) and goes on, so the launch always ends; its output is then
  *     undefined and the workspace must be re-initialised (tk_workspace_init) before the next call. */
@@ -548,6 +549,7 @@ int tk_expert_tail_embed(const void* x, int ldx, const void* norm_w, const void*
  * fp32 accumulators instead of the bf16 operands. */
 #define TK_SV_MAX_LAYERS 20
 #define TK_DENOISE_MAX_STEPS 1000
+#define TK_DENOISE_POLLS 200000 /* about 0.1 s */
 typedef struct tk_sv_weights {
   const void* wqkv; /* tk_pack_bf16_weight(rope_half = 32): q | k | v rows (1600), cross layers: q rows only (960) */
   const void* wo;   /* tk_pack_bf16_weight of [720, 960] */
@@ -581,6 +583,7 @@ typedef struct tk_sv_denoise_args {
   const int *pos, *pos0;            /* int32 [M]: rotary positions of the self and of the cross layers (clamped) */
   const float *rope_cos, *rope_sin; /* fp32 [positions, 32] */
   int positions;
+  int polls;                    /* bound of every wait between the blocks: 0 TK_DENOISE_POLLS, negative not one poll */
   const float *emb_w, *emb_b;   /* folded first linear of the suffix embedding: fp32 [720, 32], [steps, 720]; SiLU follows */
   const float *time_w, *time_b; /* its second linear: fp32 [720, 720], [720] */
   const float *act_w, *act_b;   /* action projection: fp32 [32, 720], [32] or NULL */
@@ -591,8 +594,8 @@ typedef struct tk_sv_denoise_args {
 } tk_sv_denoise_args;
 size_t tk_sv_denoise_xchg_bytes(int layers);
 /* `args` is a host structure, read before the call returns.  The launch needs one free compute unit per block (256
- * blocks: TK_EINVAL on a smaller device) and waits between its blocks, each wait bounded by tk_set_handoff_spin(): if
- * other work keeps blocks from running that long, the launch ends with NaNs in `out` and the caller falls back to the
+ * blocks: TK_EINVAL on a smaller device) and waits between its blocks, each wait bounded by args->polls: if other
+ * work keeps blocks from running that long, the launch ends with NaNs in `out` and the caller falls back to the
  * separate launches. */
 int tk_sv_denoise(const tk_sv_denoise_args* args, void* stream);
 
@@ -621,6 +624,7 @@ typedef struct tk_pi_denoise_args {
   const int* pos;  /* int32 [M] (clamped) */
   const float *rope_cos, *rope_sin; /* fp32 [positions, 128]; bf16 arithmetic */
   int positions;
+  int polls;                  /* as in tk_sv_denoise_args */
   const float *emb_w, *emb_b; /* fp32 [1024, 32], [1024] */
   const float* act_w;         /* fp32 [32, 1024] */
   const float* mods;

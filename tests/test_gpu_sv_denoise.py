@@ -59,17 +59,31 @@ def test_one_launch_matches_the_launches_per_layer(model, m, p):
 
 @torch.inference_mode()
 def test_a_run_whose_waits_give_up_ends_with_nans_and_leaves_nothing_behind(model):
-    # forced from the host: with a bound of zero polls no wave waits; every block still runs to its end
+    # forced from the host: without a single poll no wave waits; every block still runs to its end
     case = _case(model, 50, 65)
     want = _run(model, *case)
-    prev = tk.set_handoff_spin(0)
+    model.denoise_plan.polls = -1
     try:
         lost = _run(model, *case)
         torch.cuda.synchronize()
     finally:
-        tk.set_handoff_spin(prev)
+        model.denoise_plan.polls = 0
     assert torch.isnan(lost).any()
     assert torch.equal(_run(model, *case), want)
+
+
+@torch.inference_mode()
+def test_the_single_launch_ffns_bound_is_not_the_loops(model):
+    # the process-wide bound of the single-launch feed-forward says nothing about this launch
+    case = _case(model, 50, 65)
+    want = _run(model, *case)
+    prev = tk.set_handoff_spin(0)
+    try:
+        got = _run(model, *case)
+        torch.cuda.synchronize()
+    finally:
+        tk.set_handoff_spin(prev)
+    assert torch.equal(got, want)
 
 
 def test_engine_repeats_a_starved_request_layer_by_layer(tmp_path, monkeypatch):

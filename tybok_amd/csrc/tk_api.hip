@@ -1478,6 +1478,8 @@ int tk_sv_denoise_pack(const tk_sv_weights* w, int layer, void* blob, size_t blo
   return TK_OK;
 }
 
+static int denoise_polls(int polls) { return polls == 0 ? TK_DENOISE_POLLS : polls < 0 ? 0 : polls; }
+
 int tk_sv_denoise(const tk_sv_denoise_args* h, void* stream) {
   static_assert(kSvMaxLayers == TK_SV_MAX_LAYERS, "the public and the internal layer limits agree");
   if (!h) return fail(TK_EINVAL, "sv_denoise: null argument");
@@ -1529,7 +1531,7 @@ int tk_sv_denoise(const tk_sv_denoise_args* h, void* stream) {
   a.act_b = h->act_b;
   a.blob = (const uint8_t*)h->blob;
   a.xchg = h->xchg;
-  a.spin = g_handoff_spin.load(std::memory_order_relaxed);
+  a.spin = denoise_polls(h->polls);
   if (tk_launch_sv_denoise(a, (hipStream_t)stream)) return fail(TK_ELAUNCH, "sv_denoise: launch failed");
   return TK_OK;
 }
@@ -1579,7 +1581,7 @@ int tk_pi_denoise(const tk_pi_denoise_args* h, void* stream) {
   a.mods = h->mods;
   a.blob = (const uint8_t*)h->blob;
   a.xchg = h->xchg;
-  a.spin = g_handoff_spin.load(std::memory_order_relaxed);
+  a.spin = denoise_polls(h->polls);
   if (tk_launch_pi_denoise(a, (hipStream_t)stream)) return fail(TK_ELAUNCH, "pi_denoise: launch failed");
   return TK_OK;
 }

@@ -184,7 +184,7 @@ class SvDenoiseArgs(ctypes.Structure):
         ("cross_mask", ctypes.c_uint),
         *((n, c_float) for n in ("dt", "eps")),
         *((n, c_void_p) for n in ("x0", "out", "pad", "pos", "pos0", "rope_cos", "rope_sin")),
-        ("positions", c_int),
+        *((n, c_int) for n in ("positions", "polls")),
         *((n, c_void_p) for n in ("emb_w", "emb_b", "time_w", "time_b", "act_w", "act_b", "blob", "xchg")),
         ("xchg_bytes", c_size_t),
         ("cache", SvCache * SV_MAX_LAYERS),
@@ -207,7 +207,7 @@ class PiDenoiseArgs(ctypes.Structure):
         *((n, c_int) for n in ("layers", "steps", "M", "P")),
         *((n, c_float) for n in ("dt", "eps")),
         *((n, c_void_p) for n in ("x0", "out", "pad", "pos", "rope_cos", "rope_sin")),
-        ("positions", c_int),
+        *((n, c_int) for n in ("positions", "polls")),
         *((n, c_void_p) for n in ("emb_w", "emb_b", "act_w", "mods", "blob", "xchg")),
         ("xchg_bytes", c_size_t),
         ("cache", PiCache * PI_MAX_LAYERS),

@@ -254,7 +254,8 @@ def set_ffn_fusion(on: bool) -> bool:
 
 
 def set_handoff_spin(polls: int) -> int:
-    """Bound (polls) of the wait inside the single-launch FFN; returns the previous value."""
+    """Bound (polls) of the wait inside the single-launch FFN, process-wide; returns the previous value.  (The denoising
+    launches have a bound of their own, per plan: :attr:`SvDenoisePlan.polls`.)"""
     return int(native.lib().tk_set_handoff_spin(int(polls)))
 
 
@@ -975,6 +976,7 @@ class SvDenoisePlan:
 
     HIDDEN, HEADS, KV_HEADS, HEAD_DIM, FFN, ACTION = 720, 15, 5, 64, 2048, 32
     MAX_TOKENS, MAX_TILES = 64, 16
+    polls = 0  # bound of every wait inside the launch: 0 the library's default (about 0.1 s), negative not one poll
 
     def __init__(self, layers, *, time_w, time_b, act_w, act_b, norm_out, emb_w, rope: RopeTables, eps: float, device):
         e, f = self.HIDDEN, self.FFN
@@ -1044,7 +1046,7 @@ class SvDenoisePlan:
             c.k, c.vt = k.data_ptr(), vt.data_ptr()
             c.k_sl, c.k_sh, c.vt_sh, c.vt_sd = k.stride(0), k.stride(1), vt.stride(0), vt.stride(1)
         out = torch.empty_like(x0)
-        a.steps, a.M, a.P, a.dt = int(steps), m, p, float(dt)
+        a.steps, a.M, a.P, a.dt, a.polls = int(steps), m, p, float(dt), int(self.polls)
         a.x0, a.out, a.pad, a.pos, a.pos0, a.emb_b = x0.data_ptr(), out.data_ptr(), pad.data_ptr(), pos.data_ptr(), pos0.data_ptr(), emb_b.data_ptr()
         _launch_alone(lambda: native.check(native.lib().tk_sv_denoise(ctypes.addressof(a), _stream()), "tk_sv_denoise"), x0.device)
         return out
@@ -1071,6 +1073,7 @@ class PiDenoisePlan:
 
     HIDDEN, HEADS, KV_HEADS, HEAD_DIM, FFN, ACTION = 1024, 8, 1, 256, 4096, 32
     MAX_TOKENS, MAX_TILES = 64, 40
+    polls = 0  # as in SvDenoisePlan
 
     def __init__(self, layers, *, act_w, act_b, emb_w, emb_b, rope: RopeTables, eps: float, device):
         e, f, d, nq = self.HIDDEN, self.FFN, self.HEAD_DIM, self.HEADS * self.HEAD_DIM
@@ -1153,7 +1156,7 @@ class PiDenoisePlan:
                 raise ValueError("prefix caches must be bf16 [P, 1, 256] keys and [1, 256, >= P rounded up to 32] values")
             c.k, c.vt, c.k_sl, c.vt_sd = k.data_ptr(), vt.data_ptr(), k.stride(0), vt.stride(1)
         out = torch.empty_like(x0)
-        a.steps, a.M, a.P, a.dt = self._steps, m, p, float(dt)
+        a.steps, a.M, a.P, a.dt, a.polls = self._steps, m, p, float(dt), int(self.polls)
         a.x0, a.out, a.pad, a.pos, a.mods = x0.data_ptr(), out.data_ptr(), pad.data_ptr(), pos.data_ptr(), self._mods.data_ptr()
         _launch_alone(lambda: native.check(native.lib().tk_pi_denoise(ctypes.addressof(a), _stream()), "tk_pi_denoise"), x0.device)
         return out
