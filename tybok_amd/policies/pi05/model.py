@@ -104,9 +104,9 @@ class PI05Model:
         self.head_dim = self.vd["head_dim"]
         mlp_keys = tuple(f".mlp.{p}_proj.weight" for p in ("gate", "up", "down"))
         self.p = {k: v.to(self.device) for k, v in state_dict.items() if not k.endswith(mlp_keys)}
-        self.vlm_mlp = [GatedMLP(state_dict, f"{VLM}layers.{i}.mlp.", self.device, self.fp8_llm_mlp, act="gelu_tanh", w8a8=self.fp8_llm_act) for i in range(self.depth)]
-        self.exp_mlp = [GatedMLP(state_dict, f"{EXP}layers.{i}.mlp.", self.device, self.fp8_expert_mlp, act="gelu_tanh") for i in range(self.ed["depth"])]
-        self.ws = tk.default_workspace(self.device) if self.use_hip else None
+        self.ws = tk.Workspace(self.device) if self.use_hip else None  # the model's own, as in SmolVLAModel
+        self.vlm_mlp = [GatedMLP(state_dict, f"{VLM}layers.{i}.mlp.", self.device, self.fp8_llm_mlp, act="gelu_tanh", w8a8=self.fp8_llm_act, ws=self.ws) for i in range(self.depth)]
+        self.exp_mlp = [GatedMLP(state_dict, f"{EXP}layers.{i}.mlp.", self.device, self.fp8_expert_mlp, act="gelu_tanh", ws=self.ws) for i in range(self.ed["depth"])]
         self.vt_suf = None  # zero-padded V^T of the action tokens, allocated on first use
 
         inv = 1.0 / (10000.0 ** (torch.arange(0, self.head_dim, 2, dtype=torch.int64).float() / self.head_dim))

@@ -68,8 +68,9 @@ def eager_attention(mask: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: tor
 class GatedMLP:
     """gate/up/down of one decoder layer: bf16 torch linears, or fp8 weights on the HIP kernel."""
 
-    def __init__(self, sd: dict, prefix: str, device, fp8: bool, act: str = "silu", w8a8: bool = False):
+    def __init__(self, sd: dict, prefix: str, device, fp8: bool, act: str = "silu", w8a8: bool = False, ws: tk.Workspace | None = None):
         self.act = act
+        self.ws = ws
         self.fp8 = fp8
         self.w8a8 = bool(w8a8) and fp8  # activations quantised per token too (the W8A8 tier)
         names = [prefix + n + ".weight" for n in ("gate_proj", "up_proj", "down_proj")]
@@ -95,7 +96,7 @@ class GatedMLP:
         if self.fp8:
             b, length, hidden = x.shape
             ffn = tk.w8a8_gated_ffn if self.w8a8 else tk.fp8w_gated_ffn
-            y = ffn(x.reshape(b * length, hidden), self.wgu, self.wd, self.act, resid=resid.reshape(b * length, hidden))
+            y = ffn(x.reshape(b * length, hidden), self.wgu, self.wd, self.act, resid=resid.reshape(b * length, hidden), ws=self.ws)
             return y.view(b, length, hidden)
         a = F.silu(F.linear(x, self.wg)) if self.act == "silu" else F.gelu(F.linear(x, self.wg), approximate="tanh")
         out = F.linear(a * F.linear(x, self.wu), self.wdn)
@@ -135,9 +136,11 @@ class SmolVLAModel:
         mlp_keys = tuple(f".mlp.{p}_proj.weight" for p in ("gate", "up", "down"))
         # everything except the MLP weights (owned by GatedMLP, possibly as fp8) moves as is
         self.p = {k: v.to(self.device) for k, v in state_dict.items() if not k.endswith(mlp_keys)}
-        self.vlm_mlp = [GatedMLP(state_dict, f"{TXT}layers.{i}.mlp.", self.device, self.fp8_llm_mlp) for i in range(self.num_layers)]
-        self.exp_mlp = [GatedMLP(state_dict, f"{EXP}layers.{i}.mlp.", self.device, self.fp8_expert_mlp) for i in range(cfg.n_expert_layers)]
-        self.ws = tk.default_workspace(self.device) if self.use_hip else None
+        # the model's own (128 MB): the device's default one would be shared with every other engine of the process, whose
+        # requests may run at the same time on another stream
+        self.ws = tk.Workspace(self.device) if self.use_hip else None
+        self.vlm_mlp = [GatedMLP(state_dict, f"{TXT}layers.{i}.mlp.", self.device, self.fp8_llm_mlp, ws=self.ws) for i in range(self.num_layers)]
+        self.exp_mlp = [GatedMLP(state_dict, f"{EXP}layers.{i}.mlp.", self.device, self.fp8_expert_mlp, ws=self.ws) for i in range(cfg.n_expert_layers)]
         # prefill x step-0 overlap (flow_matching.py:455-531): step-0 expert layer i runs on a second
         # stream as soon as prefill layer i has produced its K/V.  Kernels that may run at the same
         # time must not share split-K partials / counters: the side stream has its own workspace.
