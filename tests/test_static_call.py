@@ -54,3 +54,72 @@ def test_store_owned_copies_only_new_objects():
     call.forget_owned("state")
     call.store_owned(state=t)
     assert torch.equal(call.inputs["state"], t)
+
+
+class _Stream:
+    device_index = 0
+
+    def __init__(self, log, name):
+        self.log, self.name = log, name
+
+    def wait_event(self, event):
+        self.log.append((self.name, "waits for", event.at))
+
+
+class _Event:
+    at = None
+
+    def record(self, stream):
+        self.at = (stream.name, len(stream.log))
+        stream.log.append((stream.name, "done", self.at))
+
+
+def test_turns_wait_for_the_last_grid_and_for_nothing_behind_it(monkeypatch):
+    from tybok_amd import graph
+
+    log: list = []
+    a, b = _Stream(log, "a"), _Stream(log, "b")
+    current = [a]
+    monkeypatch.setattr(graph, "_turn_done", {})
+    monkeypatch.setattr(torch.cuda, "Event", _Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: current[0])
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    graph.launch_alone(lambda: log.append(("a", "grid")), "cuda")
+    log.append(("a", "unrelated work"))
+    current[0] = b
+    graph.launch_alone(lambda: log.append(("b", "grid")), "cuda")
+    first = ("a", 2)
+    assert log == [("a", "waits for", None), ("a", "grid"), ("a", "done", first), ("a", "unrelated work"),
+                   ("b", "waits for", first), ("b", "grid"), ("b", "done", ("b", 6))]  # fmt: skip
+
+
+def test_only_a_recording_that_holds_such_a_grid_takes_turns(monkeypatch):
+    from tybok_amd import graph
+
+    class Session:  # records nothing: runs the body as a capture would
+        def prime_and_capture(self, fn):
+            fn()
+            return type("Graph", (), {"replay": lambda self: None})()
+
+    turns: list = []
+
+    @graph.contextmanager
+    def turn(device=None):
+        turns.append(device)
+        yield
+
+    monkeypatch.setattr(graph, "launch_turn", turn)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: None)
+    plain = StaticCall(torch.zeros(1), x=torch.ones(1)).record(Session(), lambda x: x)
+    plain.replay()
+    assert turns == [] and not plain.takes_turn
+
+    def body(x):
+        graph.launch_alone(lambda: None, "cuda")
+        return x
+
+    loop = StaticCall(torch.zeros(1), x=torch.ones(1)).record(Session(), body)
+    assert turns == [] and loop.takes_turn
+    loop.replay()
+    assert turns == [torch.device("cpu")]

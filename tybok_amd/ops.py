@@ -13,7 +13,7 @@ from dataclasses import dataclass
 import torch
 
 from . import native
-from .graph import launch_turn
+from .graph import launch_alone
 
 ACT = {"silu": 0, "gelu_tanh": 1}
 MASK_NONE, MASK_BIDIR, MASK_CAUSAL = 0, 1, 2
@@ -955,15 +955,6 @@ def expert_tail(
     return v, x_new
 
 
-def _launch_alone(launch, device) -> None:
-    """Launch a grid whose blocks wait for each other (a recorded one takes its turn when it is replayed)."""
-    if torch.cuda.is_current_stream_capturing():
-        launch()
-    else:
-        with launch_turn(device):
-            launch()
-
-
 DENOISE_MAX_STEPS = 1000  # Euler steps of one denoising launch
 
 
@@ -1048,7 +1039,7 @@ class SvDenoisePlan:
         out = torch.empty_like(x0)
         a.steps, a.M, a.P, a.dt, a.polls = int(steps), m, p, float(dt), int(self.polls)
         a.x0, a.out, a.pad, a.pos, a.pos0, a.emb_b = x0.data_ptr(), out.data_ptr(), pad.data_ptr(), pos.data_ptr(), pos0.data_ptr(), emb_b.data_ptr()
-        _launch_alone(lambda: native.check(native.lib().tk_sv_denoise(ctypes.addressof(a), _stream()), "tk_sv_denoise"), x0.device)
+        launch_alone(lambda: native.check(native.lib().tk_sv_denoise(ctypes.addressof(a), _stream()), "tk_sv_denoise"), x0.device)
         return out
 
 
@@ -1158,7 +1149,7 @@ class PiDenoisePlan:
         out = torch.empty_like(x0)
         a.steps, a.M, a.P, a.dt, a.polls = self._steps, m, p, float(dt), int(self.polls)
         a.x0, a.out, a.pad, a.pos, a.mods = x0.data_ptr(), out.data_ptr(), pad.data_ptr(), pos.data_ptr(), self._mods.data_ptr()
-        _launch_alone(lambda: native.check(native.lib().tk_pi_denoise(ctypes.addressof(a), _stream()), "tk_pi_denoise"), x0.device)
+        launch_alone(lambda: native.check(native.lib().tk_pi_denoise(ctypes.addressof(a), _stream()), "tk_pi_denoise"), x0.device)
         return out
 
 
