@@ -1,8 +1,12 @@
 """Host logic of the recorded-call inputs (``tybok_amd.graph.StaticCall``): no GPU, no recording."""
+import contextlib
+import gc
+import weakref
+
 import pytest
 import torch
 
-from tybok_amd.graph import StaticCall
+from tybok_amd.graph import CaptureSession, GraphRunner, StaticCall
 
 
 def _call():
@@ -123,3 +127,57 @@ def test_only_a_recording_that_holds_such_a_grid_takes_turns(monkeypatch):
     assert turns == [] and loop.takes_turn
     loop.replay()
     assert turns == [torch.device("cpu")]
+
+
+class _Cycle:
+    def __init__(self, on_death):
+        self.me = self
+        weakref.finalize(self, on_death)
+
+
+def test_nothing_is_garbage_collected_while_a_graph_is_recorded(monkeypatch):
+    # a dead graph in a reference cycle (an engine that was replaced) would be destroyed inside the recording
+    recording, died_inside = [False], []
+
+    @contextlib.contextmanager
+    def graph(recorded):
+        recording[0] = True
+        yield
+        recording[0] = False
+
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", object)
+    monkeypatch.setattr(torch.cuda, "graph", graph)
+    before = gc.get_threshold()
+    gc.set_threshold(1, 1, 1)
+
+    def body():
+        for _ in range(50):
+            _Cycle(lambda: died_inside.append(recording[0]))
+
+    try:
+        CaptureSession("cpu").capture(body)
+        assert gc.isenabled()
+    finally:
+        gc.set_threshold(*before)
+    gc.collect()
+    assert len(died_inside) == 50 and not any(died_inside)
+
+
+def test_a_dropped_engine_is_freed_at_once():
+    class Engine:
+        def __init__(self):
+            self.runner = GraphRunner(self._record, "cpu")
+
+        def _record(self, key, request):
+            return (key, request)
+
+    engine = Engine()
+    assert engine.runner.entry("a", 1) == ("a", 1) and engine.runner.precapture(["b"]) and engine.runner.entry("b") == ("b", None)
+    assert GraphRunner(lambda key, request: key, "cpu").entry("c") == "c"
+    gone = weakref.ref(engine)
+    gc.disable()
+    try:
+        del engine
+        assert gone() is None
+    finally:
+        gc.enable()
