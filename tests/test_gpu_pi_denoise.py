@@ -91,6 +91,46 @@ def test_the_single_launch_ffns_bound_is_not_the_loops(model):
     assert torch.equal(got, want)
 
 
+def _request():
+    _, _, inp = cases.pi05_build(cases.PI05_CASES["small"])
+    return [[t.cuda() for t in inp["images"]], [t.cuda() for t in inp["img_masks"]], inp["lang_tokens"].cuda(), inp["lang_masks"].cuda(), *[inp["noise"].cuda()]]
+
+
+def _layer_by_layer(model, args):
+    model.persistent_loop = False
+    try:
+        return model.sample_actions(*args)
+    finally:
+        model.persistent_loop = True
+
+
+@torch.inference_mode()
+def test_a_starved_loop_of_the_model_runs_again_layer_by_layer(model, monkeypatch):
+    args = _request()
+    want = _layer_by_layer(model, args)
+    asked = []
+    monkeypatch.setattr(model.denoise_plan, "run", lambda x0, *a: asked.append(1) or torch.full_like(x0, float("nan")))
+    assert torch.equal(model.sample_actions(*args), want) and asked == [1]
+
+
+@torch.inference_mode()
+def test_a_graph_of_somebody_else_holds_the_launches_per_layer(model, monkeypatch):
+    # (its replays would not take turns with other loops, and nobody would look for NaNs)
+    from tybok_amd.graph import CaptureSession
+
+    args = _request()
+    want = _layer_by_layer(model, args)
+    session, out = CaptureSession("cuda"), []
+    session.prime(lambda: model.sample_actions(*args))
+    monkeypatch.setattr(model.denoise_plan, "run", lambda *a: pytest.fail("the graph holds the persistent loop"))
+    graph = session.capture(lambda: out.append(model.sample_actions(*args)))
+    for _ in range(3):
+        out[0].zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out[0], want)
+
+
 def test_bad_arguments_are_refused(model):
     x, caches, pad, pos = _case(model, 50, 65)
     with pytest.raises(ValueError):

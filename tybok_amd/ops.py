@@ -13,7 +13,7 @@ from dataclasses import dataclass
 import torch
 
 from . import native
-from .graph import launch_alone
+from .graph import launch_alone, replays_take_turns
 
 ACT = {"silu": 0, "gelu_tanh": 1}
 MASK_NONE, MASK_BIDIR, MASK_CAUSAL = 0, 1, 2
@@ -956,6 +956,17 @@ def expert_tail(
 
 
 DENOISE_MAX_STEPS = 1000  # Euler steps of one denoising launch
+
+
+def one_launch_allowed() -> bool:
+    """Whether the denoising loop may run as one launch here: always, but for a graph somebody else records, whose
+    replays would neither take turns nor be looked at for the NaNs of a starved launch."""
+    return not torch.cuda.is_current_stream_capturing() or replays_take_turns()
+
+
+def loop_answered(out: torch.Tensor) -> bool:
+    """Whether a denoising launch was not starved of compute units (waits for the device; a recording cannot look)."""
+    return torch.cuda.is_current_stream_capturing() or not bool(torch.isnan(out).any())
 
 
 class SvDenoisePlan:

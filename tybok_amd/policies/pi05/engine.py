@@ -338,8 +338,9 @@ class PI05Engine(ChunkRuntime, PolicyEngine):
         return self._mask_cache[key]
 
     def _core(self, images01, img_masks, tokens, masks, noise) -> torch.Tensor:
-        """The unit a graph records: the change of range of the images and the whole model."""
-        return self.model.sample_actions(images01, img_masks, tokens, masks, noise, image_range01=True)
+        """The unit a graph records: the change of range of the images and the whole model (a starved loop is the
+        request's to repeat)."""
+        return self.model.sample_actions(images01, img_masks, tokens, masks, noise, image_range01=True, unchecked=True)
 
     def _infer(self, batch: dict[str, torch.Tensor], noise: torch.Tensor | None) -> torch.Tensor:
         images, img_masks = self.prepare_images01(batch)

@@ -620,9 +620,13 @@ class PI05Model:
         out, _ = gemma_norm(hidden, modulation=self.final_mods[step])
         return self.lin("action_out_proj", out.to(torch.float32))
 
-    def sample_actions(self, images, img_masks, tokens, masks, noise, trace: dict | None = None, image_range01: bool = False) -> torch.Tensor:
+    def sample_actions(
+        self, images, img_masks, tokens, masks, noise, trace: dict | None = None, image_range01: bool = False, unchecked: bool = False
+    ) -> torch.Tensor:
         """Prefix embed, prefill, Euler loop -> ``[1, chunk, max_action_dim]`` fp32.  ``image_range01``: the images are
-        still in [0, 1] (``x * 2 - 1`` is applied here, inside the unfolding launch where that is possible)."""
+        still in [0, 1] (``x * 2 - 1`` is applied here, inside the unfolding launch where that is possible).  A loop that
+        runs as one launch and is starved of compute units by other work answers NaNs; it is then run again layer by
+        layer, which takes a look at the result and so waits for the device.  ``unchecked``: the caller does both itself."""
         capturing = self.device.type == "cuda" and torch.cuda.is_current_stream_capturing()
         if self.pad_free and not capturing:
             tokens, masks = self.pack_language(tokens, masks)  # (a recorded shape already has the bucket's length)
@@ -657,8 +661,10 @@ class PI05Model:
                 self.vt_suf = torch.zeros(kv[0][0].shape[1], self.head_dim, (s + 31) // 32 * 32, dtype=BF16, device=self.device)
             # clamp(sum(pad) + arange(s)): from the prefill's bookkeeping launch, or a launch of its own
             pos32 = suf_pos if suf_pos is not None else tk.prefix_meta(pads[0].contiguous(), None, _ROPE_POSITIONS, s, want_mask=False)[2]
-            if self.persistent_loop and tk.PiDenoisePlan.covers(s, pads.shape[1], self.num_steps):
-                return self.denoise_plan.run(x_t[0], dt, caches, pads[0], pos32)[None]
+            if self.persistent_loop and tk.PiDenoisePlan.covers(s, pads.shape[1], self.num_steps) and tk.one_launch_allowed():
+                out = self.denoise_plan.run(x_t[0], dt, caches, pads[0], pos32)[None]
+                if unchecked or tk.loop_answered(out):
+                    return out
             # (`action_in_proj` stays the library's fp32 product + cast, two launches a step: carried in the tail launch
             # of the step before -- tk_expert_tail_embed -- it sums its 32 terms in another order, and that re-draw of
             # a few bf16 roundings moved one frame's maximum error from under to over the cap held for this path)

@@ -299,8 +299,8 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
         return self._to_model_range(images01), masks
 
     def _core(self, images01, img_masks, lang_tokens, lang_masks, state, noise) -> torch.Tensor:
-        """The unit a graph records: input scaling and the whole model."""
-        return self.model.sample_actions(images01, img_masks, lang_tokens, lang_masks, state, noise, image_range01=True)
+        """The unit a graph records: input scaling and the whole model (a starved loop is the request's to repeat)."""
+        return self.model.sample_actions(images01, img_masks, lang_tokens, lang_masks, state, noise, image_range01=True, unchecked=True)
 
     def prepare_state(self, batch: dict[str, torch.Tensor]) -> torch.Tensor:
         state = batch[OBS_STATE]
