@@ -348,7 +348,7 @@ class PI05Engine(ChunkRuntime, PolicyEngine):
         if self.pad_free:
             # the language block on the bucket grid, for the eager path and the recorded shapes alike
             tokens, masks = self.model.pack_language(tokens, masks)
-        if self.graph_enabled and self._graph_runner:
+        if self._replays():
             entry = self._graph_runner.entry((len(images), int(tokens.shape[1])))
             return self._run_graph(entry, images, img_masks, tokens, masks, noise)
         noise = self._sample_noise() if noise is None else self._pad_noise(noise)

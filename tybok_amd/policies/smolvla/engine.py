@@ -311,7 +311,7 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
     def _infer(self, batch: dict[str, torch.Tensor], noise: torch.Tensor | None) -> torch.Tensor:
         images, img_masks = self.prepare_images01(batch)
         tokens, lang_masks = batch[OBS_LANGUAGE_TOKENS], batch[OBS_LANGUAGE_ATTENTION_MASK]
-        if self.graph_enabled and self._graph_runner:
+        if self._replays():
             entry = None
             try:
                 entry = self._graph_runner.entry((len(images),))
