@@ -90,3 +90,12 @@ def test_a_request_that_is_itself_nan_says_nothing_about_the_loop(served):
     engine, frame, noise, _, _ = served
     assert np.isnan(engine.predict_action_chunk(frame, noise=noise * float("nan"))).any()
     assert engine.model.persistent_loop and engine._loop_rest == 0
+
+
+def test_validate_repeats_a_starved_chunk(starved, tmp_path):
+    engine, frame, _, _, _ = starved
+    zeros = torch.zeros(1, 50, engine.config.max_action_dim)
+    chunk = torch.from_numpy(_layer_by_layer(engine, frame, zeros))[None]
+    torch.save(frame, tmp_path / "frame.pt")
+    torch.save({"chunk_post": chunk}, tmp_path / "chunk.pt")
+    assert engine.validate(str(tmp_path))["chunk_post.max"] == 0.0

@@ -270,7 +270,7 @@ class PI05Engine(ChunkRuntime, PolicyEngine):
             if dump["denoise"] is not None:
                 x_t = torch.zeros(1, cfg.chunk_size, cfg.max_action_dim, device=self.device)
                 report.compare("denoise.v_t", m.velocity_at(pads, kv, x_t, 0.5), dump["denoise"]["v_t"])
-        chunk = self._infer(batch, torch.zeros(1, cfg.chunk_size, cfg.max_action_dim, device=self.device))[:, :, : cfg.action_feature_shape[0]]
+        chunk = self._answer(batch, torch.zeros(1, cfg.chunk_size, cfg.max_action_dim, device=self.device))[0]
         if "chunk" in dump["chunk"]:
             report.compare("chunk", chunk, dump["chunk"]["chunk"].reshape(chunk.shape))
         post = self.unnormalizer.unnormalize(chunk, ACTION, "ACTION")

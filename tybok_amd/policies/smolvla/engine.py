@@ -214,7 +214,7 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
                 te = sinusoidal_time_embedding(torch.tensor([0.5]), cfg.expert_hidden_size, cfg.min_period, cfg.max_period)
                 v_t = m.denoise_step(pads, keys, values, m.expert_prefix_kv(keys, values), x_t, te.float().to(self.device))
                 report.compare("denoise.v_t", v_t, dump["denoise"]["v_t"])
-        chunk = self._infer(batch, torch.zeros(1, cfg.chunk_size, cfg.max_action_dim, device=self.device))[:, :, : cfg.action_feature_shape[0]]
+        chunk = self._answer(batch, torch.zeros(1, cfg.chunk_size, cfg.max_action_dim, device=self.device))[0]
         if "chunk" in dump["chunk"]:
             report.compare("chunk", chunk, dump["chunk"]["chunk"].reshape(chunk.shape))
         post = self.unnormalizer.unnormalize(chunk, ACTION, "ACTION")
