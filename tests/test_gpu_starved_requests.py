@@ -10,15 +10,15 @@ pytestmark = pytest.mark.gpu
 ALL = dict(tl_fused_expert=True, tl_fp8_expert_mlp=True, tl_fp8_llm_mlp=True)
 
 
-def _engine(name, tmp_path, graph):
+def _engine(name, tmp_path, graph, **kw):
     from tybok_amd.policies.synthetic import write_pi05_checkpoint, write_smolvla_checkpoint
     from tybok_amd.registry import create_engine
 
     if name == "smolvla":
         ckpt = write_smolvla_checkpoint(str(tmp_path), cameras=1, seed=5, num_vlm_layers=2, vision_layers=1, num_steps=2)
-        return create_engine(ckpt, device="cuda", graph=graph, warmup=False, seed=3, tl_llm_fused_attn=True, **ALL)
+        return create_engine(ckpt, device="cuda", graph=graph, warmup=False, seed=3, tl_llm_fused_attn=True, **ALL, **kw)
     ckpt = write_pi05_checkpoint(str(tmp_path), cameras=1, seed=5, depth=2, vision_layers=1, num_steps=2)
-    return create_engine(ckpt, device="cuda", graph=graph, warmup=False, seed=3, tl_llm_flash_attn=True, pad_free=True, **ALL)
+    return create_engine(ckpt, device="cuda", graph=graph, warmup=False, seed=3, tl_llm_flash_attn=True, pad_free=True, **ALL, **kw)
 
 
 @pytest.fixture(params=[(n, g) for n in ("smolvla", "pi05") for g in (False, True)], ids=lambda p: f"{p[0]}-{'graph' if p[1] else 'eager'}", scope="module")
@@ -99,3 +99,20 @@ def test_validate_repeats_a_starved_chunk(starved, tmp_path):
     torch.save(frame, tmp_path / "frame.pt")
     torch.save({"chunk_post": chunk}, tmp_path / "chunk.pt")
     assert engine.validate(str(tmp_path))["chunk_post.max"] == 0.0
+
+
+def test_the_loop_can_be_switched_off(served, tmp_path):
+    # for a GPU that other processes work on as well: recorded shapes follow, outside a request
+    engine, frame, noise, loop, layers = served
+    turns = lambda: {call.takes_turn for call in engine._graph_runner._shapes.values()}  # noqa: E731
+    recorded = set() if not engine.graph_enabled else {False}
+    for on, want, takes in ((False, layers, recorded), (True, loop, {not r for r in recorded})):
+        engine.set_persistent_loop(on)
+        assert turns() == takes
+        for _ in range(3):
+            assert np.array_equal(engine.predict_action_chunk(frame, noise=noise), want)
+    name = "smolvla" if "smolvla" in type(engine).__module__ else "pi05"
+    without = _engine(name, tmp_path, engine.graph_requested, persistent_loop=False)
+    assert without.model.denoise_plan is None and np.array_equal(without.predict_action_chunk(frame, noise=noise), layers)
+    with pytest.raises(ValueError):
+        without.set_persistent_loop(True)

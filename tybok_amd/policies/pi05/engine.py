@@ -20,6 +20,8 @@ flags wired to the HIP kernels:
                           (tybok/policies/pi05/engine.py:510-541,612-630; flow_matching.py:725-760)
 * ``skip_empty_images``   eager path only: a masked-out camera slot behind a real one skips the vision tower and
                           contributes zero rows (flow_matching.py:415-437); inert under ``graph``, as in the reference
+* ``persistent_loop``     ``False`` keeps the denoising loop on one launch per phase: for a GPU that other processes
+                          work on as well (no counterpart in the reference)
 
 ``compile_model`` and Real-Time Chunking are not implemented here and are rejected when requested.
 """
@@ -117,6 +119,7 @@ class PI05Engine(ChunkRuntime, PolicyEngine):
         camera_alias: dict[str, str] | None = None,
         tokenizer_dir: str | None = None,
         rtc_config: dict | None = None,
+        persistent_loop: bool = True,
         **kwargs: Any,
     ):
         super().__init__(checkpoint_dir, device=device)
@@ -177,6 +180,7 @@ class PI05Engine(ChunkRuntime, PolicyEngine):
             self.config, sd, self.device,
             fused_expert=self.tl_fused_expert, fp8_expert_mlp=self.tl_fp8_expert_mlp, fp8_llm_mlp=self.tl_fp8_llm_mlp, fp8_llm_act=self.fp8_llm_act,
             fused_prefill=bool(tl_llm_flash_attn), vit_mlp_dtype=self.vit_mlp_dtype, vit_lowp_attn=self.tl_fused_vit,
+            persistent_loop=persistent_loop,
         )  # fmt: skip
         del sd
 

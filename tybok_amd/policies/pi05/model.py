@@ -80,6 +80,7 @@ class PI05Model:
         fused_prefill: bool = False,
         vit_mlp_dtype: torch.dtype | None = None,
         vit_lowp_attn: bool = False,
+        persistent_loop: bool = True,
     ):
         self.cfg = cfg
         self.vit_mlp_dtype = vit_mlp_dtype
@@ -189,7 +190,7 @@ class PI05Model:
                 self.vis_dense = {n: (tk.pack_bf16_weight(w), b.contiguous()) for n, (w, b) in self.vis_lowp.items()}
         # the whole Euler loop as one persistent launch (None: the launches per layer); a request that finds it starved of
         # compute units by other work is repeated with it off
-        self.denoise_plan = self._denoise_plan()
+        self.denoise_plan = self._denoise_plan() if persistent_loop else None
         self.persistent_loop = self.denoise_plan is not None
         self.set_num_steps(cfg.num_steps)
 

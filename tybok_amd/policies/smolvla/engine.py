@@ -13,7 +13,8 @@ gateway need no change.  The tier flags select the HIP kernels:
 
 The reference's SmolVLA backend rejects the two fp8 flags (engine.py:47-55); here they are
 implemented, because the fp8 action-inference path is what this backend is for.
-``compile_model`` has no implementation here and is rejected when requested.
+``persistent_loop=False`` (no counterpart in the reference) keeps the denoising loop on one launch per phase: for a
+GPU that other processes work on as well.  ``compile_model`` has no implementation here and is rejected when requested.
 """
 
 from __future__ import annotations
@@ -93,6 +94,7 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
         tl_fused_expert: bool = False,
         tl_fp8_llm_mlp: bool = False,
         tl_fp8_expert_mlp: bool = False,
+        persistent_loop: bool = True,
     ):
         super().__init__(checkpoint_dir, device=device)
         if sampler not in ("euler", "heun"):
@@ -150,6 +152,7 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
             fused_prefill=self.tl_llm_fused_attn, fused_vit=self.tl_vit_oproj,
             # graph mode only, like the reference (smolvla/engine.py:229-237); needs both fused tiers
             overlap=bool(overlap) and bool(graph) and sampler == "euler" and str(self.device).startswith("cuda"),
+            persistent_loop=persistent_loop,
         )  # fmt: skip
         del sd
 

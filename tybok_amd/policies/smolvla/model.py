@@ -117,6 +117,7 @@ class SmolVLAModel:
         fused_prefill: bool = False,
         fused_vit: bool = False,
         overlap: bool = False,
+        persistent_loop: bool = True,
     ):
         assert cfg.vlm_config is not None
         self.cfg = cfg
@@ -186,7 +187,7 @@ class SmolVLAModel:
         self.set_num_steps(cfg.num_steps)
         # the whole Euler loop as one persistent launch (None: the launches per layer); a request that finds it starved of
         # compute units by other work is repeated with it off
-        self.denoise_plan = self._denoise_plan()
+        self.denoise_plan = self._denoise_plan() if persistent_loop else None
         self.persistent_loop = self.denoise_plan is not None
         v = cfg.vlm_config.vision_config
         side = v.image_size // v.patch_size
