@@ -154,9 +154,10 @@ def test_full_model_bf16_path_matches_reference_golden():
 
 
 def test_overlapped_step0_equals_sequential_bit_for_bit():
-    # prefill x step-0 overlap on two streams without a graph: same kernels, same inputs, same bits
+    # prefill x step-0 overlap on two streams without a graph: same kernels, same inputs, same bits.  (A loop that is one
+    # persistent launch has no step to overlap.)
     cfg, sd, inp = cases.smolvla_build(cases.SMOLVLA_CASES["small"])
-    tiers = dict(fused_expert=True, fp8_expert_mlp=True, fp8_llm_mlp=True, fused_prefill=True)
+    tiers = dict(fused_expert=True, fp8_expert_mlp=True, fp8_llm_mlp=True, fused_prefill=True, persistent_loop=False)
     seq = _gpu_chunk(cfg, sd, inp, **tiers)
     for _ in range(2):
         assert torch.equal(seq, _gpu_chunk(cfg, sd, inp, overlap=True, **tiers))
@@ -169,16 +170,19 @@ def ckpt(tmp_path_factory):
     return write_smolvla_checkpoint(str(tmp_path_factory.mktemp("smolvla_ckpt")), cameras=3, seed=5, num_vlm_layers=4, vision_layers=2, num_steps=3)
 
 
-def test_engine_api_graph_equals_eager_and_camera_keys(ckpt):
+@pytest.mark.parametrize("loop", [True, False], ids=["one-launch", "per-layer"])
+def test_engine_api_graph_equals_eager_and_camera_keys(ckpt, loop):
     from tybok_amd.registry import create_engine
 
     flags = dict(tl_fused_expert=True, tl_fp8_expert_mlp=True, tl_fp8_llm_mlp=True, tl_llm_fused_attn=True, tl_vit_oproj=True)
+    flags["persistent_loop"] = loop
     eager = create_engine(ckpt, device="cuda", graph=False, warmup=False, **flags)
     graph = create_engine(ckpt, device="cuda", graph=True, graph_cameras=(2, 3), warmup=True, seed=3, overlap=True, **flags)
     assert graph.graph_enabled and sorted(graph._graph_runner.keys()) == [(2,), (3,)]
-    # graph mode hides step 0 inside the prefill on a second stream; the eager engine is sequential:
-    # the comparisons below are therefore also overlapped == sequential, bit for bit
-    assert graph.overlap and not eager.overlap
+    # with the loop layer by layer, graph mode hides step 0 inside the prefill on a second stream; the eager engine is
+    # sequential: the comparisons below are then also overlapped == sequential, bit for bit.  A loop that is one launch
+    # overlaps nothing, and the engine says so.
+    assert graph.overlap == (not loop) and not eager.overlap
     spec = eager.describe()
     assert spec == {"model_type": "smolvla", "cameras": ["camera1", "camera2", "camera3"], "resize": [512, 512], "action_dim": 6, "chunk_size": 50}
     noise = torch.zeros(1, 50, 6)
@@ -199,6 +203,20 @@ def test_engine_api_graph_equals_eager_and_camera_keys(ckpt):
     c1 = graph.predict_action_chunk(frame)
     c2 = graph.predict_action_chunk(frame)
     assert not np.array_equal(c1, c2)
+
+
+def test_the_overlapped_path_is_the_one_that_overlap_takes(monkeypatch):
+    from tybok_amd.policies.smolvla.model import SmolVLAModel
+
+    cfg, sd, inp = cases.smolvla_build(cases.SMOLVLA_CASES["small"])
+    tiers = dict(fused_expert=True, fp8_expert_mlp=True, fp8_llm_mlp=True, fused_prefill=True, overlap=True)
+    taken = []
+    overlapped = SmolVLAModel._sample_actions_overlapped
+    monkeypatch.setattr(SmolVLAModel, "_sample_actions_overlapped", lambda self, *a: taken.append(1) or overlapped(self, *a))
+    _gpu_chunk(cfg, sd, inp, **tiers)
+    assert taken == []
+    _gpu_chunk(cfg, sd, inp, persistent_loop=False, **tiers)
+    assert taken == [1]
 
 
 def test_graph_requests_with_changing_task_noise_and_host_inputs(ckpt):

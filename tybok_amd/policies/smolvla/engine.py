@@ -165,13 +165,21 @@ class SmolVLAEngine(ChunkRuntime, PolicyEngine):
         self._token_cache: dict[str, tuple[torch.Tensor, torch.Tensor]] = {}
         self._mask_cache: dict[tuple[int, bool], torch.Tensor] = {}
         self._init_graphs(graph, "smolvla graph", log)
-        self.overlap = self.model.overlap  # step 0 of the Euler loop hidden inside the prefill (two streams)
+        if self.model.overlap and not self.overlap:
+            log.info("overlap requested: the denoising loop runs as one launch, which takes less time than nine overlapped steps; requests run sequentially")
         self._graph_fallback_warned = False
         cameras = len(self.config.image_features)
         keys = [(n,) for n in camera_counts(graph_cameras, default=cameras, max_images=cameras)]
         self._start(warmup=warmup, graph_keys=keys, profile=profile, logger=log)
 
     # ------------------------------------------------------------------ API
+    @property
+    def overlap(self) -> bool:
+        """Whether requests hide step 0 of the Euler loop inside the prefill (two streams): asked for, and their loop is
+        not one persistent launch."""
+        prefix = self._prefix_len_for(len(self.config.image_features))
+        return self.model.overlap and not self.model.runs_as_one_launch(int(self.config.chunk_size), prefix)
+
     def describe(self) -> dict[str, Any]:
         return {
             "model_type": "smolvla",

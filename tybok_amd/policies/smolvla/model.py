@@ -763,13 +763,18 @@ class SmolVLAModel:
                 x_t = self.fused_euler_step(pads, caches, x_t, step, positions, dt, h=h)
         return x_t
 
+    def runs_as_one_launch(self, tokens: int, prefix: int) -> bool:
+        """Whether the denoising loop of a request of that shape is one persistent launch."""
+        euler = getattr(self.cfg, "sampler", "euler") == "euler"
+        return euler and self.persistent_loop and tk.SvDenoisePlan.covers(tokens, prefix, self.num_steps)
+
     def sample_actions_core(self, embs, pads, att, noise, trace: dict | None = None, unchecked: bool = False) -> torch.Tensor:
         euler = getattr(self.cfg, "sampler", "euler") == "euler"
         # the loop as one launch: also where step 0 was asked to overlap the prefill (all ten steps of it take less time
         # than nine of the other path's)
         one_launch = (
-            euler and self.persistent_loop and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous()
-            and tk.SvDenoisePlan.covers(noise.shape[1], embs.shape[1], self.num_steps) and tk.one_launch_allowed()
+            self.runs_as_one_launch(noise.shape[1], embs.shape[1]) and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous()
+            and tk.one_launch_allowed()
         )  # fmt: skip
         if self.overlap and euler and not one_launch and trace is None and embs.shape[0] == 1 and noise.shape[0] == 1 and noise.dtype == torch.float32 and noise.is_contiguous():
             return self._sample_actions_overlapped(embs, pads, att, noise)
