@@ -177,6 +177,7 @@ def test_full_depth_zero_noise_chunk_against_oracle_and_noise_floor():
         )
         assert torch.isfinite(got).all()
         assert d_mean <= 1.15 * floor_mean and d_max <= 1.5 * floor_max
+        assert d_mean <= 0.55 * floor_mean  # the loop's fp32 residual rows, logits and rotation: 0.78e-3 .. 0.86e-3, 0.39 .. 0.42 of the floor
         assert e_mean <= 1.15 * self_mean and e_max <= 1.5 * self_max
         assert e_max <= 1.25e-2 and e_mean <= 3e-3
         maxima.append(e_max)

@@ -27,17 +27,29 @@ def model():
     return m
 
 
-def _case(model, m, p):
+def _case(model, m, p, with_kv=False):
     g = torch.Generator().manual_seed(1000 * m + p)
     depth = model.ed["depth"]
     kv = [tuple(torch.randn(1, 1, p, 256, generator=g).to(torch.bfloat16).cuda() for _ in range(2)) for _ in range(depth)]
     pad = torch.rand(1, p, generator=g).cuda() > 0.2
     pos = (int(pad.sum()) + torch.arange(m)).to(torch.int32).cuda()
-    return torch.randn(m, 32, generator=g).cuda(), model.attention_caches(kv), pad, pos
+    x, caches = torch.randn(m, 32, generator=g).cuda(), model.attention_caches(kv)
+    return (x, kv, caches, pad, pos) if with_kv else (x, caches, pad, pos)
 
 
 def _run(model, x, caches, pad, pos):
     return model.denoise_plan.run(x, -1.0 / model.num_steps, caches, pad[0], pos)
+
+
+def _layer_by_layer_loop(model, x, caches, pad, pos):
+    model.vt_suf = torch.zeros(1, 256, (x.shape[0] + 31) // 32 * 32, dtype=torch.bfloat16, device="cuda")
+    for step in range(model.num_steps):
+        hidden = model.lin("action_in_proj", x).to(torch.bfloat16)
+        hidden = model._denoise_layers_fused(pad, caches, hidden, pos, step)
+        _, x = tk.expert_tail(
+            hidden, model.p["action_out_proj.weight"], model.p["action_out_proj.bias"], ada=model.final_split[step], eps=1e-6, x_t=x, dt=-1.0 / model.num_steps
+        )
+    return x
 
 
 # rows: one row group, a full one, one more row, two and a bit, all four; keys: a single one and fewer tiles than splits
@@ -46,20 +58,37 @@ def _run(model, x, caches, pad, pos):
 @torch.inference_mode()
 def test_one_launch_matches_the_launches_per_layer(model, m, p):
     x, caches, pad, pos = _case(model, m, p)
-    model.vt_suf = torch.zeros(1, 256, (m + 31) // 32 * 32, dtype=torch.bfloat16, device="cuda")
-    want = x
-    for step in range(model.num_steps):
-        hidden = model.lin("action_in_proj", want).to(torch.bfloat16)
-        hidden = model._denoise_layers_fused(pad, caches, hidden, pos, step)
-        _, want = tk.expert_tail(
-            hidden, model.p["action_out_proj.weight"], model.p["action_out_proj.bias"], ada=model.final_split[step], eps=1e-6, x_t=want, dt=-1.0 / model.num_steps
-        )
+    want = _layer_by_layer_loop(model, x, caches, pad, pos)
     got = _run(model, x, caches, pad, pos)
     assert torch.isfinite(got).all()
     rel = float((got - want).norm() / (want - x).norm())
     print(f"M={m} P={p}: relative difference of the flow {rel:.3g}")
     assert rel < 2e-2  # bf16 rounding: residual rows, logits and rotary products round to bf16 there, fp32 here (3.1e-3 - 3.5e-3)
     assert torch.equal(got, _run(model, x, caches, pad, pos))  # the exchange buffers start clean again
+
+
+@pytest.mark.parametrize("m,p", [(17, 33), (50, 275), (50, 712)])
+@torch.inference_mode()
+def test_one_launch_is_no_less_precise_than_the_launches_per_layer(model, m, p):
+    # both against the same loop with every activation in fp32 (weights as they are, on the CPU)
+    from oracle import pi05 as O
+    from oracle.smolvla import Weights
+
+    cfg, sd, _ = cases.pi05_build(cases.PI05_CASES["small"])
+    shape = O.PI05Shape(depth=model.ed["depth"], num_steps=model.num_steps, chunk=m)
+    w = Weights(sd, O.fp8_linear_names(shape, True, True), act_dtype=torch.float32)
+    x, kv, caches, pad, pos = _case(model, m, p, with_kv=True)
+    kv = [tuple(t.float().cpu() for t in layer) for layer in kv]
+    ref, dt = x.cpu()[None], -1.0 / model.num_steps
+    for step in range(model.num_steps):
+        ref = ref + dt * O.denoise_step(w, shape, pad.cpu(), kv, ref, 1.0 + step * dt)
+    flow = (ref[0] - x.cpu()).norm()
+    runs = _run(model, x, caches, pad, pos), _layer_by_layer_loop(model, x, caches, pad, pos)
+    loop, layers = (float((t.cpu() - ref[0]).norm() / flow) for t in runs)
+    print(f"M={m} P={p}: distance of the flow from the fp32 run: one launch {loop:.3g}, launches per layer {layers:.3g}")
+    # fp32 residual rows, logits and rotation, each bf16 in the launches per layer: measured 0.37 - 0.40 of their distance
+    # (one draw of the same roundings from another moves it by a tenth); with rounded rows alone it would be theirs
+    assert loop <= 0.55 * layers
 
 
 @torch.inference_mode()

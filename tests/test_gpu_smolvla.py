@@ -128,6 +128,7 @@ def test_full_model_zero_noise_chunk_against_oracle_and_noise_floor(cameras):
             )
             assert torch.isfinite(got).all()
             assert d_mean <= 1.15 * floor_mean and d_max <= 1.5 * floor_max
+            assert d_mean <= 0.9 * floor_mean  # the loop's fp32 residual rows: 1.36e-3 .. 1.58e-3, 0.63 .. 0.79 of the floor
             assert e_mean <= 1.15 * self_mean and e_all <= 1.5 * self_max
             assert e_act <= 1.25e-2 and e_all <= 1.5e-2 and e_mean <= 3e-3
             if cameras == 3 and seed == 0:
