@@ -622,7 +622,7 @@ typedef struct tk_pi_denoise_args {
   float* out;
   const void* pad; /* uint8 [P] (1 = valid) or NULL */
   const int* pos;  /* int32 [M] (clamped) */
-  const float *rope_cos, *rope_sin; /* fp32 [positions, 128]; bf16 arithmetic */
+  const float *rope_cos, *rope_sin; /* fp32 [positions, 128]; rotated in fp32, rounded to bf16 once */
   int positions;
   int polls;                  /* as in tk_sv_denoise_args */
   const float *emb_w, *emb_b; /* fp32 [1024, 32], [1024] */

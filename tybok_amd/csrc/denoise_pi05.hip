@@ -4,8 +4,9 @@
 // Bound: latency, then the bytes a compute unit takes in.  A step reads 397 MB of weights (80 us at 5 TB/s) and its
 // eighteen layers are 108 dependent phases of 0.3 - 1.5 us of work each; as five launches a layer they took 47 us a layer.
 // Here 256 resident blocks run the phases back to back: block (rt, c) works on 16 of the chunk's rows with column share c
-// of 64.  Measured (50 action tokens, two cameras and 200 language tokens, 10 steps): the loop 8.5 -> 4.3 ms, 24 us a
-// layer: six hand-offs of 1.3 us or more, 0.4 - 1 us of arithmetic a phase, and 0.8 MB through each compute unit.
+// of 64.  Measured (50 action tokens, two cameras and 200 language tokens, 10 steps): the loop 8.5 -> 4.4 ms, 24 us a
+// layer (stamps of every block, mean): 1.7 - 2.4 us from a phase's result to the next one's input, 3.8 us into PC; from
+// there to the result 0.75 us in PC, 1.0 - 2.1 us in the others; 0.8 MB through each compute unit.
 //
 //   step    E0  v = final_norm(x) . Wa^T + b, x_t += dt v         32 blocks per row group, one action column each
 //           E1  hidden = x_t . Wi^T + b                           64 blocks, 16 columns each
@@ -23,8 +24,8 @@
 // on one XCD: the weights, which are too many for any cache above the XCD's, come there once for four blocks, and a
 // key split for 32.  A row group on two XCDs of its own (hand-offs 0.3 us shorter) took 2 us a layer more.
 // Weights and keys ahead: asked for at the end of the phase one or two hand-offs before theirs, 64 - 128 KiB at a time; by
-// then most waves only wait.  Asked for in the middle of a phase, their issue alone (1 - 2 us: the unit's memory pipe takes
-// 60 B/ns) stands before the phase's result (26 us a layer).  128 registers a wave is what holds them: loads under a
+// then most waves only wait.  Asked for in the middle of a phase, their issue alone stands before the phase's result
+// (26 us a layer).  128 registers a wave is what holds them: loads under a
 // branch, or carried into the next layer under one, were spilled as they arrived (31 us).
 // Keys: one block per head would read 780 KiB; eight splits of at most five tiles of 32 keys keep that at 96 KiB (two
 // cameras).

@@ -4,18 +4,16 @@
 // HAND-OFF.  Every word of an exchange buffer is all-ones (a NaN in bf16 and in fp32) until its producer writes it;
 // consumers load the data itself with device-coherent loads and look at it: a lane that still sees an all-ones word
 // asks again.  No flag, no counter, no cache flush and no wait for store acknowledgements: a hand-off costs one
-// store-to-load trip through the fabric.  Measured with a probe of rounds of this kind (256 blocks of 16 waves, four
-// groups of 64 that exchange 32 KiB among themselves, LDS reduction and barrier included): 1.25 us a round, against
-// 1.9 us with acknowledged stores + flags, and 3 us or more between the first wait of one dependent launch and that
-// of the next.  Buffers come in two sets, used by alternate denoising steps; a block rewrites its words of the idle
+// store-to-load trip through the fabric.  Measured with rounds of this kind alone (256 blocks of 16 waves, four groups of
+// 64 that exchange 32 KiB among themselves, LDS reduction and barrier included): 1.6 us a round with the gate below, 2.4 us
+// without it, 2.35 us with acknowledged stores and a flag per block instead.  Buffers come in two sets, used by alternate denoising steps; a block rewrites its words of the idle
 // set with ones one step after they were read (every path from "written" to "rewritten" runs through data that all
 // readers produced after their reads), so a word is always clean before it is used again.  (The pi0.5 loop keeps a ring
 // of four layers instead: a layer's words are rewritten at the end of the next one and used again two layers later.)
 //
-// GATE.  Loads that come back empty cost the compute unit's memory pipe as much as real ones (its sixteen waves asking
-// for a phase's whole input keep it busy for 0.4 - 1 us), so nobody asks before there is something to expect: every block
-// keeps a progress word (a line of its own, ever growing) and raises it when its input for a phase has ARRIVED, half a
-// microsecond or more before its output leaves; ONE wave of a consumer block watches its producers' words, the others
+// GATE.  Loads that come back empty cost the compute unit's memory pipe as much as real ones, so nobody asks before
+// there is something to expect: every block keeps a progress word (a line of its own, ever growing) and raises it when its
+// input for a phase has ARRIVED, 0.8 - 2.8 us before its output leaves (5 us in the cross layers' attention); ONE wave of a consumer block watches its producers' words, the others
 // wait at the block's barrier, and the first look at the data usually succeeds.
 //
 // EVERY WAIT ENDS: a wave asks at most `spin` times, then marks itself dead, goes on with what it has (ones = NaN)
