@@ -300,6 +300,7 @@ def test_engine_heun_graph_equals_eager(ckpt):
     graph = create_engine(ckpt, device="cuda", graph=True, graph_cameras=(3,), warmup=True, sampler="heun", overlap=True, **flags)
     euler = create_engine(ckpt, device="cuda", graph=False, warmup=False, **flags)
     assert not graph.overlap  # Heun keeps the sequential path
+    assert graph.model.denoise_plan is None  # ... and no second copy of the weights for a launch it does not make
     frame = eager._profile_frame(cameras=3, seed=4)
     noise = torch.zeros(1, 50, 6)
     a = eager.predict_action_chunk(frame, noise=noise)

@@ -971,7 +971,8 @@ def loop_answered(out: torch.Tensor) -> bool:
 
 class SvDenoisePlan:
     """The SmolVLA-shaped expert's weights laid out for :meth:`run`, the flow-matching loop as one persistent launch
-    (``tk_sv_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).
+    (``tk_sv_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).  A second copy of
+    the layers' packed weights, 8.2 MB each, beside the one that the launches per layer read.
 
     ``layers``: one dict per expert layer -- ``wqkv``, ``wo`` (:class:`PackedBf16Weight`), ``wgu``
     (:class:`PackedGateUp`), ``wd`` (:class:`PackedWeight`), ``norm_in``, ``norm_post`` (bf16 ``[720]``), ``cross``."""
@@ -1068,7 +1069,8 @@ def _unpack_fp8_tiles(data: torch.Tensor, n: int, k: int) -> torch.Tensor:
 
 class PiDenoisePlan:
     """The pi0.5 expert's weights laid out for :meth:`run`, the flow-matching loop as one persistent launch
-    (``tk_pi_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).
+    (``tk_pi_denoise``): built once per model, one run at a time (the exchange buffer is the plan's own).  A second copy of
+    the layers' weights, 22 MB each, beside the one that the launches per layer read.
 
     ``layers``: one dict per expert layer -- ``q``, ``k``, ``v``, ``o`` (bf16 matrices), ``wgu`` (:class:`PackedGateUp`),
     ``wd`` (:class:`PackedWeight`)."""

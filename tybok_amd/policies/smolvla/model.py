@@ -187,7 +187,8 @@ class SmolVLAModel:
         self.set_num_steps(cfg.num_steps)
         # the whole Euler loop as one persistent launch (None: the launches per layer); a request that finds it starved of
         # compute units by other work is repeated with it off
-        self.denoise_plan = self._denoise_plan() if persistent_loop else None
+        euler = getattr(cfg, "sampler", "euler") == "euler"  # (Heun steps stay launches per layer)
+        self.denoise_plan = self._denoise_plan() if persistent_loop and euler else None
         self.persistent_loop = self.denoise_plan is not None
         v = cfg.vlm_config.vision_config
         side = v.image_size // v.patch_size
