@@ -593,10 +593,10 @@ typedef struct tk_sv_denoise_args {
   tk_sv_cache cache[TK_SV_MAX_LAYERS];
 } tk_sv_denoise_args;
 size_t tk_sv_denoise_xchg_bytes(int layers);
-/* `args` is a host structure (zeroed before it is filled in: fields may be added), read before the call returns.  The launch needs one free compute unit per block (256
- * blocks: TK_EINVAL on a smaller device) and waits between its blocks, each wait bounded by args->polls: if other
- * work keeps blocks from running that long, the launch ends with NaNs in `out` and the caller falls back to the
- * separate launches. */
+/* `args` is a host structure (zeroed before it is filled in: fields may be added), read before the call returns.  The
+ * launch needs one free compute unit per block (256 blocks: TK_EINVAL on a smaller device) and waits between its blocks,
+ * each wait bounded by args->polls: if other work keeps blocks from running that long, the launch ends with NaNs in `out`
+ * and the caller falls back to the separate launches. */
 int tk_sv_denoise(const tk_sv_denoise_args* args, void* stream);
 
 /* The same for the pi0.5 expert (hidden 1024, 8 query heads of 256 over one K/V head, feed-forward 4096, AdaRMS norms
