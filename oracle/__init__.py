@@ -1,6 +1,6 @@
 """CPU restatement of the reference's fp8 action-inference path (TEST INFRASTRUCTURE ONLY).
 
-This package is the checker, never the product: only ``tests/``, ``__graft_entry__.smoke()``
+This package is the reference of the tests, never the product: only ``tests/``, ``__graft_entry__.smoke()``
 and the ``cpu_baseline`` leg of ``bench.py`` may import it.  Nothing under ``tybok_amd/`` does.
 
 Everything here is plain ``torch`` on the CPU, written from the reference's eager torch path
