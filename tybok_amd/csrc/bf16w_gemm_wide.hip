@@ -374,7 +374,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, in
         if (a.act == 1) v = unpack_16x4<F16>(pack_16x4<F16>(v));  // the linear's 16-bit output, then the activation on it
         if (a.act) {
 #pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_f(v[j]);
+          for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_rcp_f(v[j]);
         }
         *(i32x2*)(wl + l32 * EP + (nt * 32 + 8 * g + 4 * half) * 2) = pack_16x4<F16>(v);
       }

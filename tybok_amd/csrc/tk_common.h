@@ -114,12 +114,19 @@ __device__ __forceinline__ bf16x8 as_bf16x8(i32x4 v) {
 }
 
 __device__ __forceinline__ float silu_f(float x) { return x / (1.0f + __expf(-x)); }
-// gelu(x, approximate="tanh") = 0.5 x (1 + tanh(z)) = x / (1 + exp(-2z)), z = sqrt(2/pi) (x + 0.044715 x^3): the same
-// function through one exponential instead of a tanh expansion, and -2z log2(e) as x (a + b x^2).  v_rcp_f32 in place of
-// the division's ten instructions: an epilogue evaluates it for every output while the matrix pipes wait (the 555-row
-// W8A8 block 109.3 -> 107.9 us, a three-camera SmolVLA request 5.08 -> 5.05 ms).  Against 64 bits over [-12, 12]: largest
-// relative error 8.8e-6 (1.5e-5 with the division: fewer roundings in the exponent), mean 5.6e-8 (6.0e-8).
+// gelu(x, approximate="tanh") = 0.5 x (1 + tanh(z)) = x / (1 + exp(-2z)), z = sqrt(2/pi) (x + 0.044715 x^3):
+// the same function through one exponential instead of a tanh expansion.
 __device__ __forceinline__ float gelu_tanh_f(float x) {
+  const float c0 = 0.7978845608028654f;  // sqrt(2/pi)
+  const float inner = c0 * (x + 0.044715f * x * x * x);
+  return x / (1.0f + __expf(-2.0f * inner));
+}
+// The same with -2z log2(e) as x (a + b x^2) and v_rcp_f32 in place of the division's ten instructions, for epilogues that
+// evaluate it for every output of a one-generation grid while the matrix pipes wait (the 555-row W8A8 block 109.3 -> 107.9 us,
+// a three-camera SmolVLA request 5.08 -> 5.05 ms; pi0.5's weight-only prefill and denoising loop gain nothing and keep the
+// division).  Against 64 bits over [-12, 12]: largest relative error 8.8e-6 (1.5e-5 above: fewer roundings in the
+// exponent), mean 5.6e-8 (6.0e-8).
+__device__ __forceinline__ float gelu_tanh_rcp_f(float x) {
   constexpr float a = -2.302208198144325f;    // -2 sqrt(2/pi) log2(e)
   constexpr float b = -0.10294323958002849f;  // 0.044715 a
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(b, x * x, a)));

@@ -332,7 +332,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w8a8_wide_kernel(GemmArgs a, int
           const f32x4 up = unpack_bf16x4(pack_bf16x4(vu));
           f32x4 act;
 #pragma unroll
-          for (int j = 0; j < 4; ++j) act[j] = a.act == 0 ? silu_f(gg[j]) : gelu_tanh_f(gg[j]);
+          for (int j = 0; j < 4; ++j) act[j] = a.act == 0 ? silu_f(gg[j]) : gelu_tanh_rcp_f(gg[j]);
           act = unpack_bf16x4(pack_bf16x4(act));
           *(i32x2*)(wl + l32 * EP + (8 * g + 4 * half) * 2) = pack_bf16x4(act * up);
         }
@@ -416,7 +416,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void w8a8_wide_kernel(GemmArgs a, int
         const f32x4 up = unpack_bf16x4(pack_bf16x4(vu));
         f32x4 act;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) act[j] = a.act == 0 ? silu_f(gg[j]) : gelu_tanh_f(gg[j]);
+        for (int j = 0; j < 4; ++j) act[j] = a.act == 0 ? silu_f(gg[j]) : gelu_tanh_rcp_f(gg[j]);
         act = unpack_bf16x4(pack_bf16x4(act));
         *(i32x2*)(a.y + (size_t)m * a.ldy + col) = pack_bf16x4(act * up);
       }
