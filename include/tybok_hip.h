@@ -268,8 +268,8 @@ int tk_bf16w_linear(const void* x, int ldx, int x_dtype, const void* w_packed, c
  *          MLP keeps fc1's output in fp32 through the GELU, vision.py:259-273).
  *   resid: optional bf16 or fp32 [M, N] (resid_dtype TK_BF16 / TK_F32), added to the bf16-rounded result.
  *   y:     bf16 [M, N], pitch ldy (a multiple of 8, 16-byte aligned); N a multiple of 4.
- *   tile:  0 = chosen from the shape; 42, 41, 32, 31, 22, 21, 12, 11 = (32-row tiles per block, 32-column tiles per
- *          wave of a 4-wave block).
+ *   tile:  0 = chosen from the shape; 42, 41, 32, 31, 22, 21, 12, 11 = (32-row tiles per block, groups of four 32-column
+ *          tiles); 606, 404, 406, 403, 204, 202 = (32-row tiles, 32-column tiles).
  *   split_k: 0 = automatic; > 1 needs the workspace (fp32 partials, summed in split order: bit-deterministic). */
 int tk_bf16w_dense(const void* x, int ldx, const void* w_packed, const void* bias, int act, void* y, int ldy,
                    const void* resid, int ldr, int resid_dtype, int M, int N, int K, int tile, int split_k, void* ws,

@@ -241,3 +241,52 @@ def test_dense_vt_argument_rules(tk):
         tk.bf16w_dense(x.cuda(), pw, bias.cuda(), vt_out=torch.empty(4, 1, 64, 16, dtype=BF16, device="cuda"), vt_col0=128)
     with pytest.raises(RuntimeError, match="multiple of 64"):
         tk.bf16w_dense(x.cuda(), pw, bias.cuda(), vt_out=torch.empty(2, 1, 96, 32, dtype=BF16, device="cuda"), vt_col0=96)
+
+
+# the block shapes the automatic choice knows besides the ones above
+MORE_TILES = [606, 404, 406, 403, 204, 202]
+
+
+@pytest.mark.parametrize("tile", [0, 42, 41, 32, 31, 22, 21, 12, 11, *MORE_TILES])
+@pytest.mark.parametrize("m,k,n", [(1, 16, 4), (31, 48, 36), (33, 64, 64), (193, 80, 196), (129, 720, 132), (257, 208, 388), (192, 1088, 192)])
+def test_dense_block_edges_exact_on_small_integers(tk, tile, m, k, n):
+    # one row / one past a row tile / one past a block, k ranges that end inside a round of 64 (and, split, on an odd tile
+    # of 32), N % 8 == 4; columns of x behind K hold NaN (a wider buffer) and must not be read into a product.  Integer
+    # operands: exact whatever the order of summation (|sum| < 2^24; the result is rounded once to bf16).
+    g = torch.Generator().manual_seed(m + k)
+    wide = torch.full((m, k + 72), float("nan"), dtype=BF16)
+    wide[:, :k] = torch.randint(-4, 5, (m, k), generator=g).to(BF16)
+    w = torch.randint(-3, 4, (n, k), generator=g).to(BF16)
+    b = torch.randint(-8, 9, (n,), generator=g).to(BF16)
+    r = torch.randint(-16, 17, (m, (n + 15) // 8 * 8), generator=g).to(BF16)
+    x, pw = wide.cuda()[:, :k], tk.pack_bf16_weight(w.cuda())
+    lin = (wide[:, :k].float() @ w.float().t() + b.float()).to(BF16)
+    want = (lin.float() + r[:, :n].float()).to(BF16)
+    for split in [1, 2, 3]:
+        if split > 1 and (k + 31) // 32 < split:
+            continue
+        got = tk.bf16w_dense(x, pw, b.cuda(), tile=tile, split_k=split, resid=r.cuda()[:, :n], out=torch.empty(m, r.shape[1], dtype=BF16, device="cuda")[:, :n])
+        assert torch.equal(got.cpu(), want), f"tile {tile} split {split}"
+    assert torch.equal(tk.bf16w_dense(x, pw, b.cuda(), tile=tile, out=torch.empty(m, r.shape[1], dtype=BF16, device="cuda")[:, :n]).cpu(), lin)
+
+
+@pytest.mark.parametrize("tile", [404, 204])
+@pytest.mark.parametrize("bf16_math", [True, False])
+@pytest.mark.parametrize("m,k,d,heads_rot,heads_v", [(712, 2048, 256, 9, 1), (300, 960, 64, 20, 5), (257, 80, 64, 3, 2), (33, 64, 128, 1, 1), (1, 16, 64, 1, 1)])
+def test_dense_rotary_epilogue_in_more_block_shapes(tk, tile, bf16_math, m, k, d, heads_rot, heads_v):
+    test_dense_with_rotary_epilogue_gives_the_bits_of_the_three_launches(tk, tile, bf16_math, m, k, d, heads_rot, heads_v)
+
+
+@pytest.mark.parametrize("tile", MORE_TILES)
+@pytest.mark.parametrize("dt", [BF16, torch.float16])
+@pytest.mark.parametrize("b,p,k,heads,d", [(3, 1024, 768, 12, 64), (2, 256, 1152, 16, 96), (5, 32, 80, 1, 64)])
+def test_dense_writes_the_transposed_values_in_more_block_shapes(tk, tile, dt, b, p, k, heads, d):
+    test_dense_writes_the_transposed_values_of_a_packed_qkv_projection(tk, tile, dt, b, p, k, heads, d)
+
+
+@pytest.mark.parametrize("tile", MORE_TILES)
+@pytest.mark.parametrize("act", [None, "gelu_tanh", "gelu_tanh_fp32"])
+def test_dense_activation_in_more_block_shapes(tk, tile, act):
+    x, w, b = _case(300, 1152, 648, seed=1)
+    got = tk.bf16w_dense(x.cuda(), tk.pack_bf16_weight(w.cuda()), b.cuda(), act, tile=tile)
+    _close(got, _want(x, w, b, act), f"dense {act} tile={tile}", frac_exact=0.95)

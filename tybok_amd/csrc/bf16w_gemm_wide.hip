@@ -1,4 +1,4 @@
-// bf16-weight GEMM for many rows with bias / GELU / residual epilogues on gfx950: the linears of the vision
+// 16-bit-weight GEMM for many rows with bias / GELU / residual epilogues on gfx950: the linears of the vision
 // towers (q|k|v, out_proj, fc1, fc2 over 256 .. 1024 patches per camera) and the bf16 projections of the VLM
 // prefill.
 //
@@ -6,19 +6,27 @@
 //
 // Operands: x bf16 row-major; W in the 2 KiB tile order of tk_pack_bf16_weight (tile (nt, kt): two 1 KiB chunks,
 // chunk c of lane l = 8 bf16 of column nt*32 + l%32 at k = 32*kt + 16*(l/32) + 8*c), so a weight operand of
-// v_mfma_f32_32x32x16_bf16 is one coalesced 16-byte load per lane straight into registers.
-//   * a block of 4 waves owns MT*32 rows x 4*NT*32 columns and a range of k tiles; wave w owns n tiles
-//     w*NT .. w*NT+NT-1 for all rows;
-//   * the activations of a round (MT*32 rows x 64 columns) are staged once per block through LDS with whole
-//     128-byte lines per row, double buffered, one LDS barrier per round;
-//   * blocks that share weights (same n tiles and k range, different rows) get consecutive slots of ONE XCD, so
-//     a weight tile comes from HBM once and from that XCD's L2 afterwards;
+// v_mfma_f32_32x32x16_bf16 is one coalesced 16-byte load per lane.
+//   * a block owns BM*32 rows x BN*32 columns and a range of k tiles.  Four waves multiply (wave (wm, wn): TM x TN tiles,
+//     one wave a SIMD); four more only load.  Both operands go from memory to LDS without passing through registers, 64
+//     columns of k a round, into a ring of NS buffers, one barrier a round.  Loading waves of their own, because a wave
+//     that both loads and multiplies stands still at every load while the compute unit's memory pipe is busy, with its
+//     matrix instructions behind it: 128 x 128 blocks, 455 ns a round in one wave, 390 in two, and the loads alone
+//     take 350 (32 KiB; 64 KiB of cached data reach a compute unit's LDS in 485 ns, reading them back takes 219 and does
+//     not slow that down, their 16 matrix instructions a SIMD 221);
+//   * x rows land as whole 128-byte lines; the 16-byte chunks of a line are permuted by row on the way in (the lane
+//     picks its global chunk, the LDS slot is fixed by the instruction), so that operand reads of 32 rows touch all banks;
+//   * operands are read one k step (16 columns) ahead of their use; the barrier stands in the middle of a round's last step;
 //   * K splits hand fp32 partials through the workspace; the last-arriving block sums them in split order:
 //     bit-deterministic;
-//   * the epilogue passes each wave's 32-row slices through a private LDS tile and stores 16-byte row segments.
-// Tile shapes (MT, NT) from (4, 2) = 128 x 256, one block per CU, down to (1, 1) = 32 x 128 with four blocks per
-// CU: the host picks the one whose blocks are all resident at once and load the CUs evenly (co-resident blocks
-// overlap each other's first loads and epilogue, a second generation of blocks would pay both again).
+//   * the epilogue passes the block's fp32 sums through LDS and stores 16-byte row segments on all eight waves; what it
+//     reads from memory (bias, residual, rotary positions and table rows) is asked for before the products: 1 - 2 us a
+//     launch against asking behind them (the weights and vectors of a layer are cold in every request).
+// Measured (cold weights, graph replay, us; before: weights straight into the registers of the four waves that multiply):
+// SmolVLA's tower at 3 x 1024 rows q|k|v 22 -> 17.2, out_proj 11.3 -> 9.0, fc1 23.8 -> 21.2, fc2 26.3 -> 19.5; pi0.5's
+// at 2 x 256 rows 14.9 -> 12.6, 9.9 -> 8.6, 13.3 -> 11.7, 20.4 -> 19.4; pi0.5's prefill at 712 rows q|k|v with the
+// rotary epilogue 24.4 -> 14.8, o_proj 14.0 -> 12.6.  A launch of this kind that does nothing takes 1.9 us; what bounds
+// them is a compute unit's 133 bytes/ns of loads (0.35 - 0.6 us a round), then the epilogue (0.2 us per 32 x 32 tile).
 #include "tk_common.h"
 #include "tk_kernels.h"
 
@@ -30,46 +38,65 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-constexpr int NW = 4;  // waves per block
+// 16 bytes per lane from memory (base + voff) to LDS: lane l's land at lds + 16 * l.  Written as assembly so that the
+// compiler does not wait for every such load in front of the next LDS read; load_wait below waits for exactly those that
+// are needed.  Always a scalar base and a 32-bit lane offset: with 64-bit lane addresses these loads and the matrix
+// instructions of the same SIMD hold each other up (64 KiB a compute unit beside 16 matrix instructions a SIMD, which
+// take 220 ns: 690 ns with 64-bit lane addresses, 480 with a scalar base, 485 without any matrix instructions).
+__device__ __forceinline__ void dma16(unsigned voff, const void* base, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
+}
+// at most `rounds` (<= MAXR) rounds of I loads each are still on their way
+template <int I, int MAXR>
+__device__ __forceinline__ void load_wait(int rounds) {
+  if constexpr (MAXR == 0) {
+    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
+  } else {
+    if (rounds >= MAXR) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(MAXR * I) : "memory");
+    else load_wait<I, MAXR - 1>(rounds);
+  }
+}
+
 constexpr int RK = 2;  // k tiles (of 32) per round
 
 // F16: the operands are fp16 (v_mfma_f32_32x32x16_f16) instead of bf16; same tile order, same epilogues
-// ROPE (NT == 2, bf16): the weights are packed in rotary pair order -- the two tiles of a wave hold columns
+// ROPE (TN == 2, bf16): the weights are packed in rotary pair order -- the two tiles of a wave hold columns
 // (c, c + rope_half) of one head -- and the epilogue is the skinny kernel's rotary one: columns < rope_cols rotated
 // by the table row of pos[m] (fp32 products rounded separately, or every product and sum rounded to bf16), columns
 // >= vt_col0 also written transposed for the attention kernel.  No bias, activation or residual in this form.
-template <int MT, int NT, int PF, int OCC, bool F16, bool ROPE = false>
-__global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, int nblk_m, int ngroups) {
-  static_assert(!ROPE || (NT == 2 && !F16), "the rotary epilogue needs both halves of a pair in one wave");
-  constexpr int ROWS = MT * 32;
-  constexpr int ROWB = RK * 64;     // bytes of one staged activation row per round
-  constexpr int PITCH = ROWB + 16;  // conflict-free 16-byte operand reads, 16-byte aligned
-  constexpr int XBUF = ROWS * PITCH;
-  constexpr int PPR = ROWB / 16;    // 16-byte pieces per staged row
-  constexpr int XPT = ROWS * PPR / (NW * 64);
-  constexpr int TILES = MT * NT;
-  static_assert(RK == 2 && PF % 2 == 0, "a round is two phases; buffer parity follows the pipeline slot");
-  // epilogue: each wave's 32 x (NT*32) bf16 slice passes through a private LDS tile in the staging buffers' space
-  constexpr int COLS = NT * 32;      // output columns of a wave per row
-  constexpr int EP = COLS * 2 + 16;  // LDS row pitch (bytes)
-  constexpr int LPR = COLS / 8;      // lanes (16-byte chunks) per row
-  constexpr int RPI = 64 / LPR;      // rows per store instruction
-  constexpr int LDSB = 2 * XBUF > NW * 32 * EP ? 2 * XBUF : NW * 32 * EP;
-  __shared__ __align__(16) unsigned char lds[LDSB];
+template <int BM, int BN, int WGM, int WGN, int NS, int OCC, bool F16, bool ROPE = false>
+__global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel(GemmArgs a, int nblk_m, int ngroups, int by_rows) {
+  constexpr int NW = WGM * WGN;  // multiplying waves; as many more only load
+  constexpr int TM = BM / WGM, TN = BN / WGN;  // tiles of a wave
+  static_assert(BM % WGM == 0 && BN % WGN == 0 && (BM * 4) % NW == 0 && (BN * 4) % NW == 0 && NW == 4, "whole tiles and loads per wave");
+  static_assert(!ROPE || (TN == 2 && !F16), "the rotary epilogue needs both halves of a pair in one wave");
+  constexpr int AI = BM * 4 / NW, WI = BN * 4 / NW;  // loads of a wave per round
+  constexpr int STAGE = (BM + BN) * 4096;
+  constexpr int W_OFF = BM * 4096;
+  constexpr int TILES = TM * TN;
+  constexpr int SP = BN * 128 + 16;  // epilogue: the block's outputs pass through LDS in fp32, row pitch in bytes (16 rows' same column: all banks)
+  constexpr int LDSB = NS * STAGE > BM * 32 * SP ? NS * STAGE : BM * 32 * SP;
+  static_assert(LDSB * OCC <= 160 * 1024 && NS >= 2 && (AI + WI) * (NS - 1) < 64, "LDS of a CU, the load counter's range");
+  __shared__ __align__(1024) unsigned char lds[LDSB];
+  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool loader = wave >= NW;
+  const int lw = wave - NW;  // a loading wave's number
+  const int wm = wave / WGN, wn = wave % WGN;  // a multiplying wave's place
   const int half = lane >> 5;
   const int l32 = lane & 31;
 
-  // slot s of XCD x (blocks are dealt to the 8 XCDs round-robin) -> group (s / nblk_m) * 8 + x, m block
-  // s % nblk_m: the nblk_m blocks of a group (same weights) run back to back on one XCD
-  const unsigned id = blockIdx.x;
-  const unsigned slot = id >> 3;
-  const int mblock = (int)(slot % (unsigned)nblk_m);
-  const int group = (int)((slot / (unsigned)nblk_m) * 8 + (id & 7));
-  if (group >= ngroups) return;
+  // Blocks are dealt to the 8 XCDs round-robin; each XCD takes an eighth of the tiles in a row, so that no XCD has more
+  // to do than another.  The larger operand is the outer index: weights (a group: n tiles and k range) that several
+  // blocks share come from memory once and from one XCD's L2 afterwards, or (by_rows) activations do.
+  const unsigned x8 = blockIdx.x & 7, total = (unsigned)nblk_m * (unsigned)ngroups, each = total >> 3, more8 = total & 7;
+  if ((blockIdx.x >> 3) >= each + (x8 < more8)) return;
+  const unsigned lin = x8 * each + (x8 < more8 ? x8 : more8) + (blockIdx.x >> 3);
+  const int mblock = (int)(by_rows ? lin / (unsigned)ngroups : lin % (unsigned)nblk_m);
+  const int group = (int)(by_rows ? lin % (unsigned)ngroups : lin / (unsigned)nblk_m);
   const int split = group % a.ksplit;
   const int nblk = group / a.ksplit;
 
@@ -78,146 +105,200 @@ __global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, in
   const int nrounds = (kt_hi - kt_lo + RK - 1) / RK;
   const int k_end = kt_hi * 32 < a.K ? kt_hi * 32 : a.K;
 
-  const int strip = nblk * NW + wave;  // this wave's NT packed n tiles
-  const uint8_t* wbase[NT];
+  constexpr int THREADS = 2 * NW * 64, CPR = BN * 4, ITEMS = BM * 32 * CPR / THREADS;  // 16-byte pieces of outputs: per row, per thread
+  constexpr int PRE_MAX = OCC == 1 ? 4 : TILES < 4 ? 2 : 1, PRE = ITEMS < PRE_MAX ? ITEMS : PRE_MAX;  // pieces whose residual is asked for here (128 registers at two blocks a compute unit)
+  static_assert(BM * 32 * CPR % THREADS == 0, "whole pieces");
+  const int m_blk = mblock * BM * 32, n_blk = nblk * BN * 32;
+  constexpr int PPR = ROPE ? BN / 2 * 4 : 1, RITEMS = ROPE ? BM * 32 * PPR / THREADS : 1;  // rotary form: pairs of pieces, per row and per thread
+  static_assert(!ROPE || BM * 32 * PPR % THREADS == 0, "whole pieces");
+  int rope_pos[RITEMS];
+  if (ROPE) {
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    int ntg = strip * NT + nt;
-    if (ntg > a.ntiles - 1) ntg = a.ntiles - 1;  // overhanging tiles are computed on valid data, never stored
-    wbase[nt] = a.w + ((size_t)ntg * a.KT) * 2048 + lane * 16;
+    for (int i = 0; i < RITEMS; ++i) {
+      const int m = m_blk + (i * THREADS + tid) / PPR;
+      rope_pos[i] = a.rope_pos[m < a.M ? m : a.M - 1];
+    }
   }
 
-  const char* xsrc[XPT];
-  int xcol[XPT], xdst[XPT];
+  auto swz = [](int r) { return ((r >> 1) & 3) | (((r & 1) ^ ((r >> 3) & 1)) << 2); };
+  if (loader) {
+    // ---- loads.  x: instruction i of this wave brings rows 8q .. 8q + 7 of the block, q = lw * AI + i; lane l the
+    // 16-byte slot l % 8 of row 8q + l / 8, which holds the line's chunk (l % 8) ^ swz(row) ----
+    const char* xp[AI];  // the eight rows' first column of this block's k range, then on
+    unsigned xv[AI];     // the lane's chunk from there
+    unsigned xfix[2];    // last round: lanes whose chunk is past the k range take the round's first one (zeroed in LDS)
+    const int k_last = (kt_lo + (nrounds - 1) * RK) * 32;
 #pragma unroll
-  for (int i = 0; i < XPT; ++i) {
-    const int p = tid + i * NW * 64;
-    const int r = p / PPR, c = p % PPR;
-    int m = mblock * ROWS + r;
-    if (m > a.M - 1) m = a.M - 1;  // rows past M: valid data, never stored
-    xsrc[i] = (const char*)a.x + (size_t)m * a.ldx * 2;
-    xcol[i] = c * 8;
-    xdst[i] = r * PITCH + c * 16;
-  }
+    for (int i = 0; i < AI; ++i) {
+      const int r0 = mblock * (BM * 32) + 8 * (lw * AI + i), rl = lane >> 3, ch = (lane & 7) ^ swz(8 * (lw * AI + i) + rl);
+      const int b0 = r0 < a.M ? r0 : a.M - 1;  // rows past M: valid data, never stored
+      const int m = r0 + rl < a.M ? r0 + rl : a.M - 1;
+      xp[i] = (const char*)a.x + ((size_t)b0 * a.ldx + kt_lo * 32) * 2;
+      xv[i] = (unsigned)(m - b0) * (unsigned)a.ldx * 2 + ch * 16;
+      if (i < 2) xfix[i] = k_last + ch * 8 < k_end ? 0 : ch * 16;
+    }
+    // W: a round of an n tile is 4 KiB in a row (k tile, chunk); instruction i: 1 KiB of n tile q / 4, q = i * NW + lw
+    const char* wp[WI];
+#pragma unroll
+    for (int i = 0; i < WI; ++i) {
+      int ntg = nblk * BN + (i * NW + lw) / 4;
+      if (ntg > a.ntiles - 1) ntg = a.ntiles - 1;  // overhanging tiles are computed on valid data, never stored
+      wp[i] = (const char*)a.w + ((size_t)ntg * a.KT + kt_lo) * 2048 + (lw & 3) * 1024;
+    }
+    const int w_back = (lw & 2) && kt_lo + nrounds * RK > a.KT ? 2048 : 0;  // last round's second k tile past the matrix: the first one again (its x is zero)
+    const unsigned lane16 = lane * 16;
+    int ibuf = 0;  // LDS offset of the buffer that the next round is loaded into
+    auto xissue = [&](int i, int r) {
+      unsigned v = xv[i];
+      if (r == nrounds - 1) v -= xfix[i & 1];
+      dma16(v, xp[i], lds0 + (unsigned)(ibuf + (lw * AI + i) * 1024));
+      xp[i] += 128;
+    };
+    auto wissue = [&](int i, int r) {
+      const char* p = wp[i] - (r == nrounds - 1 ? w_back : 0);
+      dma16(lane16, p, lds0 + (unsigned)(ibuf + W_OFF + (i * NW + lw) * 1024));
+      wp[i] += 4096;
+    };
+    auto xzero = [&](int buf) {  // the last round's columns past the k range (this wave's rows; behind its load_wait)
+      if (k_last + RK * 32 <= k_end) return;
+#pragma unroll
+      for (int i = 0; i < AI; ++i)
+        if (xfix[i & 1]) *(i32x4*)(lds + buf + (lw * AI + i) * 1024 + lane * 16) = i32x4{0, 0, 0, 0};
+    };
+    auto inext = [&] { ibuf = ibuf + STAGE == NS * STAGE ? 0 : ibuf + STAGE; };
 
-  f32x16 acc[MT][NT];
+    // NS rounds asked for; then, round after round: its own loads are there, so are the other waves' (and every multiplying
+    // wave has left the round before, whose buffer takes round r - 1 + NS)
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int r = 0; r < NS; ++r)
+      if (r < nrounds) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+        for (int i = 0; i < AI; ++i) xissue(i, r);
+#pragma unroll
+        for (int i = 0; i < WI; ++i) wissue(i, r);
+        inext();
+      }
+    int buf = 0;
+    for (int r = 0; r < nrounds; ++r) {
+      const int ahead = nrounds - 1 - r;  // rounds asked for behind this one: at most NS - 2 of them, NS - 1 in the first round
+      if (r == 0) load_wait<AI + WI, NS - 1>(ahead);
+      else load_wait<AI + WI, NS - 2>(ahead);
+      if (r == nrounds - 1) xzero(buf);
+      lds_barrier();
+      if (r > 0 && r - 1 + NS < nrounds) {
+#pragma unroll
+        for (int i = 0; i < AI; ++i) xissue(i, r - 1 + NS);
+#pragma unroll
+        for (int i = 0; i < WI; ++i) wissue(i, r - 1 + NS);
+        inext();
+      }
+      buf = buf + STAGE == NS * STAGE ? 0 : buf + STAGE;
+    }
+  }
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int mt = 0; mt < TM; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < TN; ++nt)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
 
-  struct WFrag {
-    i32x4 w[RK][NT][2];
+  // ---- operand reads: k step s (of four) of a round = k tile s / 2, 16-byte half s % 2 ----
+  i32x4 xa[2][TM], wb[2][TN];
+  int xoff[4];
+#pragma unroll
+  for (int s = 0; s < 4; ++s) xoff[s] = (wm * TM * 32 + l32) * 128 + ((((s >> 1) * 4 + 2 * half + (s & 1)) ^ swz(l32)) << 4);
+  const int woff = W_OFF + wn * TN * 4096 + lane * 16;
+  auto read1 = [&](int set, int s, int buf, int u) {  // u in [0, TM + TN)
+    if (u < TM) xa[set][u] = *(const i32x4*)(lds + buf + xoff[s] + u * 4096);
+    else wb[set][u - TM] = *(const i32x4*)(lds + buf + woff + (u - TM) * 4096 + s * 1024);
   };
-  struct XFrag {
-    i32x4 v[XPT];
-  };
-  // One piece of each kind of work, so that a round can deal them out between its matrix instructions: a wave
-  // cannot issue anything while it waits for the matrix pipe to take its next instruction, so whatever stands
-  // between two groups of matrix instructions in program order runs with the pipe empty.
-  auto wload1 = [&](WFrag& f, int r, int j, int q) {  // q in [0, 2*NT): chunk q%2 of n tile q/2, k tile j of round r
-    int kt = kt_lo + r * RK + j;
-    if (kt > a.KT - 1) kt = a.KT - 1;  // its activation columns are zeroed
-    f.w[j][q / 2][q % 2] = *(const i32x4*)(wbase[q / 2] + (size_t)kt * 2048 + (q % 2) * 1024);
-  };
-  auto xload1 = [&](XFrag& f, int r, int i) {
-    int k = (kt_lo + r * RK) * 32 + xcol[i];
-    if (k > a.K - 8) k = a.K - 8;
-    f.v[i] = *(const i32x4*)(xsrc[i] + (size_t)k * 2);
-  };
-  auto xstore1 = [&](const XFrag& f, int r, int b, int i) {
-    const i32x4 z = {0, 0, 0, 0};
-    *(i32x4*)(lds + b * XBUF + xdst[i]) = ((kt_lo + r * RK) * 32 + xcol[i]) < k_end ? f.v[i] : z;
-  };
-  // operand fragments of the round's two k tiles, as the 16-byte halves (k steps of 16) they are read in
-  i32x4 xa[2][MT][2];
-  auto xread1 = [&](int set, int b, int j, int u) {  // u in [0, 2*MT): k step u%2 of m tile u/2, k tile j
-    xa[set][u / 2][u % 2] = *(const i32x4*)(lds + b * XBUF + ((u / 2) * 32 + l32) * PITCH + (j * 32 + 16 * half) * 2 + 16 * (u % 2));
-  };
-  auto mma1 = [&](int set, const WFrag& f, int j, int t) {  // t in [0, 2*MT*NT): k step, m tile, n tile
-    const int h2 = t / (MT * NT), mt = (t / NT) % MT, nt = t % NT;
+  auto mma1 = [&](int set, int t) {
+    const int mt = t / TN, nt = t % TN;
     if (F16)
-      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(f.w[j][nt][h2]), as_f16x8(xa[set][mt][h2]), acc[mt][nt], 0, 0, 0);
+      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(wb[set][nt]), as_f16x8(xa[set][mt]), acc[mt][nt], 0, 0, 0);
     else
-      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(f.w[j][nt][h2]), as_bf16x8(xa[set][mt][h2]), acc[mt][nt], 0, 0, 0);
+      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(wb[set][nt]), as_bf16x8(xa[set][mt]), acc[mt][nt], 0, 0, 0);
   };
 
-  // PF rounds in flight; every load is unconditional (clamped addresses; columns past the block's k range are
-  // zeroed when staged), so the loop bodies have no branch and the compiler keeps precise wait counts.  Round r,
-  // phase A: multiplies k tile 0 while k tile 1's operands are fetched from LDS, round r+1 is staged into the
-  // other LDS buffer and the weight registers that round r-1's k tile 1 has left are refilled; then the round's
-  // only barrier (a wave can write buffer b for round r+2 only after every wave has passed the barrier of round
-  // r+1, i.e. has its round-r operands in registers); phase B: fetches round r+1's first operands, multiplies k
-  // tile 1 and refills k tile 0's weight registers.  A phase never reloads registers its own matrix instructions
-  // read.  Each of a phase's 2*MT*NT matrix instructions is followed by its share of the other work (piece j of
-  // n goes to slot j * SLOTS / n), fenced so that the order stands.
-  constexpr int SLOTS = 2 * MT * NT;
-  constexpr int HS = SLOTS / 2;  // staging: stores in the first half of phase A's slots, loads in the second
-  WFrag wbuf[PF];
-  XFrag xbuf[PF];
+  // Bias and (16-bit) residual are asked for before the products: behind them they would be a round trip of their own,
+  // to memory that nothing has touched yet
+  i32x2 bias[TN][4];
+  if (!ROPE && a.bias && !loader) {
 #pragma unroll
-  for (int p = 0; p < PF; ++p) {
+    for (int nt = 0; nt < TN; ++nt)
 #pragma unroll
-    for (int i = 0; i < XPT; ++i) xload1(xbuf[p], p, i);
-#pragma unroll
-    for (int q = 0; q < 2 * NT; ++q) {
-      wload1(wbuf[p], p, 0, q);
-      wload1(wbuf[p], p, 1, q);
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < XPT; ++i) xstore1(xbuf[0], 0, 0, i);
-#pragma unroll
-  for (int i = 0; i < XPT; ++i) xload1(xbuf[0], PF, i);
-  lds_barrier();
-#pragma unroll
-  for (int u = 0; u < 2 * MT; ++u) xread1(0, 0, 0, u);
-  auto round = [&](int p, int r) {
-    const int b = p & 1;  // == r & 1: rounds advance PF at a time
-    const int pn = (p + 1) % PF, pp = (p + PF - 1) % PF;
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int i = 0; i < SLOTS; ++i) {
-      mma1(0, wbuf[p], 0, i);
-#pragma unroll
-      for (int u = 0; u < 2 * MT; ++u)
-        if (u * SLOTS / (2 * MT) == i) xread1(1, b, 1, u);
-#pragma unroll
-      for (int x = 0; x < XPT; ++x) {
-        if (x * HS / XPT == i) xstore1(xbuf[pn], r + 1, b ^ 1, x);
-        if (HS + x * HS / XPT == i) xload1(xbuf[pn], r + 1 + PF, x);
+      for (int g = 0; g < 4; ++g) {
+        const int n = n_blk + (wn * TN + nt) * 32 + 8 * g + 4 * half;
+        bias[nt][g] = *(const i32x2*)(a.bias + (n < a.N ? n : a.N - 4));  // columns past N are never stored
       }
+  }
+  i32x2 pre[PRE][2];
+  const bool res16 = !ROPE && a.resid && !a.resid_f32;
+  auto ask_res = [&](i32x2 (&r)[2], int item) {
+    const int idx = item * THREADS + tid, m = m_blk + idx / CPR, n = n_blk + idx % CPR * 8;
+    const u16* p = (const u16*)a.resid + (size_t)(m < a.M ? m : a.M - 1) * a.ldr;  // what lies outside is loaded from inside and not stored
+    r[0] = *(const i32x2*)(p + (n < a.N ? n : a.N - 4));
+    r[1] = *(const i32x2*)(p + (n + 4 < a.N ? n + 4 : a.N - 4));
+  };
+  if (res16 && !loader) {
 #pragma unroll
-      for (int q = 0; q < 2 * NT; ++q)
-        if (q * SLOTS / (2 * NT) == i) wload1(wbuf[pp], r - 1 + PF, 1, q);  // registers round r-1 finished with in its phase B
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    lds_barrier();
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < PRE; ++i) ask_res(pre[i], i);
+  }
+
+  // rotary form: the first pair of pieces' row of the tables as well (the loading waves ask when they have nothing left to load)
+  const int po = ROPE ? a.rope_half >> 5 : 1;
+  auto first_col = [&](int pair) { return ((pair / po) * 2 * po + pair % po) * 32; };  // of a pair of physical tiles (pair, 0 / 1)
+  struct RopeRow {
+    f32x4 cos[2], sin[2];
+  } early;
+  auto ask_rope = [&](RopeRow& t, int i) {
+    const int pc = (i * THREADS + tid) % PPR, ca = first_col(nblk * (BN / 2) + (pc >> 2)) + (pc & 3) * 8;
+    int pos = rope_pos[i];
+    pos = pos < 0 ? 0 : (pos > a.rope_positions - 1 ? a.rope_positions - 1 : pos);
+    const size_t at = (size_t)pos * a.rope_half + ca % (2 * a.rope_half);
 #pragma unroll
-    for (int i = 0; i < SLOTS; ++i) {
-      mma1(1, wbuf[p], 1, i);
-#pragma unroll
-      for (int u = 0; u < 2 * MT; ++u)
-        if (u * SLOTS / (2 * MT) == i) xread1(0, b ^ 1, 0, u);
-#pragma unroll
-      for (int q = 0; q < 2 * NT; ++q)
-        if (q * SLOTS / (2 * NT) == i) wload1(wbuf[p], r + PF, 0, q);  // k tile 0's registers: free since phase A
-      __builtin_amdgcn_sched_barrier(0);
+    for (int q = 0; q < 2; ++q) {
+      t.cos[q] = *(const f32x4*)(a.rope_cos + at + 4 * q);
+      t.sin[q] = *(const f32x4*)(a.rope_sin + at + 4 * q);
     }
   };
-  {
-    int it = 0;
-    for (; it + PF <= nrounds; it += PF) {
+  if (ROPE) ask_rope(early, 0);
+
+  if (!loader) {
+    lds_barrier();
+    int buf = 0;
 #pragma unroll
-      for (int p = 0; p < PF; ++p) round(p, it + p);
+    for (int u = 0; u < TM + TN; ++u) read1(0, 0, 0, u);
+
+    // Round r: k steps 0 .. 2 fetch the next step's operands between their matrix instructions; step 3 meets the other
+    // waves in its middle (round r + 1 is there) and fetches that round's first operands.
+    constexpr int RD = TM + TN, H = (TILES + 1) / 2;
+    for (int r = 0; r < nrounds; ++r) {
+#pragma unroll
+      for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+          mma1(s & 1, t);
+#pragma unroll
+          for (int u = 0; u < RD; ++u)
+            if (u * TILES / RD == t) read1((s + 1) & 1, s + 1, buf, u);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      buf = buf + STAGE == NS * STAGE ? 0 : buf + STAGE;
+#pragma unroll
+      for (int t = 0; t < H; ++t) mma1(1, t);
+      __builtin_amdgcn_sched_barrier(0);
+      if (r + 1 < nrounds) {
+        lds_barrier();
+#pragma unroll
+        for (int u = 0; u < RD; ++u) read1(0, 0, buf, u);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int t = H; t < TILES; ++t) mma1(1, t);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    const int rem = nrounds - it;  // in [0, PF)
-#pragma unroll
-    for (int q = 0; q < PF - 1; ++q)
-      if (q < rem) round(q, it + q);  // block-uniform
   }
 
   // ---- K-split hand-off: fp32 partials [(block, split)][wave][tile][group][lane][4] ----
@@ -225,33 +306,35 @@ __global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, in
   if (a.ksplit > 1) {
     unsigned long long* pbase = (unsigned long long*)a.partial + ((size_t)wave * TILES * 4 * 64 + lane) * 2;
     unsigned long long* mine = pbase + ((size_t)blk_lin * a.ksplit + split) * (NW * TILES * 4 * 64 * 2);
+    if (!loader) {
 #pragma unroll
-    for (int t = 0; t < TILES; ++t)
+      for (int t = 0; t < TILES; ++t)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c = acc[t / NT][t % NT];
-        unsigned long long* dst = mine + (size_t)(t * 4 + g) * 128;
-        st_agent64(dst, c[4 * g], c[4 * g + 1]);
-        st_agent64(dst + 1, c[4 * g + 2], c[4 * g + 3]);
-      }
-    __shared__ int s_last;
+        for (int g = 0; g < 4; ++g) {
+          const f32x16& c = acc[t / TN][t % TN];
+          unsigned long long* dst = mine + (size_t)(t * 4 + g) * 128;
+          st_agent64(dst, c[4 * g], c[4 * g + 1]);
+          st_agent64(dst + 1, c[4 * g + 2], c[4 * g + 3]);
+        }
+    }
+    int* s_last = (int*)lds;  // (the ring is idle behind the barrier)
     handoff_publish();
     __syncthreads();
     if (threadIdx.x == 0) {
       int old = __hip_atomic_fetch_add(a.counters + blk_lin, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      s_last = (old == a.ksplit - 1);
+      *s_last = (old == a.ksplit - 1);
     }
     __syncthreads();
-    if (!s_last) return;
+    if (!*s_last) return;
     handoff_acquire();
     if (threadIdx.x == 0) __hip_atomic_store(a.counters + blk_lin, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+    for (int mt = 0; mt < TM; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
+      for (int nt = 0; nt < TN; ++nt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
-    for (int s = 0; s < a.ksplit; ++s) {  // split order, whoever arrived last
+    for (int s = 0; s < (loader ? 0 : a.ksplit); ++s) {  // split order, whoever arrived last
       const unsigned long long* src = pbase + ((size_t)blk_lin * a.ksplit + s) * (NW * TILES * 4 * 64 * 2);
 #pragma unroll
       for (int t = 0; t < TILES; ++t) {
@@ -263,7 +346,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, in
         }
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-          f32x16& c = acc[t / NT][t % NT];
+          f32x16& c = acc[t / TN][t % TN];
           c[4 * g] += __uint_as_float((unsigned)raw[g][0]);
           c[4 * g + 1] += __uint_as_float((unsigned)(raw[g][0] >> 32));
           c[4 * g + 2] += __uint_as_float((unsigned)raw[g][1]);
@@ -273,37 +356,44 @@ __global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, in
     }
   }
 
-  // ---- epilogue: lane l of a tile owns row m = l % 32 and, per register group g, four consecutive columns
-  // 8g + 4*(l/32) .. +3 (the accumulators hold C^T).  Stored as they are, one instruction would touch 32 rows with
-  // 8 bytes each; each wave therefore passes its 32 rows of an m tile through a private LDS tile (a wave's LDS
-  // instructions execute in order, so it needs no barrier of its own) and stores 16-byte chunks of consecutive
-  // columns: whole row segments of NT*64 bytes per 4*NT lanes. ----
-  lds_barrier();  // every wave has left the staged activations behind
-  unsigned char* wl = lds + wave * 32 * EP;
+  // ---- epilogue: lane l of a tile holds row m = l % 32 and, per register group g, four consecutive columns
+  // 8g + 4*(l/32) .. +3 (the accumulators are C^T).  All of it goes to LDS as fp32 with the bias added; loops over
+  // 16-byte pieces of output rows, on all eight waves, then finish them. ----
+  if (res16 && loader) {
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) ask_res(pre[i], i);
+  }
+  lds_barrier();  // every wave has left the ring (or the partials) behind
+  if (!loader) {
+#pragma unroll
+    for (int mt = 0; mt < TM; ++mt)
+#pragma unroll
+      for (int nt = 0; nt < TN; ++nt)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const f32x16& c = acc[mt][nt];
+          f32x4 v = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
+          if (!ROPE && a.bias) v = v + unpack_16x4<F16>(bias[nt][g]);
+          *(f32x4*)(lds + ((wm * TM + mt) * 32 + l32) * SP + ((wn * TN + nt) * 32 + 8 * g + 4 * half) * 4) = v;
+        }
+  }
+  lds_barrier();
   if constexpr (ROPE) {
-    // logical tile of physical tile (strip, j): (strip / PO) * 2 * PO + strip % PO + j * PO, PO = rope_half / 32
-    const int po = a.rope_half >> 5;
-    const int ca0 = ((strip / po) * 2 * po + strip % po) * 32, cb0 = ca0 + a.rope_half;  // first columns of the two tiles
-    const bool rot = ca0 < a.rope_cols;
-    const int fi0 = ca0 % (2 * a.rope_half) + 4 * half;
-    const int lrow = lane / LPR, lchunk = lane % LPR;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int m0 = (mblock * MT + mt) * 32;
-      int mr = m0 + l32;
-      if (mr > a.M - 1) mr = a.M - 1;
-      int pos = a.rope_pos[mr];
-      pos = pos < 0 ? 0 : (pos > a.rope_positions - 1 ? a.rope_positions - 1 : pos);
-      const float* cs_row = a.rope_cos + (size_t)pos * a.rope_half + fi0;
-      const float* sn_row = a.rope_sin + (size_t)pos * a.rope_half + fi0;
+    for (int i = 0; i < RITEMS; ++i) {
+      const int it = i * THREADS + tid, row = it / PPR, pc = it % PPR, c8 = (pc & 3) * 8;
+      const int m = m_blk + row, ca = first_col(nblk * (BN / 2) + (pc >> 2)) + c8, cb = ca + a.rope_half;
+      RopeRow late;
+      if (i > 0) ask_rope(late, i);
+      const RopeRow& t = i > 0 ? late : early;
+      const unsigned char* src = lds + row * SP + ((pc >> 2) * 64 + c8) * 4;
+      i32x2 oa[2], ob[2];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c0 = acc[mt][0];
-        const f32x16& c1 = acc[mt][1];
-        f32x4 va = unpack_bf16x4(pack_bf16x4(f32x4{c0[4 * g], c0[4 * g + 1], c0[4 * g + 2], c0[4 * g + 3]}));
-        f32x4 vb = unpack_bf16x4(pack_bf16x4(f32x4{c1[4 * g], c1[4 * g + 1], c1[4 * g + 2], c1[4 * g + 3]}));
-        if (rot) {
-          const f32x4 cs = *(const f32x4*)(cs_row + 8 * g), sn = *(const f32x4*)(sn_row + 8 * g);
+      for (int q = 0; q < 2; ++q) {
+        f32x4 va = unpack_bf16x4(pack_bf16x4(*(const f32x4*)(src + 16 * q)));
+        f32x4 vb = unpack_bf16x4(pack_bf16x4(*(const f32x4*)(src + 128 + 16 * q)));
+        if (ca < a.rope_cols) {
+          const f32x4 cs = t.cos[q], sn = t.sin[q];
           f32x4 ra, rb;
           if (a.rope_bf16) {
             const f32x4 ac = unpack_bf16x4(pack_bf16x4(va * cs)), bs = unpack_bf16x4(pack_bf16x4(vb * sn));
@@ -320,149 +410,131 @@ __global__ __launch_bounds__(NW * 64, OCC) void bf16w_wide_kernel(GemmArgs a, in
           va = ra;
           vb = rb;
         }
-        *(i32x2*)(wl + l32 * EP + (8 * g + 4 * half) * 2) = pack_bf16x4(va);
-        *(i32x2*)(wl + l32 * EP + (32 + 8 * g + 4 * half) * 2) = pack_bf16x4(vb);
+        oa[q] = pack_bf16x4(va);
+        ob[q] = pack_bf16x4(vb);
       }
+      if (m >= a.M) continue;
+      u16* dst = a.y + (size_t)m * a.ldy;  // N is a whole number of heads in this form
+      if (ca < a.N) *(i32x4*)(dst + ca) = i32x4{oa[0][0], oa[0][1], oa[1][0], oa[1][1]};
+      if (cb < a.N) *(i32x4*)(dst + cb) = i32x4{ob[0][0], ob[0][1], ob[1][0], ob[1][1]};
+    }
+    if (a.vt) {
+      // value columns, transposed for the attention kernel: eight consecutive rows per 16-byte store, four stores in a
+      // row; rows past M stay zero (the attention kernel relies on zeros behind the last key)
+#pragma unroll 1
+      for (int it = tid; it < BM * 4 * BN * 32; it += THREADS) {
+        const int col = (it >> 2) % (BN * 32), rg = (it / (BN * 128)) * 4 + (it & 3);
+        const int n = first_col(nblk * (BN / 2) + (col >> 6)) + (col & 31) + ((col >> 5) & 1) * a.rope_half;
+        const int m0 = m_blk + 8 * rg;
+        if (n < a.vt_col0 || n >= a.N || m0 >= a.M) continue;
+        i32x4 e;
 #pragma unroll
-      for (int j = 0; j < 32 / RPI; ++j) {
-        const int row = j * RPI + lrow;
-        const int m = m0 + row;
-        const int n = (lchunk < 4 ? ca0 : cb0) + (lchunk & 3) * 8;
-        const i32x4 t = *(const i32x4*)(wl + row * EP + lchunk * 16);
-        if (m >= a.M || n >= a.N) continue;
-        *(i32x4*)(a.y + (size_t)m * a.ldy + n) = t;  // N is a multiple of 64 in this form
-      }
-      if (a.vt && ca0 >= a.vt_col0) {  // wave-uniform: vt_col0 is a multiple of the head size
-        // value columns, transposed for the attention kernel: lane = one of the wave's 64 columns, eight consecutive
-        // rows per 16-byte store; rows past M stay zero (the attention kernel relies on zeros behind the last key)
-        const int n = (lane < 32 ? ca0 : cb0) + (lane & 31);
-        if (n < a.N) {
-          u16* dst = a.vt + (size_t)(n - a.vt_col0) * a.vt_ld + m0;
-#pragma unroll
-          for (int rg = 0; rg < 4; ++rg) {
-            unsigned e[8];
-#pragma unroll
-            for (int r = 0; r < 8; ++r) e[r] = m0 + 8 * rg + r < a.M ? *(const u16*)(wl + (8 * rg + r) * EP + lane * 2) : 0u;
-            if (m0 + 8 * rg < a.M)
-              *(i32x4*)(dst + 8 * rg) = i32x4{(int)(e[0] | (e[1] << 16)), (int)(e[2] | (e[3] << 16)), (int)(e[4] | (e[5] << 16)), (int)(e[6] | (e[7] << 16))};
-          }
+        for (int r = 0; r < 4; ++r) {
+          const float lo = *(const float*)(lds + (8 * rg + 2 * r) * SP + col * 4), hi = *(const float*)(lds + (8 * rg + 2 * r + 1) * SP + col * 4);
+          e[r] = (int)pack_bf16x2(m0 + 2 * r < a.M ? lo : 0.f, m0 + 2 * r + 1 < a.M ? hi : 0.f);
         }
+        *(i32x4*)(a.vt + (size_t)(n - a.vt_col0) * a.vt_ld + m0) = e;
       }
     }
     return;
   }
-  const int ncol0 = strip * COLS;  // first output column of this wave
-  f32x4 bias[NT][4];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      int n0 = ncol0 + nt * 32 + 8 * g + 4 * half;
-      if (n0 > a.N - 4) n0 = a.N - 4;  // columns past N are never stored
-      bias[nt][g] = a.bias ? unpack_16x4<F16>(*(const i32x2*)(a.bias + n0)) : f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int it = 0; it < ITEMS; ++it) {
+    const int idx = it * THREADS + tid, row = idx / CPR, ch = idx % CPR, m = m_blk + row, n = n_blk + ch * 8;
+    const unsigned char* src = lds + row * SP + ch * 32;
+    i32x2 r16[2];
+    i32x4 r32[2];
+    if (it >= PRE && res16) ask_res(r16, it);
+    if (a.resid && a.resid_f32) {
+      const float* p = (const float*)a.resid + (size_t)(m < a.M ? m : a.M - 1) * a.ldr;
+      r32[0] = *(const i32x4*)(p + (n < a.N ? n : a.N - 4));
+      r32[1] = *(const i32x4*)(p + (n + 4 < a.N ? n + 4 : a.N - 4));
     }
-  const int lrow = lane / LPR, lchunk = lane % LPR;
+    i32x2 o[2];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
+    for (int q = 0; q < 2; ++q) {
+      f32x4 v = *(const f32x4*)(src + 16 * q);
+      if (a.act == 1) v = unpack_16x4<F16>(pack_16x4<F16>(v));  // the linear's 16-bit output, then the activation on it
+      if (a.act) {
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c = acc[mt][nt];
-        f32x4 v = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-        v = v + bias[nt][g];
-        if (a.act == 1) v = unpack_16x4<F16>(pack_16x4<F16>(v));  // the linear's 16-bit output, then the activation on it
-        if (a.act) {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_rcp_f(v[j]);
-        }
-        *(i32x2*)(wl + l32 * EP + (nt * 32 + 8 * g + 4 * half) * 2) = pack_16x4<F16>(v);
+        for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_rcp_f(v[j]);
       }
-#pragma unroll
-    for (int j = 0; j < 32 / RPI; ++j) {
-      const int row = j * RPI + lrow;
-      const int m = (mblock * MT + mt) * 32 + row;
-      const int n = ncol0 + lchunk * 8;
-      i32x4 t = *(const i32x4*)(wl + row * EP + lchunk * 16);
-      if (m >= a.M || n >= a.N) continue;
+      o[q] = pack_16x4<F16>(v);
       if (a.resid) {
-        f32x4 r0, r1 = {0.f, 0.f, 0.f, 0.f};
-        if (a.resid_f32) {
-          const f32x4* rp = (const f32x4*)((const float*)a.resid + (size_t)m * a.ldr + n);
-          r0 = rp[0];
-          if (n + 8 <= a.N) r1 = rp[1];
-        } else if (n + 8 <= a.N) {
-          const i32x4 rr = *(const i32x4*)((const u16*)a.resid + (size_t)m * a.ldr + n);
-          r0 = unpack_16x4<F16>(i32x2{rr[0], rr[1]});
-          r1 = unpack_16x4<F16>(i32x2{rr[2], rr[3]});
-        } else {
-          r0 = unpack_16x4<F16>(*(const i32x2*)((const u16*)a.resid + (size_t)m * a.ldr + n));
-        }
-        const i32x2 lo = pack_16x4<F16>(unpack_16x4<F16>(i32x2{t[0], t[1]}) + r0), hi = pack_16x4<F16>(unpack_16x4<F16>(i32x2{t[2], t[3]}) + r1);
-        t = i32x4{lo[0], lo[1], hi[0], hi[1]};
+        const f32x4 r = a.resid_f32 ? f32x4{__int_as_float(r32[q][0]), __int_as_float(r32[q][1]), __int_as_float(r32[q][2]), __int_as_float(r32[q][3])}
+                                    : unpack_16x4<F16>(it < PRE ? pre[it < PRE ? it : 0][q] : r16[q]);
+        o[q] = pack_16x4<F16>(unpack_16x4<F16>(o[q]) + r);
       }
-      u16* dst = a.y + (size_t)m * a.ldy + n;
-      if (n + 8 <= a.N) *(i32x4*)dst = t;
-      else *(i32x2*)dst = i32x2{t[0], t[1]};  // N % 8 == 4: the row's last four columns
     }
-    if (a.vt && ncol0 >= a.vt_col0) {  // wave-uniform: vt_col0 is a multiple of the wave's COLS columns
-      // value columns of a packed q|k|v projection, also written transposed for the attention kernel (no activation
-      // or residual in this form, so the LDS tile holds the final values): a lane takes one of the wave's columns
-      // and eight consecutive rows per 16-byte store.  The rows of an m tile belong to one problem (vt_rows is a
-      // multiple of 32); rows past M are written as zeros.
-      const int ccol = lane % COLS, n = ncol0 + ccol;
-      const int m0 = (mblock * MT + mt) * 32;
-      if (n < a.N && m0 < a.M) {
-        const int prob = a.vt_rows ? m0 / a.vt_rows : 0, key0 = a.vt_rows ? m0 % a.vt_rows : m0;
-        u16* dst = a.vt + (size_t)prob * a.vt_bs + (size_t)(n - a.vt_col0) * a.vt_ld + key0;
+    if (m >= a.M || n >= a.N) continue;
+    u16* dst = a.y + (size_t)m * a.ldy + n;
+    if (n + 8 <= a.N) *(i32x4*)dst = i32x4{o[0][0], o[0][1], o[1][0], o[1][1]};
+    else *(i32x2*)dst = o[0];  // N % 8 == 4: the row's last four columns
+  }
+  if (a.vt && n_blk + BN * 32 > a.vt_col0) {
+    // value columns of a packed q|k|v projection, also written transposed for the attention kernel (no activation or
+    // residual in this form): eight consecutive rows of a column per 16-byte store, four stores in a row.  The rows of
+    // an m tile belong to one problem (vt_rows is a multiple of 32); rows past M are written as zeros.
+#pragma unroll 2
+    for (int it = tid; it < BM * 4 * BN * 32; it += THREADS) {
+      const int col = (it >> 2) % (BN * 32), rg = (it / (BN * 128)) * 4 + (it & 3);
+      const int n = n_blk + col, m0 = m_blk + 8 * rg;
+      if (n < a.vt_col0 || n >= a.N || m0 >= a.M) continue;
+      i32x4 e;
 #pragma unroll
-        for (int rg = lane / COLS; rg < 4; rg += 64 / COLS) {
-          unsigned e[8];
-#pragma unroll
-          for (int r = 0; r < 8; ++r) e[r] = m0 + 8 * rg + r < a.M ? *(const u16*)(wl + (8 * rg + r) * EP + ccol * 2) : 0u;
-          if (m0 + 8 * rg < a.M)
-            *(i32x4*)(dst + 8 * rg) = i32x4{(int)(e[0] | (e[1] << 16)), (int)(e[2] | (e[3] << 16)), (int)(e[4] | (e[5] << 16)), (int)(e[6] | (e[7] << 16))};
-        }
+      for (int r = 0; r < 4; ++r) {
+        const float lo = *(const float*)(lds + (8 * rg + 2 * r) * SP + col * 4), hi = *(const float*)(lds + (8 * rg + 2 * r + 1) * SP + col * 4);
+        const float l = m0 + 2 * r < a.M ? lo : 0.f, h = m0 + 2 * r + 1 < a.M ? hi : 0.f;
+        e[r] = (int)(F16 ? pack_f16x2(l, h) : pack_bf16x2(l, h));
       }
+      const int prob = a.vt_rows ? m0 / a.vt_rows : 0, key0 = a.vt_rows ? m0 % a.vt_rows : m0;
+      *(i32x4*)(a.vt + (size_t)prob * a.vt_bs + (size_t)(n - a.vt_col0) * a.vt_ld + key0) = e;
     }
   }
 }
 
-template <int MT, int NT, int PF, int OCC>
+template <int BM, int BN, int WGM, int WGN, int NS, int OCC, bool ROPE>
 int launch(const GemmArgs& a, hipStream_t st) {
-  const int nblk_m = (a.M + MT * 32 - 1) / (MT * 32);
-  const int nblk_n = (a.ntiles + NW * NT - 1) / (NW * NT);
+  constexpr int NW = WGM * WGN;
+  const int nblk_m = (a.M + BM * 32 - 1) / (BM * 32);
+  const int nblk_n = (a.ntiles + BN - 1) / BN;
   const int ngroups = nblk_n * a.ksplit;
-  const unsigned blocks = (unsigned)((ngroups + 7) / 8) * 8u * (unsigned)nblk_m;
+  const int by_rows = a.M > a.N;
+  const unsigned blocks = ((unsigned)nblk_m * (unsigned)ngroups + 7) / 8 * 8;
   if (a.rope_pos) {
-    if constexpr (NT == 2) {
+    if constexpr (ROPE) {
       if (a.f16) return -1;
-      hipLaunchKernelGGL((bf16w_wide_kernel<MT, NT, PF, OCC, false, true>), dim3(blocks), dim3(NW * 64), 0, st, a, nblk_m, ngroups);
+      hipLaunchKernelGGL((bf16w_wide_kernel<BM, BN, WGM, WGN, NS, OCC, false, true>), dim3(blocks), dim3(2 * NW * 64), 0, st, a, nblk_m, ngroups, by_rows);
       return hipGetLastError() == hipSuccess ? 0 : -3;
     } else {
       return -1;
     }
   }
   if (a.f16)
-    hipLaunchKernelGGL((bf16w_wide_kernel<MT, NT, PF, OCC, true>), dim3(blocks), dim3(NW * 64), 0, st, a, nblk_m, ngroups);
+    hipLaunchKernelGGL((bf16w_wide_kernel<BM, BN, WGM, WGN, NS, OCC, true>), dim3(blocks), dim3(2 * NW * 64), 0, st, a, nblk_m, ngroups, by_rows);
   else
-    hipLaunchKernelGGL((bf16w_wide_kernel<MT, NT, PF, OCC, false>), dim3(blocks), dim3(NW * 64), 0, st, a, nblk_m, ngroups);
+    hipLaunchKernelGGL((bf16w_wide_kernel<BM, BN, WGM, WGN, NS, OCC, false>), dim3(blocks), dim3(2 * NW * 64), 0, st, a, nblk_m, ngroups, by_rows);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
 
 }  // namespace
 
-// tile = 10 * MT + NT
 int tk_launch_bf16w_wide(const GemmArgs& a, int tile, hipStream_t st) {
   switch (tile) {
-    case 42: return launch<4, 2, 4, 1>(a, st);
-    case 41: return launch<4, 1, 2, 2>(a, st);
-    case 32: return launch<3, 2, 2, 2>(a, st);
-    case 31: return launch<3, 1, 2, 3>(a, st);
-    case 22: return launch<2, 2, 2, 2>(a, st);
-    case 21: return launch<2, 1, 2, 4>(a, st);
-    case 12: return launch<1, 2, 2, 3>(a, st);
-    case 11: return launch<1, 1, 2, 4>(a, st);
+    case 42: return launch<4, 8, 1, 4, 3, 1, true>(a, st);
+    case 41: return launch<4, 4, 2, 2, 2, 2, false>(a, st);
+    case 32: return launch<3, 8, 1, 4, 3, 1, true>(a, st);
+    case 31: return launch<3, 4, 1, 4, 5, 1, false>(a, st);
+    case 22: return launch<2, 8, 1, 4, 4, 1, true>(a, st);
+    case 21: return launch<2, 4, 2, 2, 3, 2, false>(a, st);
+    case 12: return launch<1, 8, 1, 4, 4, 1, true>(a, st);
+    case 11: return launch<1, 4, 1, 4, 4, 2, false>(a, st);
+    case 606: return launch<6, 6, 2, 2, 3, 1, false>(a, st);
+    case 404: return launch<4, 4, 2, 2, 4, 1, true>(a, st);
+    case 406: return launch<4, 6, 2, 2, 3, 1, false>(a, st);
+    case 204: return launch<2, 4, 2, 2, 6, 1, true>(a, st);
+    case 202: return launch<2, 2, 2, 2, 5, 2, false>(a, st);
+    case 403: return launch<4, 3, 4, 1, 5, 1, false>(a, st);
   }
   return -1;
 }

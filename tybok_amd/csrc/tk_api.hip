@@ -562,33 +562,30 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
 // ---- bf16-weight linears with bias / GELU / residual epilogues (vision towers) ---------------------------------
 namespace {
 struct DenseTile {
-  int id, rows, cols;
-  int occ;  // blocks of this shape that fit one CU (registers)
+  int id, bm, bn;  // block of 32 bm rows x 32 bn columns
+  int wt, ns;      // 32 x 32 tiles of a multiplying wave, buffers in the ring
+  int occ;         // blocks of this shape that fit one CU (LDS)
+  int rope;        // the rotary form exists
 };
-constexpr DenseTile kDenseTiles[] = {{42, 128, 256, 1}, {41, 128, 128, 2}, {32, 96, 256, 2}, {31, 96, 128, 3},
-                                     {22, 64, 256, 2},  {21, 64, 128, 4},  {12, 32, 256, 3}, {11, 32, 128, 4}};
+constexpr DenseTile kDenseTiles[] = {{42, 4, 8, 8, 3, 1, 1},  {41, 4, 4, 4, 2, 2, 0},  {32, 3, 8, 6, 3, 1, 1},  {31, 3, 4, 3, 5, 1, 0},  {22, 2, 8, 4, 4, 1, 1},
+                                     {21, 2, 4, 2, 3, 2, 0},  {12, 1, 8, 2, 4, 1, 1},  {11, 1, 4, 1, 4, 2, 0},  {606, 6, 6, 9, 3, 1, 0}, {404, 4, 4, 4, 4, 1, 1},
+                                     {406, 4, 6, 6, 3, 1, 0}, {403, 4, 3, 3, 5, 1, 0}, {204, 2, 4, 2, 6, 1, 1}, {202, 2, 2, 1, 5, 2, 0}};
 
-// Estimated duration (us) of a launch with this tile and K split; the constants are fitted to timings of the
-// vision towers' and the prefill's shapes (the picked tile is within 1 % of the best one on average).  Blocks
-// that are resident together share a CU's matrix pipes and overlap each other's first loads and epilogues; every
-// further generation of blocks pays those again.  A wave issues (rows/32) * (cols/128) MFMAs per 16 columns of k
-// (18.8 ns each under full load; 30 / 35 / 45 % of that rate reached with one / two / three or more waves per
-// SIMD), and a block loads (rows + cols) * 128 bytes per 64 columns of k at about 60 KiB/us per CU.
+// Estimated duration (us) of a launch with this tile and K split.  Fitted to 3400 timings (64 shapes of the towers, the
+// prefill and random ones, every tile, splits 1 .. 6; standard error 14 %, the picked launch on average 1.1 % slower than
+// the best one).  Blocks on one CU share its memory pipe (12 ns a KiB) and matrix pipes (75 ns for a wave's tile and
+// round); a round takes no less than the round trip over the rounds on their way; the epilogue costs per tile; each
+// further generation of blocks pays all of it again.
 float dense_cost(const DenseTile& t, int M, int N, int KT, int ks, int cus) {
-  const long long blocks = (long long)((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) * ks;
-  const float kt = (float)((KT + ks - 1) / ks);
-  const float eff = t.occ >= 3 ? 0.45f : t.occ == 2 ? 0.35f : 0.3f;
-  const float mfma_us = (float)(t.rows / 32) * (float)(t.cols / 128) * 2.f * kt * 0.0188f / eff;
-  const float load_us = 0.5f * kt * (float)(t.rows + t.cols) * 0.125f / 60.f;
-  const float tile_us = mfma_us > load_us ? mfma_us : load_us;
-  float us = 0.f;
-  long long left = blocks;
-  while (left > 0) {
-    const long long gen = left < (long long)cus * t.occ ? left : (long long)cus * t.occ;
-    us += 3.f + (float)((gen + cus - 1) / cus) * tile_us;
-    left -= gen;
+  const int rows = 32 * t.bm, cols = 32 * t.bn, rounds = ((KT + ks - 1) / ks + 1) / 2;
+  const long long blocks = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * ks;
+  float us = 1.66f;
+  for (long long left = blocks; left > 0; left -= (long long)cus * t.occ) {
+    const float r = left > cus && t.occ > 1 ? 2.f : 1.f;  // blocks on a CU
+    const float load = r * (float)(t.bm + t.bn) * 4.f * 0.0122f, mul = r * (float)t.wt * 0.0751f, trip = 0.585f / (float)(t.ns - 1);
+    us += 0.014f + (float)rounds * (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip)) + r * (float)(t.bm * t.bn) * 0.203f;
   }
-  if (ks > 1) us += 1.5f + (float)blocks * (float)(t.rows * t.cols) * 8.f / 4e6f;  // fp32 partials out and back in
+  if (ks > 1) us += 4.76f + (float)blocks * (float)(t.bm * t.bn) * 0.00213f;  // fp32 partials out and back in
   return us;
 }
 }  // namespace
@@ -616,6 +613,7 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
                  int f16, const DenseRope* rope = nullptr, const DenseVt* vt = nullptr) {
   if (M <= 0 || N <= 0 || K <= 0) return fail(TK_EINVAL, "bf16w_dense: non-positive shape M=%d N=%d K=%d", M, N, K);
   if (K % 16 || ldx % 8 || ldx < K) return fail(TK_EINVAL, "bf16w_dense: K=%d must be a multiple of 16 and ldx=%d a multiple of 8 >= K", K, ldx);
+  if (M > 1 && ldx > 1 << 28) return fail(TK_EINVAL, "bf16w_dense: ldx=%d, rows of x more than 512 MiB apart", ldx);
   if (!x || !w_packed || !y) return fail(TK_EINVAL, "bf16w_dense: null pointer");
   if (!aligned16(x) || !aligned16(w_packed) || !aligned16(y) || (bias && !aligned8(bias)))
     return fail(TK_EINVAL, "bf16w_dense: x, w_packed and y must be 16-byte aligned, bias 8-byte aligned");
@@ -681,27 +679,18 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
   float best_cost = 0.f;
   for (const DenseTile& t : kDenseTiles) {
     if (tile && t.id != tile) continue;
-    if (rope && t.id % 10 != 2) continue;  // the rotary epilogue needs two n tiles per wave
-    const int blocks0 = ((M + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
-    int k1 = 1;
-    if (split_k > 0) {
-      k1 = split_k;
-    } else if (rope) {
-      // measured at the prefill's q|k|v shape (712 x 2048 -> 2560): 64 x 256 blocks, unsplit, 20.7 us; 32 x 256:
-      // 27.9, 96 x 256: 25.7, 128 x 256: 32.2; any K split 30-39 us (the partials weigh more than the idle CUs)
-      if (!tile && t.id != (M > 32 ? 22 : 12)) continue;
-    } else {
-      // few blocks and a long K: split, keeping at least 32 k tiles per split
-      k1 = cus / blocks0;
-      if (k1 > a.KT / 32) k1 = a.KT / 32;
-      if (k1 < 1) k1 = 1;
+    if (rope && !t.rope) continue;  // the rotary epilogue needs two n tiles per wave
+    // a split keeps at least 16 k tiles; none in the rotary form unless asked for (the partials weigh more than the idle CUs)
+    const int most = split_k > 0 || rope || a.KT < 32 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
+    for (int k1 = split_k > 0 ? split_k : 1, n = 0; n < most; ++k1, ++n) {
+      const float c = dense_cost(t, M, N, a.KT, k1, cus);
+      if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
     }
-    const float c = dense_cost(t, M, N, a.KT, k1, cus);
-    if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
   }
-  if (!best) return fail(TK_EINVAL, "bf16w_dense: tile=%d (0 = automatic, or 42, 41, 32, 31, 22, 21, 12, 11)", tile);
-  const int blocks0 = ((M + best->rows - 1) / best->rows) * ((N + best->cols - 1) / best->cols);
-  const size_t per_split = (size_t)best->rows * best->cols * 4;
+  if (!best) return fail(TK_EINVAL, "bf16w_dense: tile=%d (0 = automatic, or 42, 41, 32, 31, 22, 21, 12, 11, 606, 404, 406, 403, 204, 202; the rotary form: 42, 32, 22, 12, 404, 204)", tile);
+  const int rows = 32 * best->bm, cols = 32 * best->bn;
+  const int blocks0 = ((M + rows - 1) / rows) * ((N + cols - 1) / cols);
+  const size_t per_split = (size_t)rows * cols * 4;
   if (ks > 1) {
     const size_t have = ws && ws_bytes > kPartialOff ? (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes) / (per_split * blocks0) : 0;
     if ((size_t)ks > have || blocks0 > kMaxCounters) {

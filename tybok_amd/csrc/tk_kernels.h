@@ -295,7 +295,7 @@ int tk_launch_pack(const void* w0, const void* w1, void* out, int N, int K, int 
 int tk_launch_pack_bf16(const void* w, void* out, int N, int K, int pair_off, hipStream_t st);
 int tk_launch_fill_zero(int* p, int n, hipStream_t st);
 int tk_launch_decode_fp8(float* out, hipStream_t st);
-// tile = 10 * (m tiles per block) + (n tiles per wave): 42, 41, 32, 31, 22, 21, 12 or 11
+// tile = 10 * (m tiles per block) + (n tiles per block) / 4, or 100 * (m tiles) + (n tiles): one of kDenseTiles (tk_api.hip)
 int tk_launch_bf16w_wide(const GemmArgs& a, int tile, hipStream_t st);
 // plain 16-byte-per-lane read of `bytes` (a multiple of blocks * 4096) by `blocks` blocks of 256 threads
 int tk_launch_stream_read(const void* src, size_t bytes, int blocks, int* sink, hipStream_t st);
