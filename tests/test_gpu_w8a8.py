@@ -144,3 +144,26 @@ def test_w8a8_ffn_matches_oracle(tk, m, k, i, act, mode):
     # with the residual
     got_r = tk.w8a8_gated_ffn(x.cuda(), wgu, wd, act, resid=x.cuda(), ws=ws, mode=mode)
     assert torch.equal(got_r.cpu(), (got.float().cpu() + x.float()).to(BF16))
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 16, 4), (257, 48, 36), (289, 144, 132), (319, 720, 388), (130, 2064, 260)])
+@pytest.mark.parametrize("split", [0, 1, 2, 3])
+def test_w8a8_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
+    # k ranges that end inside a round of 128 (and, split, on any tile of 32), one past a row tile, N % 8 == 4; a8 is a column
+    # slice of a wider buffer of NaN codes.  Integer codes and power-of-two scales: exact whatever the order of summation.
+    if split > 1 and (k + 31) // 32 < split:
+        pytest.skip("fewer k tiles than splits")
+    g = torch.Generator().manual_seed(m + k + n)
+    a = torch.randint(-3, 4, (m, k), generator=g).float()
+    w = torch.randint(-2, 3, (n, k), generator=g).float()
+    wide = torch.full((m, (k + 31) // 16 * 16), 0x7F, dtype=torch.uint8)
+    wide[:, :k] = a.to(torch.float8_e4m3fn).view(torch.uint8)
+    sa = torch.exp2(torch.randint(-2, 3, (m,), generator=g).float())
+    sw = torch.exp2(torch.randint(-2, 3, (n,), generator=g).float())
+    r = torch.randint(-16, 17, (m, n), generator=g).to(BF16)
+    y = ((a @ w.t()) * sa[:, None] * sw[None, :]).to(BF16)
+    want = (y.float() + r.float()).to(BF16)
+    pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), sw.cuda())
+    got = tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split, resid=r.cuda())
+    assert torch.equal(got.cpu(), want)
+    assert torch.equal(tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split).cpu(), y)

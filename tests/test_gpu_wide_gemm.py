@@ -203,3 +203,41 @@ def test_prefill_size_ffn_matches_oracle_and_rows_are_independent(tk):
     assert torch.equal(yp, y[perm]), "rows must not depend on their position in the batch"
     skinny = tk.fp8w_gated_ffn(xc[:64].contiguous(), wgu, wd, "gelu_tanh")
     _close(y[:64], skinny.cpu(), "prefill-size ffn vs skinny kernel rows")
+
+
+@pytest.mark.parametrize("m,k,n", [(257, 16, 4), (256, 48, 36), (289, 80, 132), (319, 720, 388), (385, 1088, 260), (300, 4112, 68)])
+@pytest.mark.parametrize("split", [0, 1, 2, 3])
+def test_many_row_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
+    # one past a row tile or block, k ranges that end inside a round (and, split, on an odd tile of 32), N % 8 == 4; the columns
+    # of x behind K hold NaN (a wider buffer) and must not be read into a product.  Integer codes and power-of-two scales:
+    # every sum is exact in fp32 whatever its order (|sum| < 2^24), the result is rounded once to bf16.
+    if split > 1 and (k + 31) // 32 < split:
+        pytest.skip("fewer k tiles than splits")
+    g = torch.Generator().manual_seed(m + k + n)
+    wide = torch.full((m, k + 72), float("nan"), dtype=BF16)
+    wide[:, :k] = torch.randint(-4, 5, (m, k), generator=g).to(BF16)
+    w = torch.randint(-3, 4, (n, k), generator=g).float()
+    sw = torch.exp2(torch.randint(-2, 3, (n,), generator=g).float())
+    gate = torch.randint(-2, 3, (n,), generator=g).to(BF16)
+    r = torch.randint(-16, 17, (m, n), generator=g).to(BF16)
+    y = ((wide[:, :k].float() @ w.t()) * sw).to(BF16)
+    pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), sw.cuda())
+    got = tk.fp8w_gemm(wide.cuda()[:, :k], pw, split_k=split)  # rows of N % 8 == 4: 8-byte stores
+    assert torch.equal(got.cpu(), y)
+    want = ((y.float() * gate.float()).to(BF16).float() + r.float()).to(BF16)
+    buf = torch.full((m, (n + 15) // 8 * 8), 7.0, dtype=BF16, device="cuda")
+    tk.fp8w_gemm(wide.cuda()[:, :k], pw, split_k=split, gate=gate.cuda(), resid=r.cuda(), out=buf[:, :n])
+    assert torch.equal(buf[:, :n].cpu(), want) and bool((buf[:, n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("m", [256, 257, 288, 321, 385, 500, 700])
+@pytest.mark.parametrize("k,i", [(256, 512), (80, 2560), (2048, 16384)])
+def test_many_row_gated_rows_do_not_depend_on_the_block_shape(tk, m, k, i):
+    # the k tiles of a gated output are added in ascending order in every kernel and block shape of the many-row form, so
+    # a row gives the same bits whatever the number of rows beside it picks
+    x, wg, sg, wu, su, wd, sd = ffn_case(700, k, i)
+    wgu, pd = tk.pack_fp8_gate_up(wg.cuda(), sg.cuda(), wu.cuda(), su.cuda()), tk.pack_fp8_weight(torch.eye(k, i).to(torch.float8_e4m3fn).cuda(), torch.ones(k).cuda())
+    xc = x.cuda()  # (the down projection picks the first k columns of the intermediate: exact, whatever its K split)
+    want = tk.fp8w_gated_ffn(xc, wgu, pd, "gelu_tanh")
+    got = tk.fp8w_gated_ffn(xc[700 - m :].contiguous(), wgu, pd, "gelu_tanh")
+    assert torch.equal(got, want[700 - m :])

@@ -7,16 +7,7 @@
 // Operands: x bf16 row-major; W in the 2 KiB tile order of tk_pack_bf16_weight (tile (nt, kt): two 1 KiB chunks,
 // chunk c of lane l = 8 bf16 of column nt*32 + l%32 at k = 32*kt + 16*(l/32) + 8*c), so a weight operand of
 // v_mfma_f32_32x32x16_bf16 is one coalesced 16-byte load per lane.
-//   * a block owns BM*32 rows x BN*32 columns and a range of k tiles.  Four waves multiply (wave (wm, wn): TM x TN tiles,
-//     one wave a SIMD); four more only load.  Both operands go from memory to LDS without passing through registers, 64
-//     columns of k a round, into a ring of NS buffers, one barrier a round.  Loading waves of their own, because a wave
-//     that both loads and multiplies stands still at every load while the compute unit's memory pipe is busy, with its
-//     matrix instructions behind it: 128 x 128 blocks, 455 ns a round in one wave, 390 in two, and the loads alone
-//     take 350 (32 KiB; 64 KiB of cached data reach a compute unit's LDS in 485 ns, reading them back takes 219 and does
-//     not slow that down, their 16 matrix instructions a SIMD 221);
-//   * x rows land as whole 128-byte lines; the 16-byte chunks of a line are permuted by row on the way in (the lane
-//     picks its global chunk, the LDS slot is fixed by the instruction), so that operand reads of 32 rows touch all banks;
-//   * operands are read one k step (16 columns) ahead of their use; the barrier stands in the middle of a round's last step;
+// The products are those of pipe_gemm.h: loads straight to LDS on waves of their own.
 //   * K splits hand fp32 partials through the workspace; the last-arriving block sums them in split order:
 //     bit-deterministic;
 //   * the epilogue passes the block's fp32 sums through LDS and stores 16-byte row segments on all eight waves; what it
@@ -27,85 +18,36 @@
 // at 2 x 256 rows 14.9 -> 12.6, 9.9 -> 8.6, 13.3 -> 11.7, 20.4 -> 19.4; pi0.5's prefill at 712 rows q|k|v with the
 // rotary epilogue 24.4 -> 14.8, o_proj 14.0 -> 12.6.  A launch of this kind that does nothing takes 1.9 us; what bounds
 // them is a compute unit's 133 bytes/ns of loads (0.35 - 0.6 us a round), then the epilogue (0.2 us per 32 x 32 tile).
-#include "tk_common.h"
-#include "tk_kernels.h"
+#include "pipe_gemm.h"
 
 namespace {
+using namespace pipe;
 
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
-// 16 bytes per lane from memory (base + voff) to LDS: lane l's land at lds + 16 * l.  Written as assembly so that the
-// compiler does not wait for every such load in front of the next LDS read; load_wait below waits for exactly those that
-// are needed.  Always a scalar base and a 32-bit lane offset: with 64-bit lane addresses these loads and the matrix
-// instructions of the same SIMD hold each other up (64 KiB a compute unit beside 16 matrix instructions a SIMD, which
-// take 220 ns: 690 ns with 64-bit lane addresses, 480 with a scalar base, 485 without any matrix instructions).
-__device__ __forceinline__ void dma16(unsigned voff, const void* base, unsigned lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
-}
-// at most `rounds` (<= MAXR) rounds of I loads each are still on their way
-template <int I, int MAXR>
-__device__ __forceinline__ void load_wait(int rounds) {
-  if constexpr (MAXR == 0) {
-    asm volatile("s_waitcnt vmcnt(0)" : : : "memory");
-  } else {
-    if (rounds >= MAXR) asm volatile("s_waitcnt vmcnt(%0)" : : "n"(MAXR * I) : "memory");
-    else load_wait<I, MAXR - 1>(rounds);
-  }
-}
-
-constexpr int RK = 2;  // k tiles (of 32) per round
-
-// F16: the operands are fp16 (v_mfma_f32_32x32x16_f16) instead of bf16; same tile order, same epilogues
+// FP16: the operands are fp16 (v_mfma_f32_32x32x16_f16) instead of bf16; same tile order, same epilogues
 // ROPE (TN == 2, bf16): the weights are packed in rotary pair order -- the two tiles of a wave hold columns
 // (c, c + rope_half) of one head -- and the epilogue is the skinny kernel's rotary one: columns < rope_cols rotated
 // by the table row of pos[m] (fp32 products rounded separately, or every product and sum rounded to bf16), columns
 // >= vt_col0 also written transposed for the attention kernel.  No bias, activation or residual in this form.
-template <int BM, int BN, int WGM, int WGN, int NS, int OCC, bool F16, bool ROPE = false>
+template <int BM, int BN, int WGM, int WGN, int NS, int OCC, bool FP16, bool ROPE = false>
 __global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel(GemmArgs a, int nblk_m, int ngroups, int by_rows) {
-  constexpr int NW = WGM * WGN;  // multiplying waves; as many more only load
-  constexpr int TM = BM / WGM, TN = BN / WGN;  // tiles of a wave
-  static_assert(BM % WGM == 0 && BN % WGN == 0 && (BM * 4) % NW == 0 && (BN * 4) % NW == 0 && NW == 4, "whole tiles and loads per wave");
-  static_assert(!ROPE || (TN == 2 && !F16), "the rotary epilogue needs both halves of a pair in one wave");
-  constexpr int AI = BM * 4 / NW, WI = BN * 4 / NW;  // loads of a wave per round
-  constexpr int STAGE = (BM + BN) * 4096;
-  constexpr int W_OFF = BM * 4096;
-  constexpr int TILES = TM * TN;
-  constexpr int SP = BN * 128 + 16;  // epilogue: the block's outputs pass through LDS in fp32, row pitch in bytes (16 rows' same column: all banks)
-  constexpr int LDSB = NS * STAGE > BM * 32 * SP ? NS * STAGE : BM * 32 * SP;
-  static_assert(LDSB * OCC <= 160 * 1024 && NS >= 2 && (AI + WI) * (NS - 1) < 64, "LDS of a CU, the load counter's range");
-  __shared__ __align__(1024) unsigned char lds[LDSB];
-  const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) unsigned char*)lds;
+  using P = Pipe<BM, BN, WGM, WGN, NS, FP16 ? F16 : BF16>;
+  constexpr int NW = P::NW, TM = P::TM, TN = P::TN, TILES = P::TILES, SP = P::SP;
+  static_assert(!ROPE || (TN == 2 && !FP16), "the rotary epilogue needs both halves of a pair in one wave");
+  static_assert(P::LDS * OCC <= 160 * 1024, "LDS of a CU");
+  __shared__ __align__(1024) unsigned char lds[P::LDS];
+  Tile tile;
+  if (!tile_of(tile, a, nblk_m, ngroups, by_rows)) return;
+  const int mblock = tile.mblock, nblk = tile.nblk, split = tile.split;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool loader = wave >= NW;
-  const int lw = wave - NW;  // a loading wave's number
   const int wm = wave / WGN, wn = wave % WGN;  // a multiplying wave's place
   const int half = lane >> 5;
   const int l32 = lane & 31;
 
-  // Blocks are dealt to the 8 XCDs round-robin; each XCD takes an eighth of the tiles in a row, so that no XCD has more
-  // to do than another.  The larger operand is the outer index: weights (a group: n tiles and k range) that several
-  // blocks share come from memory once and from one XCD's L2 afterwards, or (by_rows) activations do.
-  const unsigned x8 = blockIdx.x & 7, total = (unsigned)nblk_m * (unsigned)ngroups, each = total >> 3, more8 = total & 7;
-  if ((blockIdx.x >> 3) >= each + (x8 < more8)) return;
-  const unsigned lin = x8 * each + (x8 < more8 ? x8 : more8) + (blockIdx.x >> 3);
-  const int mblock = (int)(by_rows ? lin / (unsigned)ngroups : lin % (unsigned)nblk_m);
-  const int group = (int)(by_rows ? lin % (unsigned)ngroups : lin / (unsigned)nblk_m);
-  const int split = group % a.ksplit;
-  const int nblk = group / a.ksplit;
-
-  const int kt_lo = split * a.kt_q + (split < a.kt_r ? split : a.kt_r);
-  const int kt_hi = kt_lo + a.kt_q + (split < a.kt_r ? 1 : 0);
-  const int nrounds = (kt_hi - kt_lo + RK - 1) / RK;
-  const int k_end = kt_hi * 32 < a.K ? kt_hi * 32 : a.K;
-
-  constexpr int THREADS = 2 * NW * 64, CPR = BN * 4, ITEMS = BM * 32 * CPR / THREADS;  // 16-byte pieces of outputs: per row, per thread
+  constexpr int THREADS = P::THREADS, CPR = BN * 4, ITEMS = BM * 32 * CPR / THREADS;  // 16-byte pieces of outputs: per row, per thread
   constexpr int PRE_MAX = OCC == 1 ? 4 : TILES < 4 ? 2 : 1, PRE = ITEMS < PRE_MAX ? ITEMS : PRE_MAX;  // pieces whose residual is asked for here (128 registers at two blocks a compute unit)
   static_assert(BM * 32 * CPR % THREADS == 0, "whole pieces");
   const int m_blk = mblock * BM * 32, n_blk = nblk * BN * 32;
@@ -120,106 +62,9 @@ __global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel
     }
   }
 
-  auto swz = [](int r) { return ((r >> 1) & 3) | (((r & 1) ^ ((r >> 3) & 1)) << 2); };
-  if (loader) {
-    // ---- loads.  x: instruction i of this wave brings rows 8q .. 8q + 7 of the block, q = lw * AI + i; lane l the
-    // 16-byte slot l % 8 of row 8q + l / 8, which holds the line's chunk (l % 8) ^ swz(row) ----
-    const char* xp[AI];  // the eight rows' first column of this block's k range, then on
-    unsigned xv[AI];     // the lane's chunk from there
-    unsigned xfix[2];    // last round: lanes whose chunk is past the k range take the round's first one (zeroed in LDS)
-    const int k_last = (kt_lo + (nrounds - 1) * RK) * 32;
-#pragma unroll
-    for (int i = 0; i < AI; ++i) {
-      const int r0 = mblock * (BM * 32) + 8 * (lw * AI + i), rl = lane >> 3, ch = (lane & 7) ^ swz(8 * (lw * AI + i) + rl);
-      const int b0 = r0 < a.M ? r0 : a.M - 1;  // rows past M: valid data, never stored
-      const int m = r0 + rl < a.M ? r0 + rl : a.M - 1;
-      xp[i] = (const char*)a.x + ((size_t)b0 * a.ldx + kt_lo * 32) * 2;
-      xv[i] = (unsigned)(m - b0) * (unsigned)a.ldx * 2 + ch * 16;
-      if (i < 2) xfix[i] = k_last + ch * 8 < k_end ? 0 : ch * 16;
-    }
-    // W: a round of an n tile is 4 KiB in a row (k tile, chunk); instruction i: 1 KiB of n tile q / 4, q = i * NW + lw
-    const char* wp[WI];
-#pragma unroll
-    for (int i = 0; i < WI; ++i) {
-      int ntg = nblk * BN + (i * NW + lw) / 4;
-      if (ntg > a.ntiles - 1) ntg = a.ntiles - 1;  // overhanging tiles are computed on valid data, never stored
-      wp[i] = (const char*)a.w + ((size_t)ntg * a.KT + kt_lo) * 2048 + (lw & 3) * 1024;
-    }
-    const int w_back = (lw & 2) && kt_lo + nrounds * RK > a.KT ? 2048 : 0;  // last round's second k tile past the matrix: the first one again (its x is zero)
-    const unsigned lane16 = lane * 16;
-    int ibuf = 0;  // LDS offset of the buffer that the next round is loaded into
-    auto xissue = [&](int i, int r) {
-      unsigned v = xv[i];
-      if (r == nrounds - 1) v -= xfix[i & 1];
-      dma16(v, xp[i], lds0 + (unsigned)(ibuf + (lw * AI + i) * 1024));
-      xp[i] += 128;
-    };
-    auto wissue = [&](int i, int r) {
-      const char* p = wp[i] - (r == nrounds - 1 ? w_back : 0);
-      dma16(lane16, p, lds0 + (unsigned)(ibuf + W_OFF + (i * NW + lw) * 1024));
-      wp[i] += 4096;
-    };
-    auto xzero = [&](int buf) {  // the last round's columns past the k range (this wave's rows; behind its load_wait)
-      if (k_last + RK * 32 <= k_end) return;
-#pragma unroll
-      for (int i = 0; i < AI; ++i)
-        if (xfix[i & 1]) *(i32x4*)(lds + buf + (lw * AI + i) * 1024 + lane * 16) = i32x4{0, 0, 0, 0};
-    };
-    auto inext = [&] { ibuf = ibuf + STAGE == NS * STAGE ? 0 : ibuf + STAGE; };
-
-    // NS rounds asked for; then, round after round: its own loads are there, so are the other waves' (and every multiplying
-    // wave has left the round before, whose buffer takes round r - 1 + NS)
-#pragma unroll
-    for (int r = 0; r < NS; ++r)
-      if (r < nrounds) {
-#pragma unroll
-        for (int i = 0; i < AI; ++i) xissue(i, r);
-#pragma unroll
-        for (int i = 0; i < WI; ++i) wissue(i, r);
-        inext();
-      }
-    int buf = 0;
-    for (int r = 0; r < nrounds; ++r) {
-      const int ahead = nrounds - 1 - r;  // rounds asked for behind this one: at most NS - 2 of them, NS - 1 in the first round
-      if (r == 0) load_wait<AI + WI, NS - 1>(ahead);
-      else load_wait<AI + WI, NS - 2>(ahead);
-      if (r == nrounds - 1) xzero(buf);
-      lds_barrier();
-      if (r > 0 && r - 1 + NS < nrounds) {
-#pragma unroll
-        for (int i = 0; i < AI; ++i) xissue(i, r - 1 + NS);
-#pragma unroll
-        for (int i = 0; i < WI; ++i) wissue(i, r - 1 + NS);
-        inext();
-      }
-      buf = buf + STAGE == NS * STAGE ? 0 : buf + STAGE;
-    }
-  }
   f32x16 acc[TM][TN];
-#pragma unroll
-  for (int mt = 0; mt < TM; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < TN; ++nt)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
-
-  // ---- operand reads: k step s (of four) of a round = k tile s / 2, 16-byte half s % 2 ----
-  i32x4 xa[2][TM], wb[2][TN];
-  int xoff[4];
-#pragma unroll
-  for (int s = 0; s < 4; ++s) xoff[s] = (wm * TM * 32 + l32) * 128 + ((((s >> 1) * 4 + 2 * half + (s & 1)) ^ swz(l32)) << 4);
-  const int woff = W_OFF + wn * TN * 4096 + lane * 16;
-  auto read1 = [&](int set, int s, int buf, int u) {  // u in [0, TM + TN)
-    if (u < TM) xa[set][u] = *(const i32x4*)(lds + buf + xoff[s] + u * 4096);
-    else wb[set][u - TM] = *(const i32x4*)(lds + buf + woff + (u - TM) * 4096 + s * 1024);
-  };
-  auto mma1 = [&](int set, int t) {
-    const int mt = t / TN, nt = t % TN;
-    if (F16)
-      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(as_f16x8(wb[set][nt]), as_f16x8(xa[set][mt]), acc[mt][nt], 0, 0, 0);
-    else
-      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(wb[set][nt]), as_bf16x8(xa[set][mt]), acc[mt][nt], 0, 0, 0);
-  };
+  P::clear(acc);
+  if (loader) P::load(a, tile, lds, wave - NW, lane);
 
   // Bias and (16-bit) residual are asked for before the products: behind them they would be a round trip of their own,
   // to memory that nothing has touched yet
@@ -265,41 +110,7 @@ __global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel
   };
   if (ROPE) ask_rope(early, 0);
 
-  if (!loader) {
-    lds_barrier();
-    int buf = 0;
-#pragma unroll
-    for (int u = 0; u < TM + TN; ++u) read1(0, 0, 0, u);
-
-    // Round r: k steps 0 .. 2 fetch the next step's operands between their matrix instructions; step 3 meets the other
-    // waves in its middle (round r + 1 is there) and fetches that round's first operands.
-    constexpr int RD = TM + TN, H = (TILES + 1) / 2;
-    for (int r = 0; r < nrounds; ++r) {
-#pragma unroll
-      for (int s = 0; s < 3; ++s)
-#pragma unroll
-        for (int t = 0; t < TILES; ++t) {
-          mma1(s & 1, t);
-#pragma unroll
-          for (int u = 0; u < RD; ++u)
-            if (u * TILES / RD == t) read1((s + 1) & 1, s + 1, buf, u);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      buf = buf + STAGE == NS * STAGE ? 0 : buf + STAGE;
-#pragma unroll
-      for (int t = 0; t < H; ++t) mma1(1, t);
-      __builtin_amdgcn_sched_barrier(0);
-      if (r + 1 < nrounds) {
-        lds_barrier();
-#pragma unroll
-        for (int u = 0; u < RD; ++u) read1(0, 0, buf, u);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int t = H; t < TILES; ++t) mma1(1, t);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  }
+  if (!loader) P::multiply(acc, tile, lds, wave, lane);
 
   // ---- K-split hand-off: fp32 partials [(block, split)][wave][tile][group][lane][4] ----
   const int blk_lin = nblk * nblk_m + mblock;
@@ -373,7 +184,7 @@ __global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel
         for (int g = 0; g < 4; ++g) {
           const f32x16& c = acc[mt][nt];
           f32x4 v = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-          if (!ROPE && a.bias) v = v + unpack_16x4<F16>(bias[nt][g]);
+          if (!ROPE && a.bias) v = v + unpack_16x4<FP16>(bias[nt][g]);
           *(f32x4*)(lds + ((wm * TM + mt) * 32 + l32) * SP + ((wn * TN + nt) * 32 + 8 * g + 4 * half) * 4) = v;
         }
   }
@@ -454,16 +265,16 @@ __global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
       f32x4 v = *(const f32x4*)(src + 16 * q);
-      if (a.act == 1) v = unpack_16x4<F16>(pack_16x4<F16>(v));  // the linear's 16-bit output, then the activation on it
+      if (a.act == 1) v = unpack_16x4<FP16>(pack_16x4<FP16>(v));  // the linear's 16-bit output, then the activation on it
       if (a.act) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) v[j] = gelu_tanh_rcp_f(v[j]);
       }
-      o[q] = pack_16x4<F16>(v);
+      o[q] = pack_16x4<FP16>(v);
       if (a.resid) {
         const f32x4 r = a.resid_f32 ? f32x4{__int_as_float(r32[q][0]), __int_as_float(r32[q][1]), __int_as_float(r32[q][2]), __int_as_float(r32[q][3])}
-                                    : unpack_16x4<F16>(it < PRE ? pre[it < PRE ? it : 0][q] : r16[q]);
-        o[q] = pack_16x4<F16>(unpack_16x4<F16>(o[q]) + r);
+                                    : unpack_16x4<FP16>(it < PRE ? pre[it < PRE ? it : 0][q] : r16[q]);
+        o[q] = pack_16x4<FP16>(unpack_16x4<FP16>(o[q]) + r);
       }
     }
     if (m >= a.M || n >= a.N) continue;
@@ -485,7 +296,7 @@ __global__ __launch_bounds__(2 * WGM * WGN * 64, 2 * OCC) void bf16w_wide_kernel
       for (int r = 0; r < 4; ++r) {
         const float lo = *(const float*)(lds + (8 * rg + 2 * r) * SP + col * 4), hi = *(const float*)(lds + (8 * rg + 2 * r + 1) * SP + col * 4);
         const float l = m0 + 2 * r < a.M ? lo : 0.f, h = m0 + 2 * r + 1 < a.M ? hi : 0.f;
-        e[r] = (int)(F16 ? pack_f16x2(l, h) : pack_bf16x2(l, h));
+        e[r] = (int)(FP16 ? pack_f16x2(l, h) : pack_bf16x2(l, h));
       }
       const int prob = a.vt_rows ? m0 / a.vt_rows : 0, key0 = a.vt_rows ? m0 % a.vt_rows : m0;
       *(i32x4*)(a.vt + (size_t)prob * a.vt_bs + (size_t)(n - a.vt_col0) * a.vt_ld + key0) = e;
@@ -500,7 +311,7 @@ int launch(const GemmArgs& a, hipStream_t st) {
   const int nblk_n = (a.ntiles + BN - 1) / BN;
   const int ngroups = nblk_n * a.ksplit;
   const int by_rows = a.M > a.N;
-  const unsigned blocks = ((unsigned)nblk_m * (unsigned)ngroups + 7) / 8 * 8;
+  const unsigned blocks = blocks_of(nblk_m, ngroups);
   if (a.rope_pos) {
     if constexpr (ROPE) {
       if (a.f16) return -1;

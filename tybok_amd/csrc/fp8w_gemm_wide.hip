@@ -1,35 +1,14 @@
-// fp8-weight GEMM for many rows (M > 64: the VLM prefill) on gfx950.
-//
-// Same operands and packed weight tiles as the skinny kernel (fp8w_gemm.hip), other balance: with
-// hundreds of rows the product is MFMA-bound, so the block tile is large enough that neither
-// operand is re-read often:
-//   * a block of 4 waves owns 128 rows x 8 packed n tiles (256 packed columns) and a range of k
-//     tiles; wave w owns n tiles 2w, 2w+1 for all 128 rows: 8 accumulator tiles of 32x32, and per
-//     k tile 16 MFMAs against 2 weight loads (straight from global memory into operand registers,
-//     1 KiB coalesced per tile, e4m3 -> bf16 in registers) and 8 LDS operand reads;
-//   * the activations of a round (128 rows x 64 columns) are staged once per block through LDS with
-//     whole 128-byte lines per row, double buffered, one LDS barrier per round;
-//   * blocks that share weights (same n tiles and k range, different rows) get consecutive slots of
-//     ONE XCD, so the weight tiles are read from HBM once and served from that XCD's L2 afterwards;
-//   * K splits (few column blocks, long K: the down projection) leave fp32 partials in the workspace and a
-//     second launch over all CUs sums them in split order and runs the epilogue -- bit-deterministic.  (A
-//     gated launch that is split keeps the one-launch form: the last-arriving block sums.  Measured at
-//     M=712, K=16384, N=2048, 5 splits: 74 -> 52 + 7.7 us; one block per output tile -- 48 of 256 CUs -- pulling
-//     31 MB of partials through 8-byte coherent loads, split after split, was a fifth of the launch.)
-//   * where the grid would fill the device twice over (the gated 2048 -> 2 x 16384 launch) a block is EIGHT waves on
-//     192 or 256 rows with the weights staged through LDS too (fp8w_tile_kernel below): half the bytes per matrix
-//     instruction through the L2, the same accumulators, partials and epilogue, the same bits.
-// The epilogues compute exactly what the skinny kernel's do (same rounding points).
-#include "tk_common.h"
-#include "tk_kernels.h"
+// fp8-weight GEMM for many rows (the VLM prefill) on gfx950: the weight-only form of pipe_fp8.h, a kernel of its own for the
+// largest grids, and the row norm in front of them.
+// Measured (us, cold weights, graph replay; before: weights straight into the registers of four multiplying waves): the
+// gated block 2048 -> 16384 -> 2048 at 288 / 330 / 555 / 712 / 968 rows 104 -> 83, 102 -> 87, 135 -> 132, 156 -> 151, 190 ->
+// 186; 960 -> 2560 -> 960 at 305 / 600 rows 39 -> 22, 41 -> 28.
+#include <atomic>
+
+#include "pipe_fp8.h"
 
 namespace {
-
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
+using pipe::lds_barrier;
 
 constexpr int NT = 2;   // n tiles per wave
 constexpr int NW = 4;   // waves per block
@@ -190,9 +169,14 @@ __device__ __forceinline__ void wide_epilogue(const GemmArgs& a, const f32x16 (&
   }
 }
 
-// EPI: 0 plain (scale, optional per-column gate, optional residual), 1 gated (gate/up tile pairs).
-// MT: 32-row tiles per block (and per wave): 4 with one block per CU, 2 with two -- co-resident blocks cover each
-// other's first loads and epilogue.  PF: rounds in flight (even: round r uses LDS buffer r % 2).
+// Grids that cover the device twice over (from 385 rows of the gated 2048 -> 2 x 16384 launch): there the power of the
+// operands' way decides the matrix pipes' clock, and the two kernels below, whose weights go through registers, are the cheaper
+// ones.  This one where 64-row blocks waste the least: 555 rows 81 us against 83 - 88 of pipe_fp8.h's kernel, 650 rows 94 - 99
+// against 100 - 102.
+// A block of four waves owns 64 rows x 256 packed columns, two blocks a CU (they cover each other's first loads and
+// epilogue); wave w owns n tiles 2w, 2w + 1 for all rows, its weights straight from memory into its registers; a round's
+// activations are staged once per block through LDS.  EPI: 0 plain, 1 gated.  PF: rounds in flight (even: round r uses LDS
+// buffer r % 2).
 template <int EPI, int MT, int PF, int OCC>
 __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int nblk_m, int ngroups) {
   constexpr int ROWS = MT * 32;
@@ -201,7 +185,6 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
   constexpr int XBUF = ROWS * PITCH;
   constexpr int PPR = ROWB / 16;           // 16-byte pieces per staged row
   constexpr int XPT = ROWS * PPR / (NW * 64);
-  constexpr int TILES = MT * NT;
   constexpr int EPB = NW * 32 * ((EPI == 0 ? NT * 32 : 32) * 2 + 16);  // the epilogue's per-wave tiles
   __shared__ __align__(16) unsigned char lds[2 * XBUF > EPB ? 2 * XBUF : EPB];
 
@@ -218,13 +201,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
   const int mblock = (int)(slot % (unsigned)nblk_m);
   const int group = (int)((slot / (unsigned)nblk_m) * 8 + (id & 7));
   if (group >= ngroups) return;
-  const int split = group % a.ksplit;
-  const int nblk = group / a.ksplit;
-
-  const int kt_lo = split * a.kt_q + (split < a.kt_r ? split : a.kt_r);
-  const int kt_hi = kt_lo + a.kt_q + (split < a.kt_r ? 1 : 0);
-  const int nrounds = (kt_hi - kt_lo + RK - 1) / RK;
-  const int k_end = kt_hi * 32 < a.K ? kt_hi * 32 : a.K;
+  const int nblk = group;
+  const int nrounds = (a.KT + RK - 1) / RK;
 
   const int strip = nblk * NW + wave;  // this wave's pair of packed n tiles
   const uint8_t* wbase[NT];
@@ -266,18 +244,18 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
   // cannot issue anything while it waits for the matrix pipe to take its next instruction, so whatever stands
   // between two groups of matrix instructions in program order runs with the pipe empty.
   auto wload1 = [&](WFrag& f, int r, int j, int nt) {  // k tile j of round r, n tile nt: one 1 KiB tile
-    int kt = kt_lo + r * RK + j;
+    int kt = r * RK + j;
     if (kt > a.KT - 1) kt = a.KT - 1;  // its activation columns are zeroed
     f.w[j][nt] = *(const i32x4*)(wbase[nt] + (size_t)kt * 1024);
   };
   auto xload1 = [&](XFrag& f, int r, int i) {
-    int k = (kt_lo + r * RK) * 32 + xcol[i];
+    int k = r * RK * 32 + xcol[i];
     if (k > a.K - 8) k = a.K - 8;
     f.v[i] = *(const i32x4*)(xsrc[i] + (size_t)k * 2);
   };
   auto xstore1 = [&](const XFrag& f, int r, int b, int i) {
     const i32x4 z = {0, 0, 0, 0};
-    *(i32x4*)(lds + b * XBUF + xdst[i]) = ((kt_lo + r * RK) * 32 + xcol[i]) < k_end ? f.v[i] : z;
+    *(i32x4*)(lds + b * XBUF + xdst[i]) = r * RK * 32 + xcol[i] < a.K ? f.v[i] : z;
   };
   // operand fragments and converted weights of two k tiles: while the MFMAs of one k tile run, the LDS reads and
   // the e4m3 -> bf16 conversions of the next one are issued between them
@@ -382,73 +360,6 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
       if (q < rem) round(q, it + q);  // block-uniform
   }
 
-  // ---- K-split hand-off: fp32 partials [(block, split)][wave][tile][group][lane][4] ----
-  const int blk_lin = nblk * nblk_m + mblock;
-  if (a.ksplit > 1 && a.split_reduce) {
-    // the partial leaves as it is (plain 16-byte stores: the kernel boundary publishes it); wide_split_reduce_kernel
-    // finishes
-    f32x4* mine = (f32x4*)a.partial + ((size_t)blk_lin * a.ksplit + split) * (NW * TILES * 4 * 64) + (size_t)wave * TILES * 4 * 64 + lane;
-#pragma unroll
-    for (int t = 0; t < TILES; ++t)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c = acc[t / NT][t % NT];
-        mine[(t * 4 + g) * 64] = f32x4{c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-      }
-    return;
-  }
-  if (a.ksplit > 1) {
-    unsigned long long* pbase = (unsigned long long*)a.partial + ((size_t)wave * TILES * 4 * 64 + lane) * 2;
-    unsigned long long* mine = pbase + ((size_t)blk_lin * a.ksplit + split) * (NW * TILES * 4 * 64 * 2);
-#pragma unroll
-    for (int t = 0; t < TILES; ++t)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c = acc[t / NT][t % NT];
-        unsigned long long* dst = mine + (size_t)(t * 4 + g) * 128;
-        st_agent64(dst, c[4 * g], c[4 * g + 1]);
-        st_agent64(dst + 1, c[4 * g + 2], c[4 * g + 3]);
-      }
-    __shared__ int s_last;
-    handoff_publish();
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      int old = __hip_atomic_fetch_add(a.counters + blk_lin, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      s_last = (old == a.ksplit - 1);
-    }
-    __syncthreads();
-    if (!s_last) return;
-    handoff_acquire();
-    if (threadIdx.x == 0) __hip_atomic_store(a.counters + blk_lin, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
-    for (int s = 0; s < a.ksplit; ++s) {  // split order, whoever arrived last
-      const unsigned long long* src = pbase + ((size_t)blk_lin * a.ksplit + s) * (NW * TILES * 4 * 64 * 2);
-      unsigned long long raw[TILES][4][2];
-#pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          raw[t][g][0] = ld_agent64(src + (size_t)(t * 4 + g) * 128);
-          raw[t][g][1] = ld_agent64(src + (size_t)(t * 4 + g) * 128 + 1);
-        }
-#pragma unroll
-      for (int t = 0; t < TILES; ++t)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          f32x16& c = acc[t / NT][t % NT];
-          c[4 * g] += __uint_as_float((unsigned)raw[t][g][0]);
-          c[4 * g + 1] += __uint_as_float((unsigned)(raw[t][g][0] >> 32));
-          c[4 * g + 2] += __uint_as_float((unsigned)raw[t][g][1]);
-          c[4 * g + 3] += __uint_as_float((unsigned)(raw[t][g][1] >> 32));
-        }
-    }
-  }
-
   // ---- epilogue ----
   constexpr int EP = wide_ep_pitch(EPI);
   static_assert(NW * 32 * EP == EPB, "the epilogue tiles fit the LDS array");
@@ -456,11 +367,10 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
   wide_epilogue<EPI, MT>(a, acc, lds + wave * 32 * EP, mblock * ROWS, strip, lane);
 }
 
-// The same product on a block of EIGHT waves that owns 2*WM*32 rows x 256 packed columns, with BOTH operands of a
-// round staged through LDS: wave (wm, wn) = (wave / 4, wave % 4) owns rows wm*WM*32 .. of the block and the n tile
-// pair wn, as a wave of the four-wave kernel does, so accumulators, partial layout and epilogue are the same -- but a
-// weight tile is fetched (and converted to bf16) once per block and serves both wave rows, which halves the bytes
-// that a CU pulls through the L2 per matrix instruction (the four-wave kernel's bound).  A round is four k steps of
+// The same where taller blocks waste no more rows: eight waves own 2*WM*32 rows x 256 packed columns, with both operands of a
+// round staged through registers and LDS: wave (wm, wn) = (wave / 4, wave % 4) owns rows wm*WM*32 .. of the block and the n
+// tile pair wn; a weight tile is fetched and converted to bf16 once per block (712 rows 95 - 98 us against 95 - 104 of
+// pipe_fp8.h's kernel, 968 rows 120 - 125 against 125 - 131).  A round is four k steps of
 // 16; operand registers of step s + 1 are read while step s multiplies; one barrier per round, before its last step:
 // by then every wave has read the round's operands out of buffer b and written its share of round r + 1 into b ^ 1.
 //   staging per thread and round: WM 16-byte pieces of x, 2 pieces of 16 fp8 weights (wave (wm, wn): k tile wm of
@@ -476,7 +386,6 @@ __global__ __launch_bounds__(512, 1) void fp8w_tile_kernel(GemmArgs a, int nblk_
   constexpr int WBUF = NW * NT * RK * 2048;  // bf16 tiles of the round: [n tile][k tile][k step][lane][16 B]
   constexpr int STAGE = XBUF + WBUF;
   constexpr int XPT = ROWS * (ROWB / 16) / (NWV * 64);
-  constexpr int TILES = WM * NT;
   constexpr int SL = WM * NT;  // matrix instructions per k step
   static_assert(XPT == WM && NWV * 32 * wide_ep_pitch(EPI) <= 2 * STAGE, "staging and epilogue tiles fit");
   extern __shared__ __align__(16) unsigned char lds[];
@@ -493,13 +402,8 @@ __global__ __launch_bounds__(512, 1) void fp8w_tile_kernel(GemmArgs a, int nblk_
   const int mblock = (int)(slot % (unsigned)nblk_m);
   const int group = (int)((slot / (unsigned)nblk_m) * 8 + (id & 7));
   if (group >= ngroups) return;
-  const int split = group % a.ksplit;
-  const int nblk = group / a.ksplit;
-
-  const int kt_lo = split * a.kt_q + (split < a.kt_r ? split : a.kt_r);
-  const int kt_hi = kt_lo + a.kt_q + (split < a.kt_r ? 1 : 0);
-  const int nrounds = (kt_hi - kt_lo + RK - 1) / RK;
-  const int k_end = kt_hi * 32 < a.K ? kt_hi * 32 : a.K;
+  const int nblk = group;
+  const int nrounds = (a.KT + RK - 1) / RK;
 
   const int strip = nblk * NW + wn;
   const uint8_t* wbase[NT];
@@ -532,18 +436,18 @@ __global__ __launch_bounds__(512, 1) void fp8w_tile_kernel(GemmArgs a, int nblk_
     i32x4 w[NT];
   };
   auto xload1 = [&](Stg& f, int r, int i) {
-    int k = (kt_lo + r * RK) * 32 + xcol;
+    int k = r * RK * 32 + xcol;
     if (k > a.K - 8) k = a.K - 8;
     f.x[i] = *(const i32x4*)(xsrc[i] + (size_t)k * 2);
   };
   auto wload1 = [&](Stg& f, int r, int nt) {
-    int kt = kt_lo + r * RK + wm;
+    int kt = r * RK + wm;
     if (kt > a.KT - 1) kt = a.KT - 1;  // its activation columns are zeroed
     f.w[nt] = *(const i32x4*)(wbase[nt] + (size_t)kt * 1024);
   };
   auto xstore1 = [&](const Stg& f, int r, int b, int i) {
     const i32x4 z = {0, 0, 0, 0};
-    *(i32x4*)(lds + b * STAGE + xdst + i * 64 * PITCH) = ((kt_lo + r * RK) * 32 + xcol) < k_end ? f.x[i] : z;
+    *(i32x4*)(lds + b * STAGE + xdst + i * 64 * PITCH) = r * RK * 32 + xcol < a.K ? f.x[i] : z;
   };
   auto wstore1 = [&](const Stg& f, int b, int q) {  // q in [0, 2*NT): k step q%2 of n tile q/2
     *(bf16x8*)(lds + b * STAGE + XBUF + ((((wn * NT + q / 2) * RK + wm) * 2 + q % 2) * 64 + lane) * 16) =
@@ -624,66 +528,9 @@ __global__ __launch_bounds__(512, 1) void fp8w_tile_kernel(GemmArgs a, int nblk_
     if (it < nrounds) round(0, it);
   }
 
-  const int blk_lin = nblk * nblk_m + mblock;
-  if (a.ksplit > 1) {  // always the two-launch form here: partials [(block, split)][wave][tile][group][lane][4]
-    f32x4* mine = (f32x4*)a.partial + ((size_t)blk_lin * a.ksplit + split) * (NWV * TILES * 4 * 64) + (size_t)wave * TILES * 4 * 64 + lane;
-#pragma unroll
-    for (int t = 0; t < TILES; ++t)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const f32x16& c = acc[t / NT][t % NT];
-        mine[(t * 4 + g) * 64] = f32x4{c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-      }
-    return;
-  }
   constexpr int EP = wide_ep_pitch(EPI);
   if (a.vec16) lds_barrier();
   wide_epilogue<EPI, WM>(a, acc, lds + wave * 32 * EP, mblock * ROWS + wm * WM * 32, strip, lane);
-}
-
-// Second launch of a K-split plain GEMM (GemmArgs::split_reduce): thread (block tile, wave, tile, lane) sums its four
-// register groups over the splits in split order -- the order and the arithmetic of the last-arriving block of the
-// one-launch form, so the same bits -- and finishes them like the scattered epilogue above.  Every CU takes part.
-template <int MT, int NWV>
-__global__ __launch_bounds__(256) void wide_split_reduce_kernel(GemmArgs a, int nblk_m, int nthreads) {
-  constexpr int TILES = MT * NT;
-  const int gid = blockIdx.x * 256 + threadIdx.x;
-  if (gid >= nthreads) return;
-  const int lane = gid & 63, half = lane >> 5, l32 = lane & 31;
-  const int t = (gid >> 6) % TILES;
-  const int wave = (gid >> 6) / TILES % NWV;
-  const int blk_lin = (gid >> 6) / (TILES * NWV);
-  const int mblock = blk_lin % nblk_m, nblk = blk_lin / nblk_m;
-  const int mt = t / NT, nt = t % NT;
-  const int strip = nblk * NW + wave % NW;
-  const f32x4* src = (const f32x4*)a.partial + (size_t)blk_lin * a.ksplit * (NWV * TILES * 4 * 64) + (size_t)wave * TILES * 4 * 64 + (size_t)t * 4 * 64 + lane;
-  f32x4 sum[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) sum[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int s = 0; s < a.ksplit; ++s) {
-    f32x4 p[4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) p[g] = src[(size_t)s * (NWV * TILES * 4 * 64) + g * 64];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) sum[g] += p[g];
-  }
-  const int m = ((mblock * (NWV / NW) + wave / NW) * MT + mt) * 32 + l32;  // (eight waves: two wave rows of MT tiles)
-  if (m >= a.M) return;
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int n0 = (strip * NT + nt) * 32 + 8 * g + 4 * half;
-    if (n0 >= a.N) continue;
-    const f32x4 sc = *(const f32x4*)(a.s0 + n0);
-    i32x2 r = pack_bf16x4(sum[g] * sc);
-    if (a.gate) r = pack_bf16x4(unpack_bf16x4(r) * unpack_bf16x4(*(const i32x2*)(a.gate + n0)));
-    if (a.resid) {
-      const f32x4 rv = a.resid_f32 ? *(const f32x4*)((const float*)a.resid + (size_t)m * a.ldr + n0)
-                                   : unpack_bf16x4(*(const i32x2*)((const u16*)a.resid + (size_t)m * a.ldr + n0));
-      r = pack_bf16x4(unpack_bf16x4(r) + rv);
-    }
-    *(i32x2*)(a.y + (size_t)m * a.ldy + n0) = r;
-  }
 }
 
 // One block per row: out = bf16 norm of the bf16 row, with the rounding points of the skinny
@@ -766,66 +613,41 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(NormRowsArgs a) {
   }
 }
 
-}  // namespace
-
-int tk_wide_cols() { return NW * NT * 32; }
-
-namespace {
-template <int EPI, int WM, int PF>
-bool launch_tile(const GemmArgs& a, dim3 grid, int nblk_m, int ngroups, hipStream_t st) {
-  constexpr int LDS = 2 * (2 * WM * 32 * (RK * 64 + 16) + NW * NT * RK * 2048);
-  static bool sized = false;  // above 64 KiB of LDS a kernel has to be told once
-  if (!sized) {
-    if (hipFuncSetAttribute((const void*)fp8w_tile_kernel<EPI, WM, PF>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return false;
-    sized = true;
-  }
-  hipLaunchKernelGGL((fp8w_tile_kernel<EPI, WM, PF>), grid, dim3(512), LDS, st, a, nblk_m, ngroups);
-  return true;
-}
-}  // namespace
-
-// a.mtiles: 32-row tiles per block: 2 or 4 (four waves, weights straight from memory), 6 or 8 (eight waves, both
-// operands through LDS; a K split of those always finishes in the reduction launch)
-int tk_launch_gemm_wide(GemmArgs a, hipStream_t st) {
-  if (a.mtiles != 2 && a.mtiles != 4 && a.mtiles != 6 && a.mtiles != 8) return -1;
-  const bool tile8 = a.mtiles > 4;
-  const int nblk_m = (a.M + a.mtiles * 32 - 1) / (a.mtiles * 32);
-  const int nblk_n = (a.ntiles + NW * NT - 1) / (NW * NT);
-  const int ngroups = nblk_n * a.ksplit;
-  const dim3 grid((unsigned)((ngroups + 7) / 8) * 8u * (unsigned)nblk_m), block(NW * 64);
-  // K splits of a plain launch with 4-column alignment: partials out, then a reduction launch over all CUs
-  a.split_reduce = a.ksplit > 1 && !a.s1 && a.vec && a.N % 4 == 0;
-  if (tile8 && a.ksplit > 1 && !a.split_reduce) return -1;
-  bool ok = true;
-  if (a.s1) {
-    if (a.mtiles == 8)
-      ok = launch_tile<1, 4, 1>(a, grid, nblk_m, ngroups, st);
-    else if (a.mtiles == 6)
-      ok = launch_tile<1, 3, 1>(a, grid, nblk_m, ngroups, st);
-    else if (a.mtiles == 4)
-      hipLaunchKernelGGL((fp8w_wide_kernel<1, 4, 4, 1>), grid, block, 0, st, a, nblk_m, ngroups);
-    else
-      hipLaunchKernelGGL((fp8w_wide_kernel<1, 2, 4, 2>), grid, block, 0, st, a, nblk_m, ngroups);
-  } else {
-    if (a.mtiles == 8)
-      ok = launch_tile<0, 4, 1>(a, grid, nblk_m, ngroups, st);
-    else if (a.mtiles == 6)
-      ok = launch_tile<0, 3, 1>(a, grid, nblk_m, ngroups, st);
-    else if (a.mtiles == 4)
-      hipLaunchKernelGGL((fp8w_wide_kernel<0, 4, 4, 1>), grid, block, 0, st, a, nblk_m, ngroups);
-    else
-      hipLaunchKernelGGL((fp8w_wide_kernel<0, 2, 4, 2>), grid, block, 0, st, a, nblk_m, ngroups);
-  }
-  if (!ok) return -3;
-  if (a.split_reduce) {
-    const int nthreads = nblk_n * nblk_m * NW * a.mtiles * NT * 64;  // one per (output tile, lane), whatever the waves
-    const dim3 rg((nthreads + 255) / 256), rb(256);
-    if (a.mtiles == 8) hipLaunchKernelGGL((wide_split_reduce_kernel<4, 8>), rg, rb, 0, st, a, nblk_m, nthreads);
-    else if (a.mtiles == 6) hipLaunchKernelGGL((wide_split_reduce_kernel<3, 8>), rg, rb, 0, st, a, nblk_m, nthreads);
-    else if (a.mtiles == 4) hipLaunchKernelGGL((wide_split_reduce_kernel<4, 4>), rg, rb, 0, st, a, nblk_m, nthreads);
-    else hipLaunchKernelGGL((wide_split_reduce_kernel<2, 4>), rg, rb, 0, st, a, nblk_m, nthreads);
-  }
+template <int EPI>
+int launch_wide(const GemmArgs& a, hipStream_t st) {
+  const int nblk_m = (a.M + 63) / 64, nblk_n = (a.ntiles + NW * NT - 1) / (NW * NT);
+  hipLaunchKernelGGL((fp8w_wide_kernel<EPI, 2, 4, 2>), dim3((unsigned)((nblk_n + 7) / 8) * 8u * (unsigned)nblk_m), dim3(NW * 64), 0, st, a, nblk_m, nblk_n);
   return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+template <int EPI, int WM>
+int launch_tile(const GemmArgs& a, hipStream_t st) {
+  constexpr int LDS = 2 * (2 * WM * 32 * (RK * 64 + 16) + NW * NT * RK * 2048);
+  static std::atomic<int> raised{0};  // more LDS than a launch gets by default: raise the kernel's limit once per process
+  if (!raised.load(std::memory_order_acquire)) {
+    if (hipFuncSetAttribute((const void*)fp8w_tile_kernel<EPI, WM, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return -3;
+    raised.store(1, std::memory_order_release);
+  }
+  const int nblk_m = (a.M + 2 * WM * 32 - 1) / (2 * WM * 32), nblk_n = (a.ntiles + NW * NT - 1) / (NW * NT);
+  hipLaunchKernelGGL((fp8w_tile_kernel<EPI, WM, 1>), dim3((unsigned)((nblk_n + 7) / 8) * 8u * (unsigned)nblk_m), dim3(512), LDS, st, a, nblk_m, nblk_n);
+  return hipGetLastError() == hipSuccess ? 0 : -3;
+}
+
+}  // namespace
+
+// tile: an id of kWideTiles (tk_api.hip); 28, 68, 88: the kernels of this file, 64, 192 or 256 rows (no K split)
+int tk_launch_gemm_wide(const GemmArgs& a, int tile, hipStream_t st) {
+  using namespace pipe;
+  switch (tile) {
+    case 28: return a.s1 ? launch_wide<1>(a, st) : launch_wide<0>(a, st);
+    case 68: return a.s1 ? launch_tile<1, 3>(a, st) : launch_tile<0, 3>(a, st);
+    case 88: return a.s1 ? launch_tile<1, 4>(a, st) : launch_tile<0, 4>(a, st);
+    case 404: return launch_fp8_pipe<BF16_FP8, 4, 4, 2, 2, 3, 2>(a, st);
+    case 408: return launch_fp8_pipe<BF16_FP8, 4, 8, 2, 2, 4, 1>(a, st);
+    case 208: return launch_fp8_pipe<BF16_FP8, 2, 8, 1, 4, 3, 2>(a, st);
+    case 204: return launch_fp8_pipe<BF16_FP8, 2, 4, 2, 2, 4, 2>(a, st);
+  }
+  return -1;
 }
 
 int tk_launch_norm_rows(NormRowsArgs a, hipStream_t st) {

@@ -88,6 +88,56 @@ int static_scratch(void** out, hipStream_t st, bool may_fail_capture) {
   return TK_OK;
 }
 
+// A block shape of the many-row kernels (pipe_gemm.h).
+struct PipeTile {
+  int id, bm, bn;  // block of 32 bm rows x 32 bn columns
+  int wt, ns;      // 32 x 32 tiles of a multiplying wave, buffers in the ring
+  int occ;         // blocks of this shape that fit one CU (LDS)
+};
+// Estimated duration (us) of a launch; kb_n: KiB that a round brings of an n tile (of an m tile 4).  Fitted to 3400 timings
+// of the 16-bit form (64 shapes of the towers, the prefill and random ones, every tile, splits 1 .. 6; standard error
+// 14 %, the picked launch on average 1.1 % slower than the best one).  Blocks on one CU share its memory pipe (12 ns a KiB)
+// and matrix pipes (75 ns for a wave's tile and round); a round takes no less than the round trip over the rounds on
+// their way; the epilogue costs per tile; each further generation of blocks pays all of it again.
+float pipe_cost(const PipeTile& t, float kb_n, int M, int N, int rounds, int ks, int cus) {
+  const int rows = 32 * t.bm, cols = 32 * t.bn;
+  const long long blocks = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * ks;
+  float us = 1.66f;
+  for (long long left = blocks; left > 0; left -= (long long)cus * t.occ) {
+    const float r = left > cus && t.occ > 1 ? 2.f : 1.f;  // blocks on a CU
+    const float load = r * ((float)t.bm * 4.f + (float)t.bn * kb_n) * 0.0122f, mul = r * (float)t.wt * 0.0751f, trip = 0.585f / (float)(t.ns - 1);
+    us += 0.014f + (float)rounds * (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip)) + r * (float)(t.bm * t.bn) * 0.203f;
+  }
+  if (ks > 1) us += 4.76f + (float)blocks * (float)(t.bm * t.bn) * 0.00213f;  // fp32 partials out and back in
+  return us;
+}
+// The forms over fp8 weights.  Where the grid covers the device several times over, the time is the matrix pipes' at the
+// clock that their operands' power leaves (712 x 2048 x 32768, weight-only: 104 us, 81 with zeros for data, 56 without the
+// loads, 55 - 61 of loads alone): padded rows and columns at 1.15 (bf16) or 1.8 PFLOP/s (fp8 x fp8), shapes that move more
+// operands per product a little slower; a fifth of that shows where the loads set the time (the split down projection
+// 16384 -> 2048 at 555 / 650 rows on blocks of 128 x 256: the whole block 3 us less than on 64 x 256).
+struct Fp8Tile {
+  PipeTile t;
+  float power;  // relative time per product
+};
+constexpr Fp8Tile kWideTiles[] = {{{408, 4, 8, 8, 4, 1}, 1.f}, {{404, 4, 4, 4, 3, 2}, 1.f}, {{208, 2, 8, 4, 3, 2}, 1.3f}, {{204, 2, 4, 2, 4, 2}, 1.3f}};
+constexpr Fp8Tile kW8a8Tiles[] = {{{408, 4, 8, 8, 3, 1}, 1.f}, {{414, 4, 4, 4, 4, 1}, 1.1f}, {{204, 2, 4, 2, 3, 2}, 1.2f}, {{604, 6, 4, 6, 4, 1}, 1.f}};
+template <int N>
+int pick_tile(const Fp8Tile (&tiles)[N], float kb_n, float flop_per_us, int M, int ncols, int K, int rounds, int ks) {
+  int best = 0;
+  float best_cost = 0.f;
+  for (const Fp8Tile& f : tiles) {
+    const PipeTile& t = f.t;
+    const float rows = (float)((M + 32 * t.bm - 1) / (32 * t.bm) * 32 * t.bm), cols = (float)((ncols + 32 * t.bn - 1) / (32 * t.bn) * 32 * t.bn);
+    const float power = f.power * 2.f * rows * cols * (float)K / flop_per_us;
+    float c = pipe_cost(t, kb_n, M, ncols, rounds, ks, device_cus()) * (0.8f + 0.2f * f.power);
+    if (c < power) c = power;
+    if (!best || c < best_cost) best = t.id, best_cost = c;
+  }
+  return best;
+}
+constexpr int kWideCols = 256;  // column unit of the many-row rules below
+
 // Optional pieces of a GEMM launch beyond y = bf16((x . W^T) * scale).
 struct GemmExtra {
   int x_f32 = 0;                  // activations are fp32 (norm prologue only)
@@ -192,11 +242,12 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
   const bool has_norm = e.norm_w || e.ada_scale;
   // (from 256 rows on, or when its 128 x 256 tiles already fill the device; below that the skinny
   // kernel's finer blocks and K splits win)
-  const int wide_blocks = ((a.ntiles * 32 + tk_wide_cols() - 1) / tk_wide_cols()) * ((M + 127) / 128);
+  const int wide_blocks = ((a.ntiles * 32 + kWideCols - 1) / kWideCols) * ((M + 127) / 128);
   if (!e.w16 && !rope && !e.x_f32 && a.vec && (M >= 256 || (M > 64 && wide_blocks >= cus)) &&
       (!has_norm || (ws && ws_bytes >= kNormOff + (size_t)M * K * 2 && (size_t)M * K * 2 <= kNormBytes))) {
-    // many rows: MFMA-bound kernel with a 128 x 256 block tile
+    // many rows
     if (plan) return TK_OK;  // (plan->skinny stays false)
+    if (ldx > 1 << 28) return fail(TK_EINVAL, "gemm: ldx=%d, rows of x more than 512 MiB apart", ldx);
     if (has_norm) {
       NormRowsArgs nr;
       nr.x = (const u16*)x;
@@ -215,56 +266,38 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
       a.norm_w = nullptr;
       a.ada_scale = a.ada_shift = nullptr;
     }
-    // 64-row blocks, two per CU, once the 128-row grid would run in several generations anyway: co-resident
-    // blocks cover each other's first loads and epilogue; few blocks keep the 128-row tile
-    a.mtiles = wide_blocks >= 2 * cus ? 2 : 4;
-    if (a.mtiles == 2 && split_k <= 1) {
-      // eight-wave blocks of 192 / 256 rows with both operands through LDS, one per CU, where a CU's share of the rows
-      // (blocks in a row on it x rows per block) is no larger than with the 64-row blocks (measured on the gated
-      // 2048 -> 2 x 16384 launch: M=712 94 -> 90 us on 192 rows, 100 us on 256 -- its 384 blocks are one and a half
-      // generations; M=512 / 968 / 1024: 256-row blocks take 6 / 8 / 9 us off the FFN)
-      const int nb = (a.ntiles * 32 + tk_wide_cols() - 1) / tk_wide_cols();
-      auto share = [&](int rows) { return ((nb * ((M + rows - 1) / rows) + cus - 1) / cus) * rows; };
-      if (share(192) <= share(64)) a.mtiles = 6;
-      if (share(256) < share(192) && share(256) <= share(64)) a.mtiles = 8;
-    }
-    const int nbn = (a.ntiles * 32 + tk_wide_cols() - 1) / tk_wide_cols();
-    int ks = split_k;
-    if (ks <= 0 && a.mtiles == 4 && !a.s1 && a.N % 4 == 0 && ws && a.KT >= 32) {
-      // Few column blocks over a long K (the down projection): 64- or 128-row blocks and the split count by a cost
-      // fitted to M = 296 .. 968 at K = 16384, N = 2048 -- the k loop of the blocks that share a CU (0.1 us per 1000
-      // row x k products), the partials' trip through memory (0.5 us per MB), the weights pulled once per row block
-      // (0.005 us per MB) and 8 us that a grid of lone four-wave 64-row blocks loses to 128-row ones.  At 296 rows
-      // 64-row blocks x 6 splits take 31.8 us where 128-row blocks x 10 take 36.2; from 552 rows on 128-row blocks.
+    // K split, from the shape alone (it decides the order of summation).  Few column blocks over a long K (the down
+    // projection): a cost fitted to M = 296 .. 968 at K = 16384, N = 2048 -- the k loop of the blocks that share a CU (0.1 us
+    // per 1000 row x k products), the partials' trip through memory (0.5 us per MB), the weights pulled once per row block
+    // (0.005 us per MB) and 8 us that a grid of lone 64-row blocks loses to 128-row ones
+    const int nbn = (a.ntiles * 32 + kWideCols - 1) / kWideCols;
+    int ks = split_k, rows = 128;
+    if (ks <= 0 && wide_blocks < 2 * cus && !a.s1 && a.N % 4 == 0 && ws && a.KT >= 32) {
       double best = 1e30;
       for (int mt = 2; mt <= 4; mt += 2)
         for (int sp = 1; sp <= 16 && sp <= a.KT / 16; ++sp) {
           const int nbm = (M + mt * 32 - 1) / (mt * 32);
           const int gens = (nbn * nbm * sp + cus - 1) / cus;
           const double loop = 1e-4 * gens * (mt * 32) * ((double)K / sp);
-          const double part = sp > 1 ? 0.5e-6 * 4.0 * sp * nbm * (mt * 32) * nbn * tk_wide_cols() : 0.0;
-          const double cost = loop + part + (mt == 2 ? 8.0 : 0.0) + 0.005e-6 * nbm * (double)K * nbn * tk_wide_cols();
-          if (cost < best) best = cost, a.mtiles = mt, ks = sp;
+          const double part = sp > 1 ? 0.5e-6 * 4.0 * sp * nbm * (mt * 32) * nbn * kWideCols : 0.0;
+          const double cost = loop + part + (mt == 2 ? 8.0 : 0.0) + 0.005e-6 * nbm * (double)K * nbn * kWideCols;
+          if (cost < best) best = cost, rows = mt * 32, ks = sp;
         }
     }
-    const int brows = a.mtiles * 32;
-    const int blocks0 = nbn * ((M + brows - 1) / brows);
     if (ks <= 0) {
       // fill the device once; a split keeps at least 16 k tiles and its partials must fit
-      ks = cus / blocks0;
+      if (wide_blocks >= 2 * cus) rows = 64;
+      ks = cus / (nbn * ((M + rows - 1) / rows));
       if (ks > a.KT / 16) ks = a.KT / 16;
       if (ks < 1) ks = 1;
     }
-    const size_t per_split = (size_t)brows * tk_wide_cols() * 4;
+    const size_t per_split = (size_t)M * a.ntiles * 32 * 4;
     if (ks > 1 && ws) {
-      const size_t fit = kPartialBytes / (per_split * blocks0);
-      const size_t have = ws_bytes > kPartialOff ? (ws_bytes - kPartialOff) / (per_split * blocks0) : 0;
-      if ((size_t)ks > fit) ks = (int)fit;
-      if ((size_t)ks > have) ks = (int)have;
-      if (ks < 1) ks = 1;
+      const size_t have = ws_bytes > kPartialOff ? (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes) / per_split : 0;
+      if ((size_t)ks > have) ks = have > 1 ? (int)have : 1;
     }
     if (ks > a.KT) ks = a.KT;
-    if (ks > 1 && (!ws || blocks0 > kMaxCounters)) {
+    if (ks > 1 && !ws) {
       if (split_k > 1) return fail(TK_EWORKSPACE, "gemm: split_k=%d needs a workspace", ks);
       ks = 1;
     }
@@ -272,8 +305,19 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
     a.kt_q = a.KT / ks;
     a.kt_r = a.KT % ks;
     a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
-    a.counters = ks > 1 ? (int*)ws : nullptr;
-    if (tk_launch_gemm_wide(a, st)) return fail(TK_ELAUNCH, "gemm: launch failed (%s)", hipGetErrorString(hipGetLastError()));
+    int tile = 0;
+    if (wide_blocks >= 2 * cus && ks == 1) {
+      // blocks of 64 rows, two per CU, or of 192 / 256 rows, one per CU, where a CU's share of the rows (blocks in a row on
+      // it x rows per block) is no larger than with 64 (measured on the gated 2048 -> 2 x 16384 launch: M=712 90 us on 192
+      // rows, 100 on 256 -- its 384 blocks are one and a half generations; M=512 / 968 / 1024: 256-row blocks)
+      auto share = [&](int rows) { return ((nbn * ((M + rows - 1) / rows) + cus - 1) / cus) * rows; };
+      tile = 28;
+      if (share(192) <= share(64)) tile = 68;
+      if (share(256) < share(192) && share(256) <= share(64)) tile = 88;
+    }
+    const int rounds = ((a.KT + ks - 1) / ks + 1) / 2;
+    if (tk_launch_gemm_wide(a, tile ? tile : pick_tile(kWideTiles, 2.f, 1.15e9f, M, a.ntiles * 32, K, rounds, ks), st))
+      return fail(TK_ELAUNCH, "gemm: launch failed (%s)", hipGetErrorString(hipGetLastError()));
     return TK_OK;
   }
   int MT = M <= 32 ? 1 : 2;
@@ -500,6 +544,7 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   if (M <= 0 || N <= 0 || K <= 0) return fail(TK_EINVAL, "w8a8: non-positive shape M=%d N=%d K=%d", M, N, K);
   if (K % 16) return fail(TK_EINVAL, "w8a8: K=%d must be a multiple of 16", K);
   if (lda % 16 || lda < K) return fail(TK_EINVAL, "w8a8: lda=%d must be >= K and a multiple of 16 (bytes)", lda);
+  if (M > 1 && lda > 1 << 29) return fail(TK_EINVAL, "w8a8: lda=%d, rows of a8 more than 512 MiB apart", lda);
   if (!a8 || !sa || !w_packed || !s0 || !y) return fail(TK_EINVAL, "w8a8: null pointer");
   if (!aligned16(a8) || !aligned16(w_packed) || !aligned16(s0) || (s1 && !aligned16(s1))) return fail(TK_EINVAL, "w8a8: a8, w_packed and the weight scales must be 16-byte aligned");
   if (N % 4 || ldy % 4 || ldy < N || !aligned8(y)) return fail(TK_EINVAL, "w8a8: N=%d and ldy=%d must be multiples of 4, ldy >= N, y 8-byte aligned", N, ldy);
@@ -527,25 +572,22 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.act = act;
   a.vec = 1;
   a.vec16 = ldy % 8 == 0 && aligned16(y) && (!resid || (aligned16(resid) && ldr % (resid_dtype == TK_F32 ? 4 : 8) == 0));
-  // 64-row blocks, two per CU, once the 128-row grid would run in several generations anyway: co-resident blocks
-  // cover each other's first loads and epilogue (gate/up at 712 rows: 73 -> 59 us); few blocks keep the 128-row tile
-  const int blocks128 = ((a.ntiles * 32 + tk_w8a8_cols() - 1) / tk_w8a8_cols()) * ((M + 127) / 128);
-  a.mtiles = blocks128 >= 2 * device_cus() ? 2 : 4;
-  const int rows = a.mtiles * 32;
-  const int blocks0 = ((a.ntiles * 32 + tk_w8a8_cols() - 1) / tk_w8a8_cols()) * ((M + rows - 1) / rows);
+  // K split, from the shape alone (it decides the order of summation)
+  const int blocks128 = ((a.ntiles * 32 + kWideCols - 1) / kWideCols) * ((M + 127) / 128);
+  const int rows = blocks128 >= 2 * device_cus() ? 64 : 128;
   int ks = split_k;
   if (ks <= 0) {
     // fill the device once; a split keeps at least 32 k tiles and its partials must fit
-    ks = device_cus() / blocks0;
+    ks = device_cus() / (((a.ntiles * 32 + kWideCols - 1) / kWideCols) * ((M + rows - 1) / rows));
     if (ks > a.KT / 32) ks = a.KT / 32;
     if (ks < 1) ks = 1;
   }
-  const size_t per_split = (size_t)rows * tk_w8a8_cols() * 4;
+  const size_t per_split = (size_t)M * a.ntiles * 32 * 4;
   if (ks > 1) {
-    const size_t have = ws && ws_bytes > kPartialOff ? (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes) / (per_split * blocks0) : 0;
-    if ((size_t)ks > have || blocks0 > kMaxCounters) {
-      if (split_k > 1) return fail(TK_EWORKSPACE, "w8a8: split_k=%d needs %zu bytes of partial space", ks, per_split * blocks0 * ks);
-      ks = have > 1 && blocks0 <= kMaxCounters ? (int)have : 1;
+    const size_t have = ws && ws_bytes > kPartialOff ? (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes) / per_split : 0;
+    if ((size_t)ks > have) {
+      if (split_k > 1) return fail(TK_EWORKSPACE, "w8a8: split_k=%d needs %zu bytes of partial space", ks, per_split * ks);
+      ks = have > 1 ? (int)have : 1;
     }
   }
   if (ks > a.KT) ks = a.KT;
@@ -553,40 +595,23 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.kt_q = a.KT / ks;
   a.kt_r = a.KT % ks;
   a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
-  a.counters = ks > 1 ? (int*)ws : nullptr;
-  if (tk_launch_w8a8_gemm(a, st)) return fail(TK_ELAUNCH, "w8a8: launch failed (%s)", hipGetErrorString(hipGetLastError()));
+  const int rounds = ((a.KT + ks - 1) / ks + 3) / 4;
+  if (tk_launch_w8a8_gemm(a, pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, a.ntiles * 32, K, rounds, ks), st))
+    return fail(TK_ELAUNCH, "w8a8: launch failed (%s)", hipGetErrorString(hipGetLastError()));
   return TK_OK;
 }
 }  // namespace
 
 // ---- bf16-weight linears with bias / GELU / residual epilogues (vision towers) ---------------------------------
 namespace {
-struct DenseTile {
-  int id, bm, bn;  // block of 32 bm rows x 32 bn columns
-  int wt, ns;      // 32 x 32 tiles of a multiplying wave, buffers in the ring
-  int occ;         // blocks of this shape that fit one CU (LDS)
-  int rope;        // the rotary form exists
-};
-constexpr DenseTile kDenseTiles[] = {{42, 4, 8, 8, 3, 1, 1},  {41, 4, 4, 4, 2, 2, 0},  {32, 3, 8, 6, 3, 1, 1},  {31, 3, 4, 3, 5, 1, 0},  {22, 2, 8, 4, 4, 1, 1},
-                                     {21, 2, 4, 2, 3, 2, 0},  {12, 1, 8, 2, 4, 1, 1},  {11, 1, 4, 1, 4, 2, 0},  {606, 6, 6, 9, 3, 1, 0}, {404, 4, 4, 4, 4, 1, 1},
-                                     {406, 4, 6, 6, 3, 1, 0}, {403, 4, 3, 3, 5, 1, 0}, {204, 2, 4, 2, 6, 1, 1}, {202, 2, 2, 1, 5, 2, 0}};
-
-// Estimated duration (us) of a launch with this tile and K split.  Fitted to 3400 timings (64 shapes of the towers, the
-// prefill and random ones, every tile, splits 1 .. 6; standard error 14 %, the picked launch on average 1.1 % slower than
-// the best one).  Blocks on one CU share its memory pipe (12 ns a KiB) and matrix pipes (75 ns for a wave's tile and
-// round); a round takes no less than the round trip over the rounds on their way; the epilogue costs per tile; each
-// further generation of blocks pays all of it again.
-float dense_cost(const DenseTile& t, int M, int N, int KT, int ks, int cus) {
-  const int rows = 32 * t.bm, cols = 32 * t.bn, rounds = ((KT + ks - 1) / ks + 1) / 2;
-  const long long blocks = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * ks;
-  float us = 1.66f;
-  for (long long left = blocks; left > 0; left -= (long long)cus * t.occ) {
-    const float r = left > cus && t.occ > 1 ? 2.f : 1.f;  // blocks on a CU
-    const float load = r * (float)(t.bm + t.bn) * 4.f * 0.0122f, mul = r * (float)t.wt * 0.0751f, trip = 0.585f / (float)(t.ns - 1);
-    us += 0.014f + (float)rounds * (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip)) + r * (float)(t.bm * t.bn) * 0.203f;
-  }
-  if (ks > 1) us += 4.76f + (float)blocks * (float)(t.bm * t.bn) * 0.00213f;  // fp32 partials out and back in
-  return us;
+constexpr PipeTile kDenseTiles[] = {{42, 4, 8, 8, 3, 1},  {41, 4, 4, 4, 2, 2},  {32, 3, 8, 6, 3, 1},  {31, 3, 4, 3, 5, 1},  {22, 2, 8, 4, 4, 1},
+                                    {21, 2, 4, 2, 3, 2},  {12, 1, 8, 2, 4, 1},  {11, 1, 4, 1, 4, 2},  {606, 6, 6, 9, 3, 1}, {404, 4, 4, 4, 4, 1},
+                                    {406, 4, 6, 6, 3, 1}, {403, 4, 3, 3, 5, 1}, {204, 2, 4, 2, 6, 1}, {202, 2, 2, 1, 5, 2}};
+constexpr int kDenseRopeTiles[] = {42, 32, 22, 12, 404, 204};  // two n tiles per wave: the rotary form
+bool dense_rope_tile(int id) {
+  for (int t : kDenseRopeTiles)
+    if (t == id) return true;
+  return false;
 }
 }  // namespace
 
@@ -674,16 +699,16 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
     a.vt_bs = vt->bs;
   }
   const int cus = device_cus();
-  const DenseTile* best = nullptr;
+  const PipeTile* best = nullptr;
   int ks = split_k > 0 ? split_k : 1;
   float best_cost = 0.f;
-  for (const DenseTile& t : kDenseTiles) {
+  for (const PipeTile& t : kDenseTiles) {
     if (tile && t.id != tile) continue;
-    if (rope && !t.rope) continue;  // the rotary epilogue needs two n tiles per wave
+    if (rope && !dense_rope_tile(t.id)) continue;
     // a split keeps at least 16 k tiles; none in the rotary form unless asked for (the partials weigh more than the idle CUs)
     const int most = split_k > 0 || rope || a.KT < 32 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
     for (int k1 = split_k > 0 ? split_k : 1, n = 0; n < most; ++k1, ++n) {
-      const float c = dense_cost(t, M, N, a.KT, k1, cus);
+      const float c = pipe_cost(t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus);
       if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
     }
   }

@@ -58,18 +58,12 @@ struct GemmArgs {
   // bf16-weight many-row kernel only: bf16 [N] bias added to the accumulator, or nullptr; there act is
   // 0 none, 1 tanh-GELU of the bf16-rounded pre-activation, 2 tanh-GELU of the fp32 pre-activation
   const unsigned short* bias;
-  // many-row fp8 kernels: 32-row tiles per block, chosen by the host (2 / 4: four-wave blocks; 6 / 8: eight-wave
-  // blocks with both operands through LDS, weight-only kernel)
-  int mtiles;
   // many-row 16-bit-weight kernel only: activations, weights, bias, output and a 16-bit residual are fp16, not bf16
   int f16;
   // single-launch gated FFN only: the hand-off words in the workspace (TK_FUSE_* below), the down blocks per row
   // block, and the bound on a down block's wait (polls)
   int* fuse;
   int fuse_consumers, fuse_spin;
-  // many-row fp8 kernels, K splits of a plain launch: 1 = every block leaves its fp32 partial in `partial` and ends;
-  // a second launch (all CUs, not one block per output tile) sums them in split order and runs the epilogue
-  int split_reduce;
 };
 // int32 words of the single-launch FFN's hand-off: a flag per (row block, gate/up strip), the number of down blocks
 // past their wait per row block, then the sticky error word
@@ -274,8 +268,8 @@ int tk_tail_embed_width();  // the embedding's input width the tail kernel is bu
 int tk_launch_kv_proj(KvProjArgs a, hipStream_t st);
 int tk_layer_norm_max_k();
 int tk_launch_layer_norm(LayerNormArgs a, hipStream_t st);
-int tk_wide_cols();  // columns of the many-row GEMM's block tile (rows: 32 * GemmArgs::mtiles)
-int tk_launch_gemm_wide(GemmArgs a, hipStream_t st);
+// many-row fp8-weight GEMM; tile: an id of kWideTiles (tk_api.hip)
+int tk_launch_gemm_wide(const GemmArgs& a, int tile, hipStream_t st);
 int tk_launch_norm_rows(NormRowsArgs a, hipStream_t st);
 int tk_launch_gemm(GemmArgs a, int MT, int NT, int mblocks, hipStream_t st);
 // the action chunk's gated FFN in one launch (32-row blocks; g: the gate/up half without a K split, d: the down half
@@ -286,10 +280,9 @@ int tk_launch_ffn_fused(GemmArgs g, GemmArgs d, int d_nt, int mblocks, hipStream
 bool tk_gemm_stream_takes(const GemmArgs& a);
 int tk_launch_gemm_stream(GemmArgs a, hipStream_t st);
 int tk_launch_gemm_stream_cut(GemmArgs a, int cut, hipStream_t st);  // measurement forms, nothing stored
-// W8A8 tier: per-token activation quantisation and the fp8 x fp8 many-row GEMM (block tile 32 * mtiles x tk_w8a8_cols())
-int tk_w8a8_cols();
+// W8A8 tier: per-token activation quantisation and the fp8 x fp8 many-row GEMM (tile: an id of kW8a8Tiles, tk_api.hip)
 int tk_quant_act_max_k();
-int tk_launch_w8a8_gemm(GemmArgs a, hipStream_t st);
+int tk_launch_w8a8_gemm(const GemmArgs& a, int tile, hipStream_t st);
 int tk_launch_quant_act_rows(QuantActArgs a, hipStream_t st);
 int tk_launch_pack(const void* w0, const void* w1, void* out, int N, int K, int interleave, hipStream_t st);
 int tk_launch_pack_bf16(const void* w, void* out, int N, int K, int pair_off, hipStream_t st);
