@@ -4,9 +4,10 @@
 // Bound: latency, then the bytes a compute unit takes in.  A step reads 397 MB of weights (80 us at 5 TB/s) and its
 // eighteen layers are 108 dependent phases of 0.3 - 1.5 us of work each; as five launches a layer they took 47 us a layer.
 // Here 256 resident blocks run the phases back to back: block (rt, c) works on 16 of the chunk's rows with column share c
-// of 64.  Measured (50 action tokens, two cameras and 200 language tokens, 10 steps): the loop 8.5 -> 4.4 ms, 24 us a
-// layer (stamps of every block, mean): 1.7 - 2.4 us from a phase's result to the next one's input, 3.8 us into PC; from
-// there to the result 0.75 us in PC, 1.0 - 2.1 us in the others; 0.8 MB through each compute unit.
+// of 64.  Measured (50 action tokens, two cameras and 200 language tokens, 10 steps): the loop 8.5 -> 4.4 ms with weights
+// asked for at the ends of the phases (24 us a layer; stamps of every block, mean: 1.7 - 2.4 us from a phase's result to
+// the next one's input, 3.8 us into PC behind 128 KiB of weights; from there to the result 0.75 us in PC, 1.0 - 2.1 us in
+// the others), 3.9 ms (21 us) as below; 0.8 MB through each compute unit.
 //
 //   step    E0  v = final_norm(x) . Wa^T + b, x_t += dt v         32 blocks per row group, one action column each
 //           E1  hidden = x_t . Wi^T + b                           64 blocks, 16 columns each
@@ -23,10 +24,16 @@
 // Place: blocks land round-robin on the eight XCDs, so block i = 64 rt + c puts the row groups' blocks of one column share
 // on one XCD: the weights, which are too many for any cache above the XCD's, come there once for four blocks, and a
 // key split for 32.  A row group on two XCDs of its own (hand-offs 0.3 us shorter) took 2 us a layer more.
-// Weights and keys ahead: asked for at the end of the phase one or two hand-offs before theirs, 64 - 128 KiB at a time; by
-// then most waves only wait.  Asked for in the middle of a phase, their issue alone stands before the phase's result
-// (26 us a layer).  128 registers a wave is what holds them: loads under a
-// branch, or carried into the next layer under one, were spilled as they arrived (31 us).
+// Weights and keys ahead: loads that the memory pipe still works on stand before the next hand-off's looks, so each set is
+// asked for where the fewest of them are on that path (the loop with three cameras, ms).
+//   * Between a phase's products and the barrier of its reduction: the values in P1 (3.90; at its arrival 4.00, at the end
+//     of P5 4.11), P5's weights in P4 (3.90; behind the barrier 4.05, at the arrival 4.01, at the end of P3 4.05).
+//   * At PC's arrival: P3's weights (at the end of P2 with half of P4's, 128 KiB stood in front of PC's input: 4.45 -> 4.28;
+//     in front of PC's barrier 4.18 against 4.11).
+//   * At a phase's end: the keys (P1), P4's weights (PC), P1's (P4; anywhere in P5 0.3 - 0.6 more).
+// With all weights in the XCD's L2 already it would be 0.4 less, but touching them there ahead of time (a load per line, by
+// waves that wait at a gate) costs 0 - 0.25.  128 registers a wave is what holds them: loads under a branch, or carried
+// into the next layer under one, were spilled as they arrived (31 us a layer).
 // Keys: one block per head would read 780 KiB; eight splits of at most five tiles of 32 keys keep that at 96 KiB (two
 // cameras).
 //
@@ -319,7 +326,6 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
   block_barrier();
   load_A(0, 0);
   load_A2(0);
-  load_V(0);
 
   for (int step = 0; step <= a.steps; ++step) {
     const int cur = PW_B + (step & 1) * HEAD_B, oth = PW_B + ((step + 1) & 1) * HEAD_B;
@@ -421,6 +427,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         for (int t = 0; t < 4; ++t)
           if (t < 2 || c < 16) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = acc[t];
         take_stats(st, in_base);
+        load_V(l);
         block_barrier();
         if (tid < 128 || (tid < 256 && c < 8)) {
           const Own ow = own_of(tid);
@@ -553,8 +560,6 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
           st_x(cx.rs, __float_as_uint(s), tid * 64 + (c & 7) * 8 + 4, base + st_s());
         }
         pin();
-        load_B(step, l);
-        load_C(l, 0);
       }
       // ---------------- PC: the splits' outputs into 32 columns of the head ----------------
       fresh();
@@ -566,6 +571,9 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         wait_x<2>(v, cx, voff, soff, [] {});
         arrived();
         announce(id_of(step, l, PH_PC));
+        pin();
+        load_B(step, l);
+        pin();
         // this lane: splits 2 g, 2 g + 1 of row r
         const float m0 = __int_as_float(v[1][0]), l0 = __int_as_float(v[1][1]), m1 = __int_as_float(v[1][2]), l1 = __int_as_float(v[1][3]);
         float mx = fmaxf(m0, m1);
@@ -583,6 +591,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         }
         buf ^= 1;
         pin();
+        load_C(l, 0);
         load_CS(step, l);
         load_C(l, 1);
       }
@@ -606,7 +615,6 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         }
         buf ^= 1;
         pin();
-        load_D(step, l);
       }
       // ---------------- P4: gate / up ----------------
       fresh();
@@ -630,6 +638,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = acc[t];
         take_stats(st, base + OFF_X1);
+        load_D(step, l);
         block_barrier();
         if (tid < 512) {
           const Own ow = own_of(tid);
@@ -670,7 +679,6 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         }
         buf ^= 1;
         pin();
-        load_V(nl);
       }
       // ---- back to all ones: the words of the layer before (this layer's P5 input is made of what every block of the
       // group, and through the keys and values every group, produced after reading them); they are written again three
