@@ -290,3 +290,15 @@ def test_dense_activation_in_more_block_shapes(tk, tile, act):
     x, w, b = _case(300, 1152, 648, seed=1)
     got = tk.bf16w_dense(x.cuda(), tk.pack_bf16_weight(w.cuda()), b.cuda(), act, tile=tile)
     _close(got, _want(x, w, b, act), f"dense {act} tile={tile}", frac_exact=0.95)
+
+
+def test_rows_of_x_more_than_4_gib_of_lane_offset_apart(tk):
+    # eight rows share a load's scalar base and 32-bit lane offsets: rows 1 GiB apart take addresses of their own
+    m, k, n, ld = 9, 208, 96, (1 << 29) + 8
+    x, w, b = _case(m, k, n, seed=5)
+    far = torch.empty((m - 1) * ld + k, dtype=BF16, device="cuda").as_strided((m, k), (ld, 1))
+    far.copy_(x)
+    pw = tk.pack_bf16_weight(w.cuda())
+    near = tk.bf16w_dense(x.cuda(), pw, b.cuda())
+    assert torch.equal(tk.bf16w_dense(far, pw, b.cuda()), near)
+    _close(near, _want(x, w, b), "rows far apart")

@@ -167,3 +167,14 @@ def test_w8a8_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
     got = tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split, resid=r.cuda())
     assert torch.equal(got.cpu(), want)
     assert torch.equal(tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split).cpu(), y)
+
+
+def test_w8a8_rows_more_than_4_gib_of_lane_offset_apart(tk):
+    m, k, n, ld = 9, 208, 96, 1 << 30  # (eight rows share a load's scalar base and 32-bit lane offsets otherwise)
+    g = torch.Generator().manual_seed(3)
+    a = torch.randint(-3, 4, (m, k), generator=g).float()
+    w = torch.randint(-2, 3, (n, k), generator=g).float()
+    far = torch.empty((m - 1) * ld + k, dtype=torch.uint8, device="cuda").as_strided((m, k), (ld, 1))
+    far.copy_(a.to(torch.float8_e4m3fn).view(torch.uint8))
+    pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), torch.ones(n).cuda())
+    assert torch.equal(tk.w8a8_gemm(far, torch.ones(m).cuda(), pw).cpu(), (a @ w.t()).to(BF16))

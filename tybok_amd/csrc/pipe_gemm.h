@@ -35,6 +35,10 @@ __device__ __forceinline__ void lds_barrier() {
 __device__ __forceinline__ void dma16(unsigned voff, const void* base, unsigned lds) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(voff), "s"(base), "s"(lds) : "memory", "m0");
 }
+// the same from an address per lane, for rows of x too far apart for a 32-bit offset
+__device__ __forceinline__ void dma16_far(const void* p, unsigned lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(p), "s"(lds) : "memory", "m0");
+}
 // at most `rounds` (<= MAXR) rounds of I loads each are still on their way
 template <int I, int MAXR>
 __device__ __forceinline__ void load_wait(int rounds) {
@@ -109,6 +113,8 @@ struct Pipe {
     // 8q + l / 8, which holds the line's chunk (l % 8) ^ swz(row)
     const char* xp[AI];  // the eight rows' first column of this block's k range, then on
     unsigned xv[AI];     // the lane's chunk from there
+    const bool far = (unsigned long long)a.ldx * (7 * XE) + 128 > 0xffffffffull;  // xv: within the row, xd: rows down
+    int xd[AI];
     unsigned xfix[2];    // last round: lanes whose chunk is past the k range take the round's first one (zeroed in LDS)
 #pragma unroll
     for (int i = 0; i < AI; ++i) {
@@ -116,7 +122,8 @@ struct Pipe {
       const int b0 = r0 < a.M ? r0 : a.M - 1;  // rows past M: valid data, never stored
       const int m = r0 + rl < a.M ? r0 + rl : a.M - 1;
       xp[i] = (const char*)a.x + ((size_t)b0 * a.ldx + t.kt_lo * 32) * XE;
-      xv[i] = (unsigned)(m - b0) * (unsigned)a.ldx * XE + ch * 16;
+      xd[i] = m - b0;
+      xv[i] = (far ? 0u : (unsigned)xd[i] * (unsigned)a.ldx * XE) + ch * 16;
       if (i < 2) xfix[i] = k_last + ch * CPC < k_end ? 0 : ch * 16;
     }
     // W: instruction i brings KiB q % PW of the round of n tile q / PW, q = i * NW + lw
@@ -137,7 +144,9 @@ struct Pipe {
       const bool last = r == nrounds - 1;
 #pragma unroll
       for (int i = 0; i < AI; ++i) {
-        dma16(last ? xv[i] - xfix[i & 1] : xv[i], xp[i], lds0 + (unsigned)(ibuf + (lw * AI + i) * 1024));
+        const unsigned v = last ? xv[i] - xfix[i & 1] : xv[i], to = lds0 + (unsigned)(ibuf + (lw * AI + i) * 1024);
+        if (far) dma16_far(xp[i] + (size_t)xd[i] * a.ldx * XE + v, to);
+        else dma16(v, xp[i], to);
         xp[i] += 128;
       }
 #pragma unroll

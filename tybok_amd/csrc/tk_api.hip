@@ -247,7 +247,6 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
       (!has_norm || (ws && ws_bytes >= kNormOff + (size_t)M * K * 2 && (size_t)M * K * 2 <= kNormBytes))) {
     // many rows
     if (plan) return TK_OK;  // (plan->skinny stays false)
-    if (ldx > 1 << 28) return fail(TK_EINVAL, "gemm: ldx=%d, rows of x more than 512 MiB apart", ldx);
     if (has_norm) {
       NormRowsArgs nr;
       nr.x = (const u16*)x;
@@ -544,7 +543,6 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   if (M <= 0 || N <= 0 || K <= 0) return fail(TK_EINVAL, "w8a8: non-positive shape M=%d N=%d K=%d", M, N, K);
   if (K % 16) return fail(TK_EINVAL, "w8a8: K=%d must be a multiple of 16", K);
   if (lda % 16 || lda < K) return fail(TK_EINVAL, "w8a8: lda=%d must be >= K and a multiple of 16 (bytes)", lda);
-  if (M > 1 && lda > 1 << 29) return fail(TK_EINVAL, "w8a8: lda=%d, rows of a8 more than 512 MiB apart", lda);
   if (!a8 || !sa || !w_packed || !s0 || !y) return fail(TK_EINVAL, "w8a8: null pointer");
   if (!aligned16(a8) || !aligned16(w_packed) || !aligned16(s0) || (s1 && !aligned16(s1))) return fail(TK_EINVAL, "w8a8: a8, w_packed and the weight scales must be 16-byte aligned");
   if (N % 4 || ldy % 4 || ldy < N || !aligned8(y)) return fail(TK_EINVAL, "w8a8: N=%d and ldy=%d must be multiples of 4, ldy >= N, y 8-byte aligned", N, ldy);
@@ -638,7 +636,6 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
                  int f16, const DenseRope* rope = nullptr, const DenseVt* vt = nullptr) {
   if (M <= 0 || N <= 0 || K <= 0) return fail(TK_EINVAL, "bf16w_dense: non-positive shape M=%d N=%d K=%d", M, N, K);
   if (K % 16 || ldx % 8 || ldx < K) return fail(TK_EINVAL, "bf16w_dense: K=%d must be a multiple of 16 and ldx=%d a multiple of 8 >= K", K, ldx);
-  if (M > 1 && ldx > 1 << 28) return fail(TK_EINVAL, "bf16w_dense: ldx=%d, rows of x more than 512 MiB apart", ldx);
   if (!x || !w_packed || !y) return fail(TK_EINVAL, "bf16w_dense: null pointer");
   if (!aligned16(x) || !aligned16(w_packed) || !aligned16(y) || (bias && !aligned8(bias)))
     return fail(TK_EINVAL, "bf16w_dense: x, w_packed and y must be 16-byte aligned, bias 8-byte aligned");
