@@ -24,10 +24,12 @@
 // weight, beside the row's partial sums of squares; 1 / rms is a factor of the whole row and multiplies the accumulator.
 // The residual stream never leaves its owner's registers and stays fp32 there.
 //
-// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.55 ms, against 4.7 ms of the launches per layer.
+// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.48 ms, against 4.7 ms of the launches per layer.
 // A layer takes 16 us (stamps of every block, mean): 1.2 - 2.0 us from a phase's result to the next one's input, and from
 // there to the result 2.8 us in the attention, 1.2 - 1.6 us in the others; in a cross layer's attention 5.2 us, 4.0 of them
-// until the scores are there: its blocks load 216 KiB (query weights, K and V hi + lo planes).
+// until the scores are there: its blocks load 216 KiB (query weights, K and V hi + lo planes).  Where those are asked for
+// (the loop, ms): weights and K in front of the gate, V behind the query reduction's barrier 2.48; V in front of that
+// barrier 2.55, behind the next one 2.53, in front of the gate 2.75; K's lo plane or both behind the gate 2.53 - 2.65.
 #include <math.h>
 
 #include <atomic>
@@ -642,10 +644,10 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = acc[t];
         take_stats(st, in_base);
-        pin();
+        block_barrier();
         load_V(vf, l, false);
         load_V(vl, l, true);
-        block_barrier();
+        pin();
         if (tid < 256) {
           const Own ow = own_of(tid);
           const float rstd = rstd_of(ow.m);
