@@ -21,7 +21,8 @@ _BF16, _F32 = 0, 1
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle alone: building torch's Stream object around it takes 2.7 us, a quarter of a single-row linear's call
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -154,11 +155,12 @@ def pack_fp8_gate_up(wg8: torch.Tensor, sg: torch.Tensor, wu8: torch.Tensor, su:
 
 
 def _check_act(x: torch.Tensor, k: int) -> tuple[int, int]:
-    if x.dtype != torch.bfloat16 or not x.is_cuda:
+    if x.dtype is not torch.bfloat16 or not x.is_cuda:
         raise TypeError("activations must be bf16 CUDA tensors")
-    if x.dim() != 2 or x.shape[1] != k or x.stride(1) != 1:
-        raise ValueError(f"activations must be [M, {k}] with unit inner stride, got {tuple(x.shape)}")
-    return x.shape[0], x.stride(0)
+    shape, stride = x.shape, x.stride()
+    if len(shape) != 2 or shape[1] != k or stride[1] != 1:
+        raise ValueError(f"activations must be [M, {k}] with unit inner stride, got {tuple(shape)}")
+    return shape[0], stride[0]
 
 
 def _resid_args(resid: torch.Tensor | None, m: int, n: int) -> tuple[int | None, int, int]:
@@ -559,6 +561,14 @@ def _eff_strides(t: torch.Tensor) -> tuple[int, int]:
     return (t.stride(0) if t.shape[0] > 1 else 0, t.stride(1) if t.shape[1] > 1 else 0)
 
 
+def _vt_ok(vt: torch.Tensor, stride: tuple[int, ...], g: int, d: int, length: int) -> bool:
+    shape = vt.shape
+    return vt.dtype is torch.bfloat16 and len(shape) == 3 and shape[0] == g and shape[1] == d and stride[2] == 1 and shape[2] >= _pad32(length)
+
+
+_MASK_TYPES = (torch.uint8, torch.bool)
+
+
 def _same_layout(k: torch.Tensor, v: torch.Tensor) -> bool:
     return k.shape == v.shape and k.stride(2) == 1 and v.stride(2) == 1 and _eff_strides(k) == _eff_strides(v)
 
@@ -686,58 +696,60 @@ def expert_attn(
     ``[P]`` or None; ``mask2d``: uint8/bool ``[M, >= P rounded up to 32]`` per-(query, prefix key)
     visibility, replaces ``prefix_pad``.  Returns bf16 ``[M, H*D]``."""
     lib = native.lib()
-    if q.dtype != torch.bfloat16 or q.dim() != 3 or q.stride(2) != 1:
+    bf = torch.bfloat16
+    q_st = q.stride()
+    if q.dtype is not bf or len(q_st) != 3 or q_st[2] != 1:
         raise TypeError("q must be bf16 [M, H, D] with a contiguous head dim")
     m, h, d = q.shape
-    bf = torch.bfloat16
-
-    def _vt_ok(vt: torch.Tensor, g: int, length: int) -> bool:
-        return vt.dtype == bf and vt.dim() == 3 and vt.shape[:2] == (g, d) and vt.stride(2) == 1 and vt.shape[2] >= _pad32(length)
-
+    # (shapes and strides are read once per tensor: each is a call into torch, and together they cost more than the launch)
     p = g = 0
     kp = kpl = vp = vpl = None
     pre_sl = pre_sh = pre_sd = pre_vsh = 0
     if prefix is not None:
-        p, g = prefix.k.shape[0], prefix.k.shape[1]
-        if prefix.k.dtype != bf or prefix.k.shape[2] != d or prefix.k.stride(2) != 1 or not _vt_ok(prefix.vt, g, p):
+        k, vt = prefix.k, prefix.vt
+        k_st, vt_st = k.stride(), vt.stride()
+        p, g, kd = k.shape
+        if k.dtype is not bf or kd != d or k_st[2] != 1 or not _vt_ok(vt, vt_st, g, d, p):
             raise ValueError("prefix must hold bf16 K [P, G, D] and V^T [G, D, >= P rounded up to 32]")
-        pre_sl, pre_sh = _eff_strides(prefix.k)
-        pre_vsh, pre_sd = prefix.vt.stride(0) if g > 1 else 0, prefix.vt.stride(1)
-        kp, vp = prefix.k.data_ptr(), prefix.vt.data_ptr()
+        pre_sl, pre_sh = k_st[0] if p > 1 else 0, k_st[1] if g > 1 else 0
+        pre_vsh, pre_sd = vt_st[0] if g > 1 else 0, vt_st[1]
+        kp, vp = k.data_ptr(), vt.data_ptr()
         if prefix.k_lo is not None:
-            if prefix.vt_lo is None or prefix.k_lo.stride() != prefix.k.stride() or prefix.vt_lo.stride() != prefix.vt.stride():
+            if prefix.vt_lo is None or prefix.k_lo.stride() != k_st or prefix.vt_lo.stride() != vt_st:
                 raise ValueError("low planes must mirror the high planes' layout")
             kpl, vpl = prefix.k_lo.data_ptr(), prefix.vt_lo.data_ptr()
     s = 0
     ks = vs = None
     suf_sl = suf_sh = suf_sd = suf_vsh = 0
     if suffix is not None:
-        s, gs = suffix.k.shape[0], suffix.k.shape[1]
+        k, vt = suffix.k, suffix.vt
+        k_st, vt_st = k.stride(), vt.stride()
+        s, gs, kd = k.shape
         if prefix is not None and gs != g:
             raise ValueError("prefix and suffix must have the same number of kv heads")
         g = gs
-        if suffix.k.dtype != bf or suffix.k.shape[2] != d or suffix.k.stride(2) != 1 or not _vt_ok(suffix.vt, g, s):
+        if k.dtype is not bf or kd != d or k_st[2] != 1 or not _vt_ok(vt, vt_st, g, d, s):
             raise ValueError("suffix must hold bf16 K [S, G, D] and V^T [G, D, >= S rounded up to 32]")
-        suf_sl, suf_sh = _eff_strides(suffix.k)
-        suf_vsh, suf_sd = suffix.vt.stride(0) if g > 1 else 0, suffix.vt.stride(1)
-        ks, vs = suffix.k.data_ptr(), suffix.vt.data_ptr()
+        suf_sl, suf_sh = k_st[0] if s > 1 else 0, k_st[1] if g > 1 else 0
+        suf_vsh, suf_sd = vt_st[0] if g > 1 else 0, vt_st[1]
+        ks, vs = k.data_ptr(), vt.data_ptr()
     pad = None
     if prefix_pad is not None:
-        pad = prefix_pad.view(torch.uint8) if prefix_pad.dtype == torch.bool else prefix_pad
-        if pad.dtype != torch.uint8 or pad.numel() != p or not pad.is_contiguous():
+        # (bool and uint8 are one byte each: no view of one as the other is needed to pass its address)
+        if prefix_pad.dtype not in _MASK_TYPES or prefix_pad.numel() != p or not prefix_pad.is_contiguous():
             raise ValueError("prefix_pad must be a contiguous uint8/bool [P]")
+        pad = prefix_pad.data_ptr()
     m2_p, m2_ld = None, 0
     if mask2d is not None:
-        m2 = mask2d.view(torch.uint8) if mask2d.dtype == torch.bool else mask2d
-        if m2.dtype != torch.uint8 or m2.dim() != 2 or m2.shape[0] != m or m2.stride(1) != 1 or m2.shape[1] < _pad32(p):
+        if mask2d.dtype not in _MASK_TYPES or mask2d.dim() != 2 or mask2d.shape[0] != m or mask2d.stride(1) != 1 or mask2d.shape[1] < _pad32(p):
             raise ValueError("mask2d must be uint8/bool [M, >= P rounded up to 32] with unit inner stride")
-        m2_p, m2_ld = m2.data_ptr(), m2.stride(0)
+        m2_p, m2_ld = mask2d.data_ptr(), mask2d.stride(0)
     if out is None:
         out = torch.empty(m, h * d, dtype=bf, device=q.device)
     ws = ws or default_workspace(q.device)
     rc = lib.tk_expert_attn(
-        q.data_ptr(), q.stride(0), q.stride(1), kp, kpl, pre_sl, pre_sh, vp, vpl, pre_sd, pre_vsh, ks, suf_sl, suf_sh,
-        vs, suf_sd, suf_vsh, _ptr(pad), m2_p, m2_ld, out.data_ptr(), out.stride(0), m, p, s, h, max(g, 1), d, mask_mode,
+        q.data_ptr(), q_st[0], q_st[1], kp, kpl, pre_sl, pre_sh, vp, vpl, pre_sd, pre_vsh, ks, suf_sl, suf_sh,
+        vs, suf_sd, suf_vsh, pad, m2_p, m2_ld, out.data_ptr(), out.stride(0), m, p, s, h, max(g, 1), d, mask_mode,
         int(logits_bf16), ws.ptr, ws.nbytes, _stream(),
     )  # fmt: skip
     native.check(rc, "tk_expert_attn")
