@@ -467,3 +467,20 @@ def test_attention_over_the_suffix_alone_and_with_whole_key_tiles_masked(tk, h, 
     want = oops.expert_attention(q, k_pre, v_pre, k_suf, v_suf, pad, mode, bf16_logits=bl)
     got = tk.expert_attn_plain(q.cuda(), k_pre.cuda(), v_pre.cuda(), k_suf.cuda(), v_suf.cuda(), pad.cuda(), mode, logits_bf16=bl)
     _close(got, want, f"attention with whole key tiles masked D={d}")
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("k", [8, 512, 520, 1024, 1032, 1536, 1544, 2048])
+def test_layer_norms_at_the_edges_of_their_load_counts(tk, dtype, k):
+    # one more 16-byte piece per lane from 512 columns to the next: full and nearly empty last pieces.  A constant row (no
+    # variance) gives b; what lies behind the rows of a wider buffer is NaN and must not enter a sum.
+    g = torch.Generator().manual_seed(k)
+    wide = torch.full((5, k + 16), float("nan"))
+    wide[:, :k] = torch.randn(5, k, generator=g) * 3.0 + 1.0
+    wide[3, :k] = 2.5
+    x, w, b = wide.to(dtype), (torch.rand(k, generator=g) + 0.5).to(dtype), torch.randn(k, generator=g).to(dtype)
+    want = torch.nn.functional.layer_norm(x[:, :k].double(), (k,), w.double(), b.double(), 1e-6)
+    got = tk.layer_norm(x.cuda()[:, :k], w.cuda(), b.cuda(), 1e-6).double().cpu()
+    # half a bf16 ulp of the result and, before it, fp32 sums of k terms of size < 16 (relative 2^-24 each, k <= 2^11)
+    assert bool(((got - want).abs() <= 2**-8 * want.abs() + 2e-3).all())
+    assert torch.equal(got[3], b.to(torch.bfloat16).double() if dtype == torch.float32 else b.double())

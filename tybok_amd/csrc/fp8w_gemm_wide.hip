@@ -569,8 +569,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(NormRowsArgs a) {
     square(xu.h);
   }
   float ss = ss0 + ss1;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+  ss = wave_sum(ss);
   if ((tid & 63) == 0) part[tid >> 6] = ss;
   __syncthreads();
   ss = (part[0] + part[1]) + (part[2] + part[3]);

@@ -132,6 +132,39 @@ __device__ __forceinline__ float gelu_tanh_rcp_f(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(b, x * x, a)));
 }
 
+// What a lane and the one 32 (16) away from it hold, in both of them: one vector instruction where __shfl_xor is a trip
+// through the LDS pipe (60 ns), for sums and maxima (same bits: both are commutative).
+__device__ __forceinline__ f32x2 both32(float v) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f32x2{__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+__device__ __forceinline__ f32x2 both16(float v) {
+  typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+  const u32x2 s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f32x2{__uint_as_float(s[0]), __uint_as_float(s[1])};
+}
+__device__ __forceinline__ float sum32(float v) { const f32x2 b = both32(v); return b[0] + b[1]; }
+__device__ __forceinline__ float sum16(float v) { const f32x2 b = both16(v); return b[0] + b[1]; }
+__device__ __forceinline__ float max32(float v) { const f32x2 b = both32(v); return fmaxf(b[0], b[1]); }
+__device__ __forceinline__ float max16(float v) { const f32x2 b = both16(v); return fmaxf(b[0], b[1]); }
+// Sum over groups of W consecutive lanes, the same additions as v += __shfl_xor(v, o) for o = W / 2, W / 4, .. 1 (bit for bit).
+template <int W = 64>
+__device__ __forceinline__ float wave_sum(float v) {
+  static_assert(W == 64 || W == 32 || W == 16 || W == 8 || W == 4 || W == 2 || W == 1, "a power of two up to the wave");
+  if (W > 32) v = sum32(v);
+  if (W > 16) v = sum16(v);
+  if (W > 8) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));  // lane ^ 8: rotated by 8 in its row
+  if (W > 4) {  // lane ^ 4: from 4 above in the even quads, from 4 below in the odd ones
+    int t = __builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x104, 0xf, 0x5, false);
+    t = __builtin_amdgcn_update_dpp(t, __float_as_int(v), 0x114, 0xf, 0xa, false);
+    v += __int_as_float(t);
+  }
+  if (W > 2) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4e, 0xf, 0xf, true));  // lane ^ 2
+  if (W > 1) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));  // lane ^ 1
+  return v;
+}
+
 // Device-coherent (agent-scope, cache write-through / cache-bypassing) accesses used for data that
 // one block hands to another inside a kernel: with them the hand-off needs no L2 flush.
 __device__ __forceinline__ void st_agent(float* p, float v) {
