@@ -178,3 +178,26 @@ def test_w8a8_rows_more_than_4_gib_of_lane_offset_apart(tk):
     far.copy_(a.to(torch.float8_e4m3fn).view(torch.uint8))
     pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), torch.ones(n).cuda())
     assert torch.equal(tk.w8a8_gemm(far, torch.ones(m).cuda(), pw).cpu(), (a @ w.t()).to(BF16))
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("k", [8, 2048, 2056, 4104, 8200, 16384])
+def test_activation_quantisation_at_the_edges_of_the_quotient(tk, k, mode):
+    # every piece count of a row, a row of all finite bf16 magnitudes, signed zeros, scales at and beyond the range in which
+    # the quotient comes from the reciprocal; whole rows of one scale each (none that rounds to 0, where a quotient has no value).  Infinities and NaN: as the division gives them.
+    g = torch.Generator().manual_seed(k)
+    rows = [torch.randn(k, generator=g) * 2.0**e for e in (-110, -100, -81, -72, -71, -70, -20, 0, 20, 70, 88, 89, 90, 100, 118)]
+    codes = 0x7F7F - torch.arange(k, dtype=torch.int32) * 7 % 0x7F00
+    rows.append(codes.to(torch.int16).view(BF16).float())
+    rows.append(torch.where(torch.arange(k) % 3 == 0, -0.0, torch.randn(k, generator=g)))
+    x = torch.stack(rows).to(BF16)
+    a8, sa = tk.quant_act_rows(x.cuda(), mode)
+    want8, want_s = oops.quantize_activation_rows(x, "bf16" if mode else "fp32")
+    assert torch.equal(sa.cpu(), want_s) and torch.equal(a8.cpu().view(torch.uint8), want8.view(torch.uint8))
+    odd = torch.randn(3, k, generator=g).to(BF16)
+    odd[0, 1], odd[1, 2], odd[2, 3], odd[2, 4] = float("inf"), float("-inf"), float("nan"), float("inf")
+    a8, sa = tk.quant_act_rows(odd.cuda(), mode)
+    s = odd.float().abs().nan_to_num(0.0, float("inf")).amax(1) / 448  # (a maximum passes NaN by)
+    q = odd.float() / s[:, None]
+    got = a8.cpu().view(torch.float8_e4m3fn).float()
+    assert torch.equal(sa.cpu(), s) and torch.equal(got.isnan(), q.isnan()) and bool((got[~q.isnan()] == 0).all())
