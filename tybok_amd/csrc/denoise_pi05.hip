@@ -522,8 +522,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
           p[e] = (vis >> (8 + e)) & 1u ? ((vis >> e) & 1u ? sv : sv + kOpenpiMask) : -INFINITY;
           tmax = fmaxf(tmax, p[e]);
         }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+        tmax = max16(tmax);
+        tmax = max32(tmax);
         if (lane < 16) sM[wave * 16 + r] = tmax;
         block_barrier();
         announce(id_of(step, l, PH_P2));
@@ -577,8 +577,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         // this lane: splits 2 g, 2 g + 1 of row r
         const float m0 = __int_as_float(v[1][0]), l0 = __int_as_float(v[1][1]), m1 = __int_as_float(v[1][2]), l1 = __int_as_float(v[1][3]);
         float mx = fmaxf(m0, m1);
-        mx = fmaxf(mx, __shfl_xor(mx, 16));
-        mx = fmaxf(mx, __shfl_xor(mx, 32));
+        mx = max16(mx);
+        mx = max32(mx);
         const float e0 = __expf(m0 - mx), e1 = __expf(m1 - mx);
         const float sum = row_sum(e0 * l0 + e1 * l1);
         const float w = __shfl((wave >> 1) & 1 ? e1 : e0, (wave >> 2) * 16 + r) / sum;

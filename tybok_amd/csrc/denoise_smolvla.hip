@@ -313,8 +313,8 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         p[e] = sv;
         tmax = fmaxf(tmax, sv);
       }
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 16));
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+      tmax = max16(tmax);
+      tmax = max32(tmax);
     }
     if (lane < 16) sM[wave * 16 + r] = tmax;
     block_barrier();

@@ -234,7 +234,7 @@ __global__ __launch_bounds__(NWV * 64) void expert_attn_kernel(AttnArgs a) {
       p[i] = sv;
       tmax = fmaxf(tmax, sv);
     }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+    tmax = max32(tmax);
     const float m_new = fmaxf(m_run, tmax);
     const float alpha = __expf(m_run - m_new);
     float lsum = 0.f;
@@ -243,7 +243,7 @@ __global__ __launch_bounds__(NWV * 64) void expert_attn_kernel(AttnArgs a) {
       p[i] = __expf(p[i] - m_new);
       lsum += p[i];
     }
-    lsum += __shfl_xor(lsum, 32);
+    lsum = sum32(lsum);
     l_run = l_run * alpha + lsum;
     m_run = m_new;
 #pragma unroll

@@ -216,7 +216,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
     p[i] = sv;
     tmax = fmaxf(tmax, sv);
   }
-  tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+  tmax = max32(tmax);
   if (half == 0) st_m[wave][l32] = tmax;
   lds_only_barrier();
   float m_new = bm;
@@ -231,7 +231,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
     p[i] = __expf(p[i] - bm);  // out-of-range keys give 0
     lsum += p[i];
   }
-  lsum += __shfl_xor(lsum, 32);
+  lsum = sum32(lsum);
   if (half == 0) st_l[wave][l32] = lsum;
   // (every wave is past its reads of the Q tile: they feed the maxima exchanged above)
   pt[wave][0][lane] = pack8(p);

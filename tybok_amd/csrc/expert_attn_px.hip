@@ -183,7 +183,7 @@ __global__ __launch_bounds__(NWV * 64) void expert_attn_px_kernel(AttnArgs a) {
     p[i] = sv;
     tmax = fmaxf(tmax, sv);
   }
-  tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+  tmax = max32(tmax);
   if (half == 0) st_m[wave][l32] = tmax;
   lds_only_barrier();
   float bm = st_m[0][l32];  // tile 0 always has a key in range: finite
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(NWV * 64) void expert_attn_px_kernel(AttnArgs a) {
     p[i] = __expf(p[i] - bm);  // out-of-range keys give 0
     lsum += p[i];
   }
-  lsum += __shfl_xor(lsum, 32);
+  lsum = sum32(lsum);
   if (half == 0) st_l[wave][l32] = lsum;
   pt[wave][0][lane] = pack8(p);
   pt[wave][1][lane] = pack8(p + 8);
@@ -367,8 +367,7 @@ __global__ __launch_bounds__(kCrossWaves * 64) void expert_cross_px_kernel(AttnA
       }
     }
     float ss = ss0 + ss1;
-#pragma unroll
-    for (int o2 = TPR / 2; o2 > 0; o2 >>= 1) ss += __shfl_xor(ss, o2);
+    ss = wave_sum<TPR>(ss);
     const float rstd = rsqrtf(ss / (float)a.qp_K + a.qp_eps);
     const int kpieces = a.qp_KT * 4;
 #pragma unroll
@@ -497,7 +496,7 @@ __global__ __launch_bounds__(kCrossWaves * 64) void expert_cross_px_kernel(AttnA
     p[i] = sv;
     tmax = fmaxf(tmax, sv);
   }
-  tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+  tmax = max32(tmax);
   if (half == 0) st_m[wave][l32] = tmax;
   lds_only_barrier();  // (every wave is past its K tile: the P^T operands go over them)
   float bm = st_m[0][l32];  // tile 0 always has a key in range: finite
@@ -509,7 +508,7 @@ __global__ __launch_bounds__(kCrossWaves * 64) void expert_cross_px_kernel(AttnA
     p[i] = __expf(p[i] - bm);  // out-of-range keys give 0
     lsum += p[i];
   }
-  lsum += __shfl_xor(lsum, 32);
+  lsum = sum32(lsum);
   if (half == 0) st_l[wave][l32] = lsum;
   i32x4(*const pt)[NWV][2][64] = (i32x4(*)[NWV][2][64])lds;  // [plane][tile][k step][lane], region A
   {

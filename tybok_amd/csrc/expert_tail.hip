@@ -89,8 +89,7 @@ __global__ __launch_bounds__(kThreads) void expert_tail_kernel(TailArgs a) {
     const float f = bf16_bits_to_f32(x[k]);
     ss = fmaf(f, f, ss);
   }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+  ss = wave_sum(ss);
   if ((tid & 63) == 0) red[tid >> 6] = ss;
   __syncthreads();
   float tot = 0.f;

@@ -373,8 +373,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& a, const int strip, c
         }
       }
       float ss = ss0 + ss1;
-#pragma unroll
-      for (int o = PPR / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+      ss = wave_sum<PPR>(ss);
       my_rstd[i] = rsqrtf(ss / (float)a.K + a.norm_eps);
     }
   } else if (PRO) {
@@ -405,8 +404,7 @@ __device__ __forceinline__ void gemm_block(const GemmArgs& a, const int strip, c
       }
     }
     float ss = ss0 + ss1;
-#pragma unroll
-    for (int o = TPR / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    ss = wave_sum<TPR>(ss);
     if (q == 0) rstd_s[r] = rsqrtf(ss / (float)a.K + a.norm_eps);
     __syncthreads();
 #pragma unroll

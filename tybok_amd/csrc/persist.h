@@ -170,8 +170,7 @@ __device__ __forceinline__ f32x2 ld_f2_if(bool here, rsrc_t rs, int voff, int so
 
 // sum over the four lanes that hold the same row of an operand
 __device__ __forceinline__ float row_sum(float v) {
-  v += __shfl_xor(v, 16);
-  return v + __shfl_xor(v, 32);
+  return sum32(sum16(v));
 }
 // sum over eight consecutive lanes (in registers: quad permutes, then the mirror of each half row)
 __device__ __forceinline__ float sum8(float v) {
