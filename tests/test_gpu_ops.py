@@ -484,3 +484,17 @@ def test_layer_norms_at_the_edges_of_their_load_counts(tk, dtype, k):
     # half a bf16 ulp of the result and, before it, fp32 sums of k terms of size < 16 (relative 2^-24 each, k <= 2^11)
     assert bool(((got - want).abs() <= 2**-8 * want.abs() + 2e-3).all())
     assert torch.equal(got[3], b.to(torch.bfloat16).double() if dtype == torch.float32 else b.double())
+
+
+@pytest.mark.parametrize("p,suf,h", [(257, 0, 8), (288, 33, 4), (545, 0, 8), (768, 40, 4)])
+def test_d256_attention_over_rounds_that_end_early(tk, p, suf, h):
+    # blocks of more than one round of eight key tiles: a last round of one tile, of the suffix's tiles alone, prefix and
+    # suffix in one round; pad mask and causal suffix; the next round's rows are asked for while this one's are in use
+    q, k_pre, v_pre, k_suf, v_suf = attn_case(1056, p, h, 1, 256, seed=p)
+    pad = torch.rand(p, generator=torch.Generator().manual_seed(p)) > 0.2
+    ks, vs = (k_suf[:suf], v_suf[:suf]) if suf else (None, None)
+    mode = oops.MASK_BIDIR if suf else oops.MASK_NONE
+    want = oops.expert_attention(q, k_pre, v_pre, ks, vs, pad, mode)
+    dev = lambda t: None if t is None else t.cuda()  # noqa: E731
+    got = tk.expert_attn_plain(q.cuda(), k_pre.cuda(), v_pre.cuda(), dev(ks), dev(vs), pad.cuda(), mode)
+    _close(got, want, f"d256 rounds P={p} S={suf}")

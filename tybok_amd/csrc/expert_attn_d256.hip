@@ -17,6 +17,9 @@
 // of one round each, and the last-arriving block merges the fp32 partials in split order, as in the
 // other attention kernel.  Many query tiles (the prefill): one block per query tile and head, no hand-off.
 #include <math.h>
+
+#include <type_traits>
+
 #include "tk_common.h"
 #include "tk_kernels.h"
 
@@ -49,8 +52,15 @@ __device__ __forceinline__ void lds_only_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// ROUNDS: a block may have more than one round (the prefill).  Bound there: the loads' trip, 8 us a round as long as a round
+// asked for its rows at its start.  So the next round's Q, K and masks are asked for as soon as this one's K is in LDS, the
+// next V^T as soon as this one's is; the operand reads go in smaller batches to leave the registers for that.  What
+// remains is mostly the LDS' own traffic (780 KiB a round, 2.5 us) and its four barriers.  280 / 555 / 968 queries and keys,
+// 8 heads: 12.7 -> 12.3 / 20.9 -> 20.0 / 27.2 -> 25.7 us.
+template <bool ROUNDS>
 __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs a) {
   constexpr int DS = kD / 16;  // k steps of Q.K^T
+  constexpr int KB = ROUNDS ? 4 : 8, JB = ROUNDS ? kWaves / 4 : kWaves;  // k steps, key tiles of a batch of operand reads
   __shared__ float st_m[kWaves][32], st_l[kWaves][32];
   // dynamic LDS: the Q tile (later the P^T operands of every key tile), then one staging tile per wave
   // (its K tile, later its V^T rows); rows of 512 bytes at a pitch that keeps 16-byte operand reads of
@@ -80,29 +90,29 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
   f32x16 o;
 #pragma unroll
   for (int i = 0; i < 16; ++i) o[i] = 0.f;
-  for (int r_lo = 0; r_lo < ntb; r_lo += kWaves) {
-  const int nt = ntb - r_lo < kWaves ? ntb - r_lo : kWaves;  // key tiles of this round, 1..kWaves
-  const int rt_lo = t_lo + r_lo;
-  const bool active = wave < nt;  // this wave has a key tile of its own
-  // (a further round: every wave must be past its reads of the last round's P^T, which the Q tile overwrites)
-  if (r_lo > 0) lds_only_barrier();
+  i32x4 qreg[2], kreg[16], vreg[16];
+  int padv;                      // per-key visibility of the prefix
+  unsigned long long m2lo, m2hi;  // per-(query, key) visibility bytes of the tile
   // ---- every load, back to back, as whole 512-byte rows (lane -> consecutive 16-byte chunks): Q by the
   // block, K (32 keys x 256 d) and V^T (this wave's 32 d rows x the block's 256 keys) per wave.  Read
   // straight into operand registers instead (one row per lane), every load instruction would touch
   // 32 cache lines for 1 KiB, and the CU's 8 waves x 48 such loads are bound by its tag-lookup rate. ----
-  i32x4 qreg[2], kreg[16], vreg[16];
+  auto ask_qk = [&](int r_lo) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));  // (addresses formed here, not kept across the rounds)
+    const int tid = wave * 64 + lane, l32 = lane & 31, half = lane >> 5, qi = mtile * 32 + l32;
+    const bool q_ok = qi < a.M;
+    const int nt = ntb - r_lo < kWaves ? ntb - r_lo : kWaves;
+    const int t = t_lo + r_lo + (wave < nt ? wave : nt - 1);  // idle waves read a valid tile and drop it
+    const bool pre = t < tp;
+    const int tt = pre ? t : t - tp, len = pre ? a.P : a.S;
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int c = tid + 512 * i, row = c >> 5, col = c & 31;
-    int m = mtile * 32 + row;
-    if (m > a.M - 1) m = a.M - 1;  // rows past M are never stored
-    qreg[i] = *(const i32x4*)(a.q + (size_t)m * a.q_sm + (size_t)h * a.q_sh + col * 8);
-  }
-  const int t = rt_lo + (active ? wave : nt - 1);  // idle waves read a valid tile and drop it
-  const bool pre = t < tp;
-  const int tt = pre ? t : t - tp;
-  const int len = pre ? a.P : a.S;
-  {
+    for (int i = 0; i < 2; ++i) {
+      const int c = tid + 512 * i, row = c >> 5, col = c & 31;
+      int m = mtile * 32 + row;
+      if (m > a.M - 1) m = a.M - 1;  // rows past M are never stored
+      qreg[i] = *(const i32x4*)(a.q + (size_t)m * a.q_sm + (size_t)h * a.q_sh + col * 8);
+    }
     const u16* kb = (pre ? a.k_pre : a.k_suf) + (size_t)g * (pre ? a.pre_sh : a.suf_sh);
     const size_t ksl = pre ? a.pre_sl : a.suf_sl;
 #pragma unroll
@@ -112,24 +122,26 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
       if (kr > len - 1) kr = len - 1;  // masked below; keeps the address valid and the value finite
       kreg[i] = *(const i32x4*)(kb + (size_t)kr * ksl + col * 8);
     }
-  }
-  // per-key visibility of the prefix (always requested, from a harmless address when unused)
-  const bool use_pad = pre && a.mask2d == nullptr && a.pad != nullptr;
-  const int key = tt * 32 + l32;
-  const int padv = *((use_pad && key < a.P) ? a.pad + key : (const uint8_t*)a.q);
-  const int pad_ok = use_pad ? (key < a.P ? padv : 0) : 1;
-  // per-(query, key) visibility bytes of the tile (prefill): eight consecutive keys per word, the keys of
-  // this lane's registers 0..7 and 8..15
-  const bool use_m2 = pre && a.mask2d != nullptr;
-  const uint8_t* mp = use_m2 ? a.mask2d + (size_t)(q_ok ? qi : a.M - 1) * a.mask_ld + tt * 32 + 8 * half : (const uint8_t*)a.q;
-  const unsigned long long m2lo = *(const unsigned long long*)mp;
-  const unsigned long long m2hi = *(const unsigned long long*)(mp + (use_m2 ? 16 : 8));
-  {
+    // per-key visibility of the prefix (always requested, from a harmless address when unused)
+    const bool use_pad = pre && a.mask2d == nullptr && a.pad != nullptr;
+    const int key = tt * 32 + l32;
+    padv = *((use_pad && key < a.P) ? a.pad + key : (const uint8_t*)a.q);
+    // per-(query, key) visibility bytes of the tile (prefill): eight consecutive keys per word, the keys of
+    // this lane's registers 0..7 and 8..15
+    const bool use_m2 = pre && a.mask2d != nullptr;
+    const uint8_t* mp = use_m2 ? a.mask2d + (size_t)(q_ok ? qi : a.M - 1) * a.mask_ld + tt * 32 + 8 * half : (const uint8_t*)a.q;
+    m2lo = *(const unsigned long long*)mp;
+    m2hi = *(const unsigned long long*)(mp + (use_m2 ? 16 : 8));
+  };
+  auto ask_v = [&](int r_lo) {
+    int lane = threadIdx.x & 63;
+    asm volatile("" : "+v"(lane));
+    const int nt = ntb - r_lo < kWaves ? ntb - r_lo : kWaves;
     // chunk col of a staged V^T row: key tile col / 4 of the block (tiles past the range: a valid
     // address, P^T is zero there), keys 8 * (col % 4) .. + 7 of that tile
     const int col = lane & 31;
     const int j = col >> 2;
-    const int tj = rt_lo + (j < nt ? j : nt - 1);
+    const int tj = t_lo + r_lo + (j < nt ? j : nt - 1);
     const bool pj = tj < tp;
     const int ttj = pj ? tj : tj - tp;
     const size_t vsd = pj ? a.pre_vt_sd : a.suf_vt_sd;
@@ -139,7 +151,19 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
       const int row = (lane + 64 * i) >> 5;
       vreg[i] = *(const i32x4*)(vb + (size_t)(32 * wave + row) * vsd);
     }
-  }
+  };
+  ask_qk(0);
+  ask_v(0);
+  // one round; `more`: another one follows, whose rows are asked for on the way
+  auto round = [&](int r_lo, auto more) {
+  const int nt = ntb - r_lo < kWaves ? ntb - r_lo : kWaves;  // key tiles of this round, 1..kWaves
+  const bool active = wave < nt;  // this wave has a key tile of its own
+  const int t = t_lo + r_lo + (active ? wave : nt - 1);
+  const bool pre = t < tp;
+  const int tt = pre ? t : t - tp;
+  const int len = pre ? a.P : a.S;
+  // (a further round: every wave must be past its reads of the last round's P^T, which the Q tile overwrites)
+  if (r_lo > 0) lds_only_barrier();
   // keep the V^T requests here: sunk below the first product (to save registers) they would leave only
   // after Q and K have arrived, one memory round trip later
   __builtin_amdgcn_sched_barrier(0);
@@ -157,21 +181,25 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
     const int c = lane + 64 * i;
     *(i32x4*)(mine + key_of_row(c >> 5) * kPitch + (c & 31) * 16) = kreg[i];  // MFMA row r holds key key_of_row(r)
   }
+  const bool use_pad = pre && a.mask2d == nullptr && a.pad != nullptr;
+  const int pad_ok = use_pad ? (tt * 32 + l32 < a.P ? padv : 0) : 1;
+  const unsigned long long v2lo = m2lo, v2hi = m2hi;
+  if constexpr (more) ask_qk(r_lo + kWaves);
   lds_only_barrier();  // the Q tile is complete (the K tile is this wave's own)
-  // operand reads in two batches of 8 k steps, each batch out before its first product waits for one
+  // operand reads in batches of 8 (4) k steps, each batch out before its first product waits for one
   // (all 16 at once would not leave registers for the V^T rows still held for the second product)
 #pragma unroll
-  for (int s0 = 0; s0 < DS; s0 += 8) {
-    i32x4 ka[8], qb[8];
+  for (int s0 = 0; s0 < DS; s0 += KB) {
+    i32x4 ka[KB], qb[KB];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
+    for (int s = 0; s < KB; ++s) {
       const int off = l32 * kPitch + (16 * (s0 + s) + 8 * half) * 2;
       ka[s] = *(const i32x4*)(mine + off);
       qb[s] = *(const i32x4*)(qs + off);
     }
     __builtin_amdgcn_sched_barrier(0);  // (the scheduler would pair each read with its product again)
 #pragma unroll
-    for (int s = 0; s < 8; ++s) sT = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka[s]), as_bf16x8(qb[s]), sT, 0, 0, 0);
+    for (int s = 0; s < KB; ++s) sT = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(ka[s]), as_bf16x8(qb[s]), sT, 0, 0, 0);
     __builtin_amdgcn_sched_barrier(0);
   }
 
@@ -196,7 +224,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
     } else if (a.mask2d) {
       // one byte (0 or 1) per key: gather bit 0 of the 8 bytes of each word
       const unsigned long long gather = 0x0102040810204080ull, ones = 0x0101010101010101ull;
-      vbits = (unsigned)(((m2lo & ones) * gather) >> 56) | ((unsigned)(((m2hi & ones) * gather) >> 56) << 8);
+      vbits = (unsigned)(((v2lo & ones) * gather) >> 56) | ((unsigned)(((v2hi & ones) * gather) >> 56) << 8);
     } else {
       const unsigned pmask = (unsigned)__ballot(pad_ok != 0);  // lanes 0..31: keys of this tile
       vbits = ((pmask >> (8 * half)) & 0xffu) | (((pmask >> (16 + 8 * half)) & 0xffu) << 8);
@@ -241,6 +269,7 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
     const int c = lane + 64 * i;
     *(i32x4*)(mine + (c >> 5) * kPitch + (c & 31) * 16) = vreg[i];  // over this wave's K tile, which it has consumed
   }
+  if constexpr (more) ask_v(r_lo + kWaves);
   lds_only_barrier();
   {
     float rl = st_l[0][l32];
@@ -252,21 +281,29 @@ __global__ __launch_bounds__(kWaves * 64) void expert_attn_d256_kernel(AttnArgs 
 #pragma unroll
   for (int i = 0; i < 16; ++i) o[i] *= alpha;  // all of a lane's registers belong to its one query
   {
-    i32x4 va[kWaves][2], pb[kWaves][2];
 #pragma unroll
-    for (int j = 0; j < kWaves; ++j)
+    for (int j0 = 0; j0 < kWaves; j0 += JB) {
+      i32x4 va[JB][2], pb[JB][2];
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        va[j][s] = *(const i32x4*)(mine + l32 * kPitch + (32 * j + 16 * s + 8 * half) * 2);
-        pb[j][s] = pt[j][s][lane];
-      }
-    __builtin_amdgcn_sched_barrier(0);
+      for (int j = 0; j < JB; ++j)
 #pragma unroll
-    for (int j = 0; j < kWaves; ++j)
+        for (int s = 0; s < 2; ++s) {
+          va[j][s] = *(const i32x4*)(mine + l32 * kPitch + (32 * (j0 + j) + 16 * s + 8 * half) * 2);
+          pb[j][s] = pt[j0 + j][s][lane];
+        }
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < 2; ++s) o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(va[j][s]), as_bf16x8(pb[j][s]), o, 0, 0, 0);
+      for (int j = 0; j < JB; ++j)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(va[j][s]), as_bf16x8(pb[j][s]), o, 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   }
-  }  // rounds
+  };
+  int r_lo = 0;
+  if (ROUNDS)
+    for (; r_lo + kWaves < ntb; r_lo += kWaves) round(r_lo, std::true_type{});
+  round(r_lo, std::false_type{});
   // this lane's output: query qi, columns 32w + 8g4 + 4*half + 0..3 for the four register groups g4
   u16* op = a.out + (size_t)(q_ok ? qi : 0) * a.out_sm + (size_t)h * kD + 32 * wave + 4 * half;
   if (a.kv_splits == 1) {
@@ -368,14 +405,15 @@ int tk_attn_d256_tiles_per_block() { return kWaves; }
 int tk_launch_attn_d256(AttnArgs a, hipStream_t st) {
   if (a.k_pre_lo || a.batch > 0 || a.kv_splits < 1 || a.kv_splits > kMaxSplits) return -1;
   if (a.tile_q < 1) return -1;
-  // more LDS than a launch gets by default: raise the kernel's limit once per process
+  // more LDS than a launch gets by default: raise the kernels' limit once per process
   static int raised = 0;
   if (!raised) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&expert_attn_d256_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess)
-      return -3;
+    for (const void* k : {reinterpret_cast<const void*>(&expert_attn_d256_kernel<false>), reinterpret_cast<const void*>(&expert_attn_d256_kernel<true>)})
+      if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsBytes) != hipSuccess) return -3;
     raised = 1;
   }
   dim3 grid(a.H, (a.M + 31) / 32, a.kv_splits);
-  hipLaunchKernelGGL(expert_attn_d256_kernel, grid, dim3(kWaves * 64), kLdsBytes, st, a);
+  if (a.tile_q + (a.tile_r ? 1 : 0) > kWaves) hipLaunchKernelGGL(expert_attn_d256_kernel<true>, grid, dim3(kWaves * 64), kLdsBytes, st, a);
+  else hipLaunchKernelGGL(expert_attn_d256_kernel<false>, grid, dim3(kWaves * 64), kLdsBytes, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }

@@ -46,17 +46,6 @@ __device__ __forceinline__ f32x16 mma16(i32x4 a, i32x4 b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(a), as_bf16x8(b), c, 0, 0, 0);
 }
 
-// max / sum of a value over the two lanes that share a query (lane l and l ^ 32), without an LDS trip:
-// v_permlane32_swap hands each half the other half's registers
-__device__ __forceinline__ float other_half_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float other_half_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 __device__ __forceinline__ void stage_barrier() {
   // LDS-only: the global prefetch of the next stage stays in flight across it
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -229,7 +218,7 @@ __global__ __launch_bounds__(QT * kGroups * 64, WPE) void tower_attn_kernel(Attn
           }
           tmax = fmaxf(tmax, fmaxf(sT[kt][i], sT[kt][i + 1]));
         }
-      tmax = other_half_max(tmax) * scale2;
+      tmax = max32(tmax) * scale2;
       if (__any(tmax > m_run)) {  // wave-uniform
         const float m_new = fmaxf(m_run, tmax);
         const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -252,7 +241,7 @@ __global__ __launch_bounds__(QT * kGroups * 64, WPE) void tower_attn_kernel(Attn
           lsum0 += p[kt][i];
           lsum1 += p[kt][i + 1];
         }
-      l_run += other_half_sum(lsum0 + lsum1);
+      l_run += sum32(lsum0 + lsum1);
       // ---- O^T += V^T . P^T (probabilities rounded to bf16, fp32 accumulation) ----
 #pragma unroll
       for (int kt = 0; kt < KT; ++kt)
