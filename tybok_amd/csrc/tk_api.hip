@@ -699,12 +699,22 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
   const PipeTile* best = nullptr;
   int ks = split_k > 0 ? split_k : 1;
   float best_cost = 0.f;
+  // A K of 8192 or more over few columns (the connector, 12288 -> 960): as many splits as fill the device with 64 x 128
+  // blocks, 32 k tiles or more each, whatever block is picked.  The cost below would take 8 splits instead of 12 at 128
+  // rows and save 2 us of a request; but the sums of such a K are what a chunk's distance from the reference arithmetic
+  // hangs on most, and they stay as short as they are (largest distance of a two-layer chunk 8.3e-3, 10.1e-3 with 8).
+  int k_from = split_k > 0 ? split_k : 1;
+  if (split_k <= 0 && !rope && a.KT >= 256) {
+    k_from = cus / (((M + 63) / 64) * ((N + 127) / 128));
+    k_from = k_from < a.KT / 32 ? k_from : a.KT / 32;
+    k_from = k_from > 1 ? k_from : 1;
+  }
   for (const PipeTile& t : kDenseTiles) {
     if (tile && t.id != tile) continue;
     if (rope && !dense_rope_tile(t.id)) continue;
     // a split keeps at least 16 k tiles; none in the rotary form unless asked for (the partials weigh more than the idle CUs)
-    const int most = split_k > 0 || rope || a.KT < 32 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
-    for (int k1 = split_k > 0 ? split_k : 1, n = 0; n < most; ++k1, ++n) {
+    const int most = split_k > 0 || rope || a.KT < 32 || a.KT >= 256 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
+    for (int k1 = k_from, n = 0; n < most; ++k1, ++n) {
       const float c = pipe_cost(t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus);
       if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
     }
