@@ -1,7 +1,7 @@
 // fp8-weight GEMM for many rows (the VLM prefill) on gfx950: the weight-only form of pipe_fp8.h, a kernel of its own for the
 // largest grids, and the row norm in front of them.
 // Measured (us, cold weights, graph replay; before: weights straight into the registers of four multiplying waves): the
-// gated block 2048 -> 16384 -> 2048 at 288 / 330 / 555 / 712 / 968 rows 104 -> 83, 102 -> 87, 135 -> 132, 156 -> 151, 190 ->
+// gated block 2048 -> 16384 -> 2048 at 288 / 330 / 555 / 712 / 968 rows 104 -> 79, 102 -> 87, 135 -> 132, 156 -> 151, 190 ->
 // 186; 960 -> 2560 -> 960 at 305 / 600 rows 39 -> 22, 41 -> 28.
 #include <atomic>
 
@@ -642,6 +642,7 @@ int tk_launch_gemm_wide(const GemmArgs& a, int tile, hipStream_t st) {
     case 68: return a.s1 ? launch_tile<1, 3>(a, st) : launch_tile<0, 3>(a, st);
     case 88: return a.s1 ? launch_tile<1, 4>(a, st) : launch_tile<0, 4>(a, st);
     case 404: return launch_fp8_pipe<BF16_FP8, 4, 4, 2, 2, 3, 2>(a, st);
+    case 304: return launch_fp8_pipe<BF16_FP8, 3, 4, 1, 4, 3, 2>(a, st);
     case 408: return launch_fp8_pipe<BF16_FP8, 4, 8, 2, 2, 4, 1>(a, st);
     case 208: return launch_fp8_pipe<BF16_FP8, 2, 8, 1, 4, 3, 2>(a, st);
     case 204: return launch_fp8_pipe<BF16_FP8, 2, 4, 2, 2, 4, 2>(a, st);

@@ -116,11 +116,13 @@ float pipe_cost(const PipeTile& t, float kb_n, int M, int N, int rounds, int ks,
 // loads, 55 - 61 of loads alone): padded rows and columns at 1.15 (bf16) or 1.8 PFLOP/s (fp8 x fp8), shapes that move more
 // operands per product a little slower; a fifth of that shows where the loads set the time (the split down projection
 // 16384 -> 2048 at 555 / 650 rows on blocks of 128 x 256: the whole block 3 us less than on 64 x 256).
+// 96 x 128 blocks, weight-only: 257 .. 288 rows are three of them and 384 rows of the others' (gated 2048 -> 2 x 16384 at 272
+// rows 54 -> 47.5 us); fp8 x fp8 they were slower there (49.5 -> 55).
 struct Fp8Tile {
   PipeTile t;
   float power;  // relative time per product
 };
-constexpr Fp8Tile kWideTiles[] = {{{408, 4, 8, 8, 4, 1}, 1.f}, {{404, 4, 4, 4, 3, 2}, 1.f}, {{208, 2, 8, 4, 3, 2}, 1.3f}, {{204, 2, 4, 2, 4, 2}, 1.3f}};
+constexpr Fp8Tile kWideTiles[] = {{{408, 4, 8, 8, 4, 1}, 1.f}, {{404, 4, 4, 4, 3, 2}, 1.f}, {{304, 3, 4, 3, 3, 2}, 1.f}, {{208, 2, 8, 4, 3, 2}, 1.3f}, {{204, 2, 4, 2, 4, 2}, 1.3f}};
 constexpr Fp8Tile kW8a8Tiles[] = {{{408, 4, 8, 8, 3, 1}, 1.f}, {{414, 4, 4, 4, 4, 1}, 1.1f}, {{204, 2, 4, 2, 3, 2}, 1.2f}, {{604, 6, 4, 6, 4, 1}, 1.f}};
 template <int N>
 int pick_tile(const Fp8Tile (&tiles)[N], float kb_n, float flop_per_us, int M, int ncols, int K, int rounds, int ks) {
