@@ -184,7 +184,8 @@ def test_w8a8_rows_more_than_4_gib_of_lane_offset_apart(tk):
 @pytest.mark.parametrize("k", [8, 2048, 2056, 4104, 8200, 16384])
 def test_activation_quantisation_at_the_edges_of_the_quotient(tk, k, mode):
     # every piece count of a row, a row of all finite bf16 magnitudes, signed zeros, scales at and beyond the range in which
-    # the quotient comes from the reciprocal; whole rows of one scale each (none that rounds to 0, where a quotient has no value).  Infinities and NaN: as the division gives them.
+    # the quotient comes from the reciprocal; whole rows of one scale each (scales that round to 0: the next test).
+    # Infinities and NaN: as the division gives them.
     g = torch.Generator().manual_seed(k)
     rows = [torch.randn(k, generator=g) * 2.0**e for e in (-110, -100, -81, -72, -71, -70, -20, 0, 20, 70, 88, 89, 90, 100, 118)]
     codes = 0x7F7F - torch.arange(k, dtype=torch.int32) * 7 % 0x7F00
@@ -201,3 +202,20 @@ def test_activation_quantisation_at_the_edges_of_the_quotient(tk, k, mode):
     q = odd.float() / s[:, None]
     got = a8.cpu().view(torch.float8_e4m3fn).float()
     assert torch.equal(sa.cpu(), s) and torch.equal(got.isnan(), q.isnan()) and bool((got[~q.isnan()] == 0).all())
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("k", [8, 2056, 16384])
+def test_activation_quantisation_of_rows_whose_scale_rounds_to_zero(tk, k, mode):
+    # amax / 448 as a bf16 value: 0 up to 448 * 2^-134 (a tie goes to the even 0), the smallest subnormal from the next
+    # bf16 above; a scale of 0 gives zero codes (+0, whatever the signs) and a finite product.  In fp32 no bf16 row's does.
+    g = torch.Generator().manual_seed(k)
+    sign = torch.where(torch.rand(k, generator=g) < 0.5, -1.0, 1.0)
+    top = 448 * 2.0**-134
+    rows = [top * torch.rand(k, generator=g) * sign, sign * 2.0**-133, torch.where(torch.arange(k) == k - 1, top, 0.0), torch.where(torch.arange(k) == 1, top * (1 + 2**-7), -0.0)]
+    x = torch.stack([*rows, torch.randn(k, generator=g) * 2.0**-126, torch.zeros(k), -torch.zeros(k)]).to(BF16)
+    a8, sa = tk.quant_act_rows(x.cuda(), mode)
+    want8, want_s = oops.quantize_activation_rows(x, "bf16" if mode else "fp32")
+    assert torch.equal(sa.cpu(), want_s) and torch.equal(a8.cpu().view(torch.uint8), want8.view(torch.uint8))
+    if mode:
+        assert bool((sa[:3] == 0).all()) and bool((a8.view(torch.uint8)[:3] == 0).all()) and float(sa[3]) > 0

@@ -1,7 +1,8 @@
 // W8A8 tier of the VLM prefill MLP on gfx950: per-token activation quantisation and the fp8 x fp8 GEMM.
 //
 //   quant_act_rows_kernel   x[M,K] bf16 -> a8[M,K] e4m3fn, sa[M] fp32 with sa = amax_k|x| / 448 and
-//                           a8 = RNE(x / sa) in fp32 (one rounding); an all-zero row gives sa = 0 and zero codes.
+//                           a8 = RNE(x / sa) in fp32 (one rounding); a row whose scale is 0 (all zeros; bf16 mode:
+//                           |x| up to 448 * 2^-134 as well, whose scale rounds to 0) gives zero codes.
 //   fp8_pipe_kernel<FP8>    (pipe_fp8.h) y[M,N] = bf16((a8 . W8^T) * sa[m] * sw[n]) on v_mfma_f32_32x32x64_f8f6f4 (e4m3 x
 //                           e4m3, fp32 accumulate, 64 k per instruction).  The order of k inside an instruction is the
 //                           same permutation for both operands (bytes 0-15 of a lane: k tile 2s, bytes 16-31: k tile
@@ -53,7 +54,7 @@ __global__ __launch_bounds__(256) void quant_act_rows_kernel(QuantActArgs a) {
   const float inv = 1.0f / sa;
   const bool plain = sa >= 0x1p-80f && sa <= 0x1p+80f;
   auto quotient = [&](float x) {
-    if (amax == 0.f) return 0.f;
+    if (sa == 0.f) return 0.f;
     if (!plain) return x / sa;
     const float y = x * inv;
     return __builtin_copysignf(fmaf(fmaf(-sa, y, x), inv, y), x);
