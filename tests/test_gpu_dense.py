@@ -314,3 +314,16 @@ def test_long_k_keeps_its_split_count(tk, m, k, n, splits):
     _close(got, _want(x, w, b), "long k")
     if splits and torch.cuda.get_device_properties(0).multi_processor_count == 256:
         assert torch.equal(got, tk.bf16w_dense(x.cuda(), pw, b.cuda(), split_k=splits))
+
+
+@pytest.mark.parametrize("m,k,n,split", [(2391, 2592, 2824, 2), (234, 3760, 11344, 5), (671, 14656, 4904, 4), (304, 15936, 3424, 12)])
+def test_explicit_split_takes_a_block_shape_whose_partials_fit(tk, m, k, n, split):
+    # the partials are whole blocks: the fastest block shape pads these outputs past the workspace's 56 MiB, others do not
+    g = torch.Generator().manual_seed(m)
+    x = torch.randint(-2, 3, (m, k), generator=g).to(BF16).cuda()
+    w = torch.randint(-1, 2, (n, k), generator=g).to(BF16).cuda()
+    pw = tk.pack_bf16_weight(w)
+    got = tk.bf16w_dense(x, pw, split_k=split)
+    assert torch.equal(got, (x.float() @ w.float().t()).to(BF16))  # integers: exact in any order
+    with pytest.raises(RuntimeError, match="needs [0-9]+ bytes of partial space"):
+        tk.bf16w_dense(x, pw, split_k=64)

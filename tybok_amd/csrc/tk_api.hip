@@ -698,9 +698,12 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
     a.vt_bs = vt->bs;
   }
   const int cus = device_cus();
+  const size_t space = ws && ws_bytes > kPartialOff ? (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes) : 0;
   const PipeTile* best = nullptr;
   int ks = split_k > 0 ? split_k : 1;
   float best_cost = 0.f;
+  bool known = false;
+  size_t need = 0;  // of an explicit split that does not fit: the smallest partials of any block shape
   // A K of 8192 or more over few columns (the connector, 12288 -> 960): as many splits as fill the device with 64 x 128
   // blocks, 32 k tiles or more each, whatever block is picked.  The cost below would take 8 splits instead of 12 at 128
   // rows and save 2 us of a request; but the sums of such a K are what a chunk's distance from the reference arithmetic
@@ -714,24 +717,27 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
   for (const PipeTile& t : kDenseTiles) {
     if (tile && t.id != tile) continue;
     if (rope && !dense_rope_tile(t.id)) continue;
+    known = true;
+    // splits whose partials (whole blocks) and counters the workspace holds: a block shape that pads the output more holds fewer
+    const size_t blocks0 = (size_t)((M + 32 * t.bm - 1) / (32 * t.bm)) * ((N + 32 * t.bn - 1) / (32 * t.bn));
+    const size_t per_split = blocks0 * (size_t)(1024 * t.bm * t.bn) * 4, fit = blocks0 <= (size_t)kMaxCounters ? space / per_split : 0;
     // a split keeps at least 16 k tiles; none in the rotary form unless asked for (the partials weigh more than the idle CUs)
     const int most = split_k > 0 || rope || a.KT < 32 || a.KT >= 256 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
-    for (int k1 = k_from, n = 0; n < most; ++k1, ++n) {
+    for (int c1 = k_from, n = 0; n < most; ++c1, ++n) {
+      int k1 = c1;
+      if (k1 > 1 && (size_t)k1 > fit) {
+        if (split_k > 1) {
+          if (!need || per_split * k1 < need) need = per_split * k1;
+          continue;
+        }
+        k1 = fit > 1 ? (int)fit : 1;
+      }
       const float c = pipe_cost(t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus);
       if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
     }
   }
-  if (!best) return fail(TK_EINVAL, "bf16w_dense: tile=%d (0 = automatic, or 42, 41, 32, 31, 22, 21, 12, 11, 606, 404, 406, 403, 204, 202; the rotary form: 42, 32, 22, 12, 404, 204)", tile);
-  const int rows = 32 * best->bm, cols = 32 * best->bn;
-  const int blocks0 = ((M + rows - 1) / rows) * ((N + cols - 1) / cols);
-  const size_t per_split = (size_t)rows * cols * 4;
-  if (ks > 1) {
-    const size_t have = ws && ws_bytes > kPartialOff ? (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes) / (per_split * blocks0) : 0;
-    if ((size_t)ks > have || blocks0 > kMaxCounters) {
-      if (split_k > 1) return fail(TK_EWORKSPACE, "bf16w_dense: split_k=%d needs %zu bytes of partial space", ks, per_split * blocks0 * ks);
-      ks = have > 1 && blocks0 <= kMaxCounters ? (int)have : 1;
-    }
-  }
+  if (!known) return fail(TK_EINVAL, "bf16w_dense: tile=%d (0 = automatic, or 42, 41, 32, 31, 22, 21, 12, 11, 606, 404, 406, 403, 204, 202; the rotary form: 42, 32, 22, 12, 404, 204)", tile);
+  if (!best) return fail(TK_EWORKSPACE, "bf16w_dense: split_k=%d needs %zu bytes of partial space", split_k, need);
   if (ks > a.KT) ks = a.KT;
   a.ksplit = ks;
   a.kt_q = a.KT / ks;
