@@ -659,6 +659,18 @@ int tk_debug_stream_read(const void* src, size_t bytes, int blocks, void* sink, 
 int tk_debug_fp8w_gemm_cut(const void* x, int ldx, const void* w_packed, const void* scale, void* y, int ldy,
                            int M, int N, int K, int cut, void* stream);
 
+/* One launch of the many-row fp8-weight kernels with a given block shape, where tk_fp8w_gemm, tk_w8a8_gemm and the gated
+ * forms take one by the shape: for tests that run every block shape over the same operands, and for timing them.
+ *   sa: NULL = weight-only (x bf16, ldx in elements; tiles 408, 404, 304, 208, 204: 100 * 32-row tiles + 32-column tiles of a
+ *       block; with split_k = 1 also 28, 68, 88, the kernels of the largest grids), otherwise the row scales of e4m3 codes
+ *       (ldx in bytes; tiles 604, 408, 414, 204).
+ *   s1: NULL = plain (scale s0, residual, weight-only: per-column gate), otherwise gated (w_packed from tk_pack_fp8_gate_up, N the
+ *       intermediate's width, act).  Other arguments as tk_fp8w_gemm; N and ldy multiples of 4.  No counterpart in the
+ * reference. */
+int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* w_packed, const void* s0, const void* s1, void* y,
+                            int ldy, const void* resid, int ldr, int resid_dtype, const void* gate, int M, int N, int K, int split_k,
+                            int act, int tile, void* ws, size_t ws_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

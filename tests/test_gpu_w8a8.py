@@ -149,6 +149,7 @@ def test_w8a8_ffn_matches_oracle(tk, m, k, i, act, mode):
 @pytest.mark.parametrize("m,k,n", [(1, 16, 4), (257, 48, 36), (289, 144, 132), (319, 720, 388), (130, 2064, 260)])
 @pytest.mark.parametrize("split", [0, 1, 2, 3])
 def test_w8a8_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
+    # what the shapes pick by themselves (64 x 128 blocks; every shape of block: the next test):
     # k ranges that end inside a round of 128 (and, split, on any tile of 32), one past a row tile, N % 8 == 4; a8 is a column
     # slice of a wider buffer of NaN codes.  Integer codes and power-of-two scales: exact whatever the order of summation.
     if split > 1 and (k + 31) // 32 < split:
@@ -167,6 +168,67 @@ def test_w8a8_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
     got = tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split, resid=r.cuda())
     assert torch.equal(got.cpu(), want)
     assert torch.equal(tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split).cpu(), y)
+
+
+W8A8_TILES = (408, 414, 204, 604)  # 64 x 128, 128 x 128 (414), 128 x 256 and 192 x 128 blocks
+
+
+def _integers(g, top, *shape):
+    return torch.randint(-top, top + 1, shape, generator=g).float()
+
+
+def _codes_before_nan(a):
+    m, k = a.shape
+    wide = torch.full((m, (k + 31) // 16 * 16), 0x7F, dtype=torch.uint8)
+    wide[:, :k] = a.to(torch.float8_e4m3fn).view(torch.uint8)
+    return wide.cuda()[:, :k]
+
+
+@pytest.mark.parametrize("tile", W8A8_TILES)
+@pytest.mark.parametrize("k", [16, 48, 144, 720, 2064, 4112])
+def test_every_w8a8_block_shape_exact_on_small_integers(tk, tile, k):
+    # rows and columns one (four) past a block and short of one, one row alone; K inside a round, more rounds than the ring
+    # holds; even and uneven splits; NaN codes behind K, residuals, a pitch that allows only 8-byte stores (N + 4) and one with
+    # room behind N.  Exact: |sum| <= 6 * 4112 times powers of two, rounded once to bf16 each time.
+    rows, cols = (128, 128) if tile == 414 else (tile // 100 * 32, tile % 100 * 32)
+    for m, n in ((rows + 1, cols + 4), (1, 4), (2 * rows - 31, 36), (rows, 2 * cols - 60)):
+        g = torch.Generator().manual_seed(m + k + n)
+        a, w = _integers(g, 3, m, k), _integers(g, 2, n, k)
+        sa, sw = torch.exp2(_integers(g, 2, m)), torch.exp2(_integers(g, 2, n))
+        r = _integers(g, 16, m, n).to(BF16)
+        y = ((a @ w.t()) * sa[:, None] * sw[None, :]).to(BF16)
+        full = (y.float() + r.float()).to(BF16)
+        pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), sw.cuda())
+        x, sac, rc = _codes_before_nan(a), sa.cuda(), r.cuda()
+        for split in (s for s in (1, 2, 3, 5) if s <= (k + 31) // 32):
+            assert torch.equal(tk.many_rows_gemm(x, pw, tile, sa=sac, split_k=split).cpu(), y), (m, n, split)
+            for pitch in (n + 4, (n + 15) // 8 * 8):
+                buf = torch.full((m, pitch), 7.0, dtype=BF16, device="cuda")
+                tk.many_rows_gemm(x, pw, tile, sa=sac, split_k=split, resid=rc, out=buf[:, :n])
+                assert torch.equal(buf[:, :n].cpu(), full) and bool((buf[:, n:] == 7.0).all()), (m, n, split, pitch)
+            assert torch.equal(tk.many_rows_gemm(x, pw, tile, sa=sac, split_k=split, resid=rc.float()).cpu(), full), (m, n, split)
+
+
+@pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
+@pytest.mark.parametrize("m,k,i", [(1, 16, 32), (65, 80, 96), (129, 720, 160), (193, 2064, 32), (257, 144, 544)])
+def test_every_w8a8_block_shape_gives_the_same_gated_bits(tk, m, k, i, act):
+    # exact gate and up sums whatever the shape and the split, then one epilogue: the same bits from all of them
+    g = torch.Generator().manual_seed(m + k + i)
+    a, wg, wu = _integers(g, 3, m, k), _integers(g, 2, i, k), _integers(g, 2, i, k)
+    sa, sg, su = torch.exp2(_integers(g, 1, m)), torch.exp2(_integers(g, 1, i) - 5), torch.exp2(_integers(g, 1, i) - 5)
+    pre, up = ((a @ w.t()) * sa[:, None] * s for w, s in ((wg, sg), (wu, su)))
+    want = (oops.act_fn(act, pre.to(BF16)).float() * up.to(BF16).float()).to(BF16)
+    wgu = tk.pack_fp8_gate_up(wg.to(torch.float8_e4m3fn).cuda(), sg, wu.to(torch.float8_e4m3fn).cuda(), su)
+    x, sac = _codes_before_nan(a), sa.cuda()
+    first = None
+    for tile in W8A8_TILES:
+        for split in (1,) if k < 64 else (1, 2):
+            buf = torch.full((m, i + 4), 7.0, dtype=BF16, device="cuda")
+            got = tk.many_rows_gemm(x, wgu, tile, sa=sac, split_k=split, act=act)
+            tk.many_rows_gemm(x, wgu, tile, sa=sac, split_k=split, act=act, out=buf[:, :i])
+            first = got if first is None else first
+            assert torch.equal(got, first) and torch.equal(buf[:, :i], first) and bool((buf[:, i:] == 7.0).all()), (tile, split)
+    _close(first, want, f"w8a8 gated M={m} K={k} I={i}")
 
 
 def test_w8a8_rows_more_than_4_gib_of_lane_offset_apart(tk):

@@ -76,8 +76,8 @@ def test_many_row_gemm_matches_skinny_kernel_rows(tk):
 @pytest.mark.parametrize("m", [712, 1024])
 def test_eight_wave_blocks_give_the_four_wave_kernels_bits(tk, m):
     # wide launches with enough column blocks run on eight-wave blocks of 192 (M=712) or 256 (M=1024) rows that stage
-    # both operands through LDS; a 256-row slice of the same input stays on the four-wave kernel.  A row's k tiles are
-    # accumulated in the same order in both, so the shared rows must agree bit for bit -- with and without a residual.
+    # both operands through LDS; a 256-row slice of the same input takes another kernel and block shape.  A row's k tiles are
+    # accumulated in the same order in all of them, so the shared rows must agree bit for bit -- with and without a residual.
     k, n = 256, 32768
     x, w8, s = gemm_case(m, k, n)
     pw = tk.pack_fp8_weight(w8.cuda(), s.cuda())
@@ -208,7 +208,8 @@ def test_prefill_size_ffn_matches_oracle_and_rows_are_independent(tk):
 @pytest.mark.parametrize("m,k,n", [(257, 16, 4), (256, 48, 36), (289, 80, 132), (319, 720, 388), (385, 1088, 260), (300, 4112, 68)])
 @pytest.mark.parametrize("split", [0, 1, 2, 3])
 def test_many_row_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
-    # one past a row tile or block, k ranges that end inside a round (and, split, on an odd tile of 32), N % 8 == 4; the columns
+    # what the shapes pick by themselves (64 x 128 blocks; every shape of block: the next test): one past a row tile or block,
+    # k ranges that end inside a round (and, split, on an odd tile of 32), N % 8 == 4; the columns
     # of x behind K hold NaN (a wider buffer) and must not be read into a product.  Integer codes and power-of-two scales:
     # every sum is exact in fp32 whatever its order (|sum| < 2^24), the result is rounded once to bf16.
     if split > 1 and (k + 31) // 32 < split:
@@ -241,3 +242,66 @@ def test_many_row_gated_rows_do_not_depend_on_the_block_shape(tk, m, k, i):
     want = tk.fp8w_gated_ffn(xc, wgu, pd, "gelu_tanh")
     got = tk.fp8w_gated_ffn(xc[700 - m :].contiguous(), wgu, pd, "gelu_tanh")
     assert torch.equal(got, want[700 - m :])
+
+
+TILES = (408, 404, 304, 208, 204)  # 100 * (32-row tiles) + (32-column tiles) of a block
+WHOLE = (28, 68, 88)  # the kernels of the largest grids, 64, 192 and 256 rows x 256 columns, no K split
+
+
+def _block(tile):
+    return {28: (64, 256), 68: (192, 256), 88: (256, 256)}.get(tile, (tile // 100 * 32, tile % 100 * 32))
+
+
+def _integers(g, top, *shape):
+    return torch.randint(-top, top + 1, shape, generator=g).float()
+
+
+@pytest.mark.parametrize("tile", TILES + WHOLE)
+@pytest.mark.parametrize("k", [16, 80, 720, 1088, 4112])
+def test_every_block_shape_exact_on_small_integers(tk, tile, k):
+    # rows and columns one (four) past a block and short of one, one row alone; K inside a round, an odd tile of 32, more
+    # rounds than the ring holds; even and uneven splits; NaN behind K, a gate, a residual, a pitch that allows only 8-byte
+    # stores (N + 4) and one with room behind N.  Exact: |sum| <= 12 * 4112 in quarters, rounded once to bf16 each time.
+    rows, cols = _block(tile)
+    for m, n in ((rows + 1, cols + 4), (1, 4), (2 * rows - 31, 36), (rows, 2 * cols - 60)):
+        g = torch.Generator().manual_seed(m + k + n)
+        wide = torch.full((m, k + 72), float("nan"), dtype=BF16)
+        wide[:, :k] = _integers(g, 4, m, k).to(BF16)
+        w, sw = _integers(g, 3, n, k), torch.exp2(_integers(g, 2, n))
+        gate, r = _integers(g, 2, n).to(BF16), _integers(g, 16, m, n).to(BF16)
+        y = ((wide[:, :k].float() @ w.t()) * sw).to(BF16)
+        full = ((y.float() * gate.float()).to(BF16).float() + r.float()).to(BF16)
+        pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), sw.cuda())
+        x, rc = wide.cuda()[:, :k], r.cuda()
+        for split in (1,) if tile in WHOLE else (s for s in (1, 2, 3, 5) if s <= (k + 31) // 32):
+            assert torch.equal(tk.many_rows_gemm(x, pw, tile, split_k=split).cpu(), y), (m, n, split)
+            for pitch in (n + 4, (n + 15) // 8 * 8):
+                buf = torch.full((m, pitch), 7.0, dtype=BF16, device="cuda")
+                tk.many_rows_gemm(x, pw, tile, split_k=split, gate=gate.cuda(), resid=rc, out=buf[:, :n])
+                assert torch.equal(buf[:, :n].cpu(), full) and bool((buf[:, n:] == 7.0).all()), (m, n, split, pitch)
+            f32 = tk.many_rows_gemm(x, pw, tile, split_k=split, resid=rc.float())
+            assert torch.equal(f32.cpu(), (y.float() + r.float()).to(BF16)), (m, n, split)
+
+
+@pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
+@pytest.mark.parametrize("m,k,i", [(1, 16, 32), (65, 80, 96), (97, 720, 160), (129, 1088, 288), (193, 2064, 32), (257, 96, 544)])
+def test_every_block_shape_gives_the_same_gated_bits(tk, m, k, i, act):
+    # exact gate and up sums whatever the shape and the split, then one epilogue: the same bits from all of them
+    g = torch.Generator().manual_seed(m + k + i)
+    wide = torch.full((m, k + 72), float("nan"), dtype=BF16)
+    wide[:, :k] = _integers(g, 4, m, k).to(BF16)
+    wg, wu = (_integers(g, 3, i, k) for _ in range(2))
+    sg, su = (torch.exp2(_integers(g, 1, i) - 6) for _ in range(2))
+    a, u = ((wide[:, :k].float() @ w.t()) * s for w, s in ((wg, sg), (wu, su)))
+    want = (oops.act_fn(act, a.to(BF16)).float() * u.to(BF16).float()).to(BF16)
+    wgu = tk.pack_fp8_gate_up(wg.to(torch.float8_e4m3fn).cuda(), sg, wu.to(torch.float8_e4m3fn).cuda(), su)
+    x = wide.cuda()[:, :k]
+    first = None
+    for tile in TILES + WHOLE:
+        for split in (1,) if tile in WHOLE or k < 64 else (1, 2):
+            buf = torch.full((m, i + 4), 7.0, dtype=BF16, device="cuda")
+            got = tk.many_rows_gemm(x, wgu, tile, split_k=split, act=act)
+            tk.many_rows_gemm(x, wgu, tile, split_k=split, act=act, out=buf[:, :i])
+            first = got if first is None else first
+            assert torch.equal(got, first) and torch.equal(buf[:, :i], first) and bool((buf[:, i:] == 7.0).all()), (tile, split)
+    _close(first, want, f"gated M={m} K={k} I={i}")

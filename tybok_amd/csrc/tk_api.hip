@@ -155,6 +155,7 @@ struct GemmExtra {
   void* vt = nullptr;  // transposed copy of the columns >= vt_col0 (rotary epilogue)
   int vt_col0 = 0, vt_ld = 0;
   int clear_counters = 0;  // zero the arrival counters a split launch uses right before it (shared static scratch)
+  int tile = 0;            // many-row kernels with this block shape, whatever the rules would take (tests, measurements)
 };
 
 // What gemm_common decided for a launch it was asked to plan instead of run.
@@ -245,7 +246,7 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
   // (from 256 rows on, or when its 128 x 256 tiles already fill the device; below that the skinny
   // kernel's finer blocks and K splits win)
   const int wide_blocks = ((a.ntiles * 32 + kWideCols - 1) / kWideCols) * ((M + 127) / 128);
-  if (!e.w16 && !rope && !e.x_f32 && a.vec && (M >= 256 || (M > 64 && wide_blocks >= cus)) &&
+  if (!e.w16 && !rope && !e.x_f32 && a.vec && (e.tile || M >= 256 || (M > 64 && wide_blocks >= cus)) &&
       (!has_norm || (ws && ws_bytes >= kNormOff + (size_t)M * K * 2 && (size_t)M * K * 2 <= kNormBytes))) {
     // many rows
     if (plan) return TK_OK;  // (plan->skinny stays false)
@@ -306,8 +307,8 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
     a.kt_q = a.KT / ks;
     a.kt_r = a.KT % ks;
     a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
-    int tile = 0;
-    if (wide_blocks >= 2 * cus && ks == 1) {
+    int tile = e.tile;
+    if (!tile && wide_blocks >= 2 * cus && ks == 1) {
       // blocks of 64 rows, two per CU, or of 192 / 256 rows, one per CU, where a CU's share of the rows (blocks in a row on
       // it x rows per block) is no larger than with 64 (measured on the gated 2048 -> 2 x 16384 launch: M=712 90 us on 192
       // rows, 100 on 256 -- its 384 blocks are one and a half generations; M=512 / 968 / 1024: 256-row blocks)
@@ -321,6 +322,7 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
       return fail(TK_ELAUNCH, "gemm: launch failed (%s)", hipGetErrorString(hipGetLastError()));
     return TK_OK;
   }
+  if (e.tile) return fail(TK_EINVAL, "gemm: the many-row kernels do not take these operands");
   int MT = M <= 32 ? 1 : 2;
   // The action chunk (33..64 rows) over a small weight matrix is a latency-bound launch: two blocks
   // of 32 rows per strip halve each block's staging, normalisation and product work and put twice
@@ -541,7 +543,7 @@ int tk_fp8w_gated_ffn(const void* x, int ldx, const void* wgu_packed, const void
 namespace {
 int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, const float* s0, const float* s1, void* y, int ldy,
                 const void* resid, int ldr, int resid_dtype, int M, int N, int K, int split_k, int act, void* ws, size_t ws_bytes,
-                hipStream_t st) {
+                hipStream_t st, int tile = 0) {
   if (M <= 0 || N <= 0 || K <= 0) return fail(TK_EINVAL, "w8a8: non-positive shape M=%d N=%d K=%d", M, N, K);
   if (K % 16) return fail(TK_EINVAL, "w8a8: K=%d must be a multiple of 16", K);
   if (lda % 16 || lda < K) return fail(TK_EINVAL, "w8a8: lda=%d must be >= K and a multiple of 16 (bytes)", lda);
@@ -596,7 +598,7 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.kt_r = a.KT % ks;
   a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
   const int rounds = ((a.KT + ks - 1) / ks + 3) / 4;
-  if (tk_launch_w8a8_gemm(a, pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, a.ntiles * 32, K, rounds, ks), st))
+  if (tk_launch_w8a8_gemm(a, tile ? tile : pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, a.ntiles * 32, K, rounds, ks), st))
     return fail(TK_ELAUNCH, "w8a8: launch failed (%s)", hipGetErrorString(hipGetLastError()));
   return TK_OK;
 }
@@ -1631,6 +1633,28 @@ int tk_debug_fp8w_gemm_cut(const void* x, int ldx, const void* w_packed, const v
   if (plan.skinny || plan.a.ksplit != 1 || tk_launch_gemm_stream_cut(plan.a, cut, (hipStream_t)stream))
     return fail(TK_EINVAL, "gemm_cut: only for shapes the 16-round weight-streaming kernel takes unsplit (K = 2048, at most 64 rows), cut 1..4");
   return TK_OK;
+}
+
+int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* w_packed, const void* s0, const void* s1, void* y, int ldy,
+                            const void* resid, int ldr, int resid_dtype, const void* gate, int M, int N, int K, int split_k, int act,
+                            int tile, void* ws, size_t ws_bytes, void* stream) {
+  if (act != TK_ACT_SILU && act != TK_ACT_GELU_TANH) return fail(TK_EINVAL, "many_rows: unknown activation %d", act);
+  if (s1 && (resid || gate)) return fail(TK_EINVAL, "many_rows: the gated form has no residual or per-column gate");
+  if (N % 4 || ldy % 4 || !aligned8(y)) return fail(TK_EINVAL, "many_rows: N=%d and ldy=%d must be multiples of 4, y 8-byte aligned", N, ldy);
+  bool known = false;
+  if (sa) {
+    for (const Fp8Tile& t : kW8a8Tiles) known |= t.t.id == tile;
+    if (!known || gate) return fail(TK_EINVAL, "many_rows: W8A8 has no tile %d, and no per-column gate", tile);
+    return w8a8_common(x, ldx, (const float*)sa, w_packed, (const float*)s0, (const float*)s1, y, ldy, resid, ldr, resid_dtype, M, N, K,
+                       split_k, act, ws, ws_bytes, (hipStream_t)stream, tile);
+  }
+  for (const Fp8Tile& t : kWideTiles) known |= t.t.id == tile;
+  const bool whole = tile == 28 || tile == 68 || tile == 88;  // the kernels without a K split
+  if (!known && !(whole && split_k == 1)) return fail(TK_EINVAL, "many_rows: weight-only has no tile %d for split_k=%d", tile, split_k);
+  GemmExtra e;
+  e.tile = tile;
+  return gemm_common(x, ldx, w_packed, (const float*)s0, (const float*)s1, y, ldy, resid, ldr, resid_dtype, gate, M, N, K, split_k, act,
+                     ws, ws_bytes, (hipStream_t)stream, e);
 }
 
 int tk_debug_decode_fp8(void* out_f32, void* stream) {

@@ -158,6 +158,11 @@ SIGNATURES: dict[str, tuple] = {
     "tk_pi_denoise": (c_int, [c_void_p, c_void_p]),
     "tk_debug_decode_fp8": (c_int, [c_void_p, c_void_p]),
     "tk_debug_stream_read": (c_int, [c_void_p, c_size_t, c_int, c_void_p, c_void_p]),
+    "tk_debug_many_rows_gemm": (
+        c_int,
+        [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p]
+        + [c_int] * 6 + [c_void_p, c_size_t, c_void_p],
+    ),  # fmt: skip
     "tk_debug_fp8w_gemm_cut": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }
 

@@ -1375,3 +1375,31 @@ def decode_fp8_table(device: torch.device | str = "cuda") -> torch.Tensor:
     out = torch.empty(256, dtype=torch.float32, device=device)
     native.check(native.lib().tk_debug_decode_fp8(out.data_ptr(), _stream()), "tk_debug_decode_fp8")
     return out
+
+
+def many_rows_gemm(
+    x: torch.Tensor, w: PackedWeight | PackedGateUp, tile: int, *, sa: torch.Tensor | None = None, act: str = "gelu_tanh",
+    resid: torch.Tensor | None = None, gate: torch.Tensor | None = None, split_k: int = 1, out: torch.Tensor | None = None,
+    ws: Workspace | None = None,
+) -> torch.Tensor:  # fmt: skip
+    """One launch of the many-row fp8-weight kernels with the block shape ``tile``, for tests and timing: :func:`fp8w_gemm`, with
+    ``sa`` :func:`w8a8_gemm`, or the gate/up half of either gated form, which take a shape by the sizes of the call."""
+    gated = isinstance(w, PackedGateUp)
+    n = w.i if gated else w.n
+    if sa is None:
+        m, ldx = _check_act(x, w.k)
+    else:
+        x = x.view(torch.uint8)
+        if x.dim() != 2 or x.shape[1] != w.k or x.stride(1) != 1 or sa.dtype != torch.float32 or sa.numel() != x.shape[0] or not sa.is_contiguous():
+            raise ValueError(f"x must be e4m3fn codes [M, {w.k}] with unit inner stride and sa contiguous fp32 [M]")
+        m, ldx = x.shape[0], x.stride(0)
+    if out is None:
+        out = torch.empty(m, n, dtype=torch.bfloat16, device=x.device)
+    rp, ldr, rdt = _resid_args(resid, m, n)
+    ws = ws or default_workspace(x.device)
+    rc = native.lib().tk_debug_many_rows_gemm(
+        x.data_ptr(), ldx, _ptr(sa), w.data.data_ptr(), (w.scale_gate if gated else w.scale).data_ptr(), w.scale_up.data_ptr() if gated else None,
+        out.data_ptr(), out.stride(0), rp, ldr, rdt, _gate_ptr(gate, n), m, n, w.k, split_k, ACT[act], tile, ws.ptr, ws.nbytes, _stream(),
+    )  # fmt: skip
+    native.check(rc, "tk_debug_many_rows_gemm")
+    return out
