@@ -663,7 +663,7 @@ int tk_debug_fp8w_gemm_cut(const void* x, int ldx, const void* w_packed, const v
  * forms take one by the shape: for tests that run every block shape over the same operands, and for timing them.
  *   sa: NULL = weight-only (x bf16, ldx in elements; tiles 408, 404, 304, 208, 204: 100 * 32-row tiles + 32-column tiles of a
  *       block; with split_k = 1 also 28, 68, 88, the kernels of the largest grids), otherwise the row scales of e4m3 codes
- *       (ldx in bytes; tiles 604, 408, 414, 204).
+ *       (ldx in bytes; tiles 604, 408, 414, 204; with split_k = 1 also 28).
  *   s1: NULL = plain (scale s0, residual, weight-only: per-column gate), otherwise gated (w_packed from tk_pack_fp8_gate_up, N the
  *       intermediate's width, act).  Other arguments as tk_fp8w_gemm; N and ldy multiples of 4.  No counterpart in the
  * reference. */

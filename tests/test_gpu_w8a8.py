@@ -170,7 +170,7 @@ def test_w8a8_gemm_edges_exact_on_small_integers(tk, m, k, n, split):
     assert torch.equal(tk.w8a8_gemm(wide.cuda()[:, :k], sa.cuda(), pw, split_k=split).cpu(), y)
 
 
-W8A8_TILES = (408, 414, 204, 604)  # 64 x 128, 128 x 128 (414), 128 x 256 and 192 x 128 blocks
+W8A8_TILES = (408, 414, 204, 604, 28)  # 128 x 256, 128 x 128, 64 x 128, 192 x 128 blocks; 64 x 256 with weights in registers, no K split
 
 
 def _integers(g, top, *shape):
@@ -190,7 +190,7 @@ def test_every_w8a8_block_shape_exact_on_small_integers(tk, tile, k):
     # rows and columns one (four) past a block and short of one, one row alone; K inside a round, more rounds than the ring
     # holds; even and uneven splits; NaN codes behind K, residuals, a pitch that allows only 8-byte stores (N + 4) and one with
     # room behind N.  Exact: |sum| <= 6 * 4112 times powers of two, rounded once to bf16 each time.
-    rows, cols = (128, 128) if tile == 414 else (tile // 100 * 32, tile % 100 * 32)
+    rows, cols = {414: (128, 128), 28: (64, 256)}.get(tile, (tile // 100 * 32, tile % 100 * 32))
     for m, n in ((rows + 1, cols + 4), (1, 4), (2 * rows - 31, 36), (rows, 2 * cols - 60)):
         g = torch.Generator().manual_seed(m + k + n)
         a, w = _integers(g, 3, m, k), _integers(g, 2, n, k)
@@ -200,7 +200,7 @@ def test_every_w8a8_block_shape_exact_on_small_integers(tk, tile, k):
         full = (y.float() + r.float()).to(BF16)
         pw = tk.pack_fp8_weight(w.to(torch.float8_e4m3fn).cuda(), sw.cuda())
         x, sac, rc = _codes_before_nan(a), sa.cuda(), r.cuda()
-        for split in (s for s in (1, 2, 3, 5) if s <= (k + 31) // 32):
+        for split in (1,) if tile == 28 else (s for s in (1, 2, 3, 5) if s <= (k + 31) // 32):
             assert torch.equal(tk.many_rows_gemm(x, pw, tile, sa=sac, split_k=split).cpu(), y), (m, n, split)
             for pitch in (n + 4, (n + 15) // 8 * 8):
                 buf = torch.full((m, pitch), 7.0, dtype=BF16, device="cuda")
@@ -222,7 +222,7 @@ def test_every_w8a8_block_shape_gives_the_same_gated_bits(tk, m, k, i, act):
     x, sac = _codes_before_nan(a), sa.cuda()
     first = None
     for tile in W8A8_TILES:
-        for split in (1,) if k < 64 else (1, 2):
+        for split in (1,) if tile == 28 or k < 64 else (1, 2):
             buf = torch.full((m, i + 4), 7.0, dtype=BF16, device="cuda")
             got = tk.many_rows_gemm(x, wgu, tile, sa=sac, split_k=split, act=act)
             tk.many_rows_gemm(x, wgu, tile, sa=sac, split_k=split, act=act, out=buf[:, :i])

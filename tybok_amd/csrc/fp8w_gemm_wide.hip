@@ -9,165 +9,12 @@
 
 namespace {
 using pipe::lds_barrier;
+using pipe::wide_ep_pitch;
+using pipe::wide_epilogue;
 
-constexpr int NT = 2;   // n tiles per wave
-constexpr int NW = 4;   // waves per block
-constexpr int RK = 2;   // k tiles per round
-
-// LDS row pitch (bytes) of a wave's private 32-row output tile in wide_epilogue
-__host__ __device__ constexpr int wide_ep_pitch(int epi) { return (epi == 0 ? NT * 32 : 32) * 2 + 16; }
-
-// Epilogue of a wave that holds MT x NT accumulator tiles: rows row0 .. row0 + MT*32 - 1, packed n tiles strip*NT ..
-// (EPI 1: the (gate, up) pair of output columns strip*32 ..).  wl: the wave's private LDS tile of 32 rows x
-// wide_ep_pitch(EPI) bytes (used when the output is 16-byte aligned); the caller has made sure that no wave still
-// reads what that space held before.
-template <int EPI, int MT>
-__device__ __forceinline__ void wide_epilogue(const GemmArgs& a, const f32x16 (&acc)[MT][NT], unsigned char* wl, int row0, int strip, int lane) {
-  const int half = lane >> 5;
-  const int l32 = lane & 31;
-  // ---- epilogue: lane l of a tile owns row m = l % 32 and, per register group g, four
-  // consecutive columns 8g + 4*(l/32) .. +3 (the accumulators hold C^T) ----
-  if (a.vec16) {
-    // Coalesced stores: a lane holds, per tile, row l % 32 and four 4-column pieces 16 bytes apart -- stored as
-    // they are, one instruction would touch 32 rows with 16 bytes each.  Each wave therefore passes its 32 rows of
-    // an m tile through a private LDS tile (a wave's LDS instructions execute in order, so it needs no barrier
-    // of its own) and stores them as 16-byte chunks of consecutive columns: whole 64- or 128-byte row segments
-    // per 4 or 8 lanes.
-    constexpr int COLS = EPI == 0 ? NT * 32 : 32;  // output columns of a wave per row
-    constexpr int EP = COLS * 2 + 16;              // LDS row pitch (bytes)
-    constexpr int LPR = COLS / 8;                  // lanes (16-byte chunks) per row
-    constexpr int RPI = 64 / LPR;                  // rows per store instruction
-    static_assert(EP == wide_ep_pitch(EPI), "the callers size the LDS tiles by wide_ep_pitch");
-    const int ncol0 = EPI == 0 ? strip * NT * 32 : strip * 32;  // first output column of this wave
-    f32x4 sc0[EPI == 0 ? NT : 1][4], sc1[4], gt[EPI == 0 ? NT : 1][4];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      if (EPI == 0) {
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          int n0 = (strip * NT + nt) * 32 + 8 * g + 4 * half;
-          if (n0 > a.N - 4) n0 = a.N - 4;  // columns past N are never stored
-          sc0[EPI == 0 ? nt : 0][g] = *(const f32x4*)(a.s0 + n0);
-          if (a.gate) gt[EPI == 0 ? nt : 0][g] = unpack_bf16x4(*(const i32x2*)(a.gate + n0));
-        }
-      } else {
-        int col = strip * 32 + 8 * g + 4 * half;
-        if (col > a.N - 4) col = a.N - 4;
-        sc0[0][g] = *(const f32x4*)(a.s0 + col);
-        sc1[g] = *(const f32x4*)(a.s1 + col);
-      }
-    }
-    const int lrow = lane / LPR, lchunk = lane % LPR;
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        if (EPI == 0) {
-#pragma unroll
-          for (int nt = 0; nt < NT; ++nt) {
-            const f32x16& c = acc[mt][nt];
-            const f32x4 v = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-            i32x2 r = pack_bf16x4(v * sc0[EPI == 0 ? nt : 0][g]);
-            if (a.gate) r = pack_bf16x4(unpack_bf16x4(r) * gt[EPI == 0 ? nt : 0][g]);
-            *(i32x2*)(wl + l32 * EP + (nt * 32 + 8 * g + 4 * half) * 2) = r;
-          }
-        } else {
-          const f32x16& cg = acc[mt][0];
-          const f32x16& cu = acc[mt][1];
-          const f32x4 vg = {cg[4 * g], cg[4 * g + 1], cg[4 * g + 2], cg[4 * g + 3]};
-          const f32x4 vu = {cu[4 * g], cu[4 * g + 1], cu[4 * g + 2], cu[4 * g + 3]};
-          const f32x4 gg = unpack_bf16x4(pack_bf16x4(vg * sc0[0][g]));
-          const f32x4 up = unpack_bf16x4(pack_bf16x4(vu * sc1[g]));
-          f32x4 act;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) act[j] = a.act == 0 ? silu_f(gg[j]) : gelu_tanh_f(gg[j]);
-          act = unpack_bf16x4(pack_bf16x4(act));
-          *(i32x2*)(wl + l32 * EP + (8 * g + 4 * half) * 2) = pack_bf16x4(act * up);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < 32 / RPI; ++j) {
-        const int row = j * RPI + lrow;
-        const int m = row0 + mt * 32 + row;
-        const int n = ncol0 + lchunk * 8;
-        i32x4 t = *(const i32x4*)(wl + row * EP + lchunk * 16);
-        if (m >= a.M || n >= a.N) continue;
-        if (EPI == 0 && a.resid) {
-          // bf16(y + resid) on the bf16-rounded product, as the scattered path computes it
-          f32x4 r0, r1 = {0.f, 0.f, 0.f, 0.f};
-          if (a.resid_f32) {
-            const f32x4* rp = (const f32x4*)((const float*)a.resid + (size_t)m * a.ldr + n);
-            r0 = rp[0];
-            if (n + 8 <= a.N) r1 = rp[1];
-          } else if (n + 8 <= a.N) {
-            const i32x4 rr = *(const i32x4*)((const u16*)a.resid + (size_t)m * a.ldr + n);
-            r0 = unpack_bf16x4(i32x2{rr[0], rr[1]});
-            r1 = unpack_bf16x4(i32x2{rr[2], rr[3]});
-          } else {
-            r0 = unpack_bf16x4(*(const i32x2*)((const u16*)a.resid + (size_t)m * a.ldr + n));
-          }
-          const i32x2 lo = pack_bf16x4(unpack_bf16x4(i32x2{t[0], t[1]}) + r0), hi = pack_bf16x4(unpack_bf16x4(i32x2{t[2], t[3]}) + r1);
-          t = i32x4{lo[0], lo[1], hi[0], hi[1]};
-        }
-        u16* dst = a.y + (size_t)m * a.ldy + n;
-        if (n + 8 <= a.N) *(i32x4*)dst = t;
-        else *(i32x2*)dst = i32x2{t[0], t[1]};  // N % 8 == 4: the row's last four columns
-      }
-    }
-    return;
-  }
-  if (EPI == 0) {
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n0 = (strip * NT + nt) * 32 + 8 * g + 4 * half;
-        if (n0 >= a.N) continue;
-        const f32x4 sc = *(const f32x4*)(a.s0 + n0);
-        f32x4 gt = {0.f, 0.f, 0.f, 0.f};
-        if (a.gate) gt = unpack_bf16x4(*(const i32x2*)(a.gate + n0));
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const int m = row0 + mt * 32 + l32;
-          if (m >= a.M) continue;
-          const f32x16& c = acc[mt][nt];
-          f32x4 v = {c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]};
-          i32x2 r = pack_bf16x4(v * sc);
-          if (a.gate) r = pack_bf16x4(unpack_bf16x4(r) * gt);
-          if (a.resid) {
-            const f32x4 rv = a.resid_f32 ? *(const f32x4*)((const float*)a.resid + (size_t)m * a.ldr + n0)
-                                         : unpack_bf16x4(*(const i32x2*)((const u16*)a.resid + (size_t)m * a.ldr + n0));
-            r = pack_bf16x4(unpack_bf16x4(r) + rv);
-          }
-          *(i32x2*)(a.y + (size_t)m * a.ldy + n0) = r;
-        }
-      }
-  } else {
-    // tile pair (gate, up) of logical columns strip*32 ..; I % 32 == 0
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int col = strip * 32 + 8 * g + 4 * half;
-      if (col >= a.N) continue;
-      const f32x4 scg = *(const f32x4*)(a.s0 + col), scu = *(const f32x4*)(a.s1 + col);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int m = row0 + mt * 32 + l32;
-        if (m >= a.M) continue;
-        const f32x16& cg = acc[mt][0];
-        const f32x16& cu = acc[mt][1];
-        const f32x4 vg = {cg[4 * g], cg[4 * g + 1], cg[4 * g + 2], cg[4 * g + 3]};
-        const f32x4 vu = {cu[4 * g], cu[4 * g + 1], cu[4 * g + 2], cu[4 * g + 3]};
-        const f32x4 gg = unpack_bf16x4(pack_bf16x4(vg * scg));
-        const f32x4 up = unpack_bf16x4(pack_bf16x4(vu * scu));
-        f32x4 act;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) act[j] = a.act == 0 ? silu_f(gg[j]) : gelu_tanh_f(gg[j]);
-        act = unpack_bf16x4(pack_bf16x4(act));
-        *(i32x2*)(a.y + (size_t)m * a.ldy + col) = pack_bf16x4(act * up);
-      }
-    }
-  }
-}
+constexpr int NT = pipe::WIDE_NT;  // n tiles per wave
+constexpr int NW = 4;              // waves per block
+constexpr int RK = 2;              // k tiles per round
 
 // Grids that cover the device twice over (from 385 rows of the gated 2048 -> 2 x 16384 launch): there the power of the
 // operands' way decides the matrix pipes' clock, and the two kernels below, whose weights go through registers, are the cheaper
@@ -364,7 +211,7 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
   constexpr int EP = wide_ep_pitch(EPI);
   static_assert(NW * 32 * EP == EPB, "the epilogue tiles fit the LDS array");
   if (a.vec16) lds_barrier();  // every wave has left the staged activations behind
-  wide_epilogue<EPI, MT>(a, acc, lds + wave * 32 * EP, mblock * ROWS, strip, lane);
+  wide_epilogue<pipe::BF16_FP8, EPI, MT>(a, acc, lds + wave * 32 * EP, mblock * ROWS, strip, lane);
 }
 
 // The same where taller blocks waste no more rows: eight waves own 2*WM*32 rows x 256 packed columns, with both operands of a
@@ -530,7 +377,7 @@ __global__ __launch_bounds__(512, 1) void fp8w_tile_kernel(GemmArgs a, int nblk_
 
   constexpr int EP = wide_ep_pitch(EPI);
   if (a.vec16) lds_barrier();
-  wide_epilogue<EPI, WM>(a, acc, lds + wave * 32 * EP, mblock * ROWS + wm * WM * 32, strip, lane);
+  wide_epilogue<pipe::BF16_FP8, EPI, WM>(a, acc, lds + wave * 32 * EP, mblock * ROWS + wm * WM * 32, strip, lane);
 }
 
 // One block per row: out = bf16 norm of the bf16 row, with the rounding points of the skinny

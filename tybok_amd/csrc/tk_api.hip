@@ -597,6 +597,17 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.kt_q = a.KT / ks;
   a.kt_r = a.KT % ks;
   a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
+  if (!tile && ks == 1 && blocks128 >= 2 * device_cus()) {
+    // rows a CU works through (blocks in a row on it x rows per block), per 256 columns: w8a8_wide_kernel where its 64-row blocks
+    // leave the fewest
+    auto share = [&](int rows, int cols) {
+      const long long blocks = (long long)((M + rows - 1) / rows) * ((a.ntiles * 32 + cols - 1) / cols);
+      return (blocks + device_cus() - 1) / device_cus() * rows * cols / 256;
+    };
+    tile = 28;
+    for (const Fp8Tile& t : kW8a8Tiles)
+      if (share(32 * t.t.bm, 32 * t.t.bn) <= share(64, 256)) tile = 0;
+  }
   const int rounds = ((a.KT + ks - 1) / ks + 3) / 4;
   if (tk_launch_w8a8_gemm(a, tile ? tile : pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, a.ntiles * 32, K, rounds, ks), st))
     return fail(TK_ELAUNCH, "w8a8: launch failed (%s)", hipGetErrorString(hipGetLastError()));
@@ -1644,7 +1655,7 @@ int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* 
   bool known = false;
   if (sa) {
     for (const Fp8Tile& t : kW8a8Tiles) known |= t.t.id == tile;
-    if (!known || gate) return fail(TK_EINVAL, "many_rows: W8A8 has no tile %d, and no per-column gate", tile);
+    if (!(known || (tile == 28 && split_k == 1)) || gate) return fail(TK_EINVAL, "many_rows: W8A8 has no tile %d, and no per-column gate", tile);
     return w8a8_common(x, ldx, (const float*)sa, w_packed, (const float*)s0, (const float*)s1, y, ldy, resid, ldr, resid_dtype, M, N, K,
                        split_k, act, ws, ws_bytes, (hipStream_t)stream, tile);
   }

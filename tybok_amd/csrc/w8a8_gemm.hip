@@ -81,14 +81,174 @@ __global__ __launch_bounds__(256) void quant_act_rows_kernel(QuantActArgs a) {
   }
 }
 
+// Rows whose share of a compute unit comes out smallest in 64-row blocks, two a CU (577 .. 640, 769 .. 896 rows of the gated
+// 2048 -> 2 x 16384 launch): 608 / 800 / 896 rows 58.1 / 74.6 / 77.3 us against 61.9 / 79.2 / 81.4 of fp8_pipe_kernel's
+// blocks of 128 x 256, whose last generation is half empty there (graph replay, cold weights).  A block that also loads on waves of its own does not
+// fit a CU twice: registers.
+// A block of four waves owns 64 rows x 256 packed columns; wave w owns n tiles 2w, 2w + 1 for all rows, its weights straight from
+// memory into its registers; a round's activations (128 columns) are staged once per block through LDS.  No K split.
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void w8a8_wide_kernel(GemmArgs a, int nblk_m, int ngroups) {
+  using namespace pipe;
+  constexpr int MT = 2, NT = WIDE_NT, NW = 4;  // 32-row tiles of a block, n tiles of a wave, waves
+  constexpr int RK = 4, PF = 3;                // k tiles of a round (two 64-wide product steps), rounds in flight
+  constexpr int PITCH = RK * 32 + 16, XBUF = MT * 32 * PITCH;  // of the staged rows
+  constexpr int PPR = RK * 2, XPT = MT * 32 * PPR / (NW * 64);  // 16-byte pieces per staged row, per thread
+  constexpr int EPB = NW * 32 * wide_ep_pitch(EPI);
+  __shared__ __align__(16) unsigned char lds[2 * XBUF > EPB ? 2 * XBUF : EPB];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5;
+  const int l32 = lane & 31;
+
+  // slot s of XCD x (blocks are dealt to the 8 XCDs round-robin) -> group (s / nblk_m) * 8 + x, m block s % nblk_m: the
+  // nblk_m blocks of a group (same weights) run back to back on one XCD
+  const unsigned slot = blockIdx.x >> 3;
+  const int mblock = (int)(slot % (unsigned)nblk_m);
+  const int nblk = (int)((slot / (unsigned)nblk_m) * 8 + (blockIdx.x & 7));
+  if (nblk >= ngroups) return;
+  const int nrounds = (a.KT + RK - 1) / RK;
+  const int strip = nblk * NW + wave;  // this wave's pair of packed n tiles
+  const uint8_t* wbase[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) {
+    int ntg = strip * NT + nt;
+    if (ntg > a.ntiles - 1) ntg = a.ntiles - 1;  // overhanging tiles are computed on valid data, never stored
+    wbase[nt] = a.w + ((size_t)ntg * a.KT) * 1024 + lane * 16;
+  }
+  const char* xsrc[XPT];
+  int xcol[XPT], xdst[XPT];
+#pragma unroll
+  for (int i = 0; i < XPT; ++i) {
+    const int p = tid + i * NW * 64, r = p / PPR, c = p % PPR;
+    int m = mblock * MT * 32 + r;
+    if (m > a.M - 1) m = a.M - 1;  // rows past M: valid data, never stored
+    xsrc[i] = (const char*)a.x + (size_t)m * a.ldx;
+    xcol[i] = c * 16;
+    xdst[i] = r * PITCH + c * 16;
+  }
+  f32x16 acc[MT][NT];
+#pragma unroll
+  for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[mt][nt][i] = 0.f;
+
+  struct WFrag {
+    i32x4 w[RK][NT];
+  };
+  struct XFrag {
+    i32x4 v[XPT];
+  };
+  // One piece of each kind of work, so that a round can deal them out between its matrix instructions: a wave cannot issue
+  // anything while it waits for the matrix pipe to take its next instruction.
+  auto wload1 = [&](WFrag& f, int r, int st, int q) {  // q in [0, 2*NT): k tile 2*st + q/NT of round r, n tile q%NT
+    const int j = 2 * st + q / NT, nt = q % NT;
+    int kt = r * RK + j;
+    if (kt > a.KT - 1) kt = a.KT - 1;  // its activation columns are zeroed
+    f.w[j][nt] = *(const i32x4*)(wbase[nt] + (size_t)kt * 1024);
+  };
+  auto xload1 = [&](XFrag& f, int r, int i) {
+    int k = r * RK * 32 + xcol[i];
+    if (k > a.K - 16) k = a.K - 16;
+    f.v[i] = *(const i32x4*)(xsrc[i] + k);
+  };
+  auto xstore1 = [&](const XFrag& f, int r, int b, int i) {
+    const i32x4 z = {0, 0, 0, 0};
+    *(i32x4*)(lds + b * XBUF + xdst[i]) = r * RK * 32 + xcol[i] < a.K ? f.v[i] : z;
+  };
+  i32x4 xa[2][MT][2];  // operands of the round's two steps, as the 16-byte halves they are read in
+  auto xread1 = [&](int st, int b, int u) {  // u in [0, 2*MT): half u%2 of m tile u/2
+    xa[st][u / 2][u % 2] = *(const i32x4*)(lds + b * XBUF + ((u / 2) * 32 + l32) * PITCH + st * 64 + 16 * half + 32 * (u % 2));
+  };
+  auto mma1 = [&](const WFrag& f, int st, int t) {  // t in [0, MT*NT): m tile t/NT, n tile t%NT
+    const int mt = t / NT, nt = t % NT;
+    const i32x4 wl = f.w[2 * st][nt], wh = f.w[2 * st + 1][nt], xl = xa[st][mt][0], xh = xa[st][mt][1];
+    acc[mt][nt] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(i32x8{wl[0], wl[1], wl[2], wl[3], wh[0], wh[1], wh[2], wh[3]},
+                                                                  i32x8{xl[0], xl[1], xl[2], xl[3], xh[0], xh[1], xh[2], xh[3]},
+                                                                  acc[mt][nt], 0, 0, 0, 0, 0, 0);
+  };
+  // PF rounds in flight, every load unconditional (clamped addresses; columns past K are zeroed when staged).  Round r,
+  // phase A: multiplies step 0 while step 1's operands are fetched from LDS, round r+1 is staged into the other LDS buffer
+  // and the weight registers that round r-1's step 1 has left are refilled; then the round's only barrier (a wave writes
+  // buffer b for round r+2 only after every wave has passed the barrier of round r+1, with its round-r operands in
+  // registers); phase B: fetches round r+1's first operands, multiplies step 1 and refills step 0's weight registers.  A
+  // phase never reloads registers its own matrix instructions read.
+  constexpr int SLOTS = MT * NT;
+  static_assert(SLOTS == 2 * MT && SLOTS >= 2 * NT && 2 * XPT <= SLOTS, "one operand read per slot; the other pieces fit");
+  WFrag wbuf[PF];
+  XFrag xbuf[PF];
+#pragma unroll
+  for (int p = 0; p < PF; ++p) {
+#pragma unroll
+    for (int i = 0; i < XPT; ++i) xload1(xbuf[p], p, i);
+#pragma unroll
+    for (int q = 0; q < 2 * NT; ++q) {
+      wload1(wbuf[p], p, 0, q);
+      wload1(wbuf[p], p, 1, q);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < XPT; ++i) xstore1(xbuf[0], 0, 0, i);
+#pragma unroll
+  for (int i = 0; i < XPT; ++i) xload1(xbuf[0], PF, i);
+  lds_barrier();
+#pragma unroll
+  for (int u = 0; u < 2 * MT; ++u) xread1(0, 0, u);
+  auto round = [&](int p, int r) {
+    const int b = r & 1;
+    const int pn = (p + 1) % PF, pp = (p + PF - 1) % PF;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      mma1(wbuf[p], 0, i);
+      xread1(1, b, i);
+      if (i < XPT) xstore1(xbuf[pn], r + 1, b ^ 1, i);
+      if (i >= SLOTS - XPT) xload1(xbuf[pn], r + 1 + PF, i - (SLOTS - XPT));
+      if (i < 2 * NT) wload1(wbuf[pp], r - 1 + PF, 1, i);  // the registers round r-1 finished with in its phase B
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < SLOTS; ++i) {
+      mma1(wbuf[p], 1, i);
+      xread1(0, b ^ 1, i);
+      if (i < 2 * NT) wload1(wbuf[p], r + PF, 0, i);  // step 0's registers: free since phase A
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int it = 0;
+  for (; it + PF <= nrounds; it += PF) {
+#pragma unroll
+    for (int p = 0; p < PF; ++p) round(p, it + p);
+  }
+#pragma unroll
+  for (int q = 0; q < PF - 1; ++q)
+    if (q < nrounds - it) round(q, it + q);  // block-uniform
+
+  if (a.vec16) lds_barrier();  // every wave has left the staged activations behind
+  wide_epilogue<FP8, EPI, MT>(a, acc, lds + wave * 32 * wide_ep_pitch(EPI), mblock * MT * 32, strip, lane);
+}
+
 }  // namespace
 
 int tk_quant_act_max_k() { return kQuantMaxPieces * 256 * 8; }
 
-// tile: an id of kW8a8Tiles (tk_api.hip)
+// tile: an id of kW8a8Tiles (tk_api.hip), or 28: w8a8_wide_kernel (no K split)
 int tk_launch_w8a8_gemm(const GemmArgs& a, int tile, hipStream_t st) {
   using namespace pipe;
   switch (tile) {
+    case 28: {
+      const int nblk_m = (a.M + 63) / 64, nblk_n = (a.ntiles + 7) / 8;
+      const dim3 grid((unsigned)((nblk_n + 7) / 8) * 8u * (unsigned)nblk_m), block(256);
+      if (a.s1) hipLaunchKernelGGL(w8a8_wide_kernel<1>, grid, block, 0, st, a, nblk_m, nblk_n);
+      else hipLaunchKernelGGL(w8a8_wide_kernel<0>, grid, block, 0, st, a, nblk_m, nblk_n);
+      return hipGetLastError() == hipSuccess ? 0 : -3;
+    }
     case 604: return launch_fp8_pipe<FP8, 6, 4, 2, 2, 4, 1>(a, st);
     case 414: return launch_fp8_pipe<FP8, 4, 4, 2, 2, 4, 1>(a, st);
     case 408: return launch_fp8_pipe<FP8, 4, 8, 2, 2, 3, 1>(a, st);
