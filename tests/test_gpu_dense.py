@@ -316,6 +316,17 @@ def test_long_k_keeps_its_split_count(tk, m, k, n, splits):
         assert torch.equal(got, tk.bf16w_dense(x.cuda(), pw, b.cuda(), split_k=splits))
 
 
+@pytest.mark.parametrize("m,k,n,splits", [(700, 16384, 2048, 2), (1500, 12288, 960, 2), (300, 8192, 4096, 2), (500, 16384, 2048, 4), (968, 12304, 2048, 1), (40, 8160, 96, 8)])
+def test_long_k_is_split_further_where_that_pays(tk, m, k, n, splits):
+    # more splits than fill the device with 64 x 128 blocks (1, 1, 1, 2, 1) where the cost model says so; 8160 columns are its choice
+    x, w, b = _case(m, k, n, seed=10)
+    pw = tk.pack_bf16_weight(w.cuda())
+    got = tk.bf16w_dense(x.cuda(), pw, b.cuda())
+    _close(got, _want(x, w, b), "long k")
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert torch.equal(got, tk.bf16w_dense(x.cuda(), pw, b.cuda(), split_k=splits))
+
+
 @pytest.mark.parametrize("m,k,n,split", [(2391, 2592, 2824, 2), (234, 3760, 11344, 5), (671, 14656, 4904, 4), (304, 15936, 3424, 12)])
 def test_explicit_split_takes_a_block_shape_whose_partials_fit(tk, m, k, n, split):
     # the partials are whole blocks: the fastest block shape pads these outputs past the workspace's 56 MiB, others do not

@@ -99,16 +99,19 @@ struct PipeTile {
 // 14 %, the picked launch on average 1.1 % slower than the best one).  Blocks on one CU share its memory pipe (12 ns a KiB)
 // and matrix pipes (75 ns for a wave's tile and round); a round takes no less than the round trip over the rounds on
 // their way; the epilogue costs per tile; each further generation of blocks pays all of it again.
-float pipe_cost(const PipeTile& t, float kb_n, int M, int N, int rounds, int ks, int cus) {
+// long_k: K > 8160, fitted to 12000 timings with cold weights (112 shapes of 64 .. 1500 rows, K 8192 .. 16384, 320 .. 4096
+// columns; the picked launch on average 2.7 % slower than the best one): the round trip sets the time of shallow rings, and a
+// split costs by its partials rather than by itself.
+float pipe_cost(const PipeTile& t, float kb_n, int M, int N, int rounds, int ks, int cus, bool long_k = false) {
   const int rows = 32 * t.bm, cols = 32 * t.bn;
   const long long blocks = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * ks;
   float us = 1.66f;
   for (long long left = blocks; left > 0; left -= (long long)cus * t.occ) {
     const float r = left > cus && t.occ > 1 ? 2.f : 1.f;  // blocks on a CU
-    const float load = r * ((float)t.bm * 4.f + (float)t.bn * kb_n) * 0.0122f, mul = r * (float)t.wt * 0.0751f, trip = 0.585f / (float)(t.ns - 1);
+    const float load = r * ((float)t.bm * 4.f + (float)t.bn * kb_n) * 0.0122f, mul = r * (float)t.wt * 0.0751f, trip = (long_k ? 0.66f : 0.585f) / (float)(t.ns - 1);
     us += 0.014f + (float)rounds * (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip)) + r * (float)(t.bm * t.bn) * 0.203f;
   }
-  if (ks > 1) us += 4.76f + (float)blocks * (float)(t.bm * t.bn) * 0.00213f;  // fp32 partials out and back in
+  if (ks > 1) us += (long_k ? 2.5f : 4.76f) + (float)blocks * (float)(t.bm * t.bn) * (long_k ? 0.004f : 0.00213f);  // fp32 partials out and back in
   return us;
 }
 // The forms over fp8 weights.  Where the grid covers the device several times over, the time is the matrix pipes' at the
@@ -717,15 +720,20 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
   float best_cost = 0.f;
   bool known = false;
   size_t need = 0;  // of an explicit split that does not fit: the smallest partials of any block shape
-  // A K of 8192 or more over few columns (the connector, 12288 -> 960): as many splits as fill the device with 64 x 128
-  // blocks, 32 k tiles or more each, whatever block is picked.  The cost below would take 8 splits instead of 12 at 128
-  // rows and save 2 us of a request; but the sums of such a K are what a chunk's distance from the reference arithmetic
-  // hangs on most, and they stay as short as they are (largest distance of a two-layer chunk 8.3e-3, 10.1e-3 with 8).
-  int k_from = split_k > 0 ? split_k : 1;
-  if (split_k <= 0 && !rope && a.KT >= 256) {
-    k_from = cus / (((M + 63) / 64) * ((N + 127) / 128));
-    k_from = k_from < a.KT / 32 ? k_from : a.KT / 32;
-    k_from = k_from > 1 ? k_from : 1;
+  // Splits to choose from.  K up to 8160: any that leaves 16 k tiles, at most 8; the rotary form none unless asked for (the
+  // partials weigh more than the idle CUs).  Above: 32 k tiles or more each, and at least as many as fill the device with
+  // 64 x 128 blocks, so that the connector of the vision tower (64 rows a camera, 12288 -> 960) keeps its 12 / 12 / 10 / 8
+  // splits and with them its bits (free to choose, 8 at 128 rows would save 2 us of a request).  That number alone is too few
+  // where the rows fill the device without a split: 700 x 16384 -> 2048 109 us in 1 split, 65 in 2; 1500 x 16384 -> 960 113, 69.
+  const bool long_k = a.KT >= 256;
+  int k_from = split_k > 0 ? split_k : 1, k_to = k_from;
+  if (split_k <= 0 && !rope) {
+    if (long_k) {
+      k_from = cus / (((M + 63) / 64) * ((N + 127) / 128));
+      k_from = k_from < a.KT / 32 ? k_from : a.KT / 32;
+      k_from = k_from > 1 ? k_from : 1;
+    }
+    k_to = long_k ? a.KT / 32 : a.KT < 32 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
   }
   for (const PipeTile& t : kDenseTiles) {
     if (tile && t.id != tile) continue;
@@ -734,9 +742,7 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
     // splits whose partials (whole blocks) and counters the workspace holds: a block shape that pads the output more holds fewer
     const size_t blocks0 = (size_t)((M + 32 * t.bm - 1) / (32 * t.bm)) * ((N + 32 * t.bn - 1) / (32 * t.bn));
     const size_t per_split = blocks0 * (size_t)(1024 * t.bm * t.bn) * 4, fit = blocks0 <= (size_t)kMaxCounters ? space / per_split : 0;
-    // a split keeps at least 16 k tiles; none in the rotary form unless asked for (the partials weigh more than the idle CUs)
-    const int most = split_k > 0 || rope || a.KT < 32 || a.KT >= 256 ? 1 : a.KT / 16 < 8 ? a.KT / 16 : 8;
-    for (int c1 = k_from, n = 0; n < most; ++c1, ++n) {
+    for (int c1 = k_from; c1 <= k_to; ++c1) {
       int k1 = c1;
       if (k1 > 1 && (size_t)k1 > fit) {
         if (split_k > 1) {
@@ -745,7 +751,7 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
         }
         k1 = fit > 1 ? (int)fit : 1;
       }
-      const float c = pipe_cost(t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus);
+      const float c = pipe_cost(t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus, long_k);
       if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
     }
   }
