@@ -209,6 +209,16 @@ def test_every_w8a8_block_shape_exact_on_small_integers(tk, tile, k):
             assert torch.equal(tk.many_rows_gemm(x, pw, tile, sa=sac, split_k=split, resid=rc.float()).cpu(), full), (m, n, split)
 
 
+@pytest.mark.parametrize("m,k,n", [(1000, 48, 8196), (961, 1536, 8192), (960, 1536, 8192), (1000, 1552, 8192), (1025, 2048, 7940), (1024, 2048, 8192)])
+def test_w8a8_gemm_where_the_rules_change_kernels(tk, m, k, n):
+    # short K over a full generation of 64 x 256 blocks (512 on 256 CUs; 1536 columns, 2048 from 1025 rows on) and one step beside it
+    g = torch.Generator().manual_seed(m + k)
+    a, w = _integers(g, 2, m, k).cuda(), _integers(g, 1, n, k).cuda()
+    sa, sw = torch.exp2(_integers(g, 1, m)).cuda(), torch.exp2(_integers(g, 1, n)).cuda()
+    got = tk.w8a8_gemm(a.to(torch.float8_e4m3fn), sa, tk.pack_fp8_weight(w.to(torch.float8_e4m3fn), sw))
+    assert torch.equal(got, ((a @ w.t()) * sa[:, None] * sw[None, :]).to(BF16))
+
+
 @pytest.mark.parametrize("act", ["gelu_tanh", "silu"])
 @pytest.mark.parametrize("m,k,i", [(1, 16, 32), (65, 80, 96), (129, 720, 160), (193, 2064, 32), (257, 144, 544)])
 def test_every_w8a8_block_shape_gives_the_same_gated_bits(tk, m, k, i, act):

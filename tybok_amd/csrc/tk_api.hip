@@ -600,16 +600,23 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.kt_q = a.KT / ks;
   a.kt_r = a.KT % ks;
   a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
-  if (!tile && ks == 1 && blocks128 >= 2 * device_cus()) {
-    // rows a CU works through (blocks in a row on it x rows per block), per 256 columns: w8a8_wide_kernel where its 64-row blocks
-    // leave the fewest
+  if (!tile && ks == 1) {
+    // w8a8_wide_kernel, two blocks a CU, one's epilogue under the other's products: over a short K from one full generation on
+    // (us, against the best shape of fp8_pipe_kernel: 800 x 256 -> 32768 20.3 / 26.2, 1600 x 640 -> 16384 28.3 / 34.8, 800 x 1536
+    // -> 32768 52.3 / 58.5, 1600 x 2048 -> 16384 64.3 / 73.5; but 712 x 1792 -> 32768 67.2 / 59.8), otherwise where its 64-row
+    // blocks leave a CU the fewest rows (blocks in a row on it x rows per block, per 256 columns).
     auto share = [&](int rows, int cols) {
       const long long blocks = (long long)((M + rows - 1) / rows) * ((a.ntiles * 32 + cols - 1) / cols);
       return (blocks + device_cus() - 1) / device_cus() * rows * cols / 256;
     };
-    tile = 28;
-    for (const Fp8Tile& t : kW8a8Tiles)
-      if (share(32 * t.t.bm, 32 * t.t.bn) <= share(64, 256)) tile = 0;
+    const bool full = (long long)((M + 63) / 64) * ((a.ntiles * 32 + 255) / 256) >= 2 * device_cus();
+    if (full && (K <= 1536 || (K <= 2048 && M > 1024))) {
+      tile = 28;
+    } else if (blocks128 >= 2 * device_cus()) {
+      tile = 28;
+      for (const Fp8Tile& t : kW8a8Tiles)
+        if (share(32 * t.t.bm, 32 * t.t.bn) <= share(64, 256)) tile = 0;
+    }
   }
   const int rounds = ((a.KT + ks - 1) / ks + 3) / 4;
   if (tk_launch_w8a8_gemm(a, tile ? tile : pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, a.ntiles * 32, K, rounds, ks), st))
