@@ -94,24 +94,34 @@ struct PipeTile {
   int wt, ns;      // 32 x 32 tiles of a multiplying wave, buffers in the ring
   int occ;         // blocks of this shape that fit one CU (LDS)
 };
-// Estimated duration (us) of a launch; kb_n: KiB that a round brings of an n tile (of an m tile 4).  Fitted to 3400 timings
-// of the 16-bit form (64 shapes of the towers, the prefill and random ones, every tile, splits 1 .. 6; standard error
-// 14 %, the picked launch on average 1.1 % slower than the best one).  Blocks on one CU share its memory pipe (12 ns a KiB)
-// and matrix pipes (75 ns for a wave's tile and round); a round takes no less than the round trip over the rounds on
-// their way; the epilogue costs per tile; each further generation of blocks pays all of it again.
-// long_k: K > 8160, fitted to 12000 timings with cold weights (112 shapes of 64 .. 1500 rows, K 8192 .. 16384, 320 .. 4096
-// columns; the picked launch on average 2.7 % slower than the best one): the round trip sets the time of shallow rings, and a
-// split costs by its partials rather than by itself.
-float pipe_cost(const PipeTile& t, float kb_n, int M, int N, int rounds, int ks, int cus, bool long_k = false) {
+// Estimated duration (us) of a launch; kb_n: KiB that a round brings of an n tile (of an m tile 4).  Blocks on one CU share its
+// memory pipe and matrix pipes; a round takes no less than the round trip over the rounds on their way; the epilogue costs per
+// tile; each further generation of blocks pays all of it again; a split sends fp32 partials out and back in.
+struct PipeRates {
+  float launch, generation, round;  // us, whatever the shape
+  float x_kib, w_kib, tile, trip;   // us of a round: per KiB of x and of W, per 32 x 32 tile of a wave; a round trip
+  float epilogue;                   // us per 32 x 32 tile of the block
+  float split, split_tile;          // us of a split, and per tile of partials
+};
+// The 16-bit form up to K = 8160, fitted to 10000 timings with cold weights (338 shapes of 32 .. 4096 rows: the towers, the
+// prefill, a grid and random ones; every tile, splits 1 .. 8; the picked launch on average 1.4 % slower than the best one).
+// Rows of x cost more a KiB than weights, which lie in whole KiB: with one rate for both (3.6 % slower than the best) 1100 x
+// 768 -> 8192 took 28.2 us instead of 26.8, 300 x 2048 -> 4096 17.4 instead of 13.9, 712 x 2048 -> 2048 16.5 instead of 14.2.
+constexpr PipeRates kRates16 = {0.6f, 0.025f, 0.038f, 0.02f, 0.013f, 0.058f, 1.f, 0.115f, 2.4f, 0.0048f};
+// K above: 12000 timings (112 shapes of 64 .. 1500 rows, K 8192 .. 16384, 320 .. 4096 columns; 2.7 % slower than the best).
+constexpr PipeRates kRates16LongK = {1.66f, 0.014f, 0.f, 0.0122f, 0.0122f, 0.0751f, 0.66f, 0.203f, 2.5f, 0.004f};
+// Over fp8 weights (pick_tile).
+constexpr PipeRates kRatesFp8 = {1.66f, 0.014f, 0.f, 0.0122f, 0.0122f, 0.0751f, 0.585f, 0.203f, 4.76f, 0.00213f};
+float pipe_cost(const PipeRates& p, const PipeTile& t, float kb_n, int M, int N, int rounds, int ks, int cus) {
   const int rows = 32 * t.bm, cols = 32 * t.bn;
   const long long blocks = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * ks;
-  float us = 1.66f;
+  float us = p.launch;
   for (long long left = blocks; left > 0; left -= (long long)cus * t.occ) {
     const float r = left > cus && t.occ > 1 ? 2.f : 1.f;  // blocks on a CU
-    const float load = r * ((float)t.bm * 4.f + (float)t.bn * kb_n) * 0.0122f, mul = r * (float)t.wt * 0.0751f, trip = (long_k ? 0.66f : 0.585f) / (float)(t.ns - 1);
-    us += 0.014f + (float)rounds * (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip)) + r * (float)(t.bm * t.bn) * 0.203f;
+    const float load = r * ((float)t.bm * 4.f * p.x_kib + (float)t.bn * kb_n * p.w_kib), mul = r * (float)t.wt * p.tile, trip = p.trip / (float)(t.ns - 1);
+    us += p.generation + (float)rounds * (p.round + (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip))) + r * (float)(t.bm * t.bn) * p.epilogue;
   }
-  if (ks > 1) us += (long_k ? 2.5f : 4.76f) + (float)blocks * (float)(t.bm * t.bn) * (long_k ? 0.004f : 0.00213f);  // fp32 partials out and back in
+  if (ks > 1) us += p.split + (float)blocks * (float)(t.bm * t.bn) * p.split_tile;
   return us;
 }
 // The forms over fp8 weights.  Where the grid covers the device several times over, the time is the matrix pipes' at the
@@ -135,7 +145,7 @@ int pick_tile(const Fp8Tile (&tiles)[N], float kb_n, float flop_per_us, int M, i
     const PipeTile& t = f.t;
     const float rows = (float)((M + 32 * t.bm - 1) / (32 * t.bm) * 32 * t.bm), cols = (float)((ncols + 32 * t.bn - 1) / (32 * t.bn) * 32 * t.bn);
     const float power = f.power * 2.f * rows * cols * (float)K / flop_per_us;
-    float c = pipe_cost(t, kb_n, M, ncols, rounds, ks, device_cus()) * (0.8f + 0.2f * f.power);
+    float c = pipe_cost(kRatesFp8, t, kb_n, M, ncols, rounds, ks, device_cus()) * (0.8f + 0.2f * f.power);
     if (c < power) c = power;
     if (!best || c < best_cost) best = t.id, best_cost = c;
   }
@@ -758,7 +768,7 @@ int dense_common(const void* x, int ldx, const void* w_packed, const void* bias,
         }
         k1 = fit > 1 ? (int)fit : 1;
       }
-      const float c = pipe_cost(t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus, long_k);
+      const float c = pipe_cost(long_k ? kRates16LongK : kRates16, t, 4.f, M, N, ((a.KT + k1 - 1) / k1 + 1) / 2, k1, cus);
       if (!best || c < best_cost) best = &t, best_cost = c, ks = k1;
     }
   }
