@@ -100,26 +100,28 @@ struct PipeTile {
 struct PipeRates {
   float launch, generation, round;  // us, whatever the shape
   float x_kib, w_kib, tile, trip;   // us of a round: per KiB of x and of W, per 32 x 32 tile of a wave; a round trip
-  float epilogue;                   // us per 32 x 32 tile of the block
+  float epilogue, under;            // us per 32 x 32 tile of the block; the part of it that shows where blocks follow on a CU that
+                                    // holds two, one's epilogue under the other's products
   float split, split_tile;          // us of a split, and per tile of partials
 };
 // The 16-bit form up to K = 8160, fitted to 10000 timings with cold weights (338 shapes of 32 .. 4096 rows: the towers, the
 // prefill, a grid and random ones; every tile, splits 1 .. 8; the picked launch on average 1.4 % slower than the best one).
 // Rows of x cost more a KiB than weights, which lie in whole KiB: with one rate for both (3.6 % slower than the best) 1100 x
 // 768 -> 8192 took 28.2 us instead of 26.8, 300 x 2048 -> 4096 17.4 instead of 13.9, 712 x 2048 -> 2048 16.5 instead of 14.2.
-constexpr PipeRates kRates16 = {0.6f, 0.025f, 0.038f, 0.02f, 0.013f, 0.058f, 1.f, 0.115f, 2.4f, 0.0048f};
+constexpr PipeRates kRates16 = {0.6f, 0.025f, 0.038f, 0.02f, 0.013f, 0.058f, 1.f, 0.115f, 0.3f, 2.4f, 0.0048f};
 // K above: 12000 timings (112 shapes of 64 .. 1500 rows, K 8192 .. 16384, 320 .. 4096 columns; 2.7 % slower than the best).
-constexpr PipeRates kRates16LongK = {1.66f, 0.014f, 0.f, 0.0122f, 0.0122f, 0.0751f, 0.66f, 0.203f, 2.5f, 0.004f};
+constexpr PipeRates kRates16LongK = {1.66f, 0.014f, 0.f, 0.0122f, 0.0122f, 0.0751f, 0.66f, 0.203f, 1.f, 2.5f, 0.004f};
 // Over fp8 weights (pick_tile).
-constexpr PipeRates kRatesFp8 = {1.66f, 0.014f, 0.f, 0.0122f, 0.0122f, 0.0751f, 0.585f, 0.203f, 4.76f, 0.00213f};
+constexpr PipeRates kRatesFp8 = {1.66f, 0.014f, 0.f, 0.0122f, 0.0122f, 0.0751f, 0.585f, 0.203f, 1.f, 4.76f, 0.00213f};
 float pipe_cost(const PipeRates& p, const PipeTile& t, float kb_n, int M, int N, int rounds, int ks, int cus) {
   const int rows = 32 * t.bm, cols = 32 * t.bn;
   const long long blocks = (long long)((M + rows - 1) / rows) * ((N + cols - 1) / cols) * ks;
+  const float epilogue = (float)(t.bm * t.bn) * p.epilogue * (t.occ > 1 && blocks > (long long)cus * t.occ ? p.under : 1.f);
   float us = p.launch;
   for (long long left = blocks; left > 0; left -= (long long)cus * t.occ) {
     const float r = left > cus && t.occ > 1 ? 2.f : 1.f;  // blocks on a CU
     const float load = r * ((float)t.bm * 4.f * p.x_kib + (float)t.bn * kb_n * p.w_kib), mul = r * (float)t.wt * p.tile, trip = p.trip / (float)(t.ns - 1);
-    us += p.generation + (float)rounds * (p.round + (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip))) + r * (float)(t.bm * t.bn) * p.epilogue;
+    us += p.generation + (float)rounds * (p.round + (load > mul ? (load > trip ? load : trip) : (mul > trip ? mul : trip))) + r * epilogue;
   }
   if (ks > 1) us += p.split + (float)blocks * (float)(t.bm * t.bn) * p.split_tile;
   return us;
