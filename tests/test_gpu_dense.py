@@ -306,8 +306,8 @@ def test_rows_of_x_more_than_4_gib_of_lane_offset_apart(tk):
 
 @pytest.mark.parametrize("m,k,n,splits", [(64, 12288, 960, 12), (192, 12288, 960, 10), (256, 8192, 960, 8), (40, 8176, 96, None), (33, 8208, 96, 8)])
 def test_long_k_keeps_its_split_count(tk, m, k, n, splits):
-    # from 8192 columns on the number of splits (and with it the bits) follows from the shape alone: as many as fill a 256-CU
-    # device with 64 x 128 blocks, at least 32 k tiles each; below, the cost model's choice
+    # from 8161 columns on (256 k tiles) the least number of splits is what fills a 256-CU device with 64 x 128 blocks, at least 32
+    # k tiles each, and these shapes take it: the connector's bits hang on it
     x, w, b = _case(m, k, n, seed=9)
     pw = tk.pack_bf16_weight(w.cuda())
     got = tk.bf16w_dense(x.cuda(), pw, b.cuda())

@@ -14,9 +14,11 @@
 //     reads from memory (bias, residual, rotary positions and table rows) is asked for before the products: 1 - 2 us a
 //     launch against asking behind them (the weights and vectors of a layer are cold in every request).
 // Measured (cold weights, graph replay, us; before: weights straight into the registers of the four waves that multiply):
-// SmolVLA's tower at 3 x 1024 rows q|k|v 22 -> 17.2, out_proj 11.3 -> 9.0, fc1 23.8 -> 21.2, fc2 26.3 -> 19.5; pi0.5's
-// at 2 x 256 rows 14.9 -> 12.6, 9.9 -> 8.6, 13.3 -> 11.7, 20.4 -> 19.4; pi0.5's prefill at 712 rows q|k|v with the
-// rotary epilogue 24.4 -> 14.8, o_proj 14.0 -> 12.6.  A launch of this kind that does nothing takes 1.9 us; what bounds
+// SmolVLA's tower at 3 x 1024 rows q|k|v 21.4 -> 17.8, out_proj 14.4 -> 10.2, fc1 25.8 -> 22.1, fc2 29.0 -> 21.7; pi0.5's
+// at 2 x 256 rows 13.0 -> 12.4, 10.7 -> 9.4, 14.4 -> 12.7, 22.9 -> 20.8; pi0.5's prefill at 712 rows q|k|v with the
+// rotary epilogue 24.4 -> 14.8, o_proj 15.1 -> 13.3.  Slower than before: K below 600 with the weights already in the L2s (48 x
+// 256 -> 112 3.5 -> 4.2), and grids just over a generation of 128 x 128 blocks (1100 rows and 8192 columns, K 256 .. 1536: 8 - 18 %,
+// where the former kernel held three 96 x 128 blocks a CU).  A launch of this kind that does nothing takes 1.9 us; what bounds
 // them is a compute unit's 133 bytes/ns of loads (0.35 - 0.6 us a round), then the epilogue (0.2 us per 32 x 32 tile).
 #include "pipe_gemm.h"
 

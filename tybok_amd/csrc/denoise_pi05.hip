@@ -407,8 +407,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
 
     for (int l = 0; l < a.layers; ++l) {
       const int base = slot(l);
-      // the layer whose first weights and values are asked for in this one (behind the last one: dropped.  Asked for under a
-      // condition, their registers would be live through the whole layer)
+      // the layer whose first weights are asked for in this one (behind the last one: dropped.  Asked for under a condition,
+      // their registers would be live through the whole layer)
       const int nl = l + 1 < a.layers ? l + 1 : 0, nstep = nl || step + 1 == a.steps ? step : step + 1;
       const int in_base = l == 0 ? cur + OFF_HID : slot(l - 1) + OFF_X2;  // the layer's input rows
       i32x4 kf[8];  // this wave's 16 keys

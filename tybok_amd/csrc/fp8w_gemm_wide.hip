@@ -1,8 +1,8 @@
 // fp8-weight GEMM for many rows (the VLM prefill) on gfx950: the weight-only form of pipe_fp8.h, a kernel of its own for the
 // largest grids, and the row norm in front of them.
 // Measured (us, cold weights, graph replay; before: weights straight into the registers of four multiplying waves): the
-// gated block 2048 -> 16384 -> 2048 at 288 / 330 / 555 / 712 / 968 rows 104 -> 79, 102 -> 87, 135 -> 132, 156 -> 151, 190 ->
-// 186; 960 -> 2560 -> 960 at 305 / 600 rows 39 -> 22, 41 -> 28.
+// gated block 2048 -> 16384 -> 2048 at 288 / 320 / 555 / 712 / 968 rows 94 -> 78, 100 -> 87, 132 -> 129, 153 -> 149, 189 ->
+// 187; 960 -> 2560 -> 960 at 305 / 600 rows 41 -> 24, 42 -> 29.
 #include <atomic>
 
 #include "pipe_fp8.h"
@@ -17,9 +17,9 @@ constexpr int NW = 4;              // waves per block
 constexpr int RK = 2;              // k tiles per round
 
 // Grids that cover the device twice over (from 385 rows of the gated 2048 -> 2 x 16384 launch): there the power of the
-// operands' way decides the matrix pipes' clock, and the two kernels below, whose weights go through registers, are the cheaper
-// ones.  This one where 64-row blocks waste the least: 555 rows 81 us against 83 - 88 of pipe_fp8.h's kernel, 650 rows 94 - 99
-// against 100 - 102.
+// operands' way decides the matrix pipes' clock, and the two kernels below, whose weights go through registers, are about level
+// with pipe_fp8.h's.  This one where 64-row blocks waste the least: 555 / 640 / 800 rows 79 / 83 / 110 us against 77 / 79 / 106
+// of its 128 x 128 blocks, all shapes timed in turn on one card; on another 555 rows 81 against 83 - 88.
 // A block of four waves owns 64 rows x 256 packed columns, two blocks a CU (they cover each other's first loads and
 // epilogue); wave w owns n tiles 2w, 2w + 1 for all rows, its weights straight from memory into its registers; a round's
 // activations are staged once per block through LDS.  EPI: 0 plain, 1 gated.  PF: rounds in flight (even: round r uses LDS
@@ -216,8 +216,8 @@ __global__ __launch_bounds__(NW * 64, OCC) void fp8w_wide_kernel(GemmArgs a, int
 
 // The same where taller blocks waste no more rows: eight waves own 2*WM*32 rows x 256 packed columns, with both operands of a
 // round staged through registers and LDS: wave (wm, wn) = (wave / 4, wave % 4) owns rows wm*WM*32 .. of the block and the n
-// tile pair wn; a weight tile is fetched and converted to bf16 once per block (712 rows 95 - 98 us against 95 - 104 of
-// pipe_fp8.h's kernel, 968 rows 120 - 125 against 125 - 131).  A round is four k steps of
+// tile pair wn; a weight tile is fetched and converted to bf16 once per block (512 / 712 / 968 rows 61 / 93 / 118 us against 64 /
+// 93 / 122 of the best shape of pipe_fp8.h's kernel).  A round is four k steps of
 // 16; operand registers of step s + 1 are read while step s multiplies; one barrier per round, before its last step:
 // by then every wave has read the round's operands out of buffer b and written its share of round r + 1 into b ^ 1.
 //   staging per thread and round: WM 16-byte pieces of x, 2 pieces of 16 fp8 weights (wave (wm, wn): k tile wm of

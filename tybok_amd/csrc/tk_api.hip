@@ -283,10 +283,10 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
       a.norm_w = nullptr;
       a.ada_scale = a.ada_shift = nullptr;
     }
-    // K split, from the shape alone (it decides the order of summation).  Few column blocks over a long K (the down
-    // projection): a cost fitted to M = 296 .. 968 at K = 16384, N = 2048 -- the k loop of the blocks that share a CU (0.1 us
-    // per 1000 row x k products), the partials' trip through memory (0.5 us per MB), the weights pulled once per row block
-    // (0.005 us per MB) and 8 us that a grid of lone 64-row blocks loses to 128-row ones
+    // K split: from the shape, the CU count and the workspace, not from the block shape picked below (it decides the order of
+    // summation).  Few column blocks over a long K (the down projection): a cost fitted to M = 296 .. 968 at K = 16384, N = 2048
+    // on kernels of 64 and 128 x 256 blocks that are gone; kept for its bits.  Its terms: the k loop of the blocks that
+    // share a CU, the partials' trip through memory, the weights pulled once per row block and 8 us that 64-row blocks lost.
     const int nbn = (a.ntiles * 32 + kWideCols - 1) / kWideCols;
     int ks = split_k, rows = 128;
     if (ks <= 0 && wide_blocks < 2 * cus && !a.s1 && a.N % 4 == 0 && ws && a.KT >= 32) {
@@ -298,7 +298,7 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
           const double loop = 1e-4 * gens * (mt * 32) * ((double)K / sp);
           const double part = sp > 1 ? 0.5e-6 * 4.0 * sp * nbm * (mt * 32) * nbn * kWideCols : 0.0;
           const double cost = loop + part + (mt == 2 ? 8.0 : 0.0) + 0.005e-6 * nbm * (double)K * nbn * kWideCols;
-          if (cost < best) best = cost, rows = mt * 32, ks = sp;
+          if (cost < best) best = cost, ks = sp;
         }
     }
     if (ks <= 0) {
@@ -589,7 +589,8 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.act = act;
   a.vec = 1;
   a.vec16 = ldy % 8 == 0 && aligned16(y) && (!resid || (aligned16(resid) && ldr % (resid_dtype == TK_F32 ? 4 : 8) == 0));
-  // K split, from the shape alone (it decides the order of summation)
+  // K split: from the shape, the CU count and the workspace, not from the block shape picked below (it decides the order of
+  // summation); the 64 and 128 x 256 blocks that it counts are gone
   const int blocks128 = ((a.ntiles * 32 + kWideCols - 1) / kWideCols) * ((M + 127) / 128);
   const int rows = blocks128 >= 2 * device_cus() ? 64 : 128;
   int ks = split_k;

@@ -121,11 +121,13 @@ __device__ __forceinline__ float gelu_tanh_f(float x) {
   const float inner = c0 * (x + 0.044715f * x * x * x);
   return x / (1.0f + __expf(-2.0f * inner));
 }
-// The same with -2z log2(e) as x (a + b x^2) and v_rcp_f32 in place of the division's ten instructions, for epilogues that
-// evaluate it for every output of a one-generation grid while the matrix pipes wait (the 555-row W8A8 block 109.3 -> 107.9 us,
-// a three-camera SmolVLA request 5.08 -> 5.05 ms; pi0.5's weight-only prefill and denoising loop gain nothing and keep the
-// division).  Against 64 bits over [-12, 12]: largest relative error 8.8e-6 (1.5e-5 above: fewer roundings in the
-// exponent), mean 5.6e-8 (6.0e-8).
+// The same with -2z log2(e) as x (a + b x^2) and v_rcp_f32 in place of the division's ten instructions: the 16-bit linears and
+// the W8A8 block (555 rows 109.3 -> 107.9 us; a three-camera SmolVLA request 5.08 -> 5.05 ms).  Rounded to bf16 both give the
+// same for every bf16 argument; of all fp16 arguments 4 (5 above) miss the fp16 value nearest to the exact one, of 8.4 million
+// fp32 arguments 4535 (4553 above) the nearest bf16 value; mean relative error over N(0, 1) before that rounding 4.8e-8 - 9e-8
+// (4.7e-8 above).  pi0.5's weight-only prefill and denoising loop gain nothing from it and keep the division, and with it
+// the chunks they had: with the other flips of a rounding one test's chunk came to 1.03e-2 of the reference arithmetic's,
+// bound 1e-2.
 __device__ __forceinline__ float gelu_tanh_rcp_f(float x) {
   constexpr float a = -2.302208198144325f;    // -2 sqrt(2/pi) log2(e)
   constexpr float b = -0.10294323958002849f;  // 0.044715 a

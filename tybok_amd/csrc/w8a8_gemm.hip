@@ -8,7 +8,7 @@
 //                           same permutation for both operands (bytes 0-15 of a lane: k tile 2s, bytes 16-31: k tile
 //                           2s+1), which a dot product does not see.  Measured (us, before: weights straight into the
 //                           registers of four multiplying waves): the whole block 2048 -> 16384 -> 2048, quantisations
-//                           included, at 256 / 288 / 555 / 712 / 968 rows 67 -> 62, 84 -> 77, 109 -> 103, 126 -> 117, 152 -> 144.
+//                           included, at 256 / 288 / 555 / 712 / 968 rows 63 -> 60, 82 -> 71, 105 -> 96, 124 -> 110, 151 -> 135.
 #include "pipe_fp8.h"
 
 namespace {
