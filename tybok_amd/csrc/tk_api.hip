@@ -617,7 +617,8 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
     // w8a8_wide_kernel, two blocks a CU, one's epilogue under the other's products: over a short K from one full generation on
     // (us, against the best shape of fp8_pipe_kernel: 800 x 256 -> 32768 20.3 / 26.2, 1600 x 640 -> 16384 28.3 / 34.8, 800 x 1536
     // -> 32768 52.3 / 58.5, 1600 x 2048 -> 16384 64.3 / 73.5; but 712 x 1792 -> 32768 67.2 / 59.8), otherwise where its 64-row
-    // blocks leave a CU the fewest rows (blocks in a row on it x rows per block, per 256 columns).
+    // blocks leave a CU the fewest rows (blocks in a row on it x rows per block, per 256 columns, by the shape's time per product:
+    // 128 x 128 blocks leave as few at 577 .. 640 and 769 .. 896 rows of the gated 2048 -> 2 x 16384 launch and are slower).
     auto share = [&](int rows, int cols) {
       const long long blocks = (long long)((M + rows - 1) / rows) * ((a.ntiles * 32 + cols - 1) / cols);
       return (blocks + device_cus() - 1) / device_cus() * rows * cols / 256;
@@ -628,7 +629,7 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
     } else if (blocks128 >= 2 * device_cus()) {
       tile = 28;
       for (const Fp8Tile& t : kW8a8Tiles)
-        if (share(32 * t.t.bm, 32 * t.t.bn) <= share(64, 256)) tile = 0;
+        if ((float)share(32 * t.t.bm, 32 * t.t.bn) * t.power <= (float)share(64, 256)) tile = 0;
     }
   }
   const int rounds = ((a.KT + ks - 1) / ks + 3) / 4;
