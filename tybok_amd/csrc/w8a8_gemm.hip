@@ -18,9 +18,10 @@ namespace {
 // `(x / s).to(float8_e4m3fn)` (quotient rounded to bf16, then to fp8): sa = float(bf16(amax / 448)).
 // Bound: memory (a 555 x 16384 row block is 18 MB in, 9 MB out) once the loads of a row are all on their way together (NP of
 // them a thread, none under a branch: at the join behind one each would be waited for) and a quotient costs four
-// instructions: 555 rows of 2048 / 16384 columns 3.8 -> 2.8 / 9.4 -> 8.3 us, 811 of 16384 12.7 -> 10.5.
+// instructions (bf16 mode, one division a value before): 555 rows of 2048 / 16384 columns 4.4 -> 3.3 / 10.3 -> 7.1 us, 968 of 16384
+// 14.6 -> 10.4.
 constexpr int kQuantMaxPieces = 8;  // 16-byte pieces of a row per thread: K <= 8 * 256 * 8 = 16384
-template <int NP>
+template <int NP, bool BF16_MODE>
 __global__ __launch_bounds__(256) void quant_act_rows_kernel(QuantActArgs a) {
   __shared__ float part[4];
   const int tid = threadIdx.x;
@@ -46,39 +47,42 @@ __global__ __launch_bounds__(256) void quant_act_rows_kernel(QuantActArgs a) {
   __syncthreads();
   amax = fmaxf(fmaxf(part[0], part[1]), fmaxf(part[2], part[3]));
   float sa = amax / 448.0f;
-  if (a.mode == 1) sa = round_bf16(sa);
+  if (BF16_MODE) sa = round_bf16(sa);
   if (tid == 0) a.sa[blockIdx.x] = sa;
   // The IEEE quotient, as the elementwise reference computes it, from the correctly rounded reciprocal: one product and one
   // correction by the exact remainder are again correctly rounded (Markstein).  The sign is the numerator's (the remainder
   // of -0 is +0).  Scales whose reciprocal or remainders would leave the range of normal numbers take the division.
   const float inv = 1.0f / sa;
-  const bool plain = sa >= 0x1p-80f && sa <= 0x1p+80f;
-  auto quotient = [&](float x) {
-    if (sa == 0.f) return 0.f;
-    if (!plain) return x / sa;
-    const float y = x * inv;
-    return __builtin_copysignf(fmaf(fmaf(-sa, y, x), inv, y), x);
-  };
   unsigned char* dst = (unsigned char*)a.a8 + (size_t)blockIdx.x * a.lda;
+  auto codes = [&](auto quotient) {
 #pragma unroll
-  for (int i = 0; i < NP; ++i) {
-    const int p = tid + i * 256;
-    if (p >= pieces) continue;
-    float q[8];
+    for (int i = 0; i < NP; ++i) {
+      const int p = tid + i * 256;
+      if (p >= pieces) continue;
+      float q[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const unsigned u = (unsigned)v[i][e >> 1];
-      q[e] = quotient(__uint_as_float((e & 1) ? (u & 0xffff0000u) : (u << 16)));
-      if (a.mode == 1) q[e] = round_bf16(q[e]);
+      for (int e = 0; e < 8; ++e) {
+        const unsigned u = (unsigned)v[i][e >> 1];
+        q[e] = quotient(__uint_as_float((e & 1) ? (u & 0xffff0000u) : (u << 16)));
+        if (BF16_MODE) q[e] = round_bf16(q[e]);
+      }
+      // four fp32 -> four e4m3fn (RNE, saturating at +-448) per conversion pair
+      int lo = 0, hi = 0;
+      lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], lo, false);
+      lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
+      hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], hi, false);
+      hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], hi, true);
+      *(i32x2*)(dst + (size_t)p * 8) = i32x2{lo, hi};
     }
-    // four fp32 -> four e4m3fn (RNE, saturating at +-448) per conversion pair
-    int lo = 0, hi = 0;
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], lo, false);
-    lo = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], lo, true);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[4], q[5], hi, false);
-    hi = __builtin_amdgcn_cvt_pk_fp8_f32(q[6], q[7], hi, true);
-    *(i32x2*)(dst + (size_t)p * 8) = i32x2{lo, hi};
-  }
+  };
+  // the row's choice in front of the loop: inside, every element carries both branches (1 x 15776, bf16 mode, 6.2 us instead of 3.8)
+  if (sa >= 0x1p-80f && sa <= 0x1p+80f)
+    codes([&](float x) {
+      const float y = x * inv;
+      return __builtin_copysignf(fmaf(fmaf(-sa, y, x), inv, y), x);
+    });
+  else
+    codes([&](float x) { return sa == 0.f ? 0.f : x / sa; });
 }
 
 // Rows whose share of a compute unit comes out smallest in 64-row blocks, two a CU (577 .. 640, 769 .. 896 rows of the gated
@@ -257,12 +261,18 @@ int tk_launch_w8a8_gemm(const GemmArgs& a, int tile, hipStream_t st) {
   return -1;
 }
 
+template <bool BF16_MODE>
+static void launch_quant(int np, dim3 grid, dim3 block, const QuantActArgs& a, hipStream_t st) {
+  if (np <= 1) hipLaunchKernelGGL((quant_act_rows_kernel<1, BF16_MODE>), grid, block, 0, st, a);
+  else if (np <= 2) hipLaunchKernelGGL((quant_act_rows_kernel<2, BF16_MODE>), grid, block, 0, st, a);
+  else if (np <= 4) hipLaunchKernelGGL((quant_act_rows_kernel<4, BF16_MODE>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((quant_act_rows_kernel<kQuantMaxPieces, BF16_MODE>), grid, block, 0, st, a);
+}
+
 int tk_launch_quant_act_rows(QuantActArgs a, hipStream_t st) {
   const int np = (a.K / 8 + 255) / 256;
   const dim3 grid(a.M), block(256);
-  if (np <= 1) hipLaunchKernelGGL(quant_act_rows_kernel<1>, grid, block, 0, st, a);
-  else if (np <= 2) hipLaunchKernelGGL(quant_act_rows_kernel<2>, grid, block, 0, st, a);
-  else if (np <= 4) hipLaunchKernelGGL(quant_act_rows_kernel<4>, grid, block, 0, st, a);
-  else hipLaunchKernelGGL(quant_act_rows_kernel<kQuantMaxPieces>, grid, block, 0, st, a);
+  if (a.mode == 1) launch_quant<true>(np, grid, block, a, st);
+  else launch_quant<false>(np, grid, block, a, st);
   return hipGetLastError() == hipSuccess ? 0 : -3;
 }
