@@ -671,6 +671,10 @@ int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* 
                             int ldy, const void* resid, int ldr, int resid_dtype, const void* gate, int M, int N, int K, int split_k,
                             int act, int tile, void* ws, size_t ws_bytes, void* stream);
 
+/* The block shape (a tile of tk_debug_many_rows_gemm) that a W8A8 launch with that many K splits takes on the current device (256
+ * CUs where there is none); gated: N is the intermediate's width.  For tests of the rule.  No counterpart in the reference. */
+int tk_debug_w8a8_tile(int M, int N, int K, int gated, int split_k);
+
 #ifdef __cplusplus
 }
 #endif

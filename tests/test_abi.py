@@ -49,6 +49,21 @@ def test_host_only_entry_points():
     assert b"bad argument" in lib.tk_last_error()
 
 
+@pytest.mark.parametrize("m,n,k,gated,tile", [
+    # gate/up of the largest prefill: 64-row blocks at 577 .. 640 and 769 .. 896 rows, where they leave a CU the fewest rows
+    (512, 16384, 2048, 1, 408), (555, 16384, 2048, 1, 604), (577, 16384, 2048, 1, 28), (608, 16384, 2048, 1, 28), (640, 16384, 2048, 1, 28), (641, 16384, 2048, 1, 408),
+    (768, 16384, 2048, 1, 408), (769, 16384, 2048, 1, 28), (800, 16384, 2048, 1, 28), (896, 16384, 2048, 1, 28), (968, 16384, 2048, 1, 408),
+    # short K: from a full generation of 64 x 256 blocks on
+    (960, 8192, 1536, 0, 408), (961, 8192, 1536, 0, 28), (800, 32768, 256, 0, 28), (1600, 16384, 2048, 0, 28), (712, 32768, 1792, 0, 408), (300, 2560, 960, 0, 204),
+])  # fmt: skip
+def test_w8a8_block_shapes_by_the_sizes(m, n, k, gated, tile):
+    from tybok_amd import native
+
+    if not os.path.exists(native.library_path()):
+        pytest.skip("libtybok_hip.so not built")
+    assert native.lib().tk_debug_w8a8_tile(m, n, k, gated, 1) == tile
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from tybok_amd import native
 

@@ -556,6 +556,27 @@ int tk_fp8w_gated_ffn(const void* x, int ldx, const void* wgu_packed, const void
 
 // ---- W8A8 tier ---------------------------------------------------------------------------------
 namespace {
+// Block shape of a W8A8 launch; ncols: packed columns, ks: K splits.
+int w8a8_tile(int M, int ncols, int K, int ks) {
+  const int cus = device_cus(), KT = (K + 31) / 32;
+  if (ks == 1) {
+    // 28: w8a8_wide_kernel, two blocks a CU, one's epilogue under the other's products: over a short K from one full generation on
+    // (us, against the best shape of fp8_pipe_kernel: 800 x 256 -> 32768 20.3 / 26.2, 1600 x 640 -> 16384 28.3 / 34.8, 800 x 1536
+    // -> 32768 52.3 / 58.5, 1600 x 2048 -> 16384 64.3 / 73.5; but 712 x 1792 -> 32768 67.2 / 59.8), otherwise where its 64-row
+    // blocks leave a CU the fewest rows (blocks in a row on it x rows per block, per 256 columns, by the shape's time per product:
+    // 128 x 128 blocks leave as few at 577 .. 640 and 769 .. 896 rows of the gated 2048 -> 2 x 16384 launch and are slower).
+    auto blocks = [&](int rows, int cols) { return (long long)((M + rows - 1) / rows) * ((ncols + cols - 1) / cols); };
+    auto share = [&](int rows, int cols) { return (float)((blocks(rows, cols) + cus - 1) / cus * rows * cols / 256); };
+    if (blocks(64, 256) >= 2 * cus && (K <= 1536 || (K <= 2048 && M > 1024))) return 28;
+    if (blocks(128, kWideCols) >= 2 * cus) {
+      bool fewest = true;
+      for (const Fp8Tile& t : kW8a8Tiles) fewest &= share(32 * t.t.bm, 32 * t.t.bn) * t.power > share(64, 256);
+      if (fewest) return 28;
+    }
+  }
+  return pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, ncols, K, ((KT + ks - 1) / ks + 3) / 4, ks);
+}
+
 int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, const float* s0, const float* s1, void* y, int ldy,
                 const void* resid, int ldr, int resid_dtype, int M, int N, int K, int split_k, int act, void* ws, size_t ws_bytes,
                 hipStream_t st, int tile = 0) {
@@ -613,27 +634,7 @@ int w8a8_common(const void* a8, int lda, const float* sa, const void* w_packed, 
   a.kt_q = a.KT / ks;
   a.kt_r = a.KT % ks;
   a.partial = ks > 1 ? (float*)((char*)ws + kPartialOff) : nullptr;
-  if (!tile && ks == 1) {
-    // w8a8_wide_kernel, two blocks a CU, one's epilogue under the other's products: over a short K from one full generation on
-    // (us, against the best shape of fp8_pipe_kernel: 800 x 256 -> 32768 20.3 / 26.2, 1600 x 640 -> 16384 28.3 / 34.8, 800 x 1536
-    // -> 32768 52.3 / 58.5, 1600 x 2048 -> 16384 64.3 / 73.5; but 712 x 1792 -> 32768 67.2 / 59.8), otherwise where its 64-row
-    // blocks leave a CU the fewest rows (blocks in a row on it x rows per block, per 256 columns, by the shape's time per product:
-    // 128 x 128 blocks leave as few at 577 .. 640 and 769 .. 896 rows of the gated 2048 -> 2 x 16384 launch and are slower).
-    auto share = [&](int rows, int cols) {
-      const long long blocks = (long long)((M + rows - 1) / rows) * ((a.ntiles * 32 + cols - 1) / cols);
-      return (blocks + device_cus() - 1) / device_cus() * rows * cols / 256;
-    };
-    const bool full = (long long)((M + 63) / 64) * ((a.ntiles * 32 + 255) / 256) >= 2 * device_cus();
-    if (full && (K <= 1536 || (K <= 2048 && M > 1024))) {
-      tile = 28;
-    } else if (blocks128 >= 2 * device_cus()) {
-      tile = 28;
-      for (const Fp8Tile& t : kW8a8Tiles)
-        if ((float)share(32 * t.t.bm, 32 * t.t.bn) * t.power <= (float)share(64, 256)) tile = 0;
-    }
-  }
-  const int rounds = ((a.KT + ks - 1) / ks + 3) / 4;
-  if (tk_launch_w8a8_gemm(a, tile ? tile : pick_tile(kW8a8Tiles, 4.f, 1.8e9f, M, a.ntiles * 32, K, rounds, ks), st))
+  if (tk_launch_w8a8_gemm(a, tile ? tile : w8a8_tile(M, a.ntiles * 32, K, ks), st))
     return fail(TK_ELAUNCH, "w8a8: launch failed (%s)", hipGetErrorString(hipGetLastError()));
   return TK_OK;
 }
@@ -1693,6 +1694,11 @@ int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* 
   e.tile = tile;
   return gemm_common(x, ldx, w_packed, (const float*)s0, (const float*)s1, y, ldy, resid, ldr, resid_dtype, gate, M, N, K, split_k, act,
                      ws, ws_bytes, (hipStream_t)stream, e);
+}
+
+int tk_debug_w8a8_tile(int M, int N, int K, int gated, int split_k) {
+  if (M <= 0 || N <= 0 || K <= 0 || split_k <= 0) return fail(TK_EINVAL, "w8a8_tile: non-positive argument");
+  return w8a8_tile(M, (N + 31) / 32 * 32 * (gated ? 2 : 1), K, split_k);
 }
 
 int tk_debug_decode_fp8(void* out_f32, void* stream) {
