@@ -8,11 +8,14 @@ of exiting too: tybok/policies/fastwam/kernels/coop_grid.h:20-27).
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from ctypes import c_char_p, c_float, c_int, c_longlong, c_size_t, c_void_p
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libtybok_hip.so")
 _lib: ctypes.CDLL | None = None
+_calls = None
 
 # name -> (restype, argtypes); mirrors include/tybok_hip.h one to one
 SIGNATURES: dict[str, tuple] = {
@@ -246,3 +249,21 @@ def check(rc: int, what: str) -> None:
     if rc != 0:
         msg = lib().tk_last_error()
         raise RuntimeError(f"{what} failed ({rc}): {msg.decode() if msg else 'unknown error'}")
+
+
+def calls():
+    """The extension module of the launching entry points (``csrc/tk_calls.cpp``): ``calls().tk_name(...)`` takes tensors for
+    pointers, launches on torch's current stream (the entry's last argument, not passed) and raises like :func:`check`."""
+    global _calls
+    if _calls is None:
+        import torch  # noqa: F401  (its libraries have to be in the process)
+
+        lib()
+        path = os.path.join(os.path.dirname(_LIB_PATH), "tk_calls.so")
+        if not os.path.exists(path):
+            raise RuntimeError(f"{path} is missing: build it with `python -m tybok_amd.csrc.build`")
+        loader = importlib.machinery.ExtensionFileLoader("tk_calls", path)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("tk_calls", path, loader=loader))
+        loader.exec_module(module)
+        _calls = module
+    return _calls

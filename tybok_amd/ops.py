@@ -25,6 +25,19 @@ def _stream() -> int:
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
+_bound = None
+
+
+def _calls():
+    """The launching entry points on tensors (:func:`native.calls`); they find the workspace of a call that names none here."""
+    global _bound
+    if _bound is None:
+        module = native.calls()
+        module.set_workspaces(_default_ws, default_workspace)
+        _bound = module
+    return _bound
+
+
 def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
@@ -194,18 +207,7 @@ def fp8w_gemm(
     ws: Workspace | None = None,
 ) -> torch.Tensor:
     """``bf16((x @ W8^T) * scale)`` (``* gate[n]``, ``+ residual``) for ``x [M, K]`` bf16."""
-    lib = native.lib()
-    m, ldx = _check_act(x, w.k)
-    if out is None:
-        out = torch.empty(m, w.n, dtype=torch.bfloat16, device=x.device)
-    rp, ldr, rdt = _resid_args(resid, m, w.n)
-    ws = ws or default_workspace(x.device)
-    rc = lib.tk_fp8w_gemm(
-        x.data_ptr(), ldx, w.data.data_ptr(), w.scale.data_ptr(), out.data_ptr(), out.stride(0), rp, ldr, rdt,
-        _gate_ptr(gate, w.n), m, w.n, w.k, split_k, ws.ptr, ws.nbytes, _stream(),
-    )  # fmt: skip
-    native.check(rc, "tk_fp8w_gemm")
-    return out
+    return _calls().fp8w_gemm(x, w.data, w.scale, w.n, w.k, resid, gate, out, split_k, ws)
 
 
 def fp8w_gated_ffn(
@@ -225,29 +227,9 @@ def fp8w_gated_ffn(
     """``down(act(gate(x)) * up(x))`` (``* gate[n]``, ``+ residual``) for ``x [M, K]`` bf16;
     with ``norm_w`` (RMSNorm) or ``ada = (scale, shift)`` (adaptive RMSNorm) the input is first
     normalised inside the gate/up launch."""
-    lib = native.lib()
-    m, ldx = _check_act(x, wgu.k)
-    if wd.k != wgu.i or wd.n != wgu.k:
-        raise ValueError("down weight must be [K, I]")
-    if out is None:
-        out = torch.empty(m, wd.n, dtype=torch.bfloat16, device=x.device)
-    rp, ldr, rdt = _resid_args(resid, m, wd.n)
-    ws = ws or default_workspace(x.device)
-    if norm_w is not None or ada is not None:
-        rc = lib.tk_fp8w_norm_gated_ffn(
-            x.data_ptr(), ldx, _norm_ptr(norm_w, wgu.k), float(eps), *_ada_ptrs(ada, wgu.k), wgu.data.data_ptr(), wgu.scale_gate.data_ptr(),
-            wgu.scale_up.data_ptr(), wd.data.data_ptr(), wd.scale.data_ptr(), out.data_ptr(), out.stride(0), rp, ldr, rdt,
-            _gate_ptr(gate, wd.n), m, wgu.k, wgu.i, ACT[act], ws.ptr, ws.nbytes, _stream(),
-        )  # fmt: skip
-        native.check(rc, "tk_fp8w_norm_gated_ffn")
-        return out
-    rc = lib.tk_fp8w_gated_ffn(
-        x.data_ptr(), ldx, wgu.data.data_ptr(), wgu.scale_gate.data_ptr(), wgu.scale_up.data_ptr(),
-        wd.data.data_ptr(), wd.scale.data_ptr(), out.data_ptr(), out.stride(0), rp, ldr, rdt,
-        _gate_ptr(gate, wd.n), m, wgu.k, wgu.i, ACT[act], ws.ptr, ws.nbytes, _stream(),
+    return _calls().fp8w_gated_ffn(
+        x, wgu.data, wgu.scale_gate, wgu.scale_up, wgu.i, wgu.k, wd.data, wd.scale, wd.n, wd.k, ACT[act], resid, gate, norm_w, eps, ada, out, ws,
     )  # fmt: skip
-    native.check(rc, "tk_fp8w_gated_ffn")
-    return out
 
 
 def set_ffn_fusion(on: bool) -> bool:
@@ -263,13 +245,12 @@ def set_handoff_spin(polls: int) -> int:
 
 def quant_act_rows(x: torch.Tensor, mode: int = 0) -> tuple[torch.Tensor, torch.Tensor]:
     """Per-token e4m3fn quantisation of ``x [M, K]`` bf16 -> ``(a8 [M, K] float8_e4m3fn, sa [M] fp32)``."""
-    lib = native.lib()
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.stride(1) != 1:
         raise TypeError("activations must be a bf16 CUDA matrix with unit inner stride")
     m, k = x.shape
     a8 = torch.empty(m, k, dtype=torch.uint8, device=x.device)
     sa = torch.empty(m, dtype=torch.float32, device=x.device)
-    native.check(lib.tk_quant_act_rows(x.data_ptr(), x.stride(0), a8.data_ptr(), k, sa.data_ptr(), m, k, int(mode), _stream()), "tk_quant_act_rows")
+    _calls().tk_quant_act_rows(x, x.stride(0), a8, k, sa, m, k, int(mode))
     return a8.view(torch.float8_e4m3fn), sa
 
 
@@ -278,7 +259,6 @@ def w8a8_gemm(
     split_k: int = 0, ws: Workspace | None = None,
 ) -> torch.Tensor:  # fmt: skip
     """``bf16((a8 @ W8^T) * sa[m] * sw[n])`` (``+ residual``) on the fp8 matrix instruction."""
-    lib = native.lib()
     if a8.dtype == torch.float8_e4m3fn:
         a8 = a8.view(torch.uint8)
     if a8.dtype != torch.uint8 or a8.dim() != 2 or a8.shape[1] != w.k or a8.stride(1) != 1:
@@ -290,11 +270,10 @@ def w8a8_gemm(
         out = torch.empty(m, w.n, dtype=torch.bfloat16, device=a8.device)
     rp, ldr, rdt = _resid_args(resid, m, w.n)
     ws = ws or default_workspace(a8.device)
-    rc = lib.tk_w8a8_gemm(
-        a8.data_ptr(), a8.stride(0), sa.data_ptr(), w.data.data_ptr(), w.scale.data_ptr(), out.data_ptr(), out.stride(0), rp, ldr, rdt,
-        m, w.n, w.k, split_k, ws.ptr, ws.nbytes, _stream(),
+    _calls().tk_w8a8_gemm(
+        a8, a8.stride(0), sa, w.data, w.scale, out, out.stride(0), rp, ldr, rdt,
+        m, w.n, w.k, split_k, ws.buf, ws.nbytes,
     )  # fmt: skip
-    native.check(rc, "tk_w8a8_gemm")
     return out
 
 
@@ -307,20 +286,18 @@ def w8a8_gated_ffn(
     tybok/policies/pi05/models/triton_prefill_mlp.py:26-59), ``"fp32"`` = one rounding."""
     if mode not in ("fp32", "bf16"):
         raise ValueError(f"unknown quantisation mode {mode!r}")
-    lib = native.lib()
     m, ldx = _check_act(x, wgu.k)
     if wd.k != wgu.i or wd.n != wgu.k:
         raise ValueError("down weight must be [K, I]")
     if out is None:
-        out = torch.empty(m, wd.n, dtype=torch.bfloat16, device=x.device)
+        out = _calls().empty_bf16(x, m, wd.n)
     rp, ldr, rdt = _resid_args(resid, m, wd.n)
     ws = ws or default_workspace(x.device)
-    rc = lib.tk_w8a8_gated_ffn(
-        x.data_ptr(), ldx, wgu.data.data_ptr(), wgu.scale_gate.data_ptr(), wgu.scale_up.data_ptr(), wd.data.data_ptr(),
-        wd.scale.data_ptr(), out.data_ptr(), out.stride(0), rp, ldr, rdt, m, wgu.k, wgu.i, ACT[act], 1 if mode == "bf16" else 0,
-        ws.ptr, ws.nbytes, _stream(),
+    _calls().tk_w8a8_gated_ffn(
+        x, ldx, wgu.data, wgu.scale_gate, wgu.scale_up, wd.data,
+        wd.scale, out, out.stride(0), rp, ldr, rdt, m, wgu.k, wgu.i, ACT[act], 1 if mode == "bf16" else 0,
+        ws.buf, ws.nbytes,
     )  # fmt: skip
-    native.check(rc, "tk_w8a8_gated_ffn")
     return out
 
 
@@ -376,7 +353,6 @@ def bf16w_dense(
     linear output (what ``gelu(linear(x))`` on bf16 tensors computes), ``"gelu_tanh_fp32"`` to the fp32 one (a GEMM
     with the activation in its epilogue).  ``tile`` picks the block tile (0 = by shape).  With fp16 activations and
     a weight packed from an fp16 matrix every 16-bit operand is fp16 (``tk_f16w_dense``: pi0.5's fp16 tower tiers)."""
-    lib = native.lib()
     if w.rope_half:
         raise ValueError("bf16w_dense takes weights packed in natural tile order (rope_half = 0)")
     dt = w.dtype
@@ -406,18 +382,13 @@ def bf16w_dense(
         nb, ng, nd, npk = vt_out.shape
         if nb * npk != m or npk % 32 or ng * nd != w.n - vt_col0:
             raise ValueError("vt_out: B * P must equal M, P be a multiple of 32 and G * D equal N - vt_col0")
-        rc = lib.tk_bf16w_dense_vt(
-            x.data_ptr(), ldx, w.data.data_ptr(), None if bias is None else bias.data_ptr(), out.data_ptr(), out.stride(0), vt_out.data_ptr(),
-            vt_col0, vt_out.stride(2), npk, vt_out.stride(0), int(dt == torch.float16), m, w.n, w.k, tile, split_k, ws.ptr, ws.nbytes, _stream(),
+        _calls().tk_bf16w_dense_vt(
+            x, ldx, w.data, bias, out, out.stride(0), vt_out,
+            vt_col0, vt_out.stride(2), npk, vt_out.stride(0), int(dt == torch.float16), m, w.n, w.k, tile, split_k, ws.buf, ws.nbytes,
         )  # fmt: skip
-        native.check(rc, "tk_bf16w_dense_vt")
         return out
-    entry = lib.tk_f16w_dense if dt == torch.float16 else lib.tk_bf16w_dense
-    rc = entry(
-        x.data_ptr(), ldx, w.data.data_ptr(), None if bias is None else bias.data_ptr(), _DENSE_ACTS[act], out.data_ptr(),
-        out.stride(0), rp, ldr, rdt, m, w.n, w.k, tile, split_k, ws.ptr, ws.nbytes, _stream(),
-    )  # fmt: skip
-    native.check(rc, "tk_f16w_dense" if dt == torch.float16 else "tk_bf16w_dense")
+    entry = _calls().tk_f16w_dense if dt == torch.float16 else _calls().tk_bf16w_dense
+    entry(x, ldx, w.data, bias, _DENSE_ACTS[act], out, out.stride(0), rp, ldr, rdt, m, w.n, w.k, tile, split_k, ws.buf, ws.nbytes)
     return out
 
 
@@ -440,7 +411,6 @@ def bf16w_dense_rope(
     rotary pair order (``pack_bf16_weight(w, rope_half)``), the columns ``< rope_cols`` rotated by the table row of
     ``rope_pos[m]``, and with ``vt_out [N - vt_col0, >= M rounded up to 32]`` the columns from ``vt_col0`` on also
     written transposed -- a many-row prefill's q|k|v projection in one launch (``tk_bf16w_dense_rope``)."""
-    lib = native.lib()
     if w.dtype != torch.bfloat16 or not w.rope_half or rope.half != w.rope_half:
         raise ValueError("the weight must be bf16, packed in rotary pair order with the tables' rope_half")
     if x.dtype != torch.bfloat16 or not x.is_cuda or x.dim() != 2 or x.shape[1] != w.k or x.stride(1) != 1:
@@ -451,7 +421,7 @@ def bf16w_dense_rope(
     if rope.cos.dtype != torch.float32 or not rope.cos.is_contiguous() or not rope.sin.is_contiguous():
         raise ValueError("rotary tables must be contiguous fp32")
     if out is None:
-        out = torch.empty(m, w.n, dtype=torch.bfloat16, device=x.device)
+        out = _calls().empty_bf16(x, m, w.n)
     if out.dtype != torch.bfloat16 or out.shape != (m, w.n) or out.stride(1) != 1:
         raise ValueError("out must be bf16 [M, N] with unit inner stride")
     vt_p, vt_ld = None, 0
@@ -460,12 +430,11 @@ def bf16w_dense_rope(
             raise ValueError("vt_out must be bf16 [N - vt_col0, >= M] with unit inner stride")
         vt_p, vt_ld = vt_out.data_ptr(), vt_out.stride(0)
     ws = ws or default_workspace(x.device)
-    rc = lib.tk_bf16w_dense_rope(
-        x.data_ptr(), x.stride(0), w.data.data_ptr(), out.data_ptr(), out.stride(0), rope_pos.data_ptr(), rope.cos.data_ptr(),
-        rope.sin.data_ptr(), rope.positions, rope_cols, rope.half, int(rope_bf16), vt_p, vt_col0, vt_ld, m, w.n, w.k, tile, split_k,
-        ws.ptr, ws.nbytes, _stream(),
+    _calls().tk_bf16w_dense_rope(
+        x, x.stride(0), w.data, out, out.stride(0), rope_pos, rope.cos,
+        rope.sin, rope.positions, rope_cols, rope.half, int(rope_bf16), vt_p, vt_col0, vt_ld, m, w.n, w.k, tile, split_k,
+        ws.buf, ws.nbytes,
     )  # fmt: skip
-    native.check(rc, "tk_bf16w_dense_rope")
     return out
 
 
@@ -512,7 +481,6 @@ def bf16w_linear(
     transposed) or a (gated) residual epilogue.  ``ada = (scale, shift)``, fp32 ``[K]`` each,
     selects the adaptive RMSNorm prologue instead of ``norm_w``; ``rope_bf16`` the bf16-arithmetic
     rotation."""
-    lib = native.lib()
     if not x.is_cuda or x.dim() != 2 or x.shape[1] != w.k or x.stride(1) != 1:
         raise ValueError(f"activations must be CUDA [M, {w.k}] with unit inner stride")
     if x.dtype == torch.float32:
@@ -525,7 +493,7 @@ def bf16w_linear(
         raise TypeError("activations must be bf16 or fp32")
     m = x.shape[0]
     if out is None:
-        out = torch.empty(m, w.n, dtype=torch.bfloat16, device=x.device)
+        out = _calls().empty_bf16(x, m, w.n)
     rp, ldr, rdt = _resid_args(resid, m, w.n)
     pos_p = cos_p = sin_p = None
     positions = half = 0
@@ -546,12 +514,11 @@ def bf16w_linear(
             raise ValueError("vt_out must be bf16 [N - vt_col0, >= M] with unit inner stride")
         vt_p, vt_ld = vt_out.data_ptr(), vt_out.stride(0)
     ws = ws or default_workspace(x.device)
-    rc = lib.tk_bf16w_linear(
-        x.data_ptr(), x.stride(0), xdt, w.data.data_ptr(), _norm_ptr(norm_w, w.k), float(eps), *_ada_ptrs(ada, w.k),
-        pos_p, cos_p, sin_p, positions, rope_cols, half, int(rope_bf16), vt_p, vt_col0, vt_ld, out.data_ptr(),
-        out.stride(0), rp, ldr, rdt, _gate_ptr(gate, w.n), m, w.n, w.k, split_k, ws.ptr, ws.nbytes, _stream(),
+    _calls().tk_bf16w_linear(
+        x, x.stride(0), xdt, w.data, _norm_ptr(norm_w, w.k), float(eps), *_ada_ptrs(ada, w.k),
+        pos_p, cos_p, sin_p, positions, rope_cols, half, int(rope_bf16), vt_p, vt_col0, vt_ld, out,
+        out.stride(0), rp, ldr, rdt, _gate_ptr(gate, w.n), m, w.n, w.k, split_k, ws.buf, ws.nbytes,
     )  # fmt: skip
-    native.check(rc, "tk_bf16w_linear")
     return out
 
 
@@ -559,14 +526,6 @@ def _eff_strides(t: torch.Tensor) -> tuple[int, int]:
     """(row, head) element strides of a ``[L, G, D]`` view; a size-1 dim never advances, so its
     stride is reported as 0 whatever torch recorded for it."""
     return (t.stride(0) if t.shape[0] > 1 else 0, t.stride(1) if t.shape[1] > 1 else 0)
-
-
-def _vt_ok(vt: torch.Tensor, stride: tuple[int, ...], g: int, d: int, length: int) -> bool:
-    shape = vt.shape
-    return vt.dtype is torch.bfloat16 and len(shape) == 3 and shape[0] == g and shape[1] == d and stride[2] == 1 and shape[2] >= _pad32(length)
-
-
-_MASK_TYPES = (torch.uint8, torch.bool)
 
 
 def _same_layout(k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -604,7 +563,6 @@ def prepare_prefix_kv(k: torch.Tensor, v: torch.Tensor) -> PrefixKV:
 
     bf16: ``k`` is used in place, ``v`` is transposed.  fp32: both are split into bf16 hi + lo planes.
     """
-    lib = native.lib()
     if k.dtype != v.dtype or k.dtype not in (torch.bfloat16, torch.float32):
         raise TypeError("prefix K/V must both be bf16 or both fp32")
     if not _same_layout(k, v):
@@ -615,13 +573,10 @@ def prepare_prefix_kv(k: torch.Tensor, v: torch.Tensor) -> PrefixKV:
     vt = torch.empty(g, d, _pad32(p), **bf)
     if k.dtype == torch.float32:
         k_hi, k_lo, vt_lo = torch.empty(p, g, d, **bf), torch.empty(p, g, d, **bf), torch.empty_like(vt)
-        rc = lib.tk_attn_prepare_kv(k.data_ptr(), v.data_ptr(), _F32, sl, sh, p, g, d, k_hi.data_ptr(), k_lo.data_ptr(),
-                                    vt.data_ptr(), vt_lo.data_ptr(), vt.shape[2], _stream())  # fmt: skip
-        native.check(rc, "tk_attn_prepare_kv")
+        _calls().tk_attn_prepare_kv(k, v, _F32, sl, sh, p, g, d, k_hi, k_lo,
+                                    vt, vt_lo, vt.shape[2])  # fmt: skip
         return PrefixKV(k_hi, vt, k_lo, vt_lo)
-    rc = lib.tk_attn_prepare_kv(None, v.data_ptr(), _BF16, sl, sh, p, g, d, None, None, vt.data_ptr(), None, vt.shape[2],
-                                _stream())  # fmt: skip
-    native.check(rc, "tk_attn_prepare_kv")
+    _calls().tk_attn_prepare_kv(None, v, _BF16, sl, sh, p, g, d, None, None, vt, None, vt.shape[2])  # fmt: skip
     return PrefixKV(k, vt)
 
 
@@ -630,7 +585,6 @@ def project_prefix_kv(k: torch.Tensor, v: torch.Tensor, wk: torch.Tensor, wv: to
     ``k, v [P, KV]`` bf16 rows (views with a contiguous last dim and the same row stride), ``wk, wv
     [N, KV]`` fp32 -> :class:`PrefixKV` of ``float(k) @ wk.T`` / ``float(v) @ wv.T`` as bf16 hi + lo
     planes (``[P, N/d, d]`` and ``[N/d, d, P rounded up to 32]``).  One launch."""
-    lib = native.lib()
     bf = torch.bfloat16
     if k.dtype != bf or v.dtype != bf or wk.dtype != torch.float32 or wv.dtype != torch.float32:
         raise TypeError("project_prefix_kv: k, v bf16 and wk, wv fp32")
@@ -643,9 +597,8 @@ def project_prefix_kv(k: torch.Tensor, v: torch.Tensor, wk: torch.Tensor, wv: to
     opts = dict(dtype=bf, device=k.device)
     k_hi, k_lo = torch.empty(p, g, d, **opts), torch.empty(p, g, d, **opts)
     vt_hi, vt_lo = torch.empty(g, d, _pad32(p), **opts), torch.empty(g, d, _pad32(p), **opts)
-    rc = lib.tk_expert_kv_project(k.data_ptr(), v.data_ptr(), k.stride(0), p, kv, wk.data_ptr(), wv.data_ptr(), n, k_hi.data_ptr(),
-                                  k_lo.data_ptr(), vt_hi.data_ptr(), vt_lo.data_ptr(), vt_hi.shape[2], _stream())  # fmt: skip
-    native.check(rc, "tk_expert_kv_project")
+    _calls().tk_expert_kv_project(k, v, k.stride(0), p, kv, wk, wv, n, k_hi,
+                                  k_lo, vt_hi, vt_lo, vt_hi.shape[2])  # fmt: skip
     return PrefixKV(k_hi, vt_hi, k_lo, vt_lo)
 
 
@@ -695,65 +648,12 @@ def expert_attn(
     """Attention of ``q [M, H, D]`` over ``[prefix; suffix]`` keys.  ``prefix_pad``: uint8/bool
     ``[P]`` or None; ``mask2d``: uint8/bool ``[M, >= P rounded up to 32]`` per-(query, prefix key)
     visibility, replaces ``prefix_pad``.  Returns bf16 ``[M, H*D]``."""
-    lib = native.lib()
-    bf = torch.bfloat16
-    q_st = q.stride()
-    if q.dtype is not bf or len(q_st) != 3 or q_st[2] != 1:
-        raise TypeError("q must be bf16 [M, H, D] with a contiguous head dim")
-    m, h, d = q.shape
-    # (shapes and strides are read once per tensor: each is a call into torch, and together they cost more than the launch)
-    p = g = 0
-    kp = kpl = vp = vpl = None
-    pre_sl = pre_sh = pre_sd = pre_vsh = 0
+    k = vt = k_lo = vt_lo = ks = vs = None
     if prefix is not None:
-        k, vt = prefix.k, prefix.vt
-        k_st, vt_st = k.stride(), vt.stride()
-        p, g, kd = k.shape
-        if k.dtype is not bf or kd != d or k_st[2] != 1 or not _vt_ok(vt, vt_st, g, d, p):
-            raise ValueError("prefix must hold bf16 K [P, G, D] and V^T [G, D, >= P rounded up to 32]")
-        pre_sl, pre_sh = k_st[0] if p > 1 else 0, k_st[1] if g > 1 else 0
-        pre_vsh, pre_sd = vt_st[0] if g > 1 else 0, vt_st[1]
-        kp, vp = k.data_ptr(), vt.data_ptr()
-        if prefix.k_lo is not None:
-            if prefix.vt_lo is None or prefix.k_lo.stride() != k_st or prefix.vt_lo.stride() != vt_st:
-                raise ValueError("low planes must mirror the high planes' layout")
-            kpl, vpl = prefix.k_lo.data_ptr(), prefix.vt_lo.data_ptr()
-    s = 0
-    ks = vs = None
-    suf_sl = suf_sh = suf_sd = suf_vsh = 0
+        k, vt, k_lo, vt_lo = prefix.k, prefix.vt, prefix.k_lo, prefix.vt_lo
     if suffix is not None:
-        k, vt = suffix.k, suffix.vt
-        k_st, vt_st = k.stride(), vt.stride()
-        s, gs, kd = k.shape
-        if prefix is not None and gs != g:
-            raise ValueError("prefix and suffix must have the same number of kv heads")
-        g = gs
-        if k.dtype is not bf or kd != d or k_st[2] != 1 or not _vt_ok(vt, vt_st, g, d, s):
-            raise ValueError("suffix must hold bf16 K [S, G, D] and V^T [G, D, >= S rounded up to 32]")
-        suf_sl, suf_sh = k_st[0] if s > 1 else 0, k_st[1] if g > 1 else 0
-        suf_vsh, suf_sd = vt_st[0] if g > 1 else 0, vt_st[1]
-        ks, vs = k.data_ptr(), vt.data_ptr()
-    pad = None
-    if prefix_pad is not None:
-        # (bool and uint8 are one byte each: no view of one as the other is needed to pass its address)
-        if prefix_pad.dtype not in _MASK_TYPES or prefix_pad.numel() != p or not prefix_pad.is_contiguous():
-            raise ValueError("prefix_pad must be a contiguous uint8/bool [P]")
-        pad = prefix_pad.data_ptr()
-    m2_p, m2_ld = None, 0
-    if mask2d is not None:
-        if mask2d.dtype not in _MASK_TYPES or mask2d.dim() != 2 or mask2d.shape[0] != m or mask2d.stride(1) != 1 or mask2d.shape[1] < _pad32(p):
-            raise ValueError("mask2d must be uint8/bool [M, >= P rounded up to 32] with unit inner stride")
-        m2_p, m2_ld = mask2d.data_ptr(), mask2d.stride(0)
-    if out is None:
-        out = torch.empty(m, h * d, dtype=bf, device=q.device)
-    ws = ws or default_workspace(q.device)
-    rc = lib.tk_expert_attn(
-        q.data_ptr(), q_st[0], q_st[1], kp, kpl, pre_sl, pre_sh, vp, vpl, pre_sd, pre_vsh, ks, suf_sl, suf_sh,
-        vs, suf_sd, suf_vsh, pad, m2_p, m2_ld, out.data_ptr(), out.stride(0), m, p, s, h, max(g, 1), d, mask_mode,
-        int(logits_bf16), ws.ptr, ws.nbytes, _stream(),
-    )  # fmt: skip
-    native.check(rc, "tk_expert_attn")
-    return out
+        ks, vs = suffix.k, suffix.vt
+    return _calls().expert_attn(q, k, vt, k_lo, vt_lo, ks, vs, prefix_pad, mask_mode, mask2d, int(logits_bf16), out, ws)
 
 
 CROSS_FUSED_MAX_K = 768    # widest hidden size the in-kernel q projection stages
@@ -777,7 +677,6 @@ def cross_attn_fused(
     mask.  ``x [M, K]`` bf16 (``K <= 768``), ``wq`` packed with ``rope_half = 32`` (head size 64),
     ``prefix`` from :func:`project_prefix_kv` / :func:`prepare_prefix_kv` of fp32 tensors with at most
     256 keys.  Returns bf16 ``[M, H*64]``; equals :func:`bf16w_linear` + :func:`expert_attn`."""
-    lib = native.lib()
     bf = torch.bfloat16
     if x.dtype != bf or x.dim() != 2 or x.stride(1) != 1 or norm_w.dtype != bf:
         raise TypeError("cross_attn_fused: x [M, K] and norm_w must be bf16, x rows contiguous")
@@ -798,15 +697,14 @@ def cross_attn_fused(
         if pad.dtype != torch.uint8 or pad.numel() != p or not pad.is_contiguous():
             raise ValueError("prefix_pad must be a contiguous uint8/bool [P]")
     if out is None:
-        out = torch.empty(m, h * d, dtype=bf, device=x.device)
+        out = _calls().empty_bf16(x, m, h * d)
     pre_sl, pre_sh = _eff_strides(prefix.k)
-    rc = lib.tk_expert_cross_attn_fused(
-        x.data_ptr(), x.stride(0), norm_w.data_ptr(), float(eps), wq.data.data_ptr(), k, rope_pos.data_ptr(), rope.cos.data_ptr(),
-        rope.sin.data_ptr(), rope.cos.shape[0], prefix.k.data_ptr(), prefix.k_lo.data_ptr(), pre_sl, pre_sh, prefix.vt.data_ptr(),
-        prefix.vt_lo.data_ptr(), prefix.vt.stride(1), prefix.vt.stride(0) if g > 1 else 0, _ptr(pad), out.data_ptr(), out.stride(0),
-        m, p, h, g, d, _stream(),
+    _calls().tk_expert_cross_attn_fused(
+        x, x.stride(0), norm_w, float(eps), wq.data, k, rope_pos, rope.cos,
+        rope.sin, rope.cos.shape[0], prefix.k, prefix.k_lo, pre_sl, pre_sh, prefix.vt,
+        prefix.vt_lo, prefix.vt.stride(1), prefix.vt.stride(0) if g > 1 else 0, pad, out, out.stride(0),
+        m, p, h, g, d,
     )  # fmt: skip
-    native.check(rc, "tk_expert_cross_attn_fused")
     return out
 
 
@@ -824,7 +722,6 @@ def batched_attn(
     contiguous head dim), ``vt [B, G, D, >= P rounded up to 32]`` (V transposed, zero padded) ->
     bf16 ``[B, M, H*D]``.  ``scale`` multiplies the logits (default ``D ** -0.5``; a head padded with
     zero columns up to a supported ``D`` passes the scale of its true size)."""
-    lib = native.lib()
     bf = torch.bfloat16
     if q.dtype == torch.float16:
         # fp16 operands (pi0.5's fused tower): fp32 logits, probabilities rounded to fp16, bf16 output
@@ -844,12 +741,11 @@ def batched_attn(
     if out is None:
         out = torch.empty(b, m, h * d, dtype=bf, device=q.device)
     ws = ws or default_workspace(q.device)
-    rc = lib.tk_batched_attn(
-        q.data_ptr(), q.stride(0), q.stride(1), q.stride(2), k.data_ptr(), k.stride(0), k.stride(1), k.stride(2) if g > 1 else 0,
-        vt.data_ptr(), vt.stride(0), vt.stride(2), vt.stride(1) if g > 1 else 0, out.data_ptr(), out.stride(0), out.stride(1),
-        b, m, p, h, g, d, int(logits_bf16), float(scale or 0.0), ws.ptr, ws.nbytes, _stream(),
+    _calls().tk_batched_attn(
+        q, q.stride(0), q.stride(1), q.stride(2), k, k.stride(0), k.stride(1), k.stride(2) if g > 1 else 0,
+        vt, vt.stride(0), vt.stride(2), vt.stride(1) if g > 1 else 0, out, out.stride(0), out.stride(1),
+        b, m, p, h, g, d, int(logits_bf16), float(scale or 0.0), ws.buf, ws.nbytes,
     )  # fmt: skip
-    native.check(rc, "tk_batched_attn")
     return out
 
 
@@ -868,7 +764,6 @@ def transpose_v(v: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Te
     """``v [B, P, G, D]`` bf16 (a view with a contiguous head dim, e.g. into a packed q|k|v buffer) ->
     ``vt [B, G, D, P rounded up to 32]`` with zero-filled padding keys: the V^T operand of
     :func:`batched_attn`, one launch for all problems.  ``D`` in {64, 96}."""
-    lib = native.lib()
     if v.dtype not in (torch.bfloat16, torch.float16) or v.dim() != 4 or v.stride(3) != 1:
         raise TypeError("v must be a 4-D bf16 (or fp16) tensor with a contiguous head dim")
     b, p, g, d = v.shape
@@ -876,11 +771,10 @@ def transpose_v(v: torch.Tensor, *, out: torch.Tensor | None = None) -> torch.Te
         out = torch.empty(b, g, d, _pad32(p), dtype=v.dtype, device=v.device)
     if out.shape[:3] != (b, g, d) or out.shape[3] < _pad32(p) or out.stride(3) != 1 or out.dtype != v.dtype:
         raise ValueError("out must be [B, G, D, >= P rounded up to 32] of v's type with contiguous keys")
-    rc = lib.tk_batched_transpose_v(
-        v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
-        out.shape[3], b, p, g, d, _stream(),
+    _calls().tk_batched_transpose_v(
+        v, v.stride(0), v.stride(1), v.stride(2), out, out.stride(0), out.stride(1), out.stride(2),
+        out.shape[3], b, p, g, d,
     )  # fmt: skip
-    native.check(rc, "tk_batched_transpose_v")
     return out
 
 
@@ -923,7 +817,6 @@ def expert_tail(
     ``x_t [M, N]`` -- the Euler update ``x_t + dt * v``.  Returns ``(v or None, x_new or None)``.
     ``embed = (E [J, N] fp32, c [J] fp32 or None, "none" | "silu", out [M, J] fp32 or bf16)``: the same launch
     also writes ``out = act(x_new @ E^T + c)``, the next step's suffix embedding."""
-    lib = native.lib()
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.stride(1) != 1:
         raise TypeError("x must be bf16 [M, K] with unit inner stride")
     m, k = x.shape
@@ -952,18 +845,16 @@ def expert_tail(
             raise ValueError("embed out must be fp32 or bf16 [M, J] with unit inner stride")
         if eact not in ("none", "silu"):
             raise ValueError(f"embed activation {eact!r}")
-        rc = lib.tk_expert_tail_embed(
-            x.data_ptr(), x.stride(0), _norm_ptr(norm_w, k), *_ada_ptrs(ada, k), float(eps), w.data_ptr(), _ptr(bias), _ptr(v),
-            _ptr(x_t), _ptr(x_new), float(dt), m, n, k, ew.data_ptr(), _ptr(eb), j, 1 if eact == "silu" else 0, eout.data_ptr(),
-            eout.stride(0), _BF16 if eout.dtype == torch.bfloat16 else _F32, _stream(),
+        _calls().tk_expert_tail_embed(
+            x, x.stride(0), _norm_ptr(norm_w, k), *_ada_ptrs(ada, k), float(eps), w, bias, v,
+            x_t, x_new, float(dt), m, n, k, ew, eb, j, 1 if eact == "silu" else 0, eout,
+            eout.stride(0), _BF16 if eout.dtype == torch.bfloat16 else _F32,
         )  # fmt: skip
-        native.check(rc, "tk_expert_tail_embed")
         return v, x_new
-    rc = lib.tk_expert_tail(
-        x.data_ptr(), x.stride(0), _norm_ptr(norm_w, k), *_ada_ptrs(ada, k), float(eps), w.data_ptr(), _ptr(bias), _ptr(v),
-        _ptr(x_t), _ptr(x_new), float(dt), m, n, k, _stream(),
+    _calls().tk_expert_tail(
+        x, x.stride(0), _norm_ptr(norm_w, k), *_ada_ptrs(ada, k), float(eps), w, bias, v,
+        x_t, x_new, float(dt), m, n, k,
     )  # fmt: skip
-    native.check(rc, "tk_expert_tail")
     return v, x_new
 
 
@@ -1182,7 +1073,6 @@ def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float, ou
     """``bf16(LayerNorm(x) * w + b)`` over the last dim of ``x [..., K]`` (fp32 with fp32 parameters, or
     bf16 with bf16 parameters; contiguous rows), statistics in fp32.  One launch, bf16 result -- or, for fp32 rows
     and ``out_dtype=torch.float16``, an fp16 one."""
-    lib = native.lib()
     if x.dtype not in (torch.float32, torch.bfloat16) or w.dtype != x.dtype or b.dtype != x.dtype:
         raise TypeError("layer_norm: x, w, b must all be fp32 or all bf16")
     k = x.shape[-1]
@@ -1193,15 +1083,13 @@ def layer_norm(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, eps: float, ou
         if x.dtype != torch.float32:
             raise TypeError("layer_norm: the fp16 result is built for fp32 rows")
         y = torch.empty(x2.shape, dtype=torch.float16, device=x.device)
-        rc = lib.tk_layer_norm_f16(x2.data_ptr(), x2.stride(0), w.contiguous().data_ptr(), b.contiguous().data_ptr(), float(eps),
-                                   y.data_ptr(), y.stride(0), x2.shape[0], k, _stream())  # fmt: skip
-        native.check(rc, "tk_layer_norm_f16")
+        _calls().tk_layer_norm_f16(x2, x2.stride(0), w.contiguous(), b.contiguous(), float(eps),
+                                   y, y.stride(0), x2.shape[0], k)  # fmt: skip
         return y.view(x.shape)
-    y = torch.empty(x2.shape, dtype=torch.bfloat16, device=x.device)
+    y = _calls().empty_bf16(x, *x2.shape)
     dt = _F32 if x.dtype == torch.float32 else _BF16
-    rc = lib.tk_layer_norm(x2.data_ptr(), x2.stride(0), dt, w.contiguous().data_ptr(), b.contiguous().data_ptr(), dt, float(eps),
-                           y.data_ptr(), y.stride(0), x2.shape[0], k, _stream())  # fmt: skip
-    native.check(rc, "tk_layer_norm")
+    _calls().tk_layer_norm(x2, x2.stride(0), dt, w.contiguous(), b.contiguous(), dt, float(eps),
+                           y, y.stride(0), x2.shape[0], k)  # fmt: skip
     return y.view(x.shape)
 
 
@@ -1213,7 +1101,6 @@ def add_layer_norm(
     ``float(r)``, bf16 ``x`` rounds the sum once) and ``bf16(LayerNorm(x) * w + b)`` of the sum, one launch.
     Returns ``(x, normalised)``; ``x`` must own contiguous rows.  ``y_rows`` (int32, one entry per row of the
     flattened ``x``, a permutation): normalised row ``m`` is written as row ``y_rows[m]`` (bf16 result only)."""
-    lib = native.lib()
     if x.dtype not in (torch.float32, torch.bfloat16) or w.dtype != x.dtype or b.dtype != x.dtype or r.dtype != torch.bfloat16:
         raise TypeError("add_layer_norm: x, w, b all fp32 or all bf16; r bf16")
     k = x.shape[-1]
@@ -1226,25 +1113,22 @@ def add_layer_norm(
         if x.dtype != torch.float32 or y_rows is not None:
             raise TypeError("add_layer_norm: the fp16 result is built for fp32 rows in place")
         y = torch.empty(x2.shape, dtype=torch.float16, device=x.device)
-        rc = lib.tk_add_layer_norm_f16(x2.data_ptr(), x2.stride(0), r2.data_ptr(), r2.stride(0), x2.data_ptr(), x2.stride(0),
-                                       w.contiguous().data_ptr(), b.contiguous().data_ptr(), float(eps), y.data_ptr(), y.stride(0),
-                                       x2.shape[0], k, _stream())  # fmt: skip
-        native.check(rc, "tk_add_layer_norm_f16")
+        _calls().tk_add_layer_norm_f16(x2, x2.stride(0), r2, r2.stride(0), x2, x2.stride(0),
+                                       w.contiguous(), b.contiguous(), float(eps), y, y.stride(0),
+                                       x2.shape[0], k)  # fmt: skip
         return x, y.view(x.shape)
-    y = torch.empty(x2.shape, dtype=torch.bfloat16, device=x.device)
+    y = _calls().empty_bf16(x, *x2.shape)
     dt = _F32 if x.dtype == torch.float32 else _BF16
     if y_rows is not None:
         if y_rows.dtype != torch.int32 or y_rows.numel() < x2.shape[0] or not y_rows.is_contiguous() or y_rows.device != x.device:
             raise ValueError("add_layer_norm: y_rows must be a contiguous int32 tensor on x's device with an entry per row")
-        rc = lib.tk_add_layer_norm_rows(x2.data_ptr(), x2.stride(0), dt, r2.data_ptr(), r2.stride(0), x2.data_ptr(), x2.stride(0),
-                                        w.contiguous().data_ptr(), b.contiguous().data_ptr(), dt, float(eps), y.data_ptr(), y.stride(0),
-                                        y_rows.data_ptr(), x2.shape[0], k, _stream())  # fmt: skip
-        native.check(rc, "tk_add_layer_norm_rows")
+        _calls().tk_add_layer_norm_rows(x2, x2.stride(0), dt, r2, r2.stride(0), x2, x2.stride(0),
+                                        w.contiguous(), b.contiguous(), dt, float(eps), y, y.stride(0),
+                                        y_rows, x2.shape[0], k)  # fmt: skip
         return x, y.view(x.shape)
-    rc = lib.tk_add_layer_norm(x2.data_ptr(), x2.stride(0), dt, r2.data_ptr(), r2.stride(0), x2.data_ptr(), x2.stride(0),
-                               w.contiguous().data_ptr(), b.contiguous().data_ptr(), dt, float(eps), y.data_ptr(), y.stride(0),
-                               x2.shape[0], k, _stream())  # fmt: skip
-    native.check(rc, "tk_add_layer_norm")
+    _calls().tk_add_layer_norm(x2, x2.stride(0), dt, r2, r2.stride(0), x2, x2.stride(0),
+                               w.contiguous(), b.contiguous(), dt, float(eps), y, y.stride(0),
+                               x2.shape[0], k)  # fmt: skip
     return x, y.view(x.shape)
 
 
@@ -1252,7 +1136,6 @@ def rms_norm_rows(x: torch.Tensor, *, norm_w: torch.Tensor | None = None, ada: t
     """RMSNorm of bf16 rows ``x [M, K]`` into a new bf16 tensor: Llama (``norm_w`` bf16 ``[K]``) or
     Gemma / adaptive (``ada = (scale, shift)`` fp32 ``[K]``: ``(x * rstd) * (1 + scale) + shift``).  The
     norm prologue of the fused projections as one launch, for projections that run as a library GEMM."""
-    lib = native.lib()
     if x.dtype != torch.bfloat16 or x.dim() != 2 or x.stride(1) != 1:
         raise TypeError("rms_norm_rows: x must be a 2-D bf16 tensor with contiguous rows")
     if (norm_w is None) == (ada is None):
@@ -1262,29 +1145,26 @@ def rms_norm_rows(x: torch.Tensor, *, norm_w: torch.Tensor | None = None, ada: t
         raise TypeError("rms_norm_rows: norm_w must be bf16 [K]")
     if ada is not None and any(t.dtype != torch.float32 or t.numel() != k or not t.is_contiguous() for t in ada):
         raise TypeError("rms_norm_rows: ada scale / shift must be contiguous fp32 [K]")
-    y = torch.empty(m, k, dtype=torch.bfloat16, device=x.device)
-    rc = lib.tk_rms_norm_rows(
-        x.data_ptr(), x.stride(0), norm_w.contiguous().data_ptr() if norm_w is not None else None,
-        ada[0].data_ptr() if ada is not None else None, ada[1].data_ptr() if ada is not None else None, float(eps),
-        y.data_ptr(), y.stride(0), m, k, _stream(),
+    y = _calls().empty_bf16(x, m, k)
+    _calls().tk_rms_norm_rows(
+        x, x.stride(0), norm_w.contiguous() if norm_w is not None else None,
+        ada[0] if ada is not None else None, ada[1] if ada is not None else None, float(eps),
+        y, y.stride(0), m, k,
     )  # fmt: skip
-    native.check(rc, "tk_rms_norm_rows")
     return y
 
 
 def rope_rows(y: torch.Tensor, rope: RopeTables, rope_pos: torch.Tensor, rope_cols: int, *, rope_bf16: bool = False) -> torch.Tensor:
     """Rotary embedding in place on the first ``rope_cols`` columns of a bf16 projection output
     ``y [M, N]`` (heads of ``2 * rope.half`` columns), int32 positions ``[M]``.  Returns ``y``."""
-    lib = native.lib()
     if y.dtype != torch.bfloat16 or y.dim() != 2 or y.stride(1) != 1:
         raise TypeError("rope_rows: y must be a 2-D bf16 tensor with contiguous rows")
     if rope_pos.dtype != torch.int32 or rope_pos.numel() != y.shape[0] or not rope_pos.is_contiguous():
         raise TypeError("rope_rows: positions must be contiguous int32 [M]")
     if rope_cols > y.shape[1]:
         raise ValueError("rope_rows: rope_cols exceeds the row width")
-    rc = lib.tk_rope_rows(y.data_ptr(), y.stride(0), rope_pos.data_ptr(), rope.cos.data_ptr(), rope.sin.data_ptr(), rope.positions,
-                          int(rope_cols), rope.half, int(rope_bf16), y.shape[0], _stream())  # fmt: skip
-    native.check(rc, "tk_rope_rows")
+    _calls().tk_rope_rows(y, y.stride(0), rope_pos, rope.cos, rope.sin, rope.positions,
+                          int(rope_cols), rope.half, int(rope_bf16), y.shape[0])  # fmt: skip
     return y
 
 
@@ -1293,7 +1173,6 @@ def prefix_meta(pad: torch.Tensor, att: torch.Tensor | None, rope_positions: int
     ``(mask2d uint8 [P, P rounded up to 32] or None, pos32 int32 [P], suf_pos int32 [suffix_len] or None)``:
     the prefill's 2-D visibility ``(cumsum(att)[j] <= cumsum(att)[i]) & pad[i] & pad[j]``, the prefix positions
     ``clamp(cumsum(pad) - 1)`` and the action tokens' positions ``clamp(sum(pad) + s)``."""
-    lib = native.lib()
     if pad.dtype != torch.bool or pad.dim() != 1 or not pad.is_contiguous():
         raise TypeError("prefix_meta: pad must be a contiguous 1-D bool tensor")
     if att is not None and (att.dtype != torch.bool or att.shape != pad.shape or not att.is_contiguous()):
@@ -1303,9 +1182,8 @@ def prefix_meta(pad: torch.Tensor, att: torch.Tensor | None, rope_positions: int
     mask2d = torch.empty(p_len, p_pad, dtype=torch.uint8, device=pad.device) if want_mask else None
     pos32 = torch.empty(p_len, dtype=torch.int32, device=pad.device)
     suf = torch.empty(suffix_len, dtype=torch.int32, device=pad.device) if suffix_len > 0 else None
-    rc = lib.tk_prefix_meta(pad.data_ptr(), _ptr(att), p_len, p_pad, int(rope_positions), int(suffix_len), _ptr(mask2d), pos32.data_ptr(),
-                            _ptr(suf), _stream())  # fmt: skip
-    native.check(rc, "tk_prefix_meta")
+    _calls().tk_prefix_meta(pad, att, p_len, p_pad, int(rope_positions), int(suffix_len), mask2d, pos32,
+                            suf)  # fmt: skip
     return mask2d, pos32, suf
 
 
@@ -1313,7 +1191,6 @@ def patchify_images(images, patch: int, scale: float = 1.0, shift: float = 0.0, 
     """Up to four fp32 images ``[1, 3, H, W]`` (or ``[3, H, W]``) -> ``[n, (H/patch) * (W/patch), 3 * patch * patch]``
     rows of ``x * scale + shift`` in the order of ``unfold``: the patch embedding's GEMM input, in bf16 (patch sizes
     that are multiples of 8) or fp32 (any even patch size)."""
-    lib = native.lib()
     images = list(images)
     if not 1 <= len(images) <= 4:
         raise ValueError("patchify_images: one to four images")
@@ -1324,10 +1201,8 @@ def patchify_images(images, patch: int, scale: float = 1.0, shift: float = 0.0, 
     if out_dtype not in (torch.bfloat16, torch.float32):
         raise TypeError("patchify_images: bf16 or fp32 patch rows")
     out = torch.empty(len(images), (h // patch) * (w // patch), 3 * patch * patch, dtype=out_dtype, device=images[0].device)
-    ptrs = [img.data_ptr() for img in images] + [None] * (4 - len(images))
-    fn = lib.tk_patchify_images if out_dtype == torch.bfloat16 else lib.tk_patchify_images_f32
-    rc = fn(*ptrs, len(images), h, w, int(patch), float(scale), float(shift), out.data_ptr(), _stream())
-    native.check(rc, "tk_patchify_images")
+    fn = _calls().tk_patchify_images if out_dtype == torch.bfloat16 else _calls().tk_patchify_images_f32
+    fn(*images, *[None] * (4 - len(images)), len(images), h, w, int(patch), float(scale), float(shift), out)
     return out
 
 
@@ -1338,7 +1213,6 @@ def prefix_rows(img, img_scale: float, table, tokens, tok_scale: float, last=Non
     in fp32 or rounded to bf16 (``out_dtype``).  With ``cam_flags`` (a bool tensor of one element per camera) and
     ``tok_flags`` (bool ``[n_tok]``) also the pad flags ``[1, P]`` of those rows (the closing rows are always valid);
     returns ``(rows, flags or None)``."""
-    lib = native.lib()
     bf = torch.bfloat16
     if img.dtype not in (bf, torch.float32) or table.dtype != bf or tokens.dtype != torch.int64 or (last is not None and last.dtype != torch.float32):
         raise TypeError("prefix_rows: img bf16 or fp32, table bf16, tokens int64, last fp32")
@@ -1360,13 +1234,12 @@ def prefix_rows(img, img_scale: float, table, tokens, tok_scale: float, last=Non
         if any(f.dtype != torch.bool or f.numel() != 1 for f in cam_flags) or tok_flags.dtype != torch.bool:
             raise TypeError("prefix_rows: flags are bool tensors")
         flags = torch.empty(1, total, dtype=torch.bool, device=img.device)
-        fl = [f.data_ptr() for f in cam_flags] + [None] * (4 - cams)
-    rc = lib.tk_prefix_rows(
-        img.data_ptr(), _BF16 if img.dtype == bf else _F32, n_img, float(img_scale), table.data_ptr(), tokens.data_ptr(), n_tok, table.shape[0],
-        float(tok_scale), None if last is None else last.data_ptr(), n_last, out.data_ptr(), _BF16 if out_dtype == bf else _F32, h, *fl, cams,
-        tok_flags.data_ptr() if flags is not None else None, flags.data_ptr() if flags is not None else None, _stream(),
+        fl = cam_flags + [None] * (4 - cams)
+    _calls().tk_prefix_rows(
+        img, _BF16 if img.dtype == bf else _F32, n_img, float(img_scale), table, tokens, n_tok, table.shape[0],
+        float(tok_scale), last, n_last, out, _BF16 if out_dtype == bf else _F32, h, *fl, cams,
+        tok_flags if flags is not None else None, flags if flags is not None else None,
     )  # fmt: skip
-    native.check(rc, "tk_prefix_rows")
     return out, flags
 
 
