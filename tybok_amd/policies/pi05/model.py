@@ -528,6 +528,10 @@ class PI05Model:
                 )  # fmt: skip
             k = qkv[:, nq : nq + nkv].view(p_len, g, d)
             cache = tk.PrefixKV(k, vt_all[i].view(g, d, p_pad))
+            kv.append((k.transpose(0, 1)[None], qkv[:, nq + nkv :].view(p_len, g, d).transpose(0, 1)[None]))
+            caches.append(cache)
+            if i + 1 == self.depth:  # run for the keys and values: nothing reads the rows behind the last layer's
+                break
             att = tk.expert_attn(qkv[:, :nq].view(p_len, heads, d), cache, None, None, tk.MASK_NONE, mask2d=mask2d, logits_bf16=True, ws=self.ws)
             if many_rows:
                 out = tk.bf16w_dense(att, self.vlm_o[i], resid=hidden, ws=self.ws)  # bf16(bf16(att . Wo^T) + hidden), as below
@@ -542,8 +546,6 @@ class PI05Model:
             else:
                 h, _ = gemma_norm(out[None], weight=self.p[f"{VLM}layers.{i}.post_attention_layernorm.weight"])
                 hidden = mlp(h, out[None])[0]
-            kv.append((k.transpose(0, 1)[None], qkv[:, nq + nkv :].view(p_len, g, d).transpose(0, 1)[None]))
-            caches.append(cache)
         return (kv, caches, suf_pos) if suffix_len else (kv, caches)
 
     # ------------------------------------------------------------------ denoising

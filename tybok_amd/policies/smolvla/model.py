@@ -513,7 +513,8 @@ class SmolVLAModel:
 
     def _prefill_layer_fused(self, i: int, hidden: torch.Tensor, c: dict) -> torch.Tensor:
         """One VLM layer on the fused launches: norm + q|k|v + RoPE, attention under the 2-D prefix
-        mask, o_proj + residual, gated FFN.  Fills ``qkv_all[i]`` / ``vt_all[i]`` (the layer's K/V cache)."""
+        mask, o_proj + residual, gated FFN.  Fills ``qkv_all[i]`` / ``vt_all[i]`` (the layer's K/V cache).  The last
+        layer ends there: the prefill is run for its caches, and nothing reads the rows behind them."""
         h_q, h_kv, d = self.heads, self.kv_heads, self.head_dim
         nq, nkv = h_q * d, h_kv * d
         p_len, p_pad = c["p_len"], c["p_pad"]
@@ -522,6 +523,8 @@ class SmolVLAModel:
             hidden, self.vlm_qkv[i], norm_w=self.p[lp + "input_layernorm.weight"], eps=self.eps, rope=self.rope_tables,
             rope_pos=c["pos32"], rope_cols=nq + nkv, vt_out=c["vt_all"][i], vt_col0=nq + nkv, out=c["qkv_all"][i], ws=self.ws,
         )  # fmt: skip
+        if i + 1 == self.num_layers:
+            return hidden
         cache = tk.PrefixKV(qkv[:, nq : nq + nkv].view(p_len, h_kv, d), c["vt_all"][i].view(h_kv, d, p_pad))
         att = tk.expert_attn(qkv[:, :nq].view(p_len, h_q, d), cache, None, None, tk.MASK_NONE, mask2d=c["mask2d"], ws=self.ws)
         out = tk.bf16w_linear(att, self.vlm_o[i], resid=hidden, ws=self.ws)
