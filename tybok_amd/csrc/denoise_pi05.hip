@@ -83,7 +83,7 @@ constexpr int L_XT = L_L + kWaves * 16 * 4;       // x_t [32][16]
 constexpr int L_WI = L_XT + A * 16 * 4;           // this block's rows of the action embedding [16][32]
 constexpr int L_Q = L_WI + 16 * A * 4;            // the query tile, B operand order
 constexpr int L_P = L_Q + D / 32 * 1024;          // probabilities of the block's key tiles, B operand order
-constexpr int L_ROPE = L_P + TILES * 1024;        // (cos, sin) pairs of 128 threads
+constexpr int L_ROPE = L_P + TILES * 1024;        // (cos, sin) pairs of 128 column pairs
 constexpr int L_KV = L_ROPE + 128 * 16;           // prefix caches of every layer
 constexpr int LDS_B = L_KV + kPiMaxLayers * (int)sizeof(PiCache);
 static_assert(LDS_B <= 160 * 1024, "one block's LDS");
@@ -146,14 +146,13 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
   };
 
   // ---- constants of the whole run ----
-  if (tid < 128) {
-    const Own ow = own_of(tid);
-    const int mg = rt * 16 + ow.m;
+  if (tid < 128) {  // row tid / 8, columns n = 2 (tid & 7) and the next
+    const int mg = rt * 16 + (tid >> 3), n = 2 * (tid & 7);
     int p = a.pos[mg < a.M ? mg : a.M - 1];
     p = p < 0 ? 0 : (p > a.positions - 1 ? a.positions - 1 : p);
     f32x2* const o = (f32x2*)(lds + L_ROPE + tid * 16);
-    o[0] = *(const f32x2*)(a.rope_cos + (size_t)p * (D / 2) + 16 * (c & 7) + ow.n);
-    o[1] = *(const f32x2*)(a.rope_sin + (size_t)p * (D / 2) + 16 * (c & 7) + ow.n);
+    o[0] = *(const f32x2*)(a.rope_cos + (size_t)p * (D / 2) + 16 * (c & 7) + n);
+    o[1] = *(const f32x2*)(a.rope_sin + (size_t)p * (D / 2) + 16 * (c & 7) + n);
   }
   if (tid < a.layers * (int)(sizeof(PiCache) / 4)) ((int*)(lds + L_KV))[tid] = ((const int*)a.cache)[tid];
   if (tid < A * 16) {
@@ -179,43 +178,42 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
 
   // where this thread's words go, within a layer of the ring.  P1, q and k: the two words of a rotary pair; v: of two tiles
   auto q_s = [&]() { return OFF_Q + rt * Q_B + (c >> 3) * 8192 + ((c & 7) >> 1) * 1024 + (c & 1) * 512; };
-  auto kv_off = [&](int& off, int& step) {  // blocks 0..15, threads 128..255
+  auto kv_off = [&](const Own& ow, int& off, int& step) {  // blocks 0..15, threads 256..511
     if (c < 8) {
-      off = OFF_K + rt * K_B + (c >> 1) * 1024 + (c & 1) * 512 + own_of(tid).word;
+      off = OFF_K + rt * K_B + (c >> 1) * 1024 + (c & 1) * 512 + ow.word;
       step = 4096;
-    } else {
-      const int vq = ((tid >> 6) & 1) * 4 + (tid & 3), vd = (tid >> 2) & 15;  // key pair and column
-      off = OFF_V + (rt >> 1) * V_B + 2 * (c - 8) * 1024 + ((rt & 1) * 2 + (vq >> 2)) * 256 + vd * 16 + (vq & 3) * 4;
+    } else {  // keys n, n + 1 of column m
+      off = OFF_V + (rt >> 1) * V_B + 2 * (c - 8) * 1024 + (rt & 1) * 512 + ow.word;
       step = 1024;
     }
   };
   auto po_s = [&](int split) { return OFF_PO + rt * PO_B + ((c & 56) + split) * 16384; };
-  auto st_s = [&]() { return OFF_ST + rt * ST_B + (c >> 3) * 1024; };
+  auto st_s = [&]() { return OFF_ST + rt * ST_B + (c >> 3) * 1024; };  // [pair of splits][row] of two (maximum, sum)
+  auto st_w = [&]() { return ((c & 7) >> 1) * 256 + (c & 1) * 8 + lane * 16; };  // lanes < 16
   auto att_s = [&]() { return OFF_ATT + rt * ATT_B + c * 1024; };
   auto x_s = [&]() { return rt * X_B + (c >> 1) * 1024 + (c & 1) * 512; };
-  auto ss_s = [&]() { return rt * X_B + KE * 1024 + c * 4; };
+  auto ss_s = [&]() { return rt * X_B + KE * 1024 + c * 64; };
   auto h_s = [&]() { return OFF_HF + rt * HF_B + 2 * c * 1024; };
   auto xt_s = [&]() { return OFF_XT + rt * XT_B + c * 64; };
 
-  float res0 = 0.f, res1 = 0.f;  // the residual stream: row m, columns 16 c + n, n + 1 (threads < 128)
+  float res0 = 0.f, res1 = 0.f;  // the residual stream: row m, columns 16 c + n, n + 1 (threads < 256)
   auto put_hidden = [&](const Own& ow, f32x2 s, int base) {
-    st_x(cx.rs, pack_bf16x2(res0 * (1.0f + s[0]), res1 * (1.0f + s[1])), ow.word, base + x_s());
-    const float ss = sum8(fmaf(res0, res0, res1 * res1));
-    if ((tid & 7) == 0) st_x(cx.rs, __float_as_uint(ss), ow.m * 256, base + ss_s());
+    if (ow.put) st_x(cx.rs, pack_bf16x2(res0 * (1.0f + s[0]), res1 * (1.0f + s[1])), ow.word, base + x_s());
+    const float ss = own_row_sum(fmaf(res0, res0, res1 * res1));
+    if (ow.put && ow.n == 0) st_x(cx.rs, __float_as_uint(ss), ow.m * 4, base + ss_s());
   };
   auto add_gated = [&](f32x2 y, f32x2 gate) {
     res0 = fmaf(y[0], gate[0], res0);
     res1 = fmaf(y[1], gate[1], res1);
   };
-  auto poison_hidden = [&](int base) {
-    const Own ow = own_of(tid);
-    st_x(cx.rs, 0xffffffffu, ow.word, base + x_s());
-    if ((tid & 7) == 0) st_x(cx.rs, 0xffffffffu, ow.m * 256, base + ss_s());
+  auto poison_hidden = [&](const Own& ow, int base) {
+    if (ow.put) st_x(cx.rs, 0xffffffffu, ow.word, base + x_s());
+    if (ow.put && ow.n == 0) st_x(cx.rs, 0xffffffffu, ow.m * 4, base + ss_s());
   };
   // the sums of squares of the 16 rows: an extra piece of the last four waves, 16 of the 64 column shares each
   auto ask_stats = [&](i32x4& st, int base) {
     const int k = wave - (kWaves - 4);
-    st = ld_x(cx.rs, lane_at(k >= 0, r * 256 + g * 16), base_at(k >= 0, base + rt * X_B + KE * 1024 + k * 64));
+    st = ld_x(cx.rs, lane_at(k >= 0, lane * 16), base_at(k >= 0, base + rt * X_B + KE * 1024 + k * 1024));
   };
   auto take_stats = [&](i32x4& st, int base) {
     const int k = wave - (kWaves - 4);
@@ -229,8 +227,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         pin();
         ask_stats(st, base);
       }
-      const float ss = row_sum(__int_as_float(st[0]) + __int_as_float(st[1]) + __int_as_float(st[2]) + __int_as_float(st[3]));
-      if (lane < 16) sq_s()[k * 16 + lane] = ss;
+      const float ss = share_sum(st);
+      if ((lane & 12) == 0) sq_s()[k * 16 + share_row(lane)] = ss;
     }
   };
   auto rstd_of = [&](int m) { return rsqrtf((sq_s()[m] + sq_s()[16 + m] + sq_s()[32 + m] + sq_s()[48 + m]) * (1.0f / E) + a.eps); };
@@ -246,8 +244,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
     wait_all<4>(v, cx, voff, soff);
   };
   // a rotary pair of two columns -> two words
-  auto rotate = [&](f32x2 va, f32x2 vb, unsigned& wa, unsigned& wb) {
-    const f32x2 cs = ((const f32x2*)(lds + L_ROPE + (tid & 127) * 16))[0], sn = ((const f32x2*)(lds + L_ROPE + (tid & 127) * 16))[1];
+  auto rotate = [&](f32x2 va, f32x2 vb, int slot, unsigned& wa, unsigned& wb) {
+    const f32x2 cs = ((const f32x2*)(lds + L_ROPE + slot * 16))[0], sn = ((const f32x2*)(lds + L_ROPE + slot * 16))[1];
     float ra[2], rb[2];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
@@ -266,9 +264,10 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int t = 0; t < 2; ++t) wA[t][i] = ld_w(wr, lane * 16, l * W_LAYER + W_QKV + ((2 * c + t) * KE + wave + 16 * i) * 1024);
-    const bool second = tid >= 128;  // (wave-uniform)
-    const int n4 = second && c >= 8 ? ((tid >> 2) & 15) * 4 : own_of(tid).n * 4;
-    const int share = __builtin_amdgcn_readfirstlane(second ? 64 + c : c);
+    const bool second = wave >= 4;
+    const Own ow = own_of(tid);
+    const int n4 = second && c >= 8 ? ow.m * 4 : ow.n * 4;
+    const int share = second ? 64 + c : c;
     bq0 = ld_f2_if(share < 80, mr, n4, ml + M_BQ + share * 128);
     bq1 = ld_f2_if(share < 80, mr, n4, ml + M_BQ + share * 128 + 64);
   };
@@ -291,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
     for (int i = 0; i < 4; ++i) wC[q][i] = ld_w(wr, lane * 16, l * W_LAYER + W_GU + (p * KE + (wave & 7) + 8 * i) * 1024);
   };
   auto load_CS = [&](int step, int l) {
-    const int ml = (step * (a.layers + 1) + l) * M_LAYER, f = 64 * ((tid >> 7) & 3) + own_of(tid).n * 4;
+    const int ml = (step * (a.layers + 1) + l) * M_LAYER, f = 64 * (wave >> 2) + own_of(tid).n * 4;
     scg = ld_f2(wr, f, l * W_LAYER + W_SG + 256 * c);
     scu = ld_f2(wr, f, l * W_LAYER + W_SU + 256 * c);
     bg = ld_f2(mr, f, ml + M_BG + 256 * c);
@@ -388,7 +387,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
     // ---------------- E1: action embedding ----------------
     fresh();
     announce(id_of(step, -1, PH_E1));
-    if (tid < 128) {
+    if (tid < 256) {
       const Own ow = own_of(tid);
       const f32x2 s = ld_f2(mr, ow.n * 4, step * (a.layers + 1) * M_LAYER + M_SIN + 64 * c);
       const f32x2 b = *(const f32x2*)(a.emb_b + 16 * c + ow.n);
@@ -422,41 +421,36 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         announce(id_of(step, l, PH_P1));
         f32x4 acc[4];
 #pragma unroll
-        for (int t = 0; t < 4; ++t) acc[t] = mfma(wA[t][1], x[1], mfma(wA[t][0], x[0], f32x4{0.f, 0.f, 0.f, 0.f}));
+        for (int t = 0; t < 4; ++t) {
+          const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+          // (V^T: the operands swapped, a lane then owns a column and four consecutive keys)
+          acc[t] = t >= 2 && c >= 8 ? mfma(x[1], wA[t][1], mfma(x[0], wA[t][0], z)) : mfma(wA[t][1], x[1], mfma(wA[t][0], x[0], z));
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t)
-          if (t < 2 || c < 16) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = acc[t];
+          if (t < 2 || c < 16) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = acc[t];
         take_stats(st, in_base);
         load_V(l);
         block_barrier();
-        if (tid < 128 || (tid < 256 && c < 8)) {
+        if (wave < 4 || (wave < 8 && c < 16)) {
           const Own ow = own_of(tid);
-          const float rstd = rstd_of(ow.m);
-          const int t = tid < 128 ? 0 : 2;
-          const f32x2 va = sum_part<16, 4, 8>(part(), 0, t, ow.off) * rstd + bq0, vb = sum_part<16, 4, 8>(part(), 0, t + 1, ow.off) * rstd + bq1;
+          const int t = wave < 4 ? 0 : 2;
+          const f32x2 va = sum_part<16, 4>(part(), 0, t, ow), vb = sum_part<16, 4>(part(), 0, t + 1, ow);
           unsigned wa, wb;
-          rotate(va, vb, wa, wb);
+          if (t == 0 || c < 8) {
+            const float rstd = rstd_of(ow.m);
+            rotate(va * rstd + bq0, vb * rstd + bq1, ow.m * 8 + (ow.n >> 1), wa, wb);
+          } else {
+            const float r0 = rstd_of(ow.n), r1 = rstd_of(ow.n + 1);
+            wa = pack_bf16x2(va[0] * r0 + bq0[0], va[1] * r1 + bq0[0]);
+            wb = pack_bf16x2(vb[0] * r0 + bq1[0], vb[1] * r1 + bq1[0]);
+          }
           int off = ow.word + q_s(), d = 4096;
-          if (t) kv_off(off, d);
-          st_x(cx.rs, wa, off, base);
-          st_x(cx.rs, wb, off + d, base);
-        } else if (tid < 256 && c < 16) {
-          // V^T words: rows 2 vq, 2 vq + 1 of column vd of both tiles
-          const int vq = ((tid >> 6) & 1) * 4 + (tid & 3), vd = (tid >> 2) & 15;
-          const int o0 = ((vd >> 2) * 16 + 2 * vq) * 16 + (vd & 3) * 4;
-          float s[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-#pragma unroll 2
-          for (int w2 = 0; w2 < 16; ++w2)
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-              s[t][0] += *(const float*)(part() + (w2 * 4 + 2 + t) * 1024 + o0);
-              s[t][1] += *(const float*)(part() + (w2 * 4 + 2 + t) * 1024 + o0 + 16);
-            }
-          const float r0 = rstd_of(2 * vq), r1 = rstd_of(2 * vq + 1);
-          int off, d;
-          kv_off(off, d);
-          st_x(cx.rs, pack_bf16x2(s[0][0] * r0 + bq0[0], s[0][1] * r1 + bq0[0]), off, base);
-          st_x(cx.rs, pack_bf16x2(s[1][0] * r0 + bq1[0], s[1][1] * r1 + bq1[0]), off + d, base);
+          if (t) kv_off(ow, off, d);
+          if (ow.put) {
+            st_x(cx.rs, wa, off, base);
+            st_x(cx.rs, wb, off + d, base);
+          }
         }
         buf ^= 1;
         pin();
@@ -527,9 +521,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         if (lane < 16) sM[wave * 16 + r] = tmax;
         block_barrier();
         announce(id_of(step, l, PH_P2));
-        float bm = sM[r];
-#pragma unroll
-        for (int w = 1; w < 2 * TILES; ++w) bm = fmaxf(bm, sM[w * 16 + r]);
+        static_assert(2 * TILES <= 12, "three tiles per lane (without keys: -inf)");
+        const float bm = max16(max32(fmaxf(fmaxf(sM[g * 16 + r], sM[(g + 4) * 16 + r]), sM[(g + 8) * 16 + r])));
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           p[e] = (vis >> (8 + e)) & 1u ? __expf(p[e] - bm) : 0.f;  // (a block without keys: bm is -inf)
@@ -552,12 +545,9 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
             if (tp + j >= t0 && tp + j < t1) o = mfma(vs[j], *(const i32x4*)(lds + L_P + (tp + j - t0) * 1024 + lane * 16), o);
         }
         st_x4(cx.rs, __builtin_bit_cast(i32x4, o), lane * 16, base + po_s(c & 7) + wave * 1024);
-        if (tid < 16) {
-          float s = 0.f;
-#pragma unroll
-          for (int w = 0; w < 2 * TILES; ++w) s += sL[w * 16 + tid];
-          st_x(cx.rs, __float_as_uint(bm), tid * 64 + (c & 7) * 8, base + st_s());
-          st_x(cx.rs, __float_as_uint(s), tid * 64 + (c & 7) * 8 + 4, base + st_s());
+        if (wave == 0) {
+          const float sum = row_sum(sL[g * 16 + r] + sL[(g + 4) * 16 + r] + sL[(g + 8) * 16 + r]);
+          if (lane < 16) st_x2(cx.rs, __float_as_uint(bm), __float_as_uint(sum), st_w(), base + st_s());
         }
         pin();
       }
@@ -566,7 +556,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
       {
         gate(0xffull << (c & 56), id_of(step, l, PH_P2));
         i32x4 v[2];
-        const int voff[2] = {lane * 16, r * 64 + g * 16};
+        const int voff[2] = {lane * 16, lane * 16};
         const int soff[2] = {base + po_s(wave >> 1) + (2 * (c & 7) + (wave & 1)) * 1024, base + st_s()};
         wait_x<2>(v, cx, voff, soff, [] {});
         arrived();
@@ -582,12 +572,12 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         const float e0 = __expf(m0 - mx), e1 = __expf(m1 - mx);
         const float sum = row_sum(e0 * l0 + e1 * l1);
         const float w = __shfl((wave >> 1) & 1 ? e1 : e0, (wave >> 2) * 16 + r) / sum;
-        *(f32x4*)(part() + wave * 1024 + lane * 16) = __builtin_bit_cast(f32x4, v[0]) * w;
+        *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = __builtin_bit_cast(f32x4, v[0]) * w;
         block_barrier();
-        if (tid < 256) {
+        if (tid < 512) {
           const Own ow = own_of(tid);
-          const f32x2 o = sum_part<8, 2>(part(), 0, tid >> 7, ow.off);
-          st_x(cx.rs, pack_bf16x2(o[0], o[1]), (tid >> 7) * 512 + ow.word, base + att_s());
+          const f32x2 o = sum_part<8, 2>(part(), 0, wave >> 2, ow);
+          if (ow.put) st_x(cx.rs, pack_bf16x2(o[0], o[1]), (wave >> 2) * 512 + ow.word, base + att_s());
         }
         buf ^= 1;
         pin();
@@ -606,11 +596,11 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc = mfma(wB[i], v[i], acc);
-        *(f32x4*)(part() + wave * 1024 + lane * 16) = acc;
+        *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = acc;
         block_barrier();
-        if (tid < 128) {
+        if (tid < 256) {
           const Own ow = own_of(tid);
-          add_gated(sum_part<16, 1, 8>(part(), 0, 0, ow.off), gin);
+          add_gated(sum_part<16, 1>(part(), 0, 0, ow), gin);
           put_hidden(ow, spost, base + OFF_X1);
         }
         buf ^= 1;
@@ -636,16 +626,17 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
             acc[2 * q + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp8x8_to_bf16x8(wC[q][i][2], wC[q][i][3]), as_bf16x8(v[i]), acc[2 * q + 1], 0, 0, 0);
           }
 #pragma unroll
-        for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = acc[t];
+        for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = acc[t];
         take_stats(st, base + OFF_X1);
         load_D(step, l);
         block_barrier();
-        if (tid < 512) {
+        {
           const Own ow = own_of(tid);
-          const int w0 = (tid >> 8) * 8, t = 2 * ((tid >> 7) & 1);
+          const int w0 = (wave >> 3) * 8, t = 2 * ((wave >> 2) & 1);
           const float rstd = rstd_of(ow.m);
-          const f32x2 gt = sum_part<8, 4>(part(), w0, t, ow.off) * rstd * scg + bg, up = sum_part<8, 4>(part(), w0, t + 1, ow.off) * rstd * scu + bu;
-          st_x(cx.rs, pack_bf16x2(gelu_tanh_f(gt[0]) * up[0], gelu_tanh_f(gt[1]) * up[1]), (tid >> 7) * 512 + ow.word, base + h_s());
+          const f32x2 gt = sum_part<8, 4>(part(), w0, t, ow) * rstd * scg + bg, up = sum_part<8, 4>(part(), w0, t + 1, ow) * rstd * scu + bu;
+          const unsigned h = pack_bf16x2(gelu_tanh_f(gt[0]) * up[0], gelu_tanh_f(gt[1]) * up[1]);
+          if (ow.put) st_x(cx.rs, h, (wave >> 2) * 512 + ow.word, base + h_s());
         }
         buf ^= 1;
         pin();
@@ -670,11 +661,11 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp8x8_to_bf16x8(wD[i >> 1][2 * (i & 1)], wD[i >> 1][2 * (i & 1) + 1]), as_bf16x8(v[i]), acc, 0, 0, 0);
-        *(f32x4*)(part() + wave * 1024 + lane * 16) = acc;
+        *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = acc;
         block_barrier();
-        if (tid < 128) {
+        if (tid < 256) {
           const Own ow = own_of(tid);
-          add_gated(sum_part<16, 1, 8>(part(), 0, 0, ow.off) * scd, gpost);
+          add_gated(sum_part<16, 1>(part(), 0, 0, ow) * scd, gpost);
           put_hidden(ow, snext, base + OFF_X2);
         }
         buf ^= 1;
@@ -688,27 +679,28 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
       fresh();
       if (step > 0 || l > 0) {
         const int ob = slot(l - 1);
-        if (tid < 128) {
-          const Own ow = own_of(tid);
-          st_x(cx.rs, ones, ow.word + q_s(), ob);
-          st_x(cx.rs, ones, ow.word + q_s() + 4096, ob);
-          poison_hidden(ob + OFF_X1);
-          poison_hidden(ob + OFF_X2);
-        } else if (tid < 256 && c < 16) {
+        const Own ow = own_of(tid);
+        if (tid < 256) {
+          if (ow.put) {
+            st_x(cx.rs, ones, ow.word + q_s(), ob);
+            st_x(cx.rs, ones, ow.word + q_s() + 4096, ob);
+          }
+          poison_hidden(ow, ob + OFF_X1);
+          poison_hidden(ow, ob + OFF_X2);
+        } else if (tid < 512 && c < 16) {
           int off, d;
-          kv_off(off, d);
-          st_x(cx.rs, ones, off, ob);
-          st_x(cx.rs, ones, off + d, ob);
+          kv_off(ow, off, d);
+          if (ow.put) {
+            st_x(cx.rs, ones, off, ob);
+            st_x(cx.rs, ones, off + d, ob);
+          }
         }
         st_x4(cx.rs, ones4, lane * 16, ob + po_s(c & 7) + wave * 1024);
-        if (tid < 16) {
-          st_x(cx.rs, ones, tid * 64 + (c & 7) * 8, ob + st_s());
-          st_x(cx.rs, ones, tid * 64 + (c & 7) * 8 + 4, ob + st_s());
-        }
+        if (tid < 16) st_x2(cx.rs, ones, ones, st_w(), ob + st_s());
         if (tid < 256) st_x(cx.rs, ones, tid * 4, ob + att_s());
         if (tid < 512) st_x(cx.rs, ones, tid * 4, ob + h_s());
         if (l == 0) {
-          if (tid < 128) poison_hidden(oth + OFF_HID);
+          if (tid < 256) poison_hidden(ow, oth + OFF_HID);
           if (c < A && tid < 16) st_x(cx.rs, ones, tid * 4, oth + xt_s());
         }
       }

@@ -24,8 +24,9 @@
 // weight, beside the row's partial sums of squares; 1 / rms is a factor of the whole row and multiplies the accumulator.
 // The residual stream never leaves its owner's registers and stays fp32 there.
 //
-// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.48 ms, against 4.7 ms of the launches per layer.
-// A layer takes 16 us (stamps of every block, mean): 1.2 - 2.0 us from a phase's result to the next one's input, and from
+// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.37 ms, against 4.7 ms of the launches per layer
+// (2.45 ms with two waves reducing and the rows' sums of squares exchanged row by row: persist.h).  A layer took 16 us then
+// (stamps of every block, mean): 1.2 - 2.0 us from a phase's result to the next one's input, and from
 // there to the result 2.8 us in the attention, 1.2 - 1.6 us in the others; in a cross layer's attention 5.2 us, 4.0 of them
 // until the scores are there: its blocks load 216 KiB (query weights, K and V hi + lo planes).  Where those are asked for
 // (the loop, ms): weights and K in front of the gate, V behind the query reduction's barrier 2.48; V in front of that
@@ -59,7 +60,7 @@ constexpr int W_QKV = 0, W_O = W_QKV + 2 * NQ * KE * 1024, W_GU = W_O + NE * KO 
 
 // exchange layout (bytes): per set a head (per row group: x, h, hidden and its sums of squares), then per layer Q, K, V,
 // attention output, hidden after attention, feed-forward intermediate, hidden (hidden rows with sums of squares)
-constexpr int SS_B = 16 * 48 * 4;  // partial sums of squares: [row][column share]
+constexpr int SS_B = 48 * 16 * 4;  // partial sums of squares: [column share][row]
 constexpr int XT_B = 2048, HE_B = NE * 1024, X_B = KE * 1024 + SS_B;
 constexpr int OFF_PW = 0, PW_B = 4 * kProgressBytes;  // progress words (one set only)
 constexpr int OFF_XT = 0, OFF_HE = OFF_XT + 4 * XT_B, OFF_HID = OFF_HE + 4 * HE_B, HEAD_B = OFF_HID + 4 * X_B;
@@ -75,7 +76,7 @@ constexpr int L_L = L_M + kWaves * 16 * 4;
 constexpr int L_XT = L_L + kWaves * 16 * 4;          // x_t [32][16]
 constexpr int L_WS = L_XT + A * 16 * 4;              // this block's rows of the suffix embedding [16][32]
 constexpr int L_Q = L_WS + 16 * A * 4;               // cross layers: the query tile in operand order
-constexpr int L_ROPE = L_Q + 2048;                   // (cos, sin) pairs of P1's (128) and of the cross q's (256) threads
+constexpr int L_ROPE = L_Q + 2048;                   // (cos, sin) pairs of P1's (128) and of the cross q's (256) column pairs
 constexpr int L_KV = L_ROPE + 384 * 16;              // prefix caches of every layer
 constexpr int LDS_B = L_KV + kSvMaxLayers * (int)sizeof(SvCache);
 
@@ -139,13 +140,13 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
 
   // ---- constants of the whole run ----
   if (tid < 384) {
-    // rotary factors: threads 0..127 P1 (columns 16 (c & 1) + n of a head half), 128..383 the cross q (16 u + n)
+    // rotary factors of row t / 8, columns n = 2 (t & 7) and the next: 0..127 P1 (columns 16 (c & 1) + n of a head half),
+    // 128..383 the cross q (16 u + n)
     const int t = tid < 128 ? tid : tid - 128;
-    const Own ow = own_of(t);
-    const int mg = rt * 16 + ow.m, mc = mg < a.M ? mg : a.M - 1;
+    const int mg = rt * 16 + ((t >> 3) & 15), mc = mg < a.M ? mg : a.M - 1;
     int p = tid < 128 ? a.pos[mc] : a.pos0[mc];
     p = p < 0 ? 0 : (p > a.positions - 1 ? a.positions - 1 : p);
-    const int f = 16 * (tid < 128 ? ((c < 60 ? (c == AT ? NQ - 1 : c) : c - 15) & 1) : t >> 7) + ow.n;
+    const int f = 16 * (tid < 128 ? ((c < 60 ? (c == AT ? NQ - 1 : c) : c - 15) & 1) : t >> 7) + 2 * (t & 7);
     f32x2* const o = (f32x2*)(lds + L_ROPE + tid * 16);
     o[0] = *(const f32x2*)(a.rope_cos + (size_t)p * (D / 2) + f);
     o[1] = *(const f32x2*)(a.rope_sin + (size_t)p * (D / 2) + f);
@@ -166,11 +167,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       const int set = i & 1;
       const int b = PW_B + set * set_b + (i < 2 ? OFF_HID : HEAD_B + ((i - 2) >> 2) * LAYER_B + ((i & 2) ? OFF_X1 : OFF_X2)) + rt * X_B;
       if (lane < 32) st_x4(cx.rs, z, lane * 16, b + (KE - 1) * 1024 + 512);
-      if (lane < 16) {
-        st_x(cx.rs, 0, lane * 192 + 180, b + KE * 1024);
-        st_x(cx.rs, 0, lane * 192 + 184, b + KE * 1024);
-        st_x(cx.rs, 0, lane * 192 + 188, b + KE * 1024);
-      }
+      if (lane < 48) st_x(cx.rs, 0, lane * 4, b + KE * 1024 + NE * 64);
     }
   }
   // visibility of this wave's prefix key tile: keys 8 g .. 8 g + 7 of it in this lane; bits 8..15: keys that exist
@@ -184,10 +181,9 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   }
 
   auto q_share = [&]() { return c < NE ? c : (c >= 60 ? c - 15 : (c == AT ? NQ - 1 : -1)); };
-  // where this thread's words of P1 go (relative to the layer's buffers): the two words of a rotary pair, or of a V^T pair
-  auto p1_off = [&](int& off0, int& step) {
+  // where this thread's words of P1 go (relative to the layer's buffers): the two words of a rotary pair, or of two V^T tiles
+  auto p1_off = [&](const Own& ow, int& off0, int& step) {
     const int u = q_share(), hh = u >> 1, uu = u & 1;
-    const Own ow = own_of(tid);
     if (hh < H) {
       off0 = OFF_Q + rt * Q_B + hh * 2048 + uu * 512 + ow.word;
       step = 1024;
@@ -195,37 +191,35 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       const int kk = (rt & 1) * 16 + ow.m, row = 4 * (kk >> 3) + (kk & 3), sub = (kk >> 2) & 1;
       off0 = OFF_K + (((hh - H) * 2 + (rt >> 1)) * 2 + sub) * 2048 + (2 * uu + (ow.n >> 3)) * 256 + row * 16 + (ow.n & 7) * 2;
       step = 1024;
-    } else {
-      const int vq = ((tid >> 6) & 1) * 4 + (tid & 3), vd = (tid >> 2) & 15;  // V^T: key pair and column of this thread
-      off0 = OFF_V + ((hh - H - G) * 2 + (rt >> 1)) * 4096 + uu * 1024 + ((rt & 1) * 2 + (vq >> 2)) * 256 + vd * 16 + (vq & 3) * 4;
+    } else {  // V^T: keys n, n + 1 of column m
+      off0 = OFF_V + ((hh - H - G) * 2 + (rt >> 1)) * 4096 + uu * 1024 + (rt & 1) * 512 + ow.word;
       step = 2048;
     }
   };
   // ... and of the other phases: scalar parts of the addresses
-  auto att_s = [&]() { return OFF_ATT + rt * ATT_B + 2 * (c - AT) * 1024; };       // P2: threads < 512
-  auto x_s = [&]() { return rt * X_B + (c >> 1) * 1024 + (c & 1) * 512; };  // E2 / P3 / P5: threads < 128
-  auto ss_s = [&]() { return rt * X_B + KE * 1024 + c * 4; };
-  auto h_s = [&]() { return OFF_HF + rt * HF_B + c * 1024; };               // P4: threads < 256
+  auto att_s = [&]() { return OFF_ATT + rt * ATT_B + 2 * (c - AT) * 1024; };       // P2
+  auto x_s = [&]() { return rt * X_B + (c >> 1) * 1024 + (c & 1) * 512; };  // E2 / P3 / P5: threads < 256
+  auto ss_s = [&]() { return rt * X_B + KE * 1024 + c * 64; };
+  auto h_s = [&]() { return OFF_HF + rt * HF_B + c * 1024; };               // P4: threads < 512
   auto he_s = [&]() { return OFF_HE + rt * HE_B + c * 1024; };              // E1: threads < 256
   auto xt_s = [&]() { return OFF_XT + rt * XT_B + c * 64; };                // E0: threads < 16
 
-  float res0 = 0.f, res1 = 0.f;  // the residual stream: row m, columns 16 c + n, n + 1 (threads < 128 of blocks < 45)
-  // hidden values of threads < 128 into an exchange buffer: times the next norm's weight, squares beside
+  float res0 = 0.f, res1 = 0.f;  // the residual stream: row m, columns 16 c + n, n + 1 (threads < 256 of blocks < 45)
+  // hidden values of threads < 256 into an exchange buffer: times the next norm's weight, squares beside
   auto put_hidden = [&](const Own& ow, f32x2 nw, int base) {
-    st_x(cx.rs, pack_bf16x2(res0 * nw[0], res1 * nw[1]), ow.word, base + x_s());
-    const float ss = sum8(fmaf(res0, res0, res1 * res1));
-    if ((tid & 7) == 0) st_x(cx.rs, __float_as_uint(ss), ow.m * 192, base + ss_s());
+    if (ow.put) st_x(cx.rs, pack_bf16x2(res0 * nw[0], res1 * nw[1]), ow.word, base + x_s());
+    const float ss = own_row_sum(fmaf(res0, res0, res1 * res1));
+    if (ow.put && ow.n == 0) st_x(cx.rs, __float_as_uint(ss), ow.m * 4, base + ss_s());
   };
-  auto poison_hidden = [&](int base) {
-    const Own ow = own_of(tid);
-    st_x(cx.rs, 0xffffffffu, ow.word, base + x_s());
-    if ((tid & 7) == 0) st_x(cx.rs, 0xffffffffu, ow.m * 192, base + ss_s());
+  auto poison_hidden = [&](const Own& ow, int base) {
+    if (ow.put) st_x(cx.rs, 0xffffffffu, ow.word, base + x_s());
+    if (ow.put && ow.n == 0) st_x(cx.rs, 0xffffffffu, ow.m * 4, base + ss_s());
   };
   // the sums of squares of the 16 rows of a hidden buffer into LDS: an extra piece of the last three waves, 16 of the 48
   // column shares each, asked for with the wave's share of the rows and looked at after it
   auto ask_stats = [&](i32x4& st, int base) {
     const int k = wave - (kWaves - 3);
-    st = ld_x(cx.rs, lane_at(k >= 0, r * 192 + g * 16), base_at(k >= 0, base + rt * X_B + KE * 1024 + k * 64));
+    st = ld_x(cx.rs, lane_at(k >= 0, lane * 16), base_at(k >= 0, base + rt * X_B + KE * 1024 + k * 1024));
   };
   auto take_stats = [&](i32x4& st, int base) {
     const int k = wave - (kWaves - 3);
@@ -239,8 +233,8 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         pin();
         ask_stats(st, base);
       }
-      const float ss = row_sum(__int_as_float(st[0]) + __int_as_float(st[1]) + __int_as_float(st[2]) + __int_as_float(st[3]));
-      if (lane < 16) sq_s()[k * 16 + lane] = ss;
+      const float ss = share_sum(st);
+      if ((lane & 12) == 0) sq_s()[k * 16 + share_row(lane)] = ss;
     }
   };
   auto rstd_of = [&](int m) { return rsqrtf((sq_s()[m] + sq_s()[16 + m] + sq_s()[32 + m]) * (1.0f / E) + a.eps); };
@@ -324,16 +318,10 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
 #pragma unroll
       for (int t = 0; t < 4; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (has) {
-        float bm[kWaves];
-#pragma unroll
-        for (int w = 0; w < kWaves; ++w) bm[w] = sM[w * 16 + r];
-#pragma unroll
-        for (int d = kWaves / 2; d > 0; d >>= 1)
-#pragma unroll
-          for (int w = 0; w < d; ++w) bm[w] = fmaxf(bm[w], bm[w + d]);
+        const float bm = max16(max32(fmaxf(fmaxf(sM[g * 16 + r], sM[(g + 4) * 16 + r]), fmaxf(sM[(g + 8) * 16 + r], sM[(g + 12) * 16 + r]))));
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-          p[e] = __expf(p[e] - bm[0]);
+          p[e] = __expf(p[e] - bm);
           ls += p[e];
         }
         ls = row_sum(ls);
@@ -357,21 +345,15 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       announce(id);
       if (lane < 16) sL[wave * 16 + r] = ls;
 #pragma unroll
-      for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = o[t];
+      for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = o[t];
     }
     block_barrier();
-    if (tid < 512) {
+    {
       const Own ow = own_of(tid);
-      const f32x2 o = sum_part<kWaves, 4>(part(), 0, tid >> 7, ow.off);
-      float ls[kWaves];
-#pragma unroll
-      for (int w = 0; w < kWaves; ++w) ls[w] = sL[w * 16 + ow.m];
-#pragma unroll
-      for (int d = kWaves / 2; d > 0; d >>= 1)
-#pragma unroll
-        for (int w = 0; w < d; ++w) ls[w] += ls[w + d];
-      const float inv = 1.0f / ls[0];
-      st_x(cx.rs, pack_bf16x2(o[0] * inv, o[1] * inv), (tid >> 7) * 512 + ow.word, base + att_s());
+      const f32x2 o = sum_part<kWaves, 4>(part(), 0, wave >> 2, ow);
+      const float* const l0 = sL + ow.from * 16 + ow.m;
+      const float inv = 1.0f / sum16(sum32((l0[0] + l0[8 * 16]) + (l0[4 * 16] + l0[12 * 16])));
+      if (ow.put) st_x(cx.rs, pack_bf16x2(o[0] * inv, o[1] * inv), (wave >> 2) * 512 + ow.word, base + att_s());
     }
     buf ^= 1;
   };
@@ -401,7 +383,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       wB[i] = ld_w_if(hid && s < KO, wr, lane * 16, wl + W_O + (c * KO + s) * 1024);
     }
     nwp = ld_f2_if(hid, wr, n4, wl + W_NPOST + 64 * c);
-    const int p = 2 * c + (wave >> 3), f = 64 * ((tid >> 7) & 1) + n4;
+    const int p = 2 * c + (wave >> 3), f = 64 * ((wave >> 2) & 1) + n4;
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       const int s = (wave & 7) + 8 * i;
@@ -424,40 +406,32 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
     arrived();
     announce(id);
     f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    const bool vt = (u >> 1) >= H + G;  // V^T: the operands swapped, a lane then owns a column and four consecutive keys
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-      for (int t = 0; t < 2; ++t) acc[t] = mfma(wA[t][i], x[i], acc[t]);
+      for (int t = 0; t < 2; ++t) acc[t] = vt ? mfma(x[i], wA[t][i], acc[t]) : mfma(wA[t][i], x[i], acc[t]);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) *(f32x4*)(part() + (wave * 2 + t) * 1024 + lane * 16) = acc[t];
+    for (int t = 0; t < 2; ++t) *(f32x4*)(part() + (wave * 2 + t) * 1024 + part_slot(cx)) = acc[t];
     take_stats(st, in_base);
     block_barrier();
-    if (tid < 128) {
-      int off0, step;
-      p1_off(off0, step);
-      if ((u >> 1) < H + G) {
-        const Own ow = own_of(tid);
+    if (tid < 256) {
+      const Own ow = own_of(tid);
+      f32x2 va = sum_part<16, 2>(part(), 0, 0, ow), vb = sum_part<16, 2>(part(), 0, 1, ow);
+      unsigned wa, wb2;
+      if (!vt) {
         const float rstd = rstd_of(ow.m);
-        const f32x2 va = sum_part<16, 2>(part(), 0, 0, ow.off) * rstd, vb = sum_part<16, 2>(part(), 0, 1, ow.off) * rstd;
-        unsigned wa, wb2;
-        rotate(va, vb, tid, wa, wb2);
+        rotate(va * rstd, vb * rstd, ow.m * 8 + (ow.n >> 1), wa, wb2);
+      } else {
+        const float r0 = rstd_of(ow.n), r1 = rstd_of(ow.n + 1);
+        wa = pack_bf16x2(va[0] * r0, va[1] * r1);
+        wb2 = pack_bf16x2(vb[0] * r0, vb[1] * r1);
+      }
+      int off0, step;
+      p1_off(ow, off0, step);
+      if (ow.put) {
         st_x(cx.rs, wa, off0, base);
         st_x(cx.rs, wb2, off0 + step, base);
-      } else {
-        // V^T words: rows 2 vq, 2 vq + 1 of column vd of both tiles
-        const int vq = ((tid >> 6) & 1) * 4 + (tid & 3), vd = (tid >> 2) & 15;
-        const int o0 = ((vd >> 2) * 16 + 2 * vq) * 16 + (vd & 3) * 4;
-        float s[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-#pragma unroll
-        for (int w2 = 0; w2 < 16; ++w2)
-#pragma unroll
-          for (int t = 0; t < 2; ++t) {
-            s[t][0] += *(const float*)(part() + (w2 * 2 + t) * 1024 + o0);
-            s[t][1] += *(const float*)(part() + (w2 * 2 + t) * 1024 + o0 + 16);
-          }
-        const float r0 = rstd_of(2 * vq), r1 = rstd_of(2 * vq + 1);
-        st_x(cx.rs, pack_bf16x2(s[0][0] * r0, s[0][1] * r1), off0, base);
-        st_x(cx.rs, pack_bf16x2(s[1][0] * r0, s[1][1] * r1), off0 + step, base);
       }
     }
     if (rest) load_rest(l);
@@ -561,10 +535,10 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(__int_as_float(wt[i][e]), __int_as_float(v[i][e]), acc, 0, 0, 0);
-      *(f32x4*)(part() + wave * 1024 + lane * 16) = acc;
+      *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = acc;
       block_barrier();
-      if (tid < 128) {
-        const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow.off);
+      if (tid < 256) {
+        const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow);
         res0 = s[0] + tb[0];
         res1 = s[1] + tb[1];
         put_hidden(ow, nw, cur + OFF_HID);
@@ -642,21 +616,23 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) acc[t] = mfma(w[t][1], x[1], mfma(w[t][0], x[0], f32x4{0.f, 0.f, 0.f, 0.f}));
 #pragma unroll
-        for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + lane * 16) = acc[t];
+        for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = acc[t];
         take_stats(st, in_base);
         block_barrier();
         load_V(vf, l, false);
         load_V(vl, l, true);
         pin();
-        if (tid < 256) {
+        if (tid < 512) {
           const Own ow = own_of(tid);
           const float rstd = rstd_of(ow.m);
-          const int u = tid >> 7;
-          const f32x2 va = sum_part<16, 4, 4>(part(), 0, u, ow.off) * rstd, vb = sum_part<16, 4, 4>(part(), 0, 2 + u, ow.off) * rstd;
+          const int u = wave >> 2;
+          const f32x2 va = sum_part<16, 4>(part(), 0, u, ow) * rstd, vb = sum_part<16, 4>(part(), 0, 2 + u, ow) * rstd;
           unsigned wa, wb2;
-          rotate(va, vb, 128 + tid, wa, wb2);
-          *(unsigned*)(lds + L_Q + u * 512 + ow.word) = wa;
-          *(unsigned*)(lds + L_Q + 1024 + u * 512 + ow.word) = wb2;
+          rotate(va, vb, 128 + u * 128 + ow.m * 8 + (ow.n >> 1), wa, wb2);
+          if (ow.put) {
+            *(unsigned*)(lds + L_Q + u * 512 + ow.word) = wa;
+            *(unsigned*)(lds + L_Q + 1024 + u * 512 + ow.word) = wb2;
+          }
         }
         buf ^= 1;
         block_barrier();
@@ -677,10 +653,10 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         arrived();
         announce(id_of(step, l, PH_P3));
         const f32x4 acc = mfma(wB[1], v[1], mfma(wB[0], v[0], f32x4{0.f, 0.f, 0.f, 0.f}));
-        *(f32x4*)(part() + wave * 1024 + lane * 16) = acc;
+        *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = acc;
         block_barrier();
-        if (tid < 128) {
-          const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow.off);
+        if (tid < 256) {
+          const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow);
           res0 = s[0] + res0;
           res1 = s[1] + res1;
           put_hidden(ow, nwp, base + OFF_X1);
@@ -715,18 +691,18 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
           acc[1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wu[i], as_bf16x8(v[i]), acc[1], 0, 0, 0);
         }
 #pragma unroll
-        for (int t = 0; t < 2; ++t) *(f32x4*)(part() + (wave * 2 + t) * 1024 + lane * 16) = acc[t];
+        for (int t = 0; t < 2; ++t) *(f32x4*)(part() + (wave * 2 + t) * 1024 + part_slot(cx)) = acc[t];
         take_stats(st, base + OFF_X1);
         block_barrier();
-        if (tid < 256) {
+        if (tid < 512) {
           const Own ow = own_of(tid);
-          const int w0 = (tid >> 7) * 8;
+          const int pair = wave >> 2;
           const float rstd = rstd_of(ow.m);
-          const f32x2 gt = sum_part<8, 2>(part(), w0, 0, ow.off) * rstd * scg, up = sum_part<8, 2>(part(), w0, 1, ow.off) * rstd * scu;
+          const f32x2 gt = sum_part<8, 2>(part(), 8 * pair, 0, ow) * rstd * scg, up = sum_part<8, 2>(part(), 8 * pair, 1, ow) * rstd * scu;
           float h[2];
 #pragma unroll
           for (int j = 0; j < 2; ++j) h[j] = silu_f(gt[j]) * up[j];
-          st_x(cx.rs, pack_bf16x2(h[0], h[1]), (tid >> 7) * 512 + ow.word, base + h_s());
+          if (ow.put) st_x(cx.rs, pack_bf16x2(h[0], h[1]), pair * 512 + ow.word, base + h_s());
         }
         buf ^= 1;
       }
@@ -752,10 +728,10 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wd[i], as_bf16x8(v[i]), acc, 0, 0, 0);
-        *(f32x4*)(part() + wave * 1024 + lane * 16) = acc;
+        *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = acc;
         block_barrier();
-        if (tid < 128) {
-          const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow.off) * scd;
+        if (tid < 256) {
+          const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow) * scd;
           res0 = s[0] + res0;
           res1 = s[1] + res1;
           put_hidden(ow, nwd, base + OFF_X2);
@@ -765,18 +741,21 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       // ---------------- the idle set: this layer's words were read a step ago, back to all ones ----------------
       const unsigned ones = 0xffffffffu;
       fresh();
-      if (tid < 128) {
+      if (tid < 256) {
+        const Own ow = own_of(tid);
         if (!cross && q_share() >= 0) {
           int off0, pstep;
-          p1_off(off0, pstep);
-          st_x(cx.rs, ones, off0, obase);
-          st_x(cx.rs, ones, off0 + pstep, obase);
+          p1_off(ow, off0, pstep);
+          if (ow.put) {
+            st_x(cx.rs, ones, off0, obase);
+            st_x(cx.rs, ones, off0 + pstep, obase);
+          }
         }
         if (c < NE) {
-          poison_hidden(obase + OFF_X1);
+          poison_hidden(ow, obase + OFF_X1);
           // (the closing layer's hidden rows of the idle set are read by this step's E0: they have been by now)
-          poison_hidden(obase + OFF_X2);
-          if (l == 0) poison_hidden(oth + OFF_HID);
+          poison_hidden(ow, obase + OFF_X2);
+          if (l == 0) poison_hidden(ow, oth + OFF_HID);
         }
       }
       if (c >= AT && c < AT + H && tid < 512) st_x(cx.rs, ones, tid * 4, obase + att_s());

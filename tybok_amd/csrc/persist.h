@@ -46,6 +46,10 @@ __device__ __forceinline__ i32x4 ld_x(rsrc_t rs, int voff, int soff) {
   return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, kCoherent));
 }
 __device__ __forceinline__ void st_x(rsrc_t rs, unsigned v, int voff, int soff) { __builtin_amdgcn_raw_buffer_store_b32(v, rs, voff, soff, kCoherent); }
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void st_x2(rsrc_t rs, unsigned v0, unsigned v1, int voff, int soff) {
+  __builtin_amdgcn_raw_buffer_store_b64(u32x2{v0, v1}, rs, voff, soff, kCoherent);
+}
 __device__ __forceinline__ void st_x4(rsrc_t rs, i32x4 v, int voff, int soff) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), rs, voff, soff, kCoherent);
@@ -172,47 +176,73 @@ __device__ __forceinline__ f32x2 ld_f2_if(bool here, rsrc_t rs, int voff, int so
 __device__ __forceinline__ float row_sum(float v) {
   return sum32(sum16(v));
 }
-// sum over eight consecutive lanes (in registers: quad permutes, then the mirror of each half row)
-__device__ __forceinline__ float sum8(float v) {
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));   // lane ^ 1
-  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4e, 0xf, 0xf, true));   // lane ^ 2
-  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x141, 0xf, 0xf, true));  // 7 - lane
-}
-
-// ---- reduction of the waves' partial tiles through LDS: partials lie as [wave][tile][lane] float4; thread t of 128 owns
-// row m = t / 8 and two columns n, n + 1 of a 16 x 16 tile ----
+// ---- reduction of the waves' partial tiles through LDS ----
+// Partials lie as [wave][tile] of 1 KiB, accumulator lane (g, r) -- row r, columns 4 g .. 4 g + 3 -- at part_slot.  Four waves
+// reduce a tile, four rows each: lane = 32 h + 16 d + 4 i + j adds up row 4 (wave & 3) + i, columns 4 j .. 4 j + 3 of every
+// fourth partial (of 2 h + d on) and ends with columns 4 j + 2 h and the next; the two lanes d = 0, 1 end with the same, d = 0 stores.
+// Bound: the chain of LDS reads behind the barrier, and what the stores look like to the memory.  Measured in rounds of the
+// hand-off alone (MI355X, 32 KiB a group): two waves adding up sixteen partials of two columns 1.62 us, this split 1.37 (the
+// reads are 128 bits without bank conflicts and a quarter as many in a row); eight waves, whose stores cover 32 bytes of a line
+// each, 1.92.
+__device__ __forceinline__ int part_slot(const Ctx& cx) { return (cx.g * 16 + (cx.r ^ (4 * cx.g))) * 16; }
 struct Own {
-  int m, n;  // row and first of two columns within the tile
-  int off;   // byte offset of the two partial sums within a partial tile
-  int word;  // byte offset of the two bf16 results within the tile's half of an exchange piece
+  int m, n;   // row and first of two columns within the tile
+  int src;    // byte offset of the row's four columns within a partial tile
+  int word;   // byte offset of the two bf16 results within the tile's half of an exchange piece
+  int from;   // the first partial this lane adds up
+  bool put;   // of the two lanes with the same result the one that stores
 };
 __device__ __forceinline__ Own own_of(int t) {
-  const int dw = t & 3, chunk = (t >> 2) & 1;
+  const int j = t & 3, h = (t >> 5) & 1;
   Own o;
-  o.m = (t >> 3) & 15;
-  o.n = chunk * 8 + 2 * dw;
-  o.off = ((chunk * 2 + (dw >> 1)) * 16 + o.m) * 16 + (dw & 1) * 8;
-  o.word = chunk * 256 + o.m * 16 + dw * 4;
+  o.m = ((t >> 6) & 3) * 4 + ((t >> 2) & 3);
+  o.n = 4 * j + 2 * h;
+  o.src = (j * 16 + (o.m ^ (4 * j))) * 16;
+  o.word = (j >> 1) * 256 + o.m * 16 + (j & 1) * 8 + h * 4;
+  o.from = (t >> 4) & 3;
+  o.put = (t & 16) == 0;
   return o;
 }
-// waves w0 .. w0 + KG - 1, tile `tile` of NT per wave; BATCH partials on the way at a time
-template <int KG, int NT, int BATCH = KG>
-__device__ __forceinline__ f32x2 sum_part(const unsigned char* p, int w0, int tile, int off) {
-  f32x2 s = {0.f, 0.f};
-#pragma unroll
-  for (int b = 0; b < KG; b += BATCH) {
-    f32x2 v[BATCH];
-#pragma unroll
-    for (int w = 0; w < BATCH; ++w) v[w] = *(const f32x2*)(p + ((w0 + b + w) * NT + tile) * 1024 + off);
-#pragma unroll
-    for (int d = BATCH / 2; d > 0; d >>= 1)
-#pragma unroll
-      for (int w = 0; w < d; ++w) v[w] += v[w + d];
-    s = b == 0 ? v[0] : s + v[0];
-    if (BATCH < KG) pin();
-  }
-  return s;
+// a's sum over the lanes l, l ^ 32 in the lower half of the wave, b's in the upper; the same for l, l ^ 16 and its even and odd rows
+__device__ __forceinline__ float fold32(float a, float b) {
+  const u32x2 s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
 }
+__device__ __forceinline__ float fold16(float a, float b) {
+  const u32x2 s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+// waves w0 .. w0 + KG - 1, tile `tile` of NT per wave
+template <int KG, int NT>
+__device__ __forceinline__ f32x2 sum_part(const unsigned char* p, int w0, int tile, const Own& o) {
+  constexpr int N = KG / 4;
+  f32x4 v[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = *(const f32x4*)(p + ((w0 + o.from + 4 * i) * NT + tile) * 1024 + o.src);
+#pragma unroll
+  for (int d = N / 2; d > 0; d >>= 1)
+#pragma unroll
+    for (int i = 0; i < d; ++i) v[i] += v[i + d];
+  return f32x2{sum16(fold32(v[0][0], v[0][2])), sum16(fold32(v[0][1], v[0][3]))};
+}
+// the sum over a row's sixteen columns of what its lanes hold, in all of them
+__device__ __forceinline__ float own_row_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xb1, 0xf, 0xf, true));  // lane ^ 1
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x4e, 0xf, 0xf, true));  // lane ^ 2
+  return sum32(v);
+}
+
+// ---- sums of squares of the rows: exchanged as [column share][16 rows] floats.  A share's 64 bytes come from one block; as
+// [row][column share] every block wrote four bytes of every row's lines, and a hand-off with the sums beside its rows took
+// 2.19 us alone, against 1.62 without them and 1.36 in this order.  Sixteen shares are a wave's KiB; st: its 16 bytes of lane l,
+// share l / 4, rows 4 (l & 3) .. + 3.  The row whose sum the lane ends with (the same in four lanes): share_row ----
+__device__ __forceinline__ float share_sum(i32x4 st) {
+  float v = fold16(fold32(__int_as_float(st[0]), __int_as_float(st[2])), fold32(__int_as_float(st[1]), __int_as_float(st[3])));
+  v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x128, 0xf, 0xf, true));         // lane ^ 8
+  return v + __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x124, 0xf, 0xf, true));  // lane + 4
+}
+__device__ __forceinline__ int share_row(int lane) { return 4 * (lane & 3) + 2 * (lane >> 5) + ((lane >> 4) & 1); }
+
 __device__ __forceinline__ void block_barrier() {
   // LDS traffic only: global loads stay in flight
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
