@@ -4,10 +4,9 @@
 // Bound: latency, then the bytes a compute unit takes in.  A step reads 397 MB of weights (80 us at 5 TB/s) and its
 // eighteen layers are 108 dependent phases of 0.3 - 1.5 us of work each; as five launches a layer they took 47 us a layer.
 // Here 256 resident blocks run the phases back to back: block (rt, c) works on 16 of the chunk's rows with column share c
-// of 64.  Measured (50 action tokens, two cameras and 200 language tokens, 10 steps): the loop 8.5 -> 4.4 ms with weights
-// asked for at the ends of the phases (24 us a layer; stamps of every block, mean: 1.7 - 2.4 us from a phase's result to
-// the next one's input, 3.8 us into PC behind 128 KiB of weights; from there to the result 0.75 us in PC, 1.0 - 2.1 us in
-// the others), 3.9 ms (21 us) as below; 0.8 MB through each compute unit.
+// of 64.  Measured (50 action tokens, two cameras and 200 language tokens, 10 steps): the loop 8.5 -> 3.44 ms (19 us a layer;
+// stamps of every block, mean: 0.6 - 1.5 us from a phase's result to the next one's first input, 0.6 - 1.5 us until all of a
+// block's input is there, from there to the result 0.7 - 1.4 us); 0.8 MB through each compute unit.
 //
 //   step    E0  v = final_norm(x) . Wa^T + b, x_t += dt v         32 blocks per row group, one action column each
 //           E1  hidden = x_t . Wi^T + b                           64 blocks, 16 columns each
@@ -24,15 +23,18 @@
 // Place: blocks land round-robin on the eight XCDs, so block i = 64 rt + c puts the row groups' blocks of one column share
 // on one XCD: the weights, which are too many for any cache above the XCD's, come there once for four blocks, and a
 // key split for 32.  A row group on two XCDs of its own (hand-offs 0.3 us shorter) took 2 us a layer more.
-// Weights and keys ahead: loads that the memory pipe still works on stand before the next hand-off's looks, so each set is
-// asked for where the fewest of them are on that path (the loop with three cameras, ms).
-//   * Between a phase's products and the barrier of its reduction: the values in P1 (3.90; at its arrival 4.00, at the end
-//     of P5 4.11), P5's weights in P4 (3.90; behind the barrier 4.05, at the arrival 4.01, at the end of P3 4.05).
-//   * At PC's arrival: P3's weights (at the end of P2 with half of P4's, 128 KiB stood in front of PC's input: 4.45 -> 4.28;
-//     in front of PC's barrier 4.18 against 4.11).
-//   * At a phase's end: the keys (P1), P4's weights (PC), P1's (P4; anywhere in P5 0.3 - 0.6 more).
+// Weights and keys ahead: loads that the memory pipe still works on stand before the next hand-off's data, so each set is
+// asked for where the fewest of them are on that path (the loop, us; first figure: as below).
+//   * The keys at P1's end; the values behind the query's arrival in P2 3463 (behind P1's products 3489, at P1's end 3584; the
+//     keys in front of P1's barrier 3707, at its input 3787).
+//   * P3's weights at PC's input 3538 (in P2 3600).  P4's: half at PC's end, half at P3's input 3493 (all at PC's end 3558, at
+//     P3's input 3668; the first half at PC's input 3659).
+//   * P5's between P4's products and the barrier of its reduction 3558 (behind it 3714, at P4's input 3596).
+//   * P1's at P4's end 3805 (in P5 4017).
+// P4's and P5's weights are asked for as data that is read once: a step's weights are more than the memory-side cache holds,
+// and the others' then stay there (3550 -> 3517; P1's and P3's instead 3832, all 4073, against 3805).
 // With all weights in the XCD's L2 already it would be 0.4 less, but touching them there ahead of time (a load per line, by
-// waves that wait at a gate) costs 0 - 0.25.  128 registers a wave is what holds them: loads under a branch, or carried
+// waves that wait at a gate) costs 0 - 0.25, through the scalar cache 0.4 - 0.6.  128 registers a wave is what holds them: loads under a branch, or carried
 // into the next layer under one, were spilled as they arrived (31 us a layer).
 // Keys: one block per head would read 780 KiB; eight splits of at most five tiles of 32 keys keep that at 96 KiB (two
 // cameras).
@@ -127,7 +129,8 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
     if (tid == 0) st_x(cx.rs, (unsigned)id, 0, rt * kProgressBytes + c * 128);
   };
   auto gate = [&](unsigned long long who, int id) {
-    if (wave == kWaves - 1) watch(cx, rt * kProgressBytes, (who >> lane) & 1, id);
+    const unsigned mine = wave < 4 ? (unsigned)(who >> (16 * wave)) & 0xffff : 0;
+    if (mine) watch<16>(cx, (const char*)a.xchg + rt * kProgressBytes + wave * 2048, mine, id);
     block_barrier();
   };
   constexpr unsigned long long kAll = ~0ull, kAct = (1ull << A) - 1;
@@ -287,7 +290,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
   auto load_C = [&](int l, int q) {
     const int p = 4 * c + 2 * (wave >> 3) + q;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wC[q][i] = ld_w(wr, lane * 16, l * W_LAYER + W_GU + (p * KE + (wave & 7) + 8 * i) * 1024);
+    for (int i = 0; i < 4; ++i) wC[q][i] = ld_once(wr, lane * 16, l * W_LAYER + W_GU + (p * KE + (wave & 7) + 8 * i) * 1024);
   };
   auto load_CS = [&](int step, int l) {
     const int ml = (step * (a.layers + 1) + l) * M_LAYER, f = 64 * (wave >> 2) + own_of(tid).n * 4;
@@ -299,7 +302,7 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
   auto load_D = [&](int step, int l) {
     const int ml = (step * (a.layers + 1) + l) * M_LAYER, n4 = own_of(tid).n * 4;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) wD[i] = ld_w(wr, lane * 16, l * W_LAYER + W_D + (c * (KF / 2) + wave + 16 * i) * 1024);
+    for (int i = 0; i < 4; ++i) wD[i] = ld_once(wr, lane * 16, l * W_LAYER + W_D + (c * (KF / 2) + wave + 16 * i) * 1024);
     scd = ld_f2(wr, n4, l * W_LAYER + W_SD + 64 * c);
     gpost = ld_f2(mr, n4, ml + M_GPOST + 64 * c);
     snext = ld_f2(mr, n4, ml + M_LAYER + M_SIN + 64 * c);  // the norm that reads P5's rows
@@ -430,7 +433,6 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         for (int t = 0; t < 4; ++t)
           if (t < 2 || c < 16) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = acc[t];
         take_stats(st, in_base);
-        load_V(l);
         block_barrier();
         if (wave < 4 || (wave < 8 && c < 16)) {
           const Own ow = own_of(tid);
@@ -467,6 +469,9 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
           wait_x<1>(q, cx, voff, soff, [] {});
           *(i32x4*)(lds + L_Q + wave * 1024 + lane * 16) = q[0];
         }
+        pin();
+        load_V(l);
+        pin();
         const int t = t0 + (wave >> 1);
         // the action tokens' own keys and values: 16 keys are the rows of one row group (one that does not exist: repeat)
         i32x4 vs[2];
@@ -583,7 +588,6 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         pin();
         load_C(l, 0);
         load_CS(step, l);
-        load_C(l, 1);
       }
       // ---------------- P3: output projection, gated residual ----------------
       fresh();
@@ -593,6 +597,9 @@ __global__ __launch_bounds__(kThreads) void pi_denoise_kernel(PiDenoiseArgs a) {
         wait_pieces(v, base + OFF_ATT + rt * ATT_B, wave, 16);
         arrived();
         announce(id_of(step, l, PH_P3));
+        pin();
+        load_C(l, 1);
+        pin();
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) acc = mfma(wB[i], v[i], acc);

@@ -24,13 +24,18 @@
 // weight, beside the row's partial sums of squares; 1 / rms is a factor of the whole row and multiplies the accumulator.
 // The residual stream never leaves its owner's registers and stays fp32 there.
 //
-// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 2.37 ms, against 4.7 ms of the launches per layer
-// (2.45 ms with two waves reducing and the rows' sums of squares exchanged row by row: persist.h).  A layer took 16 us then
-// (stamps of every block, mean): 1.2 - 2.0 us from a phase's result to the next one's input, and from
-// there to the result 2.8 us in the attention, 1.2 - 1.6 us in the others; in a cross layer's attention 5.2 us, 4.0 of them
-// until the scores are there: its blocks load 216 KiB (query weights, K and V hi + lo planes).  Where those are asked for
-// (the loop, ms): weights and K in front of the gate, V behind the query reduction's barrier 2.48; V in front of that
-// barrier 2.55, behind the next one 2.53, in front of the gate 2.75; K's lo plane or both behind the gate 2.53 - 2.65.
+// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 1.98 ms, against 4.7 ms of the launches per layer.
+// A self layer takes 13.5 us (stamps of every block, mean), a cross layer 12.4: five or four hand-offs of 0.6 - 1 us from a
+// phase's result to the next one's first input, 0.3 - 0.7 us until all of a block's input is there (64 bytes a cycle), and
+// from there to the result 0.6 us in P3 and P5, 1.0 in P1 and P4, 1.7 in the attention, 3.6 us in a cross layer's.
+// Where loads are asked for (the loop, us; first figure: as below):
+//   * P1's weights: at P4's end 2185; at the end of P3 2309, at P4's input 2218, in P5 2197.
+//   * The cross layers' values: between the query's reduction and its barrier 2240; in front of the reduction 2309, behind
+//     the barrier 2300.  Their query weights and K in front of the gate (K behind it 2366).
+//   * Everything else of a layer behind P1, in the attention's blocks behind the attention (P5's at P4 2108, P4's at P3 2109,
+//     against 2070).
+// When a block raises its progress word: in the attention behind its last barrier 1979 (in front of it 2068), in P3 with its
+// partial tiles written 1973 (at its input 1985), else when the input is there (P1 behind its barrier 1996).
 #include <math.h>
 
 #include <atomic>
@@ -108,7 +113,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   auto part = [&]() { return lds + buf * PART_B; };
   auto sq_s = [&]() { return ldsf + L_RS / 4 + buf * 48; };
 
-  // progress: phase ids grow along the run; `announce` when this block's input of a phase is here, `gate` before asking
+  // progress: phase ids grow along the run; `announce` some time before this block's output of a phase leaves, `gate` before asking
   // for data that the blocks `from` .. (and the extra ones) produce in phase `id`
   enum { PH_E0, PH_E1, PH_E2, PH_P1, PH_P2, PH_P3, PH_P4, PH_P5 };
   auto id_of = [&](int step, int l, int ph) { return (step * (a.layers + 1) + l + 1) * 8 + ph; };  // E phases: l = -1
@@ -119,7 +124,8 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
     if (tid == 0) st_x(cx.rs, (unsigned)id, 0, OFF_PW + rt * kProgressBytes + c * 128);
   };
   auto gate = [&](unsigned long long who, int id) {
-    if (wave == kWaves - 1) watch(cx, OFF_PW + rt * kProgressBytes, (who >> lane) & 1, id);
+    const unsigned mine = wave < 8 ? (unsigned)(who >> (8 * wave)) & 0xff : 0;
+    if (mine) watch<8>(cx, (const char*)a.xchg + OFF_PW + rt * kProgressBytes + wave * 1024, mine, id);
     block_barrier();
   };
   constexpr unsigned long long kHid = (1ull << NE) - 1, kAtt = ((1ull << H) - 1) << AT, kAll = ~0ull, kQkv = kHid | (1ull << AT) | (15ull << 60),
@@ -342,12 +348,12 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
           }
         }
       }
-      announce(id);
       if (lane < 16) sL[wave * 16 + r] = ls;
 #pragma unroll
       for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = o[t];
     }
     block_barrier();
+    announce(id);
     {
       const Own ow = own_of(tid);
       const f32x2 o = sum_part<kWaves, 4>(part(), 0, wave >> 2, ow);
@@ -361,7 +367,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   // ---------------- P1: q | k | v ----------------
   // Weights.  Loads return in order, so a weight asked for shortly before a phase's input delays that input; and a layer's
   // weights asked for phase by phase come in bursts the fabric needs longer for than the phases last.  So P1's are asked
-  // for in P3 of the layer before, and the rest of a layer's behind P1 (behind the attention in its blocks): they arrive
+  // for in P4 of the layer before, and the rest of a layer's behind P1 (behind the attention in its blocks): they arrive
   // while the attention runs.
   i32x4 wA[2][2], wB[2], wC[3], wD[2];
   f32x2 nwp, scg, scu, scd, nwd;  // the next norm's weight (P3, P5), column scales
@@ -555,7 +561,11 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       fresh();
       if (c >= AT && c < AT + H && !cross) {
         // ---------------- P2: self attention (and the odd share of P1) ----------------
-        const int nw = tp + nsuf, h = c - AT;
+        // Keys of later rows are masked.  Only the step's first self layer waits for those of all row groups (what the step
+        // before left is overwritten behind it: nobody may be reading that still), the others for the rows up to their own
+        // (the loop 1984 -> 1969 us)
+        const bool sync = (~a.cross_mask & ((1u << l) - 1)) == 0;
+        const int last = sync ? 3 : rt, nw = tp + (sync ? nsuf : (rt >> 1) + 1), h = c - AT;
         i32x4 kf[2][2], vf[4], v[10];
         load_K(kf, l, false);
         load_V(vf, l, false);
@@ -566,7 +576,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
           // the query tile; for the waves behind the prefix also the action tokens' own keys: 32 of them are the rows of
           // two row groups (a group that does not exist: repeat)
           const int j = wave - tp, kvh = h / (H / G);
-          const bool own = wave >= tp && wave < nw, one = 16 * (2 * j + 1) >= a.M;
+          const bool own = wave >= tp && wave < nw, one = 16 * (2 * j + 1) >= a.M || 2 * j + 1 > last;
           const int rr = one ? (r & 7) : r, gg = one ? (g & 1) : g;
           int voff[10], soff[10];
 #pragma unroll
@@ -619,9 +629,6 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         for (int t = 0; t < 4; ++t) *(f32x4*)(part() + (wave * 4 + t) * 1024 + part_slot(cx)) = acc[t];
         take_stats(st, in_base);
         block_barrier();
-        load_V(vf, l, false);
-        load_V(vl, l, true);
-        pin();
         if (tid < 512) {
           const Own ow = own_of(tid);
           const float rstd = rstd_of(ow.m);
@@ -635,6 +642,9 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
           }
         }
         buf ^= 1;
+        load_V(vf, l, false);
+        load_V(vl, l, true);
+        pin();
         block_barrier();
         const i32x4 qb[2] = {*(const i32x4*)(lds + L_Q + lane * 16), *(const i32x4*)(lds + L_Q + 1024 + lane * 16)};
         attend(qb, kf, kl, vf, vl, base, id_of(step, l, PH_P2), std::true_type{}, tp);
@@ -651,9 +661,9 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         gate(kAtt, id_of(step, l, PH_P2));
         wait_tiles<2, KO>(v, cx, base + OFF_ATT + rt * ATT_B, wave, 16, [] {});
         arrived();
-        announce(id_of(step, l, PH_P3));
         const f32x4 acc = mfma(wB[1], v[1], mfma(wB[0], v[0], f32x4{0.f, 0.f, 0.f, 0.f}));
         *(f32x4*)(part() + wave * 1024 + part_slot(cx)) = acc;
+        announce(id_of(step, l, PH_P3));
         block_barrier();
         if (tid < 256) {
           const f32x2 s = sum_part<16, 1>(part(), 0, 0, ow);
@@ -661,10 +671,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
           res1 = s[1] + res1;
           put_hidden(ow, nwp, base + OFF_X1);
         }
-        load_A(l + 1, next_self);
         buf ^= 1;
-      } else {
-        load_A(l + 1, next_self);
       }
       // ---------------- P4: gate / up ----------------
       fresh();
@@ -704,6 +711,9 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
           for (int j = 0; j < 2; ++j) h[j] = silu_f(gt[j]) * up[j];
           if (ow.put) st_x(cx.rs, pack_bf16x2(h[0], h[1]), pair * 512 + ow.word, base + h_s());
         }
+        pin();
+        load_A(l + 1, next_self);
+        pin();
         buf ^= 1;
       }
       // ---------------- P5: down projection, residual ----------------

@@ -5,16 +5,21 @@
 // consumers load the data itself with device-coherent loads and look at it: a lane that still sees an all-ones word
 // asks again.  No flag, no counter, no cache flush and no wait for store acknowledgements: a hand-off costs one
 // store-to-load trip through the fabric.  Measured with rounds of this kind alone (256 blocks of 16 waves, four groups of
-// 64 that exchange 32 KiB among themselves, LDS reduction and barrier included): 1.6 us a round with the gate below, 2.4 us
-// without it, 2.35 us with acknowledged stores and a flag per block instead.  Buffers come in two sets, used by alternate denoising steps; a block rewrites its words of the idle
+// 64 that exchange 32 KiB among themselves, LDS reduction and barrier included): 1.37 us a round with a gate as below and the
+// reduction further down (1.6 as that was at first, and then 2.4 without the gate, 2.35 with acknowledged stores and a flag per
+// block instead).  Buffers come in two sets, used by alternate denoising steps; a block rewrites its words of the idle
 // set with ones one step after they were read (every path from "written" to "rewritten" runs through data that all
 // readers produced after their reads), so a word is always clean before it is used again.  (The pi0.5 loop keeps a ring
 // of four layers instead: a layer's words are rewritten at the end of the next one and used again two layers later.)
 //
 // GATE.  Loads that come back empty cost the compute unit's memory pipe as much as real ones, so nobody asks before
-// there is something to expect: every block keeps a progress word (a line of its own, ever growing) and raises it when its
-// input for a phase has ARRIVED, 0.8 - 2.8 us before its output leaves (5 us in the cross layers' attention); ONE wave of a consumer block watches its producers' words, the others
-// wait at the block's barrier, and the first look at the data usually succeeds.
+// there is something to expect: every block keeps a progress word (a line of its own, ever growing) and raises it 0.4 - 1 us
+// before a phase's output leaves; a few waves of a consumer block watch its producers' words, the others wait at the block's
+// barrier, and the first look at the data usually succeeds.  The watch goes through the scalar cache, which it empties before
+// each look: vector loads return in order, and behind the 64 - 128 KiB of weights that a block has on the way at any time a
+// look at a word took as long as those.  (SmolVLA's loop 2364 -> 2275 us, pi0.5's 3805 -> 3519; rounds alone with 128 KiB of
+// weights from memory 3.56 -> 3.29 us, without any 1.41 -> 1.52.)  A progress word is a hint: whoever has looked kLooks times
+// goes on and asks for the data.
 //
 // EVERY WAIT ENDS: a wave asks at most `spin` times, then marks itself dead, goes on with what it has (ones = NaN)
 // and never waits again, so the grid drains and the result holds NaNs, which the caller can see.  All blocks must be
@@ -69,27 +74,42 @@ __device__ __forceinline__ void pin() { asm volatile("" ::: "memory"); }
 
 // progress words of a row group: [64 blocks] at 128 bytes
 constexpr int kGroup = 64, kProgressBytes = kGroup * 128;
-__device__ __forceinline__ int ld_word(rsrc_t rs, int voff, int soff) {
-  return (int)__builtin_amdgcn_raw_buffer_load_b32(rs, voff, soff, kCoherent);
-}
-// until the words of the lanes with `mine` set have reached `id` (two looks on the way at any time)
-__device__ __forceinline__ void watch(Ctx& cx, int soff, bool mine, int id) {
-  const int voff = cx.lane * 128;
-  int u = ld_word(cx.rs, voff, soff);
-  __builtin_amdgcn_s_sleep(4);
-  pin();
-  int v = ld_word(cx.rs, voff, soff);
-  for (int n = 0;; ++n) {
-    if (__builtin_amdgcn_ballot_w64(mine && u < id) == 0 || cx.dead) break;
-    pin();
-    u = ld_word(cx.rs, voff, soff);
-    if (__builtin_amdgcn_ballot_w64(mine && v < id) == 0) break;
-    pin();
-    v = ld_word(cx.rs, voff, soff);
-    if (n >= cx.spin) {
-      cx.dead = 1;
-      break;
+constexpr int kLooks = 400;  // at most so many at the progress words: they only say when to ask for the data
+// Until the progress words of the N producers from `at` on have reached `id` (bit i of who: the i-th is one).
+// N, us of a loop: SmolVLA 2275 with eight words in each of the first eight waves, 2309 with sixteen in four; pi0.5 3454 and
+// 3442, 3550 with four words in all sixteen waves.  The first waves: the last ones instead, 2100 (SmolVLA) and 3505.
+template <int N>
+__device__ __forceinline__ void watch(const Ctx& cx, const char* at, unsigned who, int id) {
+  static_assert(N == 8 || N == 16, "words of one look");
+  at = uniform_ptr(at);
+  for (int n = 0; n < kLooks && n <= cx.spin && !cx.dead; ++n) {
+    int w[N];
+    if constexpr (N == 8) {
+      asm volatile(
+          "s_dcache_inv\n\t"
+          "s_load_dword %0, %8, 0x0\n\ts_load_dword %1, %8, 0x80\n\ts_load_dword %2, %8, 0x100\n\ts_load_dword %3, %8, 0x180\n\t"
+          "s_load_dword %4, %8, 0x200\n\ts_load_dword %5, %8, 0x280\n\ts_load_dword %6, %8, 0x300\n\ts_load_dword %7, %8, 0x380\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&s"(w[0]), "=&s"(w[1]), "=&s"(w[2]), "=&s"(w[3]), "=&s"(w[4]), "=&s"(w[5]), "=&s"(w[6]), "=&s"(w[7])
+          : "s"(at)
+          : "memory");
+    } else {
+      asm volatile(
+          "s_dcache_inv\n\t"
+          "s_load_dword %0, %16, 0x0\n\ts_load_dword %1, %16, 0x80\n\ts_load_dword %2, %16, 0x100\n\ts_load_dword %3, %16, 0x180\n\t"
+          "s_load_dword %4, %16, 0x200\n\ts_load_dword %5, %16, 0x280\n\ts_load_dword %6, %16, 0x300\n\ts_load_dword %7, %16, 0x380\n\t"
+          "s_load_dword %8, %16, 0x400\n\ts_load_dword %9, %16, 0x480\n\ts_load_dword %10, %16, 0x500\n\ts_load_dword %11, %16, 0x580\n\t"
+          "s_load_dword %12, %16, 0x600\n\ts_load_dword %13, %16, 0x680\n\ts_load_dword %14, %16, 0x700\n\ts_load_dword %15, %16, 0x780\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&s"(w[0]), "=&s"(w[1]), "=&s"(w[2]), "=&s"(w[3]), "=&s"(w[4]), "=&s"(w[5]), "=&s"(w[6]), "=&s"(w[7]),
+            "=&s"(w[8]), "=&s"(w[9]), "=&s"(w[10]), "=&s"(w[11]), "=&s"(w[12]), "=&s"(w[13]), "=&s"(w[14]), "=&s"(w[15])
+          : "s"(at)
+          : "memory");
     }
+    bool all = true;
+#pragma unroll
+    for (int i = 0; i < N; ++i) all = all && (!((who >> i) & 1) || w[i] >= id);
+    if (all) break;
   }
 }
 
@@ -165,6 +185,10 @@ __device__ __forceinline__ f32x4 mfma(i32x4 a, i32x4 b, f32x4 c) {
 // ---- weights: one blob per model in the order the kernel reads it, so that a load is one lane offset and scalars ----
 __device__ __forceinline__ i32x4 ld_w(rsrc_t rs, int voff, int soff) {
   return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0));
+}
+// the same for bytes that are not to push others out of the caches behind
+__device__ __forceinline__ i32x4 ld_once(rsrc_t rs, int voff, int soff) {
+  return __builtin_bit_cast(i32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 2));
 }
 __device__ __forceinline__ f32x2 ld_f2(rsrc_t rs, int voff, int soff) {
   return __builtin_bit_cast(f32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0));
