@@ -63,10 +63,15 @@ constexpr int W_QKV = 0, W_O = W_QKV + 2 * NQ * KE * 1024, W_GU = W_O + NE * KO 
               W_SG = W_D + NE * (KF / 2) * 1024, W_SU = W_SG + F * 4, W_SD = W_SU + F * 4, W_NIN = W_SD + E * 4, W_NPOST = W_NIN + E * 4,
               W_LAYER = (W_NPOST + E * 4 + 1023) / 1024 * 1024;
 
-// exchange layout (bytes): per set a head (per row group: x, h, hidden and its sums of squares), then per layer Q, K, V,
+// exchange layout (bytes): kSets sets, used by the steps in turn; per set a head (per row group: x, h, hidden and its sums of squares), then per layer Q, K, V,
 // attention output, hidden after attention, feed-forward intermediate, hidden (hidden rows with sums of squares)
 constexpr int SS_B = 48 * 16 * 4;  // partial sums of squares: [column share][row]
 constexpr int XT_B = 2048, HE_B = NE * 1024, X_B = KE * 1024 + SS_B;
+// A step rewrites the words of the step before with ones, and the keys and values of other row groups are the only words whose
+// writers a reader does not follow closely: it waits for all groups once a step (P2), so what it knows of one is that the step
+// before the last wait has ended there.  With three sets that is enough: a step reads words that were rewritten two steps ago.
+// With two a group that ran a whole step ahead could have read another's words of two steps ago.
+constexpr int kSets = 3;
 constexpr int OFF_PW = 0, PW_B = 4 * kProgressBytes;  // progress words (one set only)
 constexpr int OFF_XT = 0, OFF_HE = OFF_XT + 4 * XT_B, OFF_HID = OFF_HE + 4 * HE_B, HEAD_B = OFF_HID + 4 * X_B;
 constexpr int Q_B = H * 2048, KV_B = G * 2 * 4096, ATT_B = KO * 1024, HF_B = KF * 1024;
@@ -99,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   int rt = blockIdx.x >> 6, c = blockIdx.x & 63;
   if (rt * 16 >= a.M) return;
   const int set_b = HEAD_B + a.layers * LAYER_B;
-  cx.rs = make_rsrc(a.xchg, PW_B + 2u * (unsigned)set_b);
+  cx.rs = make_rsrc(a.xchg, PW_B + (unsigned)kSets * (unsigned)set_b);
   const rsrc_t wr = make_rsrc(a.blob, (unsigned)a.layers * W_LAYER + E * 4);
   int &tid = cx.tid, &lane = cx.lane, &wave = cx.wave, &g = cx.g, &r = cx.r;
   const int nsuf = (a.M + 31) >> 5, tp = (a.P + 31) >> 5;
@@ -169,12 +174,12 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
   // the half k tile behind the last hidden column, and the three unused sums of squares of a row, are zeros for good
   if (c == NE - 1) {
     const i32x4 z = {0, 0, 0, 0};
-    for (int i = wave; i < 2 * (1 + 2 * a.layers); i += kWaves) {
-      const int set = i & 1;
-      const int b = PW_B + set * set_b + (i < 2 ? OFF_HID : HEAD_B + ((i - 2) >> 2) * LAYER_B + ((i & 2) ? OFF_X1 : OFF_X2)) + rt * X_B;
-      if (lane < 32) st_x4(cx.rs, z, lane * 16, b + (KE - 1) * 1024 + 512);
-      if (lane < 48) st_x(cx.rs, 0, lane * 4, b + KE * 1024 + NE * 64);
-    }
+    for (int i = wave; i < 1 + 2 * a.layers; i += kWaves)
+      for (int set = 0; set < kSets; ++set) {
+        const int b = PW_B + set * set_b + (i == 0 ? OFF_HID : HEAD_B + ((i - 1) >> 1) * LAYER_B + ((i & 1) ? OFF_X1 : OFF_X2)) + rt * X_B;
+        if (lane < 32) st_x4(cx.rs, z, lane * 16, b + (KE - 1) * 1024 + 512);
+        if (lane < 48) st_x(cx.rs, 0, lane * 4, b + KE * 1024 + NE * 64);
+      }
   }
   // visibility of this wave's prefix key tile: keys 8 g .. 8 g + 7 of it in this lane; bits 8..15: keys that exist
   unsigned vis_in;
@@ -446,8 +451,8 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
 
   block_barrier();
 
-  for (int step = 0; step <= a.steps; ++step) {
-    const int cur = PW_B + (step & 1) * set_b, oth = PW_B + ((step + 1) & 1) * set_b;
+  int cur = PW_B, oth = PW_B + (kSets - 1) * set_b;  // this step's set and the one of the step before
+  for (int step = 0; step <= a.steps; ++step, oth = cur, cur = cur == PW_B + (kSets - 1) * set_b ? PW_B : cur + set_b) {
     // ---------------- E0: the previous step's velocity and Euler update ----------------
     fresh();
     if (step > 0) {
@@ -561,9 +566,8 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
       fresh();
       if (c >= AT && c < AT + H && !cross) {
         // ---------------- P2: self attention (and the odd share of P1) ----------------
-        // Keys of later rows are masked.  Only the step's first self layer waits for those of all row groups (what the step
-        // before left is overwritten behind it: nobody may be reading that still), the others for the rows up to their own
-        // (the loop 1984 -> 1969 us)
+        // Keys of later rows are masked.  Only the step's first self layer waits for those of all row groups (kSets), the others
+        // for the rows up to their own (the loop 1984 -> 1969 us)
         const bool sync = (~a.cross_mask & ((1u << l) - 1)) == 0;
         const int last = sync ? 3 : rt, nw = tp + (sync ? nsuf : (rt >> 1) + 1), h = c - AT;
         i32x4 kf[2][2], vf[4], v[10];
@@ -748,7 +752,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         }
         buf ^= 1;
       }
-      // ---------------- the idle set: this layer's words were read a step ago, back to all ones ----------------
+      // ---------------- the set of the step before: this layer's words were read, back to all ones ----------------
       const unsigned ones = 0xffffffffu;
       fresh();
       if (tid < 256) {
@@ -840,7 +844,7 @@ __global__ void fill_ones_kernel(i32x4* p, size_t n) {
 
 }  // namespace
 
-size_t tk_sv_denoise_exchange_bytes(int layers) { return PW_B + 2 * ((size_t)HEAD_B + (size_t)layers * LAYER_B); }
+size_t tk_sv_denoise_exchange_bytes(int layers) { return PW_B + kSets * ((size_t)HEAD_B + (size_t)layers * LAYER_B); }
 size_t tk_sv_denoise_blob_bytes() { return W_LAYER; }
 int tk_sv_denoise_max_key_tiles() { return kWaves; }
 

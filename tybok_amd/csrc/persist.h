@@ -7,9 +7,10 @@
 // store-to-load trip through the fabric.  Measured with rounds of this kind alone (256 blocks of 16 waves, four groups of
 // 64 that exchange 32 KiB among themselves, LDS reduction and barrier included): 1.37 us a round with a gate as below and the
 // reduction further down (1.6 as that was at first, and then 2.4 without the gate, 2.35 with acknowledged stores and a flag per
-// block instead).  Buffers come in two sets, used by alternate denoising steps; a block rewrites its words of the idle
-// set with ones one step after they were read (every path from "written" to "rewritten" runs through data that all
-// readers produced after their reads), so a word is always clean before it is used again.  (The pi0.5 loop keeps a ring
+// block instead).  Buffers come in sets, used by the denoising steps in turn; a block rewrites its words of the step
+// before with ones (every path from "written" to "rewritten" runs through data that all readers produced after their
+// reads), and a word is used again only where every path to its next reader runs through data that its writer produced
+// after the rewriting, so that nobody finds an old one.  (The pi0.5 loop keeps a ring
 // of four layers instead: a layer's words are rewritten at the end of the next one and used again two layers later.)
 //
 // GATE.  Loads that come back empty cost the compute unit's memory pipe as much as real ones, so nobody asks before
@@ -40,7 +41,7 @@ constexpr int kThreads = kWaves * 64;
 constexpr int kCoherent = 16;  // sc1: device scope
 
 struct Ctx {
-  rsrc_t rs;  // the exchange buffers (both sets)
+  rsrc_t rs;  // the exchange buffers (all sets)
   int tid, lane, wave, g, r;
   int spin;
   int dead;  // this wave gave up a wait
