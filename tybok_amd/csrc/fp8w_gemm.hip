@@ -803,6 +803,159 @@ __global__ void decode_fp8_kernel(float* out) {
   out[c] = bf16_bits_to_f32((u16)(cv.u & 0xffff));
 }
 
+// ---- gate/up with the bf16 RMSNorm, several strips per block ----
+// A few hundred rows (the SmolVLA prefill: 113 .. 241 of 960) over many strips: fp8w_gemm_kernel has a block per (32 rows, strip)
+// there, two or three of them on a compute unit, and what bounds them is that every one normalises its rows again (32 x 960
+// values, 1.5 - 2 us of a compute unit) behind a fetch of their 60 KiB.  Here a block normalises its 32 rows once, keeps its
+// waves' operands of them in registers (a wave walks the same k tiles of every strip) and goes through the strips
+// [strips * i / groups, strips * (i + 1) / groups) with nothing but weights to load, a strip ahead.  Same k tiles per wave, same
+// order of all sums as there: the same bits.
+// Whole blocks of 960 -> 2560 -> 960 with cold weights (48 layers in a graph), us: 113 / 177 / 241 rows 18.8 -> 17.5,
+// 19.5 -> 18.1, 23.0 -> 20.1; 720 -> 2048 -> 720 at 177 / 241 rows 14.4 -> 13.5, 15.2 -> 14.1; 784 -> 4096 -> 784 at 70 / 241
+// rows 18.5 -> 17.0, 28.2 -> 24.1.  Bound now: the rows' way to the operand registers (about half of the launch), then a
+// strip's 16 KiB exchange between the waves.
+// Up to 64 rows every pair has a compute unit of its own, or the matrix is large and its stream wants more blocks on a unit.
+// The blocks that share strips are on one XCD (the weights reach its L2 once): a group's index modulo 8 is the block's.
+template <int NR>
+__global__ __launch_bounds__(512) void norm_gate_up_kernel(GemmArgs a, int groups) {
+  constexpr int NW = 8, PPR = NW * 4, PITCH = NW * 64 + 16, XBUF = 32 * PITCH, XPT = 32 * PPR / (NW * 64);
+  constexpr int RED = NW * 2 * 4 * 64;  // f32x4: the waves' partial tiles of a strip
+  static_assert(NR * XBUF <= 2 * RED * 16, "the staged rows lie where the partial tiles go");
+  __shared__ __align__(16) f32x4 red[2 * RED];  // two strips' partials in turn: one barrier a strip
+  unsigned char* const lds = (unsigned char*)red;
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int gx = groups >> 3, slot = blockIdx.x >> 3, mblock = slot / gx;
+  const int group = (slot - mblock * gx) * 8 + (blockIdx.x & 7);
+  const int strips = a.ntiles >> 1, s_lo = strips * group / groups, s_hi = strips * (group + 1) / groups;
+  if (s_lo == s_hi) return;  // (block-uniform)
+
+  i32x4 xv[XPT][NR], nw[NR];
+  int xrow[XPT];
+  const int xcol = (tid & (PPR - 1)) * 8;
+#pragma unroll
+  for (int i = 0; i < XPT; ++i) xrow[i] = tid / PPR + i * (NW * 64 / PPR);
+#pragma unroll
+  for (int p = 0; p < NR; ++p) {
+    int k = p * NW * 32 + xcol;
+    if (k > a.K - 8) k = a.K - 8;  // keep the address inside the row; the value is dropped below
+#pragma unroll
+    for (int i = 0; i < XPT; ++i) {
+      int m = mblock * 32 + xrow[i];
+      if (m > a.M - 1) m = a.M - 1;
+      xv[i][p] = *(const i32x4*)((const u16*)a.x + (size_t)m * a.ldx + k);
+    }
+    nw[p] = *(const i32x4*)(a.norm_w + k);
+  }
+  // a strip's weights (this wave's k tiles) and the scales of this thread's columns in it
+  const int og = tid >> 7, ol = (tid & 127) >> 1, oh = tid & 1;  // output: register group, accumulator lane, half of its columns
+  const int ocol = 8 * og + 4 * (ol >> 5) + 2 * oh;
+  i32x4 w[NR][2];
+  f32x2 scg, scu;
+  auto wload = [&](int s) {
+#pragma unroll
+    for (int p = 0; p < NR; ++p) {
+      int kt = p * NW + wave;
+      if (kt > a.KT - 1) kt = a.KT - 1;
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) w[p][nt] = *(const i32x4*)(a.w + ((size_t)(2 * s + nt) * a.KT + kt) * 1024 + lane * 16);
+    }
+    scg = *(const f32x2*)(a.s0 + s * 32 + ocol);
+    scu = *(const f32x2*)(a.s1 + s * 32 + ocol);
+  };
+  wload(s_lo);
+
+  // row statistics, then the rows as bf16(w * bf16(x * rstd)) through LDS into operand order
+#pragma unroll
+  for (int i = 0; i < XPT; ++i) {
+    float ss0 = 0.f, ss1 = 0.f;
+#pragma unroll
+    for (int p = 0; p < NR; ++p) {
+      if (p * NW * 32 + xcol < a.K) {
+        union { i32x4 v; bf16x2 h[4]; } xu;
+        xu.v = xv[i][p];
+        ss0 = __builtin_amdgcn_fdot2_f32_bf16(xu.h[0], xu.h[0], ss0, false);
+        ss1 = __builtin_amdgcn_fdot2_f32_bf16(xu.h[1], xu.h[1], ss1, false);
+        ss0 = __builtin_amdgcn_fdot2_f32_bf16(xu.h[2], xu.h[2], ss0, false);
+        ss1 = __builtin_amdgcn_fdot2_f32_bf16(xu.h[3], xu.h[3], ss1, false);
+      }
+    }
+    const float rstd = rsqrtf(wave_sum<PPR>(ss0 + ss1) / (float)a.K + a.norm_eps);
+#pragma unroll
+    for (int p = 0; p < NR; ++p) {
+      union { i32x4 v; unsigned u[4]; } xu, nu, o;
+      xu.v = xv[i][p];
+      nu.v = nw[p];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const unsigned u = pack_bf16x2(__uint_as_float(xu.u[e] << 16) * rstd, __uint_as_float(xu.u[e] & 0xffff0000u) * rstd);
+        o.u[e] = pack_bf16x2(__uint_as_float(nu.u[e] << 16) * __uint_as_float(u << 16),
+                             __uint_as_float(nu.u[e] & 0xffff0000u) * __uint_as_float(u & 0xffff0000u));
+      }
+      const i32x4 z = {0, 0, 0, 0};
+      *(i32x4*)(lds + p * XBUF + xrow[i] * PITCH + xcol * 2) = p * NW * 32 + xcol < a.K ? o.v : z;
+    }
+  }
+  lds_barrier();
+  bf16x8 xa[NR][2];
+#pragma unroll
+  for (int p = 0; p < NR; ++p) {
+    const i32x4* q = (const i32x4*)(lds + p * XBUF + l32 * PITCH + (wave * 32 + 16 * half) * 2);
+    xa[p][0] = as_bf16x8(q[0]);
+    xa[p][1] = as_bf16x8(q[1]);
+  }
+  lds_barrier();  // the partial tiles go where the rows were
+
+  int buf = 0;
+  for (int s = s_lo; s < s_hi; ++s) {
+    f32x16 acc[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[nt][i] = 0.f;
+#pragma unroll
+    for (int p = 0; p < NR; ++p) {
+      bf16x8 wb[2][2];
+#pragma unroll
+      for (int nt = 0; nt < 2; ++nt) {
+        wb[nt][0] = fp8x8_to_bf16x8(w[p][nt][0], w[p][nt][1]);
+        wb[nt][1] = fp8x8_to_bf16x8(w[p][nt][2], w[p][nt][3]);
+      }
+#pragma unroll
+      for (int h2 = 0; h2 < 2; ++h2)
+#pragma unroll
+        for (int nt = 0; nt < 2; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb[nt][h2], xa[p][h2], acc[nt], 0, 0, 0);
+    }
+    const f32x2 cg = scg, cu = scu;
+    wload(s + 1 < s_hi ? s + 1 : s);  // (unconditional: behind a branch the compiler waits for every load)
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt)
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        red[buf * RED + ((wave * 2 + nt) * 4 + g) * 64 + lane] = f32x4{acc[nt][4 * g], acc[nt][4 * g + 1], acc[nt][4 * g + 2], acc[nt][4 * g + 3]};
+    lds_barrier();
+    // waves in the order of gemm_block: w + 4 onto w, then 0 .. 3
+    f32x2 own[2];
+#pragma unroll
+    for (int nt = 0; nt < 2; ++nt) {
+      f32x2 v[NW];
+#pragma unroll
+      for (int i = 0; i < NW; ++i) v[i] = *((const f32x2*)(red + buf * RED + ((i * 2 + nt) * 4 + og) * 64 + ol) + oh);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] += v[i + 4];
+      own[nt] = ((v[0] + v[1]) + v[2]) + v[3];
+    }
+    const unsigned gb = pack_bf16x2(own[0][0] * cg[0], own[0][1] * cg[1]), ub = pack_bf16x2(own[1][0] * cu[0], own[1][1] * cu[1]);
+    const float g0 = __uint_as_float(gb << 16), g1 = __uint_as_float(gb & 0xffff0000u);
+    const unsigned ab = a.act == 0 ? pack_bf16x2(silu_f(g0), silu_f(g1)) : pack_bf16x2(gelu_tanh_f(g0), gelu_tanh_f(g1));
+    const int m = mblock * 32 + (ol & 31);
+    if (m < a.M)
+      *(unsigned*)(a.y + (size_t)m * a.ldy + s * 32 + ocol) = pack_bf16x2(__uint_as_float(ab << 16) * __uint_as_float(ub << 16),
+                                                                        __uint_as_float(ab & 0xffff0000u) * __uint_as_float(ub & 0xffff0000u));
+    buf ^= 1;
+  }
+}
+
 // Pipeline depth (block rounds in flight) and k tiles per wave and round.  Measured on MI355X: 4 rounds
 // cover the weight stream's latency at the 33.5 MB shapes (2, 6 and 8 are no faster); two k tiles per
 // wave and round halve the barriers but lengthen every small launch of the denoise loop.
@@ -845,7 +998,7 @@ int launch(const GemmArgs& a, dim3 grid, int nw, hipStream_t st) {
 
 }  // namespace
 
-int tk_launch_gemm(GemmArgs a, int MT, int NT, int mblocks, hipStream_t st) {
+int tk_launch_gemm(GemmArgs a, int MT, int NT, int mblocks, int cus, hipStream_t st) {
   dim3 grid((a.ntiles + NT - 1) / NT, a.ksplit, mblocks);
   // eight waves on a 32-row block where they pay (measured per launch and in whole requests, K = 720 .. 2048): a
   // long k range of fp8 tiles (half the rounds) or a norm prologue, plain or adaptive (half the normalisation work
@@ -873,6 +1026,17 @@ int tk_launch_gemm(GemmArgs a, int MT, int NT, int mblocks, hipStream_t st) {
   if (epi == 2 || pro == 2) return -1;
   if (epi == 1) {
     if (NT != 2) return -1;
+    if (pro == 1 && MT == 1 && a.M > 64 && a.ksplit == 1 && a.N % 32 == 0 && a.KT > 2 * 8 && a.KT <= 4 * 8) {
+      // more (row block, strip) pairs than compute units: as many strips to a block as it takes, in whole eights of groups
+      const int strips = a.ntiles / 2, most = cus / (8 * mblocks) * 8;
+      if (most > 0 && strips > most) {
+        const int per = (strips + most - 1) / most, groups = ((strips + per - 1) / per + 7) / 8 * 8;
+        const dim3 g1(groups * mblocks);
+        if (a.KT <= 3 * 8) hipLaunchKernelGGL(norm_gate_up_kernel<3>, g1, dim3(512), 0, st, a, groups);
+        else hipLaunchKernelGGL(norm_gate_up_kernel<4>, g1, dim3(512), 0, st, a, groups);
+        return hipGetLastError() == hipSuccess ? 0 : -3;
+      }
+    }
     if (pro == 1) return MT == 1 ? launch<1, 2, 1, false, 1>(a, grid, nw, st) : launch<2, 2, 1, false, 1>(a, grid, nw, st);
     if (pro == 3) return MT == 1 ? launch<1, 2, 1, false, 3>(a, grid, nw, st) : launch<2, 2, 1, false, 3>(a, grid, nw, st);
     return MT == 1 ? launch<1, 2, 1, false, 0>(a, grid, nw, st) : launch<2, 2, 1, false, 0>(a, grid, nw, st);

@@ -426,7 +426,7 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
     plan->skinny = !stream;
     return TK_OK;
   }
-  int rc = stream ? tk_launch_gemm_stream(a, st) : tk_launch_gemm(a, MT, NT, mblocks, st);
+  int rc = stream ? tk_launch_gemm_stream(a, st) : tk_launch_gemm(a, MT, NT, mblocks, cus, st);
   if (rc == -1) return fail(TK_EINVAL, "gemm: this combination of weight type, prologue and epilogue is not built");
   if (rc) return fail(TK_ELAUNCH, "gemm: launch failed (%s)", hipGetErrorString(hipGetLastError()));
   return TK_OK;

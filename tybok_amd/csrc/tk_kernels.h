@@ -271,7 +271,7 @@ int tk_launch_layer_norm(LayerNormArgs a, hipStream_t st);
 // many-row fp8-weight GEMM; tile: an id of kWideTiles (tk_api.hip)
 int tk_launch_gemm_wide(const GemmArgs& a, int tile, hipStream_t st);
 int tk_launch_norm_rows(NormRowsArgs a, hipStream_t st);
-int tk_launch_gemm(GemmArgs a, int MT, int NT, int mblocks, hipStream_t st);
+int tk_launch_gemm(GemmArgs a, int MT, int NT, int mblocks, int cus, hipStream_t st);
 // the action chunk's gated FFN in one launch (32-row blocks; g: the gate/up half without a K split, d: the down half
 // with NT n tiles per strip); -1 when the pair of shapes is not one of the built combinations
 int tk_launch_ffn_fused(GemmArgs g, GemmArgs d, int d_nt, int mblocks, hipStream_t st);
