@@ -372,6 +372,13 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
   const int blocks0 = strips * mblocks;
   const int NW = 4;
   int ks = stream_ks ? stream_ks : split_k;
+  // Plain fp8 linears of 65 .. 96 k tiles on 32-row blocks: one block walks them all with eight waves in a straight line of 9 .. 12
+  // rounds (fp8w_gemm.hip) instead of handing split sums over.  Cold weights, us, as split before and whole: 2560 -> 960 at
+  // 50 / 113 / 241 rows 6.2 -> 5.6, 7.6 -> 5.9, 8.4 -> 5.9; 2304 -> 1600 at 180 rows 9.2 -> 7.1, 3072 -> 960 at 100 / 250 rows
+  // 7.0 -> 6.3, 8.7 -> 6.4.  Up to 64 blocks (few columns, or few rows and 960 columns) the splits bring idle units in: 3072 ->
+  // 250 at 250 rows 6.3 split, 6.8 whole; at ten rounds the two are level there and whole is ahead in between.
+  const int rounds8 = (a.KT + 7) / 8;
+  if (ks <= 0 && MT == 1 && !e.w16 && !gated && !has_norm && rounds8 >= 9 && rounds8 <= 12 && (blocks0 > 64 || rounds8 == 10)) ks = 1;
   if (ks <= 0) {
     // Launch-cost model (microseconds, fitted to graph-replayed launches on MI355X): the k loop costs
     // 0.35 per block round (NW k tiles) for 64-row blocks, 0.20 for 32-row blocks (0.27 with two bf16
