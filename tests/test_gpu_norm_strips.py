@@ -34,3 +34,37 @@ def test_rows_equal_calls_of_32_rows(m, k, i, act):
         want = torch.cat([tk.fp8w_gated_ffn(x[r : r + 32], wgu, wd, act, **norm) for r in range(0, m, 32)])
         assert torch.equal(got, want)
         assert got.float().abs().max() > 0
+
+
+# plain linears whose blocks walk the whole K in 9 .. 12 rounds of eight k tiles: a round of one tile, partial last tiles, whole
+# ones; one row to several row blocks; one column group, a partial tile, and a grid beyond the device
+@pytest.mark.parametrize("k", [2064, 2304, 2320, 2560, 2576, 2816, 2832, 3072])
+@pytest.mark.parametrize("m,n", [(1, 1600), (50, 960), (97, 250), (255, 960), (241, 4096)])
+def test_whole_k_linears(m, k, n):
+    g = torch.Generator().manual_seed(m + k)
+    x = torch.randn(m, k, generator=g).to(BF16).cuda()
+    w8, s = quantize_weight_rows((torch.randn(n, k, generator=g) * 0.05).cuda())
+    got = tk.fp8w_gemm(x, tk.pack_fp8_weight(w8, s)).double()
+    w = w8.double() * s.double()[:, None]
+    want = x.double() @ w.t()
+    # one rounding to bf16 (8 significant bits: half a step is 2^-8 of the value), one of the scaled sum, K fp32 additions of
+    # products of this size
+    bound = (2.0**-8 + 2.0**-23) * want.abs() + k * 2.0**-24 * (x.double().abs() @ w.abs().t())
+    assert bool(((got - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m", [65, 177, 256])
+def test_norm_of_fp32_rows_equals_calls_of_64_rows(m):
+    k, heads, kv = 960, 15, 5
+    n = (heads + 2 * kv) * 64
+    g = torch.Generator().manual_seed(m)
+    x = torch.randn(m, k, generator=g).cuda()
+    w = tk.pack_bf16_weight((torch.randn(n, k, generator=g) * 0.05).to(BF16).cuda(), rope_half=32)
+    rope = tk.RopeTables(torch.randn(512, 32, generator=g).cuda(), torch.randn(512, 32, generator=g).cuda())
+    pos = torch.arange(m, dtype=torch.int32, device="cuda")
+    norm = (1.0 + 0.1 * torch.randn(k, generator=g)).to(BF16).cuda()
+
+    def rows(lo, hi):
+        return tk.bf16w_linear(x[lo:hi], w, norm_w=norm, eps=1e-5, rope=rope, rope_pos=pos[lo:hi].contiguous(), rope_cols=(heads + kv) * 64)
+
+    assert torch.equal(rows(0, m), torch.cat([rows(r, min(r + 64, m)) for r in range(0, m, 64)]))
