@@ -1,5 +1,6 @@
 """Gate/up of a few hundred rows with the RMSNorm prologue (blocks that walk several strips) against the same rows in calls of 32,
-which run on the kernel with a block per strip: the same order of all sums, so the same bits."""
+which run on the kernel with a block per strip: the same order of all sums, so the same bits.  And the other linears of that prefill whose
+blocks changed with it: those that walk a long K whole, the projection of fp32 rows."""
 
 import pytest
 import torch
