@@ -55,7 +55,24 @@ def test_one_launch_matches_the_launches_per_layer(model, m, p):
     rel = float((got - want[0]).norm() / (want[0] - x).norm())
     print(f"M={m} P={p}: relative difference of the flow {rel:.3g}")
     assert rel < 2e-2  # bf16 rounding: the launches per layer and the plain torch path differ by 5e-3 - 1.2e-2 here
-    assert torch.equal(got, _run(model, x, caches, pad, pos))  # both exchange sets start clean again
+    assert torch.equal(got, _run(model, x, caches, pad, pos))  # every launch starts from clean exchange sets
+
+
+# A step's exchange words are used again three steps later: ten steps in one launch (every set three times or more) against ten
+# launches of one step, none of which finds a word that was ever used.  The rows go from step to step in fp32 either way, so an
+# old word that somebody reads, or one that was not set back, shows in the bits.
+@pytest.mark.parametrize("m,p", [(1, 1), (16, 32), (17, 33), (50, 241), (33, 255), (50, 448), (64, 448)])
+@torch.inference_mode()
+def test_ten_steps_in_one_launch_equal_ten_launches(model, m, p):
+    x, caches, pad, pos = _case(model, m, p)
+    steps = 10
+    emb = torch.stack([model.suffix_b_all[i % model.num_steps] for i in range(steps)])
+    want = x
+    for i in range(steps):
+        want = model.denoise_plan.run(want, 1, -1.0 / steps, emb[i : i + 1], caches, pad[0], *pos)
+    assert torch.isfinite(want).all() and not torch.equal(want, x)
+    for _ in range(3):
+        assert torch.equal(model.denoise_plan.run(x, steps, -1.0 / steps, emb, caches, pad[0], *pos), want)
 
 
 @pytest.mark.parametrize("m,p", [(17, 33), (50, 241), (64, 448)])
