@@ -73,6 +73,50 @@ def test_missing_library_fails_loudly(monkeypatch):
         native.lib()
 
 
+@pytest.mark.parametrize("other", ["torch", "python"])
+def test_an_extension_built_for_another_torch_or_python_is_not_loaded(monkeypatch, other):
+    import torch
+
+    from tybok_amd import native
+
+    if not os.path.exists(native.library_path()):
+        pytest.skip("libtybok_hip.so not built")
+    native.calls()  # this one's is there
+    monkeypatch.setattr(native, "_calls", None)
+    if other == "torch":
+        monkeypatch.setattr(torch, "__version__", "2.9.1+other")
+    else:
+        monkeypatch.setattr("sysconfig.get_config_var", lambda name: "cpython-399-x86_64-linux-gnu")
+    with pytest.raises(RuntimeError, match="built for each Python and torch.*build it with"):
+        native.calls()
+
+
+def test_an_incremental_build_for_another_torch_compiles_the_extension(monkeypatch, tmp_path):
+    import torch
+
+    from tybok_amd import native
+    from tybok_amd.csrc import build
+
+    for name in ("LIB_DIR", "OBJ_DIR"):
+        monkeypatch.setattr(build, name, str(tmp_path))
+    monkeypatch.setattr(build, "LIB_PATH", str(tmp_path / "libtybok_hip.so"))
+    monkeypatch.setattr(native, "_LIB_PATH", build.LIB_PATH)
+    made = []
+
+    def run(cmd, verbose):
+        made.append(os.path.basename(cmd[cmd.index("-o") + 1]))
+        open(cmd[cmd.index("-o") + 1], "w").close()
+
+    monkeypatch.setattr(build, "_run", run)
+    build.build_library(verbose=False)
+    made.clear()
+    build.build_library(verbose=False, incremental=True)
+    assert not [n for n in made if "tk_calls" in n]
+    monkeypatch.setattr(torch, "__version__", "2.9.1+other")
+    build.build_library(verbose=False, incremental=True)
+    assert len([n for n in made if "tk_calls" in n]) == 1
+
+
 P = 0x10000  # a 16-byte aligned stand-in for device pointers: every call below is rejected before any launch
 
 

@@ -4,7 +4,7 @@
 Layout:
 
 * ``csrc/``      hand-written HIP kernels + the C ABI (``include/tybok_hip.h``)
-* ``native``     ctypes binding of ``libtybok_hip.so``
+* ``native``     binding of ``libtybok_hip.so``: ctypes, and an extension on torch tensors for the entry points that launch
 * ``ops``        tensor-level wrappers (torch = device memory + stream only)
 * ``quant``      per-row e4m3fn weight quantisation (the checkpoint-side recipe)
 * ``base`` / ``registry`` / ``graph``  the engine API mirrored from the reference

@@ -1,10 +1,11 @@
-"""Build libtybok_hip.so for gfx950 with plain hipcc (no torch headers), and tk_calls.so, torch's side of its Python binding.
+"""Build libtybok_hip.so for gfx950 with plain hipcc (no torch headers), and the tk_calls extension, torch's side of its Python binding.
 
 Run as ``python -m tybok_amd.csrc.build`` or through ``__graft_entry__.build()``.  hipcc
 cross-compiles without a GPU; the library lands in ``tybok_amd/_lib/`` next to the package so it
 travels with the source tree.  Each translation unit is compiled to an object of its own (in
-parallel) and the objects are linked into the shared library.  tk_calls.so (host code only) is a
-CPython extension that links against it and against the torch of the running interpreter.
+parallel) and the objects are linked into the shared library.  tk_calls (host code only) is a CPython
+extension that links against it; it is compiled for the Python that runs the build and that Python's torch
+(the headers of both are needed) and has both in its file name.
 """
 
 from __future__ import annotations
@@ -16,12 +17,13 @@ import sys
 import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
+from .. import native
+
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(os.path.dirname(HERE), "_lib")
 OBJ_DIR = os.path.join(LIB_DIR, "obj")
 LIB_PATH = os.path.join(LIB_DIR, "libtybok_hip.so")
 CALLS_SOURCE = os.path.join(HERE, "tk_calls.cpp")
-CALLS_PATH = os.path.join(LIB_DIR, "tk_calls.so")
 SOURCES = ("fp8w_gemm.hip", "fp8w_gemm_stream.hip", "fp8w_gemm_wide.hip", "expert_attn.hip", "expert_attn_d256.hip", "expert_attn_px.hip", "expert_tail.hip", "expert_kv_proj.hip", "layer_norm.hip", "tower_attn.hip", "rope_rows.hip", "prefix_prep.hip", "denoise_smolvla.hip", "denoise_pi05.hip", "stream_read.hip", "w8a8_gemm.hip", "bf16w_gemm_wide.hip", "tk_api.hip")
 HEADERS = ("tk_common.h", "tk_kernels.h", "persist.h", "pipe_gemm.h", "pipe_fp8.h", os.path.join("..", "..", "include", "tybok_hip.h"))
 ARCH = "gfx950"
@@ -55,7 +57,7 @@ def _run(cmd: list[str], verbose: bool) -> None:
 
 
 def _calls_command(hipcc: str, out: str) -> list[str]:
-    """The compile line of tk_calls.so; torch's libraries are in the process before it is loaded, so it names no path to them."""
+    """The compile line of tk_calls; torch's libraries are in the process before it is loaded, so it names no path to them."""
     import torch
 
     root = os.path.dirname(torch.__file__)
@@ -85,10 +87,11 @@ def build_library(verbose: bool = True, incremental: bool = False, jobs: int = 8
         list(pool.map(lambda cmd: _run(cmd, verbose), todo))
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,-soname,libtybok_hip.so", *objects, "-o", LIB_PATH + ".tmp"], verbose)
     os.replace(LIB_PATH + ".tmp", LIB_PATH)
+    calls = native.calls_path()
     newest = max(os.path.getmtime(CALLS_SOURCE), os.path.getmtime(os.path.join(HERE, HEADERS[-1])))
-    if not (incremental and os.path.exists(CALLS_PATH) and os.path.getmtime(CALLS_PATH) >= newest):
-        _run(_calls_command(hipcc, CALLS_PATH + ".tmp"), verbose)
-        os.replace(CALLS_PATH + ".tmp", CALLS_PATH)
+    if not (incremental and os.path.exists(calls) and os.path.getmtime(calls) >= newest):
+        _run(_calls_command(hipcc, calls + ".tmp"), verbose)
+        os.replace(calls + ".tmp", calls)
     return LIB_PATH
 
 

@@ -1,6 +1,7 @@
-"""ctypes binding of ``libtybok_hip.so`` (the C ABI declared in ``include/tybok_hip.h``).
+"""Binding of ``libtybok_hip.so`` (the C ABI declared in ``include/tybok_hip.h``): :func:`lib` through ctypes, for the entry
+points that a program calls while it prepares, and :func:`calls`, an extension module on torch tensors, for the ones that launch.
 
-The library is loaded from ``tybok_amd/_lib/``; there is no fallback: if it is missing or an
+Both are loaded from ``tybok_amd/_lib/``; there is no fallback: if one is missing or an
 entry point fails, a ``RuntimeError`` is raised (the reference's native helpers raise instead
 of exiting too: tybok/policies/fastwam/kernels/coop_grid.h:20-27).
 """
@@ -11,6 +12,7 @@ import ctypes
 import importlib.machinery
 import importlib.util
 import os
+import sysconfig
 from ctypes import c_char_p, c_float, c_int, c_longlong, c_size_t, c_void_p
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib", "libtybok_hip.so")
@@ -251,17 +253,23 @@ def check(rc: int, what: str) -> None:
         raise RuntimeError(f"{what} failed ({rc}): {msg.decode() if msg else 'unknown error'}")
 
 
+def calls_path() -> str:
+    """Where the extension module of this Python and this torch lies.  It is compiled against the headers of both, and neither keeps
+    the layout of what they describe between versions; so both are in its name, and a build for others is not found."""
+    import torch
+
+    return os.path.join(os.path.dirname(_LIB_PATH), f"tk_calls.{sysconfig.get_config_var('SOABI')}.torch-{torch.__version__}.so")
+
+
 def calls():
     """The extension module of the launching entry points (``csrc/tk_calls.cpp``): ``calls().tk_name(...)`` takes tensors for
     pointers, launches on torch's current stream (the entry's last argument, not passed) and raises like :func:`check`."""
     global _calls
     if _calls is None:
-        import torch  # noqa: F401  (its libraries have to be in the process)
-
+        path = calls_path()  # (imports torch: its libraries have to be in the process)
         lib()
-        path = os.path.join(os.path.dirname(_LIB_PATH), "tk_calls.so")
         if not os.path.exists(path):
-            raise RuntimeError(f"{path} is missing: build it with `python -m tybok_amd.csrc.build`")
+            raise RuntimeError(f"{path} is missing (one is built for each Python and torch): build it with `python -m tybok_amd.csrc.build`")
         loader = importlib.machinery.ExtensionFileLoader("tk_calls", path)
         module = importlib.util.module_from_spec(importlib.util.spec_from_file_location("tk_calls", path, loader=loader))
         loader.exec_module(module)
