@@ -675,6 +675,11 @@ int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* 
  * CUs where there is none); gated: N is the intermediate's width.  For tests of the rule.  No counterpart in the reference. */
 int tk_debug_w8a8_tile(int M, int N, int K, int gated, int split_k);
 
+/* The blocks of a launch of few rows on the current device (256 CUs where there is none) with a whole workspace: 100 * rows of a
+ * block + K splits; 0 = another kernel takes it.  kind 0: tk_fp8w_gemm; 1: tk_bf16w_linear of fp32 rows with the RMSNorm and the
+ * rotary epilogue (heads of 64).  For tests of the rules.  No counterpart in the reference. */
+int tk_debug_linear_blocks(int M, int N, int K, int kind);
+
 #ifdef __cplusplus
 }
 #endif

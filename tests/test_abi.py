@@ -64,6 +64,28 @@ def test_w8a8_block_shapes_by_the_sizes(m, n, k, gated, tile):
     assert native.lib().tk_debug_w8a8_tile(m, n, k, gated, 1) == tile
 
 
+@pytest.mark.parametrize("m,n,k,blocks", [
+    # three splits of more blocks than compute units: whole at every K
+    (96, 960, 2304, 3201), (96, 960, 2560, 3201), (96, 960, 3072, 3201), (250, 960, 3072, 3201), (64, 1376, 3072, 3201),
+    # fewer: twelve rounds are split ...
+    (64, 1344, 3072, 3203), (96, 720, 3072, 3203), (64, 1280, 3072, 3203), (50, 960, 2848, 3203), (1, 32, 3072, 3203),
+    # ... and thirds that are a straight line of their own, up to a quarter of the compute units
+    (1, 128, 2304, 3203), (50, 512, 2784, 3203), (64, 1024, 2304, 3203), (64, 1056, 2304, 3201), (64, 1024, 2784, 3203), (64, 1056, 2784, 3201),
+    # the others walk the whole K, from one block on ...
+    (1, 32, 2560, 3201), (50, 960, 2560, 3201), (1, 128, 2240, 3201), (50, 512, 2400, 3201), (50, 512, 2688, 3201), (96, 720, 2816, 3201), (50, 250, 2560, 3201),
+    # ... but for a few blocks of eleven rounds with columns in no fours
+    (50, 250, 2592, 3203), (50, 250, 2816, 3203), (64, 1090, 2816, 3201),
+    # either side of the range: as the model splits them
+    (50, 960, 2048, 3201), (50, 960, 3104, 3203), (50, 960, 4096, 3204),
+])  # fmt: skip
+def test_whole_k_linears_by_the_sizes(m, n, k, blocks):
+    from tybok_amd import native
+
+    if not os.path.exists(native.library_path()):
+        pytest.skip("libtybok_hip.so not built")
+    assert native.lib().tk_debug_linear_blocks(m, n, k, 0) == blocks
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from tybok_amd import native
 

@@ -37,21 +37,23 @@ def test_rows_equal_calls_of_32_rows(m, k, i, act):
         assert got.float().abs().max() > 0
 
 
-# plain linears whose blocks walk the whole K in 9 .. 12 rounds of eight k tiles: a round of one tile, partial last tiles, whole
-# ones; one row to several row blocks; one column group, a partial tile, and a grid beyond the device
+# plain linears whose blocks walk the whole K in 9 .. 12 rounds of eight k tiles (split_k = 1: wherever the rule would split it), and
+# as the rule takes them: a round of one tile, partial last tiles, whole ones; one row to several row blocks; one column group, a
+# partial tile, and a grid beyond the device
 @pytest.mark.parametrize("k", [2064, 2304, 2320, 2560, 2576, 2816, 2832, 3072])
 @pytest.mark.parametrize("m,n", [(1, 1600), (50, 960), (97, 250), (255, 960), (241, 4096)])
 def test_whole_k_linears(m, k, n):
     g = torch.Generator().manual_seed(m + k)
     x = torch.randn(m, k, generator=g).to(BF16).cuda()
     w8, s = quantize_weight_rows((torch.randn(n, k, generator=g) * 0.05).cuda())
-    got = tk.fp8w_gemm(x, tk.pack_fp8_weight(w8, s)).double()
+    packed = tk.pack_fp8_weight(w8, s)
     w = w8.double() * s.double()[:, None]
     want = x.double() @ w.t()
     # one rounding to bf16 (8 significant bits: half a step is 2^-8 of the value), one of the scaled sum, K fp32 additions of
     # products of this size
     bound = (2.0**-8 + 2.0**-23) * want.abs() + k * 2.0**-24 * (x.double().abs() @ w.abs().t())
-    assert bool(((got - want).abs() <= bound).all())
+    for split_k in (1, 0):
+        assert bool(((tk.fp8w_gemm(x, packed, split_k=split_k).double() - want).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("m", [65, 177, 256])

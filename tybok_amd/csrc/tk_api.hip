@@ -373,12 +373,24 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
   const int NW = 4;
   int ks = stream_ks ? stream_ks : split_k;
   // Plain fp8 linears of 65 .. 96 k tiles on 32-row blocks: one block walks them all with eight waves in a straight line of 9 .. 12
-  // rounds (fp8w_gemm.hip) instead of handing split sums over.  Cold weights, us, as split before and whole: 2560 -> 960 at
-  // 50 / 113 / 241 rows 6.2 -> 5.6, 7.6 -> 5.9, 8.4 -> 5.9; 2304 -> 1600 at 180 rows 9.2 -> 7.1, 3072 -> 960 at 100 / 250 rows
-  // 7.0 -> 6.3, 8.7 -> 6.4.  Up to 64 blocks (few columns, or few rows and 960 columns) the splits bring idle units in: 3072 ->
-  // 250 at 250 rows 6.3 split, 6.8 whole; at ten rounds the two are level there and whole is ahead in between.
+  // rounds (fp8w_gemm.hip) instead of handing split sums over.  Against it stands a split by three (the model's below), where
+  // a block walks a third with four waves.  Cold weights, us, split and whole:
+  //   * More blocks than compute units in three splits (of 256: 86 blocks and more): the split's second generation costs more
+  //     than its shorter walk saves at every K: 2304 -> 960 at 96 rows 6.4 -> 5.8, 2560 -> 960 at 96 / 250 rows 7.4 -> 6.0, 8.4 ->
+  //     6.1, 3072 -> 960 at 96 / 250 rows 7.4 -> 6.7, 9.0 -> 6.8, 3072 -> 1600 at 180 rows 11.5 -> 9.2.
+  //   * Fewer, at twelve rounds, the longest walk: 3072 -> 512 at 50 rows 5.6 split, 6.2 whole; 3072 -> 720 at 96 rows 6.2 and 6.5,
+  //     2944 -> 720 at 96 rows level.
+  //   * Fewer, at nine to eleven: a split whose thirds are a straight line of their own (equal, of six or eight rounds) is ahead up
+  //     to a quarter of the compute units (2304 -> 512 at 50 rows 5.1 split, 5.4 whole; at 60 blocks and more level to 2 %
+  //     behind).  The other thirds are a loop of unknown length, and whole is up to 10 % ahead from one block on: 2560 -> 32 at one
+  //     row 5.4 -> 4.9, 2560 -> 960 at 50 rows 6.5 -> 5.9, 2688 -> 512 at 50 rows 5.9 -> 5.7; but for a few blocks of eleven rounds
+  //     and columns in no fours, whose output goes by single values (2816 -> 250 at 50 rows 6.2 split, 6.4 whole).
   const int rounds8 = (a.KT + 7) / 8;
-  if (ks <= 0 && MT == 1 && !e.w16 && !gated && !has_norm && rounds8 >= 9 && rounds8 <= 12 && (blocks0 > 64 || rounds8 == 10)) ks = 1;
+  if (ks <= 0 && MT == 1 && !e.w16 && !gated && !has_norm && rounds8 >= 9 && rounds8 <= 12) {
+    const int third = (a.KT / 3 + 3) / 4;  // rounds of four waves
+    const bool straight = a.KT % 3 == 0 && (third == 6 || third == 8), few = blocks0 * 4 <= cus;
+    if (blocks0 * 3 > cus || (rounds8 < 12 && !(few && (straight || (rounds8 == 11 && !a.vec))))) ks = 1;
+  }
   if (ks <= 0) {
     // Launch-cost model (microseconds, fitted to graph-replayed launches on MI355X): the k loop costs
     // 0.35 per block round (NW k tiles) for 64-row blocks, 0.20 for 32-row blocks (0.27 with two bf16
@@ -1706,6 +1718,25 @@ int tk_debug_many_rows_gemm(const void* x, int ldx, const void* sa, const void* 
 int tk_debug_w8a8_tile(int M, int N, int K, int gated, int split_k) {
   if (M <= 0 || N <= 0 || K <= 0 || split_k <= 0) return fail(TK_EINVAL, "w8a8_tile: non-positive argument");
   return w8a8_tile(M, (N + 31) / 32 * 32 * (gated ? 2 : 1), K, split_k);
+}
+
+int tk_debug_linear_blocks(int M, int N, int K, int kind) {
+  if (kind < 0 || kind > 1) return fail(TK_EINVAL, "linear_blocks: unknown kind %d", kind);
+  alignas(16) static char stand_in[16];  // operands of a launch that is only planned
+  void* const p = stand_in;
+  const float* const f = (const float*)p;
+  GemmExtra e;
+  if (kind == 1) {
+    e.x_f32 = e.w16 = 1;
+    e.norm_w = p;
+    e.rope_pos = (const int*)p;
+    e.rope_cos = e.rope_sin = f;
+    e.rope_positions = 1, e.rope_cols = N, e.rope_half = 32;
+  }
+  GemmPlan plan;
+  const int rc = gemm_common(p, K, p, f, nullptr, p, (N + 7) / 8 * 8, nullptr, 0, 0, nullptr, M, N, K, 0, 0, p, tk_workspace_bytes(), nullptr, e, &plan);
+  if (rc) return rc;
+  return plan.skinny ? plan.MT * 3200 + plan.a.ksplit : 0;
 }
 
 int tk_debug_decode_fp8(void* out_f32, void* stream) {

@@ -169,6 +169,7 @@ SIGNATURES: dict[str, tuple] = {
         + [c_int] * 6 + [c_void_p, c_size_t, c_void_p],
     ),  # fmt: skip
     "tk_debug_w8a8_tile": (c_int, [c_int] * 5),
+    "tk_debug_linear_blocks": (c_int, [c_int] * 4),
     "tk_debug_fp8w_gemm_cut": (c_int, [c_void_p, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_void_p]),
 }
 
