@@ -86,6 +86,24 @@ def test_whole_k_linears_by_the_sizes(m, n, k, blocks):
     assert native.lib().tk_debug_linear_blocks(m, n, k, 0) == blocks
 
 
+@pytest.mark.parametrize("m,n,k,rows", [
+    # a generation of 32-row blocks, its last row block and the next
+    (65, 1600, 960, 32), (256, 1600, 960, 32), (128, 4096, 960, 32), (129, 4096, 960, 64), (256, 4096, 960, 64), (128, 8192, 1024, 64),
+    # three of 32 rows for two of 64, and four: by the columns
+    (160, 8192, 720, 32), (200, 8192, 720, 64), (200, 8192, 960, 32), (65, 16384, 512, 32), (65, 16384, 256, 64), (256, 512, 256, 32),
+    # 64-row blocks that a K split would multiply, and that it would not
+    (200, 2560, 1344, 32), (160, 4096, 1408, 64), (113, 5120, 1408, 32), (160, 4096, 1440, 32), (200, 4096, 1440, 64),
+    # a long K; matrices of more than 16 MiB and more rows keep theirs
+    (256, 4096, 1536, 32), (256, 4096, 2048, 32), (256, 4160, 2048, 64), (257, 1600, 960, 64),
+])  # fmt: skip
+def test_blocks_of_fp32_rows_by_the_sizes(m, n, k, rows):
+    from tybok_amd import native
+
+    if not os.path.exists(native.library_path()):
+        pytest.skip("libtybok_hip.so not built")
+    assert native.lib().tk_debug_linear_blocks(m, n, k, 1) // 100 == rows
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from tybok_amd import native
 

@@ -338,6 +338,29 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
     return TK_OK;
   }
   if (e.tile) return fail(TK_EINVAL, "gemm: the many-row kernels do not take these operands");
+  // Launch-cost model (microseconds, fitted to graph-replayed launches on MI355X): the k loop costs
+  // 0.35 per block round (NW k tiles) for 64-row blocks, 0.20 for 32-row blocks (0.27 with two bf16
+  // weight tiles per wave and round), with a floor of one memory round trip; splitting K adds a partial write, an arrival
+  // count and a read-back that grows with the number of splits and steps up with every batch of four
+  // the finishing block has in flight (1.1 + 0.4 c + 1.0 per further batch), and only pays while the
+  // grid still fits the device twice over.
+  const auto model_splits = [&](int MT, int NT, int blocks0) {
+    constexpr int NW = 4;
+    int ks = 1;
+    if (blocks0 >= cus) return ks;
+    const float per_round = MT == 1 ? (e.w16 && NT == 2 ? 0.27f : 0.20f) : 0.35f;
+    float best = 1e30f;
+    // (an automatic choice never asks for more partial space than the workspace holds)
+    const size_t cap = !ws || ws_bytes <= kPartialOff ? 0 : (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes);
+    for (int c = 1; c <= 64 && c * NW <= a.KT && (c == 1 || (blocks0 * c <= 2 * cus && (size_t)blocks0 * c * MT * NT * 4096 <= cap && blocks0 * 4 <= kMaxCounters)); ++c) {
+      const int rounds = (a.KT + c * NW - 1) / (c * NW);
+      float t = rounds * per_round;
+      if (t < 1.0f) t = 1.0f;
+      if (c > 1) t += 1.1f + 0.4f * (float)c + 1.0f * (float)((c + 3) / 4 - 1);
+      if (t < best - 1e-3f) best = t, ks = c;
+    }
+    return ks;
+  };
   int MT = M <= 32 ? 1 : 2;
   // The action chunk (33..64 rows) over a small weight matrix is a latency-bound launch: two blocks
   // of 32 rows per strip halve each block's staging, normalisation and product work and put twice
@@ -347,9 +370,25 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
   // A few hundred rows (the SmolVLA prefill: 241 / 177) over a small matrix: 32-row blocks too.  With the bf16
   // RMSNorm prologue over a short K they run the prologue that requests every round up front and takes the row
   // statistics from the staged pieces (-3 us per launch inside a request); the other launches gain 0.7 us from the
-  // finer blocks, the norm of fp32 rows (the prefix's first layer) more: 960 -> 1600 at 113 / 241 rows 13.7 -> 8.5, 14.1 -> 9.2 us
+  // finer blocks
   if (M > 64 && e.norm_w && !e.x_f32 && a.KT <= 32) MT = 1;
-  if (M > 64 && M <= 256 && (size_t)a.ntiles * 32 * a.KT * 32 * (e.w16 ? 2 : 1) <= (16u << 20)) MT = 1;
+  if (M > 64 && M <= 256 && (size_t)a.ntiles * 32 * a.KT * 32 * (e.w16 ? 2 : 1) <= (16u << 20)) {
+    MT = 1;
+    // The norm of fp32 rows (the prefix's first layer) is most of what such a block does, once a generation of blocks: 32-row
+    // blocks where a unit then has fewer rows in all.  Cold weights, us, 64 and 32 rows: 960 -> 1600 at 113 / 241 rows 13.8 and 8.5,
+    // 14.1 and 9.2; 720 -> 8192 at 160 rows (two generations, three) 23.0 and 19.3.  As many rows: 960 -> 4096 at 160 rows (one, two)
+    // 14.3 and 15.4, 512 -> 8192 at 200 rows (two, four) 17.9 and 19.6, from 30 k tiles on there 960 -> 8192 32.9 and 30.8.  Below 512
+    // columns a block is mostly its start and end, and a second generation never pays: 256 -> 16384 at 200 rows 26.3 and 29.7.
+    // From 41 k tiles on a grid of less than a generation is split in K, and every part normalises again: with 64 rows 1344 ->
+    // 2560 at 200 rows 29.1 and 17.9, 1536 -> 3072 at 241 rows 37.7 and 19.4; and from 48 on they lose without a split, too (1536 ->
+    // 4096 at 256 rows 22.5 and 20.2, 2048 -> 4096 33.1 and 25.2).
+    if (e.x_f32 && a.KT < 48) {
+      const int strips2 = (a.ntiles + 1) / 2, blocks64 = strips2 * ((M + 63) / 64);
+      const int gens32 = (strips2 * ((M + 31) / 32) + cus - 1) / cus, gens64 = (blocks64 + cus - 1) / cus;
+      const bool more = gens32 > 2 * gens64 || (gens32 == 2 * gens64 && (gens64 == 1 || a.KT < 30));
+      if ((split_k > 0 ? split_k : model_splits(2, 2, blocks64)) == 1 && (more || (gens32 > 1 && a.KT < 16))) MT = 2;
+    }
+  }
   int NT = 2;
   // 33..64 rows over a large fp8 matrix with the plain epilogue: the weight-streaming schedule (two-tile strips,
   // every block 16 or 8 rounds of four k tiles) when a K split of that size about fills the device
@@ -370,7 +409,6 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
   const int mblocks = (M + 32 * MT - 1) / (32 * MT);
   const int strips = (a.ntiles + NT - 1) / NT;
   const int blocks0 = strips * mblocks;
-  const int NW = 4;
   int ks = stream_ks ? stream_ks : split_k;
   // Plain fp8 linears of 65 .. 96 k tiles on 32-row blocks: one block walks them all with eight waves in a straight line of 9 .. 12
   // rounds (fp8w_gemm.hip) instead of handing split sums over.  Against it stands a split by three (the model's below), where
@@ -391,31 +429,7 @@ int gemm_common(const void* x, int ldx, const void* w_packed, const float* s0, c
     const bool straight = a.KT % 3 == 0 && (third == 6 || third == 8), few = blocks0 * 4 <= cus;
     if (blocks0 * 3 > cus || (rounds8 < 12 && !(few && (straight || (rounds8 == 11 && !a.vec))))) ks = 1;
   }
-  if (ks <= 0) {
-    // Launch-cost model (microseconds, fitted to graph-replayed launches on MI355X): the k loop costs
-    // 0.35 per block round (NW k tiles) for 64-row blocks, 0.20 for 32-row blocks (0.27 with two bf16
-    // weight tiles per wave and round), with a floor of one memory round trip; splitting K adds a partial write, an arrival
-    // count and a read-back that grows with the number of splits and steps up with every batch of four
-    // the finishing block has in flight (1.1 + 0.4 c + 1.0 per further batch), and only pays while the
-    // grid still fits the device twice over.
-    ks = 1;
-    if (blocks0 < cus) {
-      const float per_round = MT == 1 ? (e.w16 && NT == 2 ? 0.27f : 0.20f) : 0.35f;
-      float best = 1e30f;
-      // (an automatic choice never asks for more partial space than the workspace holds)
-      const size_t cap = !ws || ws_bytes <= kPartialOff ? 0 : (ws_bytes - kPartialOff < kPartialBytes ? ws_bytes - kPartialOff : kPartialBytes);
-      for (int c = 1; c <= 64 && c * NW <= a.KT && (c == 1 || (blocks0 * c <= 2 * cus && (size_t)blocks0 * c * MT * NT * 4096 <= cap && blocks0 * 4 <= kMaxCounters)); ++c) {
-        const int rounds = (a.KT + c * NW - 1) / (c * NW);
-        float t = rounds * per_round;
-        if (t < 1.0f) t = 1.0f;
-        if (c > 1) t += 1.1f + 0.4f * (float)c + 1.0f * (float)((c + 3) / 4 - 1);
-        if (t < best - 1e-3f) {
-          best = t;
-          ks = c;
-        }
-      }
-    }
-  }
+  if (ks <= 0) ks = model_splits(MT, NT, blocks0);
   if (ks > a.KT) ks = a.KT;
   if (ks > 64) ks = 64;
   a.ksplit = ks;
