@@ -24,8 +24,9 @@
 // weight, beside the row's partial sums of squares; 1 / rms is a factor of the whole row and multiplies the accumulator.
 // The residual stream never leaves its owner's registers and stays fp32 there.
 //
-// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 1.98 ms, against 4.7 ms of the launches per layer.
-// A self layer takes 13.5 us (stamps of every block, mean), a cross layer 12.4: five or four hand-offs of 0.6 - 1 us from a
+// Measured (50 action tokens, 241 prefix tokens, 16 layers, 10 steps): 1.98 ms, against 4.7 ms of the launches per layer: 12.3 us
+// a layer and step, a step's ends included.  With stamps in every block, which the kernel pays for, a self layer takes 13.5 us
+// (mean) and a cross layer 12.4: five or four hand-offs of 0.6 - 1 us from a
 // phase's result to the next one's first input, 0.3 - 0.7 us until all of a block's input is there (64 bytes a cycle), and
 // from there to the result 0.6 us in P3 and P5, 1.0 in P1 and P4, 1.7 in the attention, 3.6 us in a cross layer's.
 // Where loads are asked for (the loop, us; first figure: as below):
@@ -767,7 +768,7 @@ __global__ __launch_bounds__(kThreads) void sv_denoise_kernel(SvDenoiseArgs a) {
         }
         if (c < NE) {
           poison_hidden(ow, obase + OFF_X1);
-          // (the closing layer's hidden rows of the idle set are read by this step's E0: they have been by now)
+          // (the closing layer's hidden rows of that set are read by this step's E0: they have been by now)
           poison_hidden(ow, obase + OFF_X2);
           if (l == 0) poison_hidden(ow, oth + OFF_HID);
         }

@@ -812,7 +812,8 @@ __global__ void decode_fp8_kernel(float* out) {
 // order of all sums as there: the same bits.
 // Whole blocks of 960 -> 2560 -> 960 with cold weights (48 layers in a graph), us: 113 / 177 / 241 rows 18.8 -> 17.5,
 // 19.5 -> 18.1, 23.0 -> 20.1; 720 -> 2048 -> 720 at 177 / 241 rows 14.4 -> 13.5, 15.2 -> 14.1; 784 -> 4096 -> 784 at 70 / 241
-// rows 18.5 -> 17.0, 28.2 -> 24.1.  Bound now: the rows' way to the operand registers (about half of the launch), then a
+// rows 18.5 -> 17.0, 28.2 -> 24.1; up to the most strips that come here 960 -> 12288 -> 960 at 65 / 255 rows 33.7 -> 25.7, 64.8 -> 46.5,
+// 960 -> 16384 -> 960 at 65 / 128 rows 41.9 -> 34.5, 50.9 -> 38.6.  Bound now: the rows' way to the operand registers (about half of the launch), then a
 // strip's 16 KiB exchange between the waves.
 // Up to 64 rows every pair has a compute unit of its own, or the matrix is large and its stream wants more blocks on a unit.
 // The blocks that share strips are on one XCD (the weights reach its L2 once): a group's index modulo 8 is the block's.
@@ -827,8 +828,7 @@ __global__ __launch_bounds__(512) void norm_gate_up_kernel(GemmArgs a, int group
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int gx = groups >> 3, slot = blockIdx.x >> 3, mblock = slot / gx;
   const int group = (slot - mblock * gx) * 8 + (blockIdx.x & 7);
-  const int strips = a.ntiles >> 1, s_lo = strips * group / groups, s_hi = strips * (group + 1) / groups;
-  if (s_lo == s_hi) return;  // (block-uniform)
+  const int strips = a.ntiles >> 1, s_lo = strips * group / groups, s_hi = strips * (group + 1) / groups;  // (more strips than groups)
 
   i32x4 xv[XPT][NR], nw[NR];
   int xrow[XPT];
@@ -986,7 +986,7 @@ int launch(const GemmArgs& a, dim3 grid, int nw, hipStream_t st) {
       if (nr == 3) return launch_nr<MT, NT, EPI, W16, PRO, MT == 1 ? 3 : 0, MT == 1 ? 8 : 4>(a, grid, st);
       if (nr == 4) return launch_nr<MT, NT, EPI, W16, PRO, MT == 1 ? 4 : 0, MT == 1 ? 8 : 4>(a, grid, st);
       if (nr == 8) return launch_nr<MT, NT, EPI, W16, PRO, MT == 1 ? 8 : 0, MT == 1 ? 8 : 4>(a, grid, st);
-      if constexpr (MT == 1 && EPI == 0 && !W16) {  // plain linears over 2064 .. 3072 columns (2560 -> 960 at 241 rows 6.8 -> 5.9 us)
+      if constexpr (MT == 1 && EPI == 0 && !W16) {  // plain linears over 2064 .. 3072 columns (2560 -> 960 at 250 rows: two splits 8.4 us, whole 6.1)
         if (nr == 9) return launch_nr<MT, NT, EPI, W16, PRO, 9, 8>(a, grid, st);
         if (nr == 10) return launch_nr<MT, NT, EPI, W16, PRO, 10, 8>(a, grid, st);
         if (nr == 11) return launch_nr<MT, NT, EPI, W16, PRO, 11, 8>(a, grid, st);

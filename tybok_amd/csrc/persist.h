@@ -19,8 +19,10 @@
 // barrier, and the first look at the data usually succeeds.  The watch goes through the scalar cache, which it empties before
 // each look: vector loads return in order, and behind the 64 - 128 KiB of weights that a block has on the way at any time a
 // look at a word took as long as those.  (SmolVLA's loop 2364 -> 2275 us, pi0.5's 3805 -> 3519; rounds alone with 128 KiB of
-// weights from memory 3.56 -> 3.29 us, without any 1.41 -> 1.52.)  A progress word is a hint: whoever has looked kLooks times
-// goes on and asks for the data.
+// weights from memory 3.56 -> 3.29 us, without any 1.41 -> 1.52.)  A scalar load goes through the XCD's own L2, which the store of a
+// block on another XCD passes by; that looks see its word in time is measured, and what public descriptions of these parts lead to
+// expect (the memory-side cache keeps track of the lines in the XCDs' L2s), but nothing rests on it: a progress word is a hint,
+// and whoever has looked kLooks times goes on and asks for the data, with loads at device scope.
 //
 // EVERY WAIT ENDS: a wave asks at most `spin` times, then marks itself dead, goes on with what it has (ones = NaN)
 // and never waits again, so the grid drains and the result holds NaNs, which the caller can see.  All blocks must be
